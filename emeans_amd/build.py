@@ -21,7 +21,7 @@ SOURCES = ["emh_api.cpp", "emh_host.cpp", "emh_ops.hip", "emh_scatter.hip", "emh
            "emh_screen3.hip", "emh_screen4.hip", "emh_screen_t1_bf3.hip", "emh_screen_t1_f32.hip",
            "emh_screen_kn_bf3_self.hip", "emh_screen_kn_bf3_any.hip",
            "emh_screen_kn_f32_self.hip", "emh_screen_kn_f32_any.hip", "emh_rescore.hip",
-           "emh_verify.hip", "emh_autok.hip", "emh_topk_long.hip", "emh_screen4kn.hip",
+           "emh_verify.hip", "emh_autok.hip", "emh_topk_long.hip", "emh_screen5.hip",
            "emh_update.hip", "emh_perm.cpp"]
 # Plain host C++ (no HIP), built by the system compiler.
 HOST_ONLY = {"emh_perm.cpp"}

@@ -322,8 +322,9 @@ int emh_create(int device, emh_ctx** out) {
     try {
       EMH_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
       for (hipEvent_t& e : c->ev_stage) EMH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-      EMH_HIP(hipMalloc(&c->small, emh::SW_WORDS * 4));
-      EMH_HIP(hipMemsetAsync(c->small, 0, emh::SW_WORDS * 4, c->stream));
+      EMH_HIP(hipMalloc(&c->small, (emh::SW_WORDS + emh::SCALE_WORDS) * 4));
+      EMH_HIP(hipMemsetAsync(c->small, 0, (emh::SW_WORDS + emh::SCALE_WORDS) * 4, c->stream));
+      c->scales = (float*)(c->small + emh::SW_WORDS);
       EMH_HIP(hipStreamSynchronize(c->stream));
     } catch (...) {
       if (c->small) (void)hipFree(c->small);
@@ -353,7 +354,7 @@ int emh_destroy(emh_ctx* c) {
                             &c->xnorm, &c->bigj, &c->chunkcnt, &c->tickets,
                             &c->preview_ticket, &c->xsplit, &c->csplit, &c->csplit_norm, &c->csplit_part,
                             &c->xpre, &c->xpre_norm, &c->tsplit, &c->tsplit_part, &c->tally_cnt,
-                            &c->klong, &c->trun, &c->kpp, &c->iscore, &c->cnorm})
+                            &c->log5, &c->klong, &c->trun, &c->kpp, &c->iscore, &c->cnorm})
       s->release();
     for (emh::Pinned* s : {&c->pin_usage, &c->pin_plan, &c->pin_small, &c->pin_order[0],
                            &c->pin_order[1], &c->pin_lab[0], &c->pin_lab[1], &c->pin_sco[0],

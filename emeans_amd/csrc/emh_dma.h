@@ -41,6 +41,16 @@ __device__ __forceinline__ void dma16o(const void* base, uint32_t off, void* lds
       : "v"(off), "s"(base), "s"(lds_addr(lds))
       : "memory");
 }
+// The same to an LDS address (wave-uniform).
+__device__ __forceinline__ void dma16a(const void* base, uint32_t off, uint32_t lds) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(off), "s"(base), "s"(lds)
+      : "memory");
+}
 __device__ __forceinline__ void dma4(const void* g, void* lds) {
   uint32_t saved;
   asm volatile(

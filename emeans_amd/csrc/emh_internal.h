@@ -151,6 +151,12 @@ enum SmallWord : int {
   SW_BAD_INIT = 8,        // set when a training run's initial centroids are not finite
   SW_WORDS = 16,
 };
+// The matrices whose fp16 lines a context may hold at once (emh_lines.h).
+enum ScaleOf : int {
+  SCALE_ROWS = 0,   // a call's rows
+  SCALE_CENTS = 1,  // a call's centroids (kNN: the data rows)
+  SCALE_WORDS = 8,
+};
 
 }  // namespace emh
 
@@ -186,6 +192,7 @@ struct emh_ctx {
   int screen = emh::SCREEN_BF3;
   size_t exact_below = emh::EXACT_BELOW;  // emh_set_exact_below
   uint32_t* small = nullptr;  // SW_WORDS u32 on the device
+  float* scales = nullptr;    // (s, 1 / s) of each SCALE_* matrix (emh_lines.h), after small
   char* scratch = nullptr;    // the device's fixed scratch block (emh_top1_noalloc)
   uint64_t fallback_total = 0;
   emh::Scratch cand, fblist, order, start, misc, knn_tmp, xnorm, bigj, chunkcnt, tickets;
@@ -202,6 +209,7 @@ struct emh_ctx {
   } xpre_of;
   emh::Scratch tsplit, tsplit_part;          // a training run's centroids, kept split by the EMA
   emh::Scratch tally_cnt;                    // a training run's label tally (chunk histograms)
+  emh::Scratch log5;                         // the one-pass screen's logs
   emh::Scratch klong;                        // top-k beyond 16: a query block's scores
   // Per-call buffers of the entry points that run many times in a row (a
   // training run's, k-means++'s, internal_scores', the assignment's norms):
@@ -481,7 +489,19 @@ inline size_t halves_blocks(size_t n) { return (n + 7) / 8; }
 // bits as u32), for a screen whose blocks would otherwise each read more than
 // PART_MAX_ONCE partials.
 constexpr size_t PART_MAX_ONCE = 1024;
-void launch_part_max(emh_ctx* c, const uint32_t* part, size_t nparts, uint32_t* out);
+// Rows as fp16 lines for the one-pass screen (emh_lines.h, emh_screen5.hip):
+// the scales of one or two matrices (nx d elements each; b may be null),
+// clearing nclear words on the way; rows ids[lo .. lo + n) (or lo ..) of x as
+// lines in out (lines_bytes(n, d)) with (|x|^2, residual) in norm, and with
+// part each of the lines_blocks(n) blocks' maxima in part[4 b ..]; the maxima
+// over those.
+void launch_scales(emh_ctx* c, const float* a, size_t na, float* sa, const float* b, size_t nb,
+                   float* sb, uint32_t* clear, int nclear);
+void launch_lines(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
+                  size_t n, const float* scale, void* out, float2* norm, const float* cnorm,
+                  uint32_t* part);
+inline size_t lines_blocks(size_t n) { return (n + 7) / 8; }
+void launch_part_max4(emh_ctx* c, const uint32_t* part, size_t nparts, uint32_t* out);
 // Bytes of fixed-block scratch launch_top1 takes for a call of n rows (an
 // upper bound: each region rounded up to 256 bytes).
 size_t top1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);

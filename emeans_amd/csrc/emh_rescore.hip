@@ -22,6 +22,15 @@ namespace {
 
 constexpr int PF = 16;  // float4 loads of each operand in flight per chain
 
+// The bound E of one row from the screen's xnorm entry: |x|^2 for the bounds
+// that screen_bound computes, E itself for BOUND_LINES.
+__device__ __forceinline__ float row_bound(float xn, const uint32_t* small, int d, bool l2,
+                                           int bound) {
+  if (bound == BOUND_LINES) return xn;
+  return screen_bound(xn, __uint_as_float(small[SW_CMAX2]), __uint_as_float(small[SW_CNMAX]), d, l2,
+                      bound);
+}
+
 // Exact fma chain of x and c (the cpu-fused dot); acc starts at +0.
 template <bool VEC4>
 __device__ __forceinline__ float chain(const float* __restrict__ xr, const float* __restrict__ cr,
@@ -143,8 +152,7 @@ __global__ __launch_bounds__(256) void k_verify(
     }
   }
   __syncthreads();
-  // One thread per row. kNN: merge (each part's list is ascending, so a part
-  // is done at its first entry not below the current L-th key), bound, decide.
+  // One thread per row. kNN: merge (a part's valid entries come first), bound, decide.
   // Top-1: per part, as k_check1 decides (a part's list holds all of its
   // centroids within thr when not full or when its last key is above thr).
   float key[L];
@@ -161,18 +169,18 @@ __global__ __launch_bounds__(256) void k_verify(
       for (int q = 0; q < parts; q++)
         for (int e = 0; e < L; e++) {
           const Cand v = c[q * L + e];
-          if (v.id == NONE || !(v.key < key[L - 1])) break;
+          if (v.id == NONE) break;
           insert<L>(key, id, v.key, v.id);
         }
     }
     int state = 0, nc = 0;
     if (rowid[tid] != NONE) {
-      const float E = screen_bound(xnorm[r0 + tid], __uint_as_float(small[SW_CMAX2]),
-                                   __uint_as_float(small[SW_CNMAX]), d, l2, bound);
+      const float E = row_bound(xnorm[r0 + tid], small, d, l2, bound);
       bool complete;
       if (KNN) {
         thr = key[kk - 1] + 2.0f * E;
-        complete = id[L - 1] == NONE || key[L - 1] > thr;
+        // (A NaN bound of the one-pass screen listed nothing.)
+        complete = (id[L - 1] == NONE || key[L - 1] > thr) && !(bound == BOUND_LINES && E != E);
         if (complete)
 #pragma unroll
           for (int e = 0; e < L - 1; e++) nc += id[e] != NONE && (key[e] <= thr || thr != thr);
@@ -195,7 +203,7 @@ __global__ __launch_bounds__(256) void k_verify(
             tot += v.id != NONE && (v.key <= thr || thr != thr);
           }
         }
-        complete = anyv && cert && tot <= C1;
+        complete = anyv && cert && tot <= C1 && !(bound == BOUND_LINES && E != E);
         if (complete) nc = tot + (l2 ? 1 : 0);
       }
       if (complete) {
@@ -425,8 +433,7 @@ __global__ __launch_bounds__(256) void k_check1(
     uint32_t inc = 0;
     int cj = 0, cert = 1;
     if (vrow) {
-      const float E = screen_bound(xn, __uint_as_float(small[SW_CMAX2]),
-                                   __uint_as_float(small[SW_CNMAX]), d, l2, bound);
+      const float E = row_bound(xn, small, d, l2, bound);
       const float thr = best + 2.0f * E;
 #pragma unroll
       for (int e = 0; e < L; e++)
@@ -696,8 +703,11 @@ __global__ __launch_bounds__(256) void k_margin(
   for (int t = 0; t < d; t++) acc = fmaf(xr[t], cr[t], acc);
   const float kx = ip ? -acc : cnorm[cd.id] - 2.0f * acc;
   float edot = 0.f;
-  const float E = screen_bound(xnorm[r], __uint_as_float(small[SW_CMAX2]),
-                               __uint_as_float(small[SW_CNMAX]), d, !ip, bound, &edot);
+  const float E = bound == BOUND_LINES
+                      ? xnorm[r]
+                      : screen_bound(xnorm[r], __uint_as_float(small[SW_CMAX2]),
+                                     __uint_as_float(small[SW_CNMAX]), d, !ip, bound, &edot);
+  if (bound == BOUND_LINES) edot = xnorm[nrows + r];
   if (!isfinite(kx) || !isfinite(E) || !(E > 0.f) || !(edot > 0.f)) return;
   const float dk = fabsf(cd.key - kx);
   const float ratio = dk / E;
@@ -705,7 +715,8 @@ __global__ __launch_bounds__(256) void k_margin(
   const float allow = (ip ? 0.f : 1.0000002f * u * (fabsf(cd.key) + fabsf(kx))) +
                       (bound == BOUND_BF16_TAGGED || bound == BOUND_F16_TAGGED
                            ? 7.63e-6f * fabsf(cd.key) + 8.9e-44f
-                           : 0.f);
+                       : bound == BOUND_LINES ? 1.526e-5f * fabsf(cd.key) + 1.8e-43f
+                                              : 0.f);
   const float dot_ratio = fmaxf(dk - allow, 0.f) / ((ip ? 1.0f : 2.0f) * edot);
   atomicAdd(&out[0], 1ull);
   if (ratio > 1.0f) atomicAdd(&out[1], 1ull);
@@ -771,9 +782,8 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
 
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                     size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
-                    float* sims, uint32_t* fb) {
+                    float* sims, uint32_t* fb, int bound) {
   const dim3 g((unsigned)((m + RK - 1) / RK));
-  const int bound = c->screen == SCREEN_F32 ? BOUND_F32 : BOUND_BF16;
   if (d % 4 == 0)
     hipLaunchKernelGGL((k_verify<LK, RK, true, true>), g, dim3(256), 0, c->stream, q, m, (int)d,
                        nullptr, (size_t)0, (int)m, data, nullptr, (int)n, 1, (int)kk, cand, parts,

@@ -77,6 +77,7 @@ enum BoundKind : int {
   BOUND_BF16 = 1,        // bf16 three-pass screen
   BOUND_BF16_TAGGED = 2, // the same with tagged keys (k_screen4, k_screen3 one tile per part)
   BOUND_F16_TAGGED = 3,  // fp16 two-pass screen with tagged keys (k_screen4 on fp16 halves)
+  BOUND_LINES = 4,       // fp16 one-pass screen (k_screen5): E of row r comes in xnorm[r]
 };
 
 // Screen error bound E on |key' - key| for one row (see emh_screen.hip):
@@ -176,15 +177,15 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
                     const Cand* cand, int parts, const float* xnorm, uint32_t* labels,
                     float* scores, uint32_t* fb, int bound, const LabelTally* tally = nullptr,
                     int L = L1);
-// The kNN screen over split operands (emh_screen4kn.hip): whether it takes a
-// call, and the call's screen (candidate lists [m][parts][LK] and the queries'
-// |q|^2, in the context's scratch); returns the parts.
-bool screen4kn_fits(emh_ctx* c, size_t m, size_t n, size_t d);
-int screen4kn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-              size_t kk, bool exclude_self, Cand** cand, float** xnorm);
+// The one-pass kNN screen (emh_screen5.hip): whether it takes a call, and the
+// call's screen (candidate lists [m][parts][LK]; the queries' E at bound[r]
+// and its dot term at bound[m + r]; in the context's scratch); returns the parts.
+bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d);
+int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
+                size_t kk, bool exclude_self, Cand** cand, float** bound);
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                     size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
-                    float* sims, uint32_t* fb);
+                    float* sims, uint32_t* fb, int bound);
 // Re-score every entry of the screen's lists (rows lo..lo+n, parts x L
 // entries each, laid out [row][part][L]) with the check's exact key and fill
 // rep's pair count, pairs beyond the bound and max |screen key - exact key| / E

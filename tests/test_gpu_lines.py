@@ -1,0 +1,92 @@
+"""The one-pass fp16 screen (k_screen5) at the sizes and inputs where its own
+parts can go wrong: tile and slab remainders, parts, the append buffers' and
+logs' overflows, and values around and beyond fp16's range. Results equal the
+oracle's bit for bit: the screen only chooses what the exact chains score."""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    from emeans_amd import HipDevice
+    d = HipDevice()
+    yield d
+    d.close()
+
+
+def _rows(n, d, seed):
+    x = np.random.default_rng(seed).standard_normal((n, d), dtype=np.float32)
+    return (x / np.linalg.norm(x, axis=1, keepdims=True)).astype(np.float32)
+
+
+def _knn(dev, q, x, kk, self_):
+    d = x.shape[1]
+    gi, gs = dev.topk(x if self_ else q, x, d, kk, self_)
+    oi, os_ = O.knn(x if self_ else q, x, d, kk, self_)
+    assert np.array_equal(gi, oi)
+    assert gs.tobytes() == os_.tobytes()
+
+
+@pytest.mark.parametrize("m,n,d,kk,self_", [
+    (256, 512, 32, 1, False),    # the smallest call, one slab
+    (257, 513, 33, 16, False),   # one past a tile of queries and of data
+    (300, 9000, 99, 10, False),  # parts of several tiles, an odd width
+    (700, 2100, 384, 16, False),
+    (767, 767, 64, 10, True),
+    (1025, 1025, 100, 16, True),
+])
+def test_knn_shapes(dev, m, n, d, kk, self_):
+    _knn(dev, _rows(m, d, m + d), _rows(n, d, n + d), kk, self_)
+
+
+def test_knn_bursts_and_crowds(dev):
+    """Runs of 40 consecutive near-duplicates overflow a row's append buffer
+    within a tile; 300 exact duplicates overflow the lists (the exact scan)."""
+    n, d = 2000, 96
+    x = _rows(n, d, 5)
+    noise = np.random.default_rng(6).standard_normal((n, d), dtype=np.float32)
+    for a in range(0, 1200, 40):
+        x[a:a + 40] = x[a] + np.float32(1e-3) * noise[a:a + 40]
+    x[1500:1800] = x[1500]
+    _knn(dev, x, x, 10, True)
+    _knn(dev, x[::5].copy(), x, 16, False)
+
+
+def test_knn_rising_similarity(dev):
+    """Data rows in order of rising similarity to every query: each one enters
+    the lists when it comes, so the logs fill and are swept."""
+    n, d, m = 8000, 64, 260
+    base = _rows(1, d, 1)[0]
+    t = np.linspace(2.0, 0.01, n, dtype=np.float32)[:, None]
+    x = base + t * _rows(n, d, 2)
+    x = (x / np.linalg.norm(x, axis=1, keepdims=True)).astype(np.float32)
+    q = (base + np.float32(0.01) * _rows(m, d, 3)).astype(np.float32)
+    _knn(dev, q, x, 16, False)
+
+
+@pytest.mark.parametrize("case", ["large", "tiny", "mixed", "beyond", "special"])
+def test_knn_ranges(dev, case):
+    """Magnitudes that the scale brings into fp16's range, rows far below the
+    others, elements that overflow fp16 (their residual is infinite: the exact
+    scan), NaN and infinite elements."""
+    m, n, d = 300, 1500, 128
+    q, x = _rows(m, d, 11), _rows(n, d, 12)
+    if case == "large":
+        q, x = q * np.float32(1e9), x * np.float32(3e12)
+    elif case == "tiny":
+        q, x = q * np.float32(1e-15), x * np.float32(1e-12)
+    elif case == "mixed":
+        s = np.array([1.0, 1e-3, 1e-6, 1e-9], np.float32)
+        q, x = q * s[np.arange(m) % 4][:, None], x * s[np.arange(n) % 4][:, None]
+    elif case == "beyond":
+        x[700] *= np.float32(1e7)
+        q[5] *= np.float32(1e8)
+    else:
+        x[100, 3], x[200, 7], x[300] = np.nan, np.inf, 0.0
+        q[7, 0], q[8, 1], q[9] = np.nan, -np.inf, 0.0
+    _knn(dev, np.ascontiguousarray(q), np.ascontiguousarray(x), 10, False)
