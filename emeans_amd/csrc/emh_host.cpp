@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "emh_internal.h"
+#include "emh_lines.h"
 
 namespace emh {
 namespace host {
@@ -629,39 +630,71 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
   next = beside([&] { fill_order(0); });
   if (draw_init)  // into h_order[1], unused until epoch 1
     init_perm = beside([&] { RandomState::permutation_into(cfg.seed, n, h_order[1]); });
-  // When the batches take the split-operand screen, every row's halves once
-  // (slab-major, with |x|^2; fp16 for the two-pass screen of SCREEN_F16,
-  // else bf16): each batch then gathers its rows' halves by id instead of
-  // splitting them again.
+  // When the batches take a split-operand screen, every row split once
+  // (slab-major; lines, or fp16 halves for the two-pass screen of
+  // SCREEN_F16): each batch then gathers its rows by id instead of splitting
+  // them again.
   SplitRows pre_rows{};
   const SplitRows* pre = nullptr;
   c->xpre_of = emh_ctx::SplitOf{};  // xpre is rewritten (or left stale) below
-  bool run_f16 = false;
+  const bool run_f16 = c->screen == SCREEN_F16;
+  float* run_scale = c->scales + 2 * SCALE_RUN;
   if (split_screen(c, bsz, d, k, sph) && n < (1u << 25)) {
-    run_f16 = c->screen == SCREEN_F16;
-    pre_rows = SplitRows{c->xpre.get(halves_bytes(n, d)), (float*)c->xpre_norm.get(n * 4), n,
-                         n * 128, run_f16};
-    launch_halves(c, x, n, d, nullptr, 0, n, (void*)pre_rows.xs, (float*)pre_rows.xn, nullptr,
-                  nullptr, run_f16);
+    pre_rows.nx = n;
+    pre_rows.f16 = run_f16;
+    if (run_f16) {
+      pre_rows.xs = c->xpre.get(halves_bytes(n, d));
+      pre_rows.xn = c->xpre_norm.get(n * 4);
+      pre_rows.slab = n * 128;
+      launch_halves(c, x, n, d, nullptr, 0, n, (void*)pre_rows.xs, (float*)pre_rows.xn, nullptr,
+                    nullptr);
+    } else {
+      pre_rows.xs = c->xpre.get(lines_bytes(n, d));
+      pre_rows.xn = c->xpre_norm.get(n * 8);
+      pre_rows.slab = n * LINE_BYTES;
+      pre_rows.scale = run_scale;
+      launch_scales(c, x, n * d, run_scale, nullptr, 0, nullptr, nullptr, 0);
+      launch_lines(c, x, n, d, nullptr, 0, n, run_scale, (void*)pre_rows.xs,
+                   (float2*)pre_rows.xn, nullptr, nullptr);
+    }
     pre = &pre_rows;
     c->xpre_of.ptr = x;  // which buffer: emh_train_dev names it once the run has ended
     c->xpre_of.n = n;
     c->xpre_of.d = d;
     c->xpre_of.f16 = run_f16;
   }
-  // L2 batches on the split-operand screen keep the centroids split for the
+  // L2 batches on a split-operand screen keep the centroids split for the
   // run: a full split after each row-norms readout (the first batch, and
   // after a revival moved rows), then the EMA rewrites the rows it moves.
+  // Centroids move within the rows' hull (or, given, towards it), so the rows'
+  // scale serves them.
   const bool keep_csplit = pre && !sph;
-  void* tsplit = keep_csplit ? c->tsplit.get(halves_bytes(k, d)) : nullptr;
-  // The bound's centroid maxima: halves_blocks(k) pairs after a full split,
-  // then one pair per EMA block, or per cluster after a small batch's update.
-  // A revival's split appends one pair per split (at most k / 2) to those.
-  const size_t tpart_pairs = halves_blocks(k) + std::max(ema_blocks(k), k) + k;
-  uint32_t* tpart_h = keep_csplit ? (uint32_t*)c->tsplit_part.get(tpart_pairs * 8) : nullptr;
-  const uint32_t* tpart_end = keep_csplit ? tpart_h + 2 * tpart_pairs : nullptr;
-  uint32_t* tpart_e = keep_csplit ? tpart_h + 2 * halves_blocks(k) : nullptr;
-  SplitCents pcents{tsplit, tpart_h, (int)halves_blocks(k), run_f16};
+  CentsOut tco{};
+  // The bound's centroid maxima, in groups of four words: halves_blocks(k)
+  // groups after a full split, then one per EMA block, or per cluster after a
+  // small batch's update. A revival's split appends one per pair (at most k /
+  // 2) to those.
+  static_assert(sizeof(uint4) == 16, "a group of maxima");
+  const size_t full_groups = run_f16 ? halves_blocks(k) : lines_blocks(k);
+  const size_t tpart_groups = full_groups + std::max(ema_blocks(k), k) + k;
+  uint32_t* tpart_h = keep_csplit ? (uint32_t*)c->tsplit_part.get(tpart_groups * 16) : nullptr;
+  const uint32_t* tpart_end = keep_csplit ? tpart_h + 4 * tpart_groups : nullptr;
+  SplitCents pcents{};
+  if (keep_csplit) {
+    tco.cs = (char*)c->tsplit.get(run_f16 ? halves_bytes(k, d) : lines_bytes(k, d));
+    tco.norm2 = (float2*)c->tsplit_norm.get(k * 8);
+    tco.scale = run_f16 ? nullptr : run_scale;
+    tco.part = tpart_h + 4 * full_groups;
+    pcents.cs = tco.cs;
+    pcents.f16 = run_f16;
+    pcents.scale = tco.scale;
+  } else if (pre && !run_f16) {
+    // Spherical: the readout is split batch by batch, at one scale (no element
+    // of a unit row is beyond 1, and the largest of d is at least d^-1/2, so
+    // the scale of the first readout keeps every later one in range).
+    pcents.scale = c->scales + 2 * SCALE_UNIT;
+  }
+  const SplitCents* pcp = pre && (keep_csplit || !run_f16) ? &pcents : nullptr;
   // When the batches' top-1 runs the screen with d % 4 == 0 (the check and
   // the queued-row scan), or the latency-bound exact scan alone (small k),
   // it tallies the labels it writes (counts and the chunk histograms of the
@@ -748,14 +781,21 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
       if (sph) {
         if (!ema_readout || readout_stale) launch_normalize_rows(c, pos.f(), k, d, readout.f());
         readout_stale = false;
+        if (step == 0 && pcents.scale)
+          launch_scales(c, readout.f(), k * d, c->scales + 2 * SCALE_UNIT, nullptr, 0, nullptr,
+                        nullptr, 0);
       } else if (norms_stale) {
         launch_row_norms(c, pos.f(), k, d, readout.f());
         norms_stale = false;
         if (keep_csplit) {
-          launch_halves(c, pos.f(), k, d, nullptr, 0, k, tsplit, (float*)c->csplit_norm.get(k * 4),
-                        readout.f(), tpart_h, run_f16);
+          if (run_f16)
+            launch_halves(c, pos.f(), k, d, nullptr, 0, k, tco.cs, (float*)tco.norm2, readout.f(),
+                          tpart_h);
+          else
+            launch_lines(c, pos.f(), k, d, nullptr, 0, k, run_scale, tco.cs, tco.norm2,
+                         readout.f(), tpart_h);
           pcents.part = tpart_h;
-          pcents.nparts = (int)halves_blocks(k);
+          pcents.nparts = (int)full_groups;
         }
       }
       const float* cents = sph ? readout.f() : pos.f();
@@ -765,7 +805,7 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
         const size_t c1 = std::min(c0 + chunk, e);
         // After the first step the previous EMA cleared the screen's words.
         launch_top1(c, x, n, d, order, c0, c1, cents, cn, k, sph, lab, sco,
-                    step > 0 && c0 == b, nullptr, pre, keep_csplit ? &pcents : nullptr,
+                    step > 0 && c0 == b, nullptr, pre, pcp,
                     tally ? &tl : nullptr);
       }
       if (!init_checked) {
@@ -798,10 +838,10 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
                     scatter_bytes(e - b, k, d, true, last) + ema_bytes(k, d), tsc);
         launch_update_small(c, x, n, d, order, b, e, lab, k, counts.u(), tcnt, tstride * k,
                             last ? pass.f() : nullptr, pos.f(), mass.f(), af, df, replace,
-                            sph ? nullptr : readout.f(), tsplit, tpart_e,
-                            sph ? readout.f() : nullptr, d_tally[buf], run_f16);
+                            sph ? nullptr : readout.f(), tco, sph ? readout.f() : nullptr,
+                            d_tally[buf]);
         if (keep_csplit) {
-          pcents.part = tpart_e;
+          pcents.part = tco.part;
           pcents.nparts = (int)k;
         }
       } else {
@@ -813,10 +853,10 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
         }
         ProfScope p(c, EMH_PROF_EMA, ema_bytes(k, d), prof_take(c, EMH_PROF_EMA));
         launch_ema(c, pos.f(), mass.f(), sums.f(), counts.u(), k, d, af, df, replace,
-                   sph ? nullptr : readout.f(), true, d_tally[buf], true, tsplit, tpart_e, tcnt,
-                   tally ? tstride * k : 0, ema_readout ? readout.f() : nullptr, run_f16);
+                   sph ? nullptr : readout.f(), true, d_tally[buf], true, tco, tcnt,
+                   tally ? tstride * k : 0, ema_readout ? readout.f() : nullptr);
         if (keep_csplit) {
-          pcents.part = tpart_e;
+          pcents.part = tco.part;
           pcents.nparts = (int)ema_blocks(k);
         }
       }
@@ -832,12 +872,11 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
             // Donors and dead are disjoint. The split also leaves the moved
             // rows' norms and (split screen) halves, and appends a bound
             // partial per pair: no full row_norms and halves pass follows.
-            uint32_t* app = keep_csplit ? const_cast<uint32_t*>(pcents.part) +  // tpart_h's
-                                              2 * (size_t)pcents.nparts
-                                        : nullptr;
-            EMH_ENSURE(!keep_csplit || app + 2 * np <= tpart_end, "bound partials overflow");
-            launch_split_fused(c, pos.f(), mass.f(), d_plan, np, d, k, readout.f(),
-                               keep_csplit ? tsplit : nullptr, app, run_f16);
+            CentsOut app = tco;
+            if (keep_csplit)
+              app.part = const_cast<uint32_t*>(pcents.part) + 4 * (size_t)pcents.nparts;  // tpart_h's
+            EMH_ENSURE(!keep_csplit || app.part + 4 * np <= tpart_end, "bound partials overflow");
+            launch_split_fused(c, pos.f(), mass.f(), d_plan, np, d, k, readout.f(), app);
             if (keep_csplit) pcents.nparts += (int)np;
           } else {
             launch_split(c, pos.f(), mass.f(), d_plan, np, d, true);
@@ -1516,17 +1555,38 @@ int emh_assign_dev(emh_ctx* c, const emh_buf* x, size_t n, size_t d, const emh_b
     // rows, in the format the screen mode takes, and nothing has written them
     // since.
     const emh_ctx::SplitOf& so = c->xpre_of;
+    const bool f16 = c->screen == emh::SCREEN_F16;
     const bool reuse = so.valid && so.ptr == x->ptr && so.serial == x->serial &&
-                       so.gen == x->gen && !x->exposed && so.d == d && n <= so.n &&
-                       so.f16 == (c->screen == emh::SCREEN_F16);
-    const emh::SplitRows pre{c->xpre.ptr, (const float*)c->xpre_norm.ptr, so.n, so.n * 128,
-                             so.f16};
+                       so.gen == x->gen && !x->exposed && so.d == d && n <= so.n && so.f16 == f16;
+    emh::SplitRows pre;
+    pre.f16 = f16;
+    if (reuse) {
+      pre.xs = c->xpre.ptr;
+      pre.xn = c->xpre_norm.ptr;
+      pre.nx = so.n;
+      pre.slab = so.n * (f16 ? 128 : emh::LINE_BYTES);
+      pre.scale = f16 ? nullptr : c->scales + 2 * emh::SCALE_RUN;
+    }
+    // Calls of several chunks on the one-pass screen: the scales and the
+    // centroids' lines once for all of them.
+    const float* cp = (const float*)cents->ptr;
+    emh::SplitCents pc;
+    bool once = false;
+    if (!f16 && n > chunk && emh::split_screen(c, chunk, d, k, metric == EMH_IP)) {
+      float* sc = c->scales + 2 * emh::SCALE_CENTS;
+      float* sx = c->scales + 2 * emh::SCALE_ROWS;
+      emh::launch_scales(c, cp, k * d, sc, reuse ? nullptr : (const float*)x->ptr, n * d, sx,
+                         nullptr, 0);
+      if (!reuse) pre.scale = sx;
+      pc = emh::split_cents(c, cp, d, k, metric == EMH_L2 ? cn.f() : nullptr, sc);
+      once = true;
+    }
     for (size_t b = 0; b < n; b += chunk) {
       const size_t e = std::min(b + chunk, n);
-      emh::launch_top1(c, (const float*)x->ptr, n, d, nullptr, b, e, (const float*)cents->ptr,
+      emh::launch_top1(c, (const float*)x->ptr, n, d, nullptr, b, e, cp,
                        metric == EMH_L2 ? cn.f() : nullptr, k, metric == EMH_IP,
                        (uint32_t*)labels->ptr, (float*)scores->ptr, false, nullptr,
-                       reuse ? &pre : nullptr);
+                       reuse || once ? &pre : nullptr, once ? &pc : nullptr);
     }
     EMH_HIP(hipStreamSynchronize(c->stream));  // cn's block is reused by the next call
   });

@@ -155,6 +155,8 @@ enum SmallWord : int {
 enum ScaleOf : int {
   SCALE_ROWS = 0,   // a call's rows
   SCALE_CENTS = 1,  // a call's centroids (kNN: the data rows)
+  SCALE_RUN = 2,    // a training run's rows (xpre), and its centroids when they lie among them
+  SCALE_UNIT = 3,   // a spherical run's readout
   SCALE_WORDS = 8,
 };
 
@@ -196,7 +198,7 @@ struct emh_ctx {
   char* scratch = nullptr;    // the device's fixed scratch block (emh_top1_noalloc)
   uint64_t fallback_total = 0;
   emh::Scratch cand, fblist, order, start, misc, knn_tmp, xnorm, bigj, chunkcnt, tickets;
-  emh::Scratch xsplit, csplit, csplit_norm, csplit_part;  // split-operand screen: a call's rows, centroids
+  emh::Scratch xsplit, xsplit_norm, csplit, csplit_norm, csplit_part;  // split-operand screens: a call's rows, centroids
   emh::Scratch xpre, xpre_norm;              // a training run's rows, split once
   // What xpre holds: the rows [0, n) of buffer `serial` at generation `gen`
   // (d dimensions, at address ptr); valid only for a buffer the library owns.
@@ -205,9 +207,9 @@ struct emh_ctx {
     const void* ptr = nullptr;
     uint64_t serial = 0, gen = 0;
     size_t n = 0, d = 0;
-    bool f16 = false;  // the halves' format (emh_halves.h)
+    bool f16 = false;  // fp16 halves (else lines)
   } xpre_of;
-  emh::Scratch tsplit, tsplit_part;          // a training run's centroids, kept split by the EMA
+  emh::Scratch tsplit, tsplit_norm, tsplit_part;  // a training run's centroids, kept split by the EMA
   emh::Scratch tally_cnt;                    // a training run's label tally (chunk histograms)
   emh::Scratch log5;                         // the one-pass screen's logs
   emh::Scratch klong;                        // top-k beyond 16: a query block's scores
@@ -306,21 +308,28 @@ void launch_normalize_rows(emh_ctx* c, const float* src, size_t rows, size_t d, 
 // clears before its screen (the fallback count and the bound maxima), so the
 // next top-1 may skip that fill. With tally, also adds counts into it. With
 // zero_counts, leaves counts at zero once read (the next batch's
-// launch_scatter_count adds into them). With csplit (norms needed), also
-// rewrites the halves (launch_halves' layout, k rows; fp16 with f16, else
-// bf16) of the rows it
-// moves and leaves the bound's centroid maxima of its ema_blocks(k) blocks in
-// cpart, as launch_halves' part does. With zero_words, also clears
+// launch_scatter_count adds into them). With co.cs (norms needed), also
+// rewrites the split rows of the centroids it moves and leaves the maxima of
+// its ema_blocks(k) blocks in co.part. With zero_words, also clears
 // zero_words[0..nzero) (a tally's chunk histograms). With readout (spherical
 // runs, no norms, d <= EMA_READOUT_MAX_D), each moved row's normalize_rows
 // readout is written there too (rows that did not move keep theirs).
+// The split centroids that the kernels which move centroids keep up to date:
+// k rows in lines (scale set: emh_lines.h; norm2[j].y is row j's residual) or,
+// without a scale, in fp16 halves. part: where the kernel leaves the bound's
+// maxima, four words a group of rows (|c|^2, cnorm, residual).
+struct CentsOut {
+  char* cs = nullptr;
+  const float* scale = nullptr;
+  float2* norm2 = nullptr;
+  uint32_t* part = nullptr;
+};
 constexpr size_t EMA_READOUT_MAX_D = 1024;
 void launch_ema(emh_ctx* c, float* pos, float* usage, const float* sums, const uint32_t* counts,
                 size_t k, size_t d, float alpha, float decay, int replace, float* norms = nullptr,
                 bool clear_screen_words = false, uint32_t* tally = nullptr,
-                bool zero_counts = false, void* csplit = nullptr, uint32_t* cpart = nullptr,
-                uint32_t* zero_words = nullptr, size_t nzero = 0, float* readout = nullptr,
-                bool f16 = false);
+                bool zero_counts = false, const CentsOut& co = CentsOut{},
+                uint32_t* zero_words = nullptr, size_t nzero = 0, float* readout = nullptr);
 size_t ema_blocks(size_t k);
 // The masses launch_ema will leave, into out (usage untouched); with
 // small_out, also a copy of the small block's words; with seq_out, then seq
@@ -343,14 +352,11 @@ void launch_check_finite(emh_ctx* c, const float* v, size_t n, uint32_t* flag);
 void launch_split(emh_ctx* c, float* pos, float* usage, const uint32_t* pairs_dev, size_t npairs,
                   size_t d, bool independent);
 // launch_split of independent pairs that also writes the two moved rows'
-// norms (L2 readout) and, when given, their halves (csplit, k rows; fp16 with
-// f16, else bf16) and
-// one bound partial pair per pair (cpart[2 q], cpart[2 q + 1]); d at most
-// SPLIT_FUSED_MAX_D.
+// norms (L2 readout) and, with co.cs, their split rows and one group of bound
+// maxima per pair (co.part[4 q ..]); d at most SPLIT_FUSED_MAX_D.
 constexpr size_t SPLIT_FUSED_MAX_D = 1024;
 void launch_split_fused(emh_ctx* c, float* pos, float* usage, const uint32_t* pairs_dev,
-                        size_t npairs, size_t d, size_t k, float* norms, void* csplit,
-                        uint32_t* cpart, bool f16);
+                        size_t npairs, size_t d, size_t k, float* norms, const CentsOut& co);
 void launch_gather_rows(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                         size_t m, float* out);
 
@@ -387,16 +393,15 @@ bool update_small(size_t n, size_t d, bool spherical);
 // Labels lo .. hi tallied into counts (and tcnt, ntcnt words) by the batch's
 // top-1 call. As launch_scatter_sums (tallied) then launch_ema with
 // clear_screen_words and zero_counts: moves the centroids that got rows
-// (pos, usage; norms and, with csplit, the halves for L2 runs, fp16 with f16;
-// readout
+// (pos, usage; norms and, with co.cs, the split rows for L2 runs; readout
 // for spherical ones), adds the sums into acc (when given) and counts into
-// tally, and leaves counts and tcnt at zero. With csplit, cpart[2 j] =
-// cpart[2 j + 1] = norms[j] bits for every cluster j (k pairs).
+// tally, and leaves counts and tcnt at zero. With co.cs, every cluster j's
+// own maxima go to co.part[4 j ..].
 void launch_update_small(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                          size_t lo, size_t hi, const uint32_t* labels, size_t k, uint32_t* counts,
                          uint32_t* tcnt, size_t ntcnt, float* acc, float* pos, float* usage,
-                         float alpha, float decay, int replace, float* norms, void* csplit,
-                         uint32_t* cpart, float* readout, uint32_t* tally, bool f16);
+                         float alpha, float decay, int replace, float* norms, const CentsOut& co,
+                         float* readout, uint32_t* tally);
 
 // ---- emh_autok.hip (kmeans_pp and internal_scores of the automatic-k callers)
 // best[i] = max(best[i], dot(x[i], x[last])), the dot in sequence without fma.
@@ -417,14 +422,19 @@ void launch_iscore_terms(emh_ctx* c, size_t n, size_t ke, const float* g, const 
 // last top-1 (launch_ema with clear_screen_words), so the fill is skipped.
 // ar: take the per-call scratch from this fixed block instead of the
 // context's buffers (no allocation; the call is not profiled).
-// Rows split into bf16 halves ahead of the calls (launch_halves over all nx
-// rows of x, slab-major with slab stride `slab` bytes), with their |x|^2:
-// the screen gathers them by id instead of splitting each call's selection.
+// The split operands' formats: fp16 lines for the one-pass screen (k_screen5;
+// every mode but SCREEN_F16), fp16 halves for the two-pass one (k_screen4).
+// Rows split ahead of the calls (launch_lines or launch_halves over all nx
+// rows of x, slab-major with slab stride `slab` bytes), with (|x|^2, residual)
+// or |x|^2 of each: the screen gathers them by id instead of splitting each
+// call's selection. Lines: with their scale (emh_lines.h); without xs, the
+// scale alone, for the call's own split.
 struct SplitRows {
-  const void* xs;
-  const float* xn;
-  size_t nx, slab;
-  bool f16 = false;  // fp16 halves (else bf16; emh_halves.h)
+  const void* xs = nullptr;
+  const void* xn = nullptr;  // float2 (lines) or float (halves) per row
+  size_t nx = 0, slab = 0;
+  bool f16 = false;          // fp16 halves (else lines)
+  const float* scale = nullptr;
 };
 // Positions per chunk of scatter_add's chunked counting sort.
 constexpr int TALLY_CP = 256;
@@ -445,14 +455,16 @@ struct LabelTally {
 bool scatter_tallied(size_t n, size_t k);
 inline size_t scatter_chunks(size_t n) { return (n + TALLY_CP - 1) / TALLY_CP; }
 inline size_t tally_stride(size_t n) { return (scatter_chunks(n) + 3) & ~(size_t)3; }
-// Centroids split ahead of the call (launch_halves over the k centroids, or
-// launch_ema's csplit for the rows it moved), with the bound's centroid
-// maxima in nparts (max |c|^2, max cnorm) pairs.
+// Centroids split ahead of the call (launch_lines or launch_halves over the k
+// centroids, or kept up to date through CentsOut), with the bound's centroid
+// maxima in nparts groups of four words (|c|^2, cnorm, residual; halves: the
+// first two of every four, too).
 struct SplitCents {
-  const void* cs;
-  const uint32_t* part;
-  int nparts;
-  bool f16 = false;  // fp16 halves (else bf16)
+  const void* cs = nullptr;
+  const uint32_t* part = nullptr;
+  int nparts = 0;
+  bool f16 = false;  // fp16 halves (else lines)
+  const float* scale = nullptr;
 };
 // pre: x's rows already split, pc: the centroids (used when the call takes
 // the split-operand screen; see split_screen).
@@ -464,9 +476,12 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
                  float* scores, bool words_clear = false, Arena* ar = nullptr,
                  const SplitRows* pre = nullptr, const SplitCents* pc = nullptr,
                  const LabelTally* tally = nullptr);
-// Whether top-1 calls of n rows with d dimensions and k centroids take the
-// split-operand screen (k_screen4), whose rows a caller may split ahead.
+// Whether top-1 calls of n rows with d dimensions and k centroids take a
+// split-operand screen, whose rows a caller may split ahead.
 bool split_screen(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);
+// The centroids as lines in the context's scratch (one call's), scale given.
+SplitCents split_cents(emh_ctx* c, const float* cents, size_t d, size_t k, const float* cnorm,
+                       const float* scale);
 // Whether top-1 calls of n rows with d dimensions and k centroids run a
 // screen (and so the check and the queued-row scan). A tallied call always
 // does, whatever its rows.
@@ -474,20 +489,17 @@ bool top1_screens(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);
 // Whether a top-1 call of n rows (and of any fewer) can tally the labels it
 // writes: the screen with d % 4 == 0, or the latency-bound exact scan.
 bool top1_tallies(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);
-// Split rows of x (n rows, or ids[lo..lo+n)) into halves in out (fp16 with
-// f16, else bf16; emh_halves.h), slab-major, with their |x|^2 in norm; with
-// part, each of the
+// Split rows of x (n rows, or ids[lo..lo+n)) into fp16 halves in out
+// (emh_halves.h), slab-major, with their |x|^2 in norm; with part, each of the
 // halves_blocks(n) blocks leaves the largest |x|^2 of its rows and the
-// largest cnorm in part[2 b], part[2 b + 1] (emh_screen4.hip). Bytes of out:
+// largest cnorm in part[4 b], part[4 b + 1] (emh_screen4.hip). Bytes of out:
 // halves_bytes(n, d).
 void launch_halves(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
-                   size_t n, void* out, float* norm, const float* cnorm, uint32_t* part,
-                   bool f16 = false);
+                   size_t n, void* out, float* norm, const float* cnorm, uint32_t* part);
 inline size_t halves_bytes(size_t n, size_t d) { return n * ((d + 31) / 32) * 128; }
 inline size_t halves_blocks(size_t n) { return (n + 7) / 8; }
-// out[0], out[1] = the largest part[2 i], part[2 i + 1] over i < nparts (f32
-// bits as u32), for a screen whose blocks would otherwise each read more than
-// PART_MAX_ONCE partials.
+// A screen whose blocks would each read more partials than this takes them
+// reduced by one workgroup ahead (launch_part_max4).
 constexpr size_t PART_MAX_ONCE = 1024;
 // Rows as fp16 lines for the one-pass screen (emh_lines.h, emh_screen5.hip):
 // the scales of one or two matrices (nx d elements each; b may be null),

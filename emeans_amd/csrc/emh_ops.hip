@@ -242,11 +242,11 @@ __device__ __forceinline__ float ema_mass(float u, uint32_t cnt, float alpha, fl
 
 // With norms != nullptr, also the squared norm of every updated row (the next
 // batch's L2 readout, assign.rs:150-155); rows without members keep theirs.
-// With csplit (norms too), also the bf16 halves of every updated row in the
-// split-operand layout of k rows (emh_halves.h), so the next batch's screen
-// need not split the centroids again (rows without members keep theirs), and
-// cpart[2 b] = cpart[2 b + 1] = the largest norms[] of block b's rows (f32
-// bits; a NaN wins): the bound's centroid maxima, as k_halves leaves them.
+// With co.cs (norms too), also the lines or halves of every updated row
+// (CentsOut, emh_halves.h), so the next batch's screen need not split the
+// centroids again (rows without members keep theirs), and the maxima of block
+// b's rows (f32 bits; a NaN wins) in co.part[4 b ..]: norms[] twice, and the
+// residuals.
 // Workgroup = EC clusters: the 256 threads update the clusters' positions
 // element by element, then lane c of the first wave adds cluster c's rounded
 // squares in order from LDS (rows padded by four floats so the EC lanes read
@@ -268,14 +268,13 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
                                              uint32_t* __restrict__ clear3,
                                              uint32_t* __restrict__ tally,
                                              uint32_t* zero_counts,  // counts itself, or null
-                                             char* __restrict__ csplit,
-                                             uint32_t* __restrict__ cpart,
+                                             const CentsOut co,
                                              uint32_t* __restrict__ zero_words, size_t nzero,
-                                             float* __restrict__ readout, int f16) {
+                                             float* __restrict__ readout) {
   // EC rows of min(d, ECH) + 4 floats (norms, or readout): the rounded
-  // squares; with csplit or readout, then as many for the values.
+  // squares; with co.cs or readout, then as many for the values.
   extern __shared__ __attribute__((aligned(16))) float sq[];
-  __shared__ float wgt[EC], cntf[EC];
+  __shared__ float wgt[EC], cntf[EC], res[EC];
   const int tid = threadIdx.x;
   const size_t j0 = (size_t)blockIdx.x * EC;
   const int nc = (int)min((size_t)EC, k - j0);
@@ -290,6 +289,7 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
     usage[j0 + tid] = ema_mass(usage[j0 + tid], cnt, alpha, decay, replace, &weight);
     wgt[tid] = cnt > 0 ? weight : -1.0f;  // -1: no rows, position unchanged
     cntf[tid] = (float)cnt;
+    res[tid] = 0.0f;
   }
   __syncthreads();
   const int seg = (int)min(d, (size_t)ECH), row = ema_row(seg);
@@ -329,17 +329,18 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
           }
           p[t] = v;
           if (norms) sq[c * row + t] = v * v;
-          if (csplit || readout) vs[c * row + t] = v;
+          if (co.cs || readout) vs[c * row + t] = v;
           if (readout) tmx = fmaxf(tmx, fabsf(v));
         }
       }
     }
     if (!norms) continue;
     __syncthreads();
-    if (csplit && tid >= WAVE) {
-      // Waves 1-3 write the halves of the pass's dimensions (c0 is a
+    if (co.cs && tid >= WAVE) {
+      // Waves 1-3 write the split rows of the pass's dimensions (c0 is a
       // multiple of 32; the last slab's dimensions past d are zero) while
-      // lanes of wave 0 run the chains.
+      // lanes of wave 0 run the chains. A row's residual is summed in any
+      // order: the bound allows for it.
       const int nq = (((int)len + 31) & ~31) >> 2;  // quads in the pass
       for (int e = tid - WAVE; e < EC * nq; e += 256 - WAVE) {
         const int cc = e / nq, t = 4 * (e % nq);
@@ -348,12 +349,8 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
         const float4 v4 = make_float4(t < len ? vr[t] : 0.0f, t + 1 < len ? vr[t + 1] : 0.0f,
                                       t + 2 < len ? vr[t + 2] : 0.0f,
                                       t + 3 < len ? vr[t + 3] : 0.0f);
-        uint2 hi, lw;
-        split_quad(v4, hi, lw, f16 != 0);
-        const size_t col = c0 + (size_t)t;
-        char* o = csplit + ((col >> 5) * k + j0 + cc) * SLAB_BYTES + quad_hi_offset((int)(col & 31) >> 2);
-        *reinterpret_cast<uint2*>(o) = hi;
-        *reinterpret_cast<uint2*>(o + 32) = lw;
+        const float r = put_quad(co, k, j0 + cc, c0 + (size_t)t, v4);
+        if (co.scale) atomicAdd(&res[cc], r);
       }
     }
     if (tid < nc && wgt[tid] >= 0.0f) nrm = ordered_sum(sq + tid * row, len, nrm);  // in order
@@ -384,15 +381,23 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
     }
   }
   if (norms && tid < nc && wgt[tid] >= 0.0f) norms[j0 + tid] = nrm;
-  if (cpart && tid < WAVE) {
-    uint32_t m = 0u;
-    if (tid < nc) m = __float_as_uint(wgt[tid] >= 0.0f ? nrm : norms[j0 + tid]);
-#pragma unroll
-    for (int o = 1; o < EC; o <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, WAVE));
-    if (tid == 0) {
-      cpart[2 * blockIdx.x] = m;
-      cpart[2 * blockIdx.x + 1] = m;
+  if (co.part && tid < WAVE) {
+    // (The last pass's barrier: every quad's residual is in.)
+    uint32_t m = 0u, mr = 0u;
+    if (tid < nc) {
+      const bool moved = wgt[tid] >= 0.0f;
+      m = __float_as_uint(moved ? nrm : norms[j0 + tid]);
+      if (co.scale) {
+        if (moved) co.norm2[j0 + tid].y = res[tid];
+        mr = __float_as_uint(moved ? res[tid] : co.norm2[j0 + tid].y);
+      }
     }
+#pragma unroll
+    for (int o = 1; o < EC; o <<= 1) {
+      m = max(m, (uint32_t)__shfl_xor((int)m, o, WAVE));
+      mr = max(mr, (uint32_t)__shfl_xor((int)mr, o, WAVE));
+    }
+    if (tid == 0) reinterpret_cast<uint4*>(co.part)[blockIdx.x] = make_uint4(m, m, mr, 0u);
   }
 }
 
@@ -533,9 +538,9 @@ __global__ __launch_bounds__(256) void k_split(float* __restrict__ pos, float* _
 // cluster), d <= SPLIT_FUSED_MAX_D, leaving also what the next batch reads of
 // the two rows it moves, as a full row_norms and halves pass would: norms[s]
 // and norms[t] (k_row_norms' in-order chain of the rounded squares); with
-// csplit their bf16 halves in the split layout of k rows; with cpart the pair
-// cpart[2 q] = cpart[2 q + 1] = the larger of the two norms (f32 bits), which
-// the caller appends to the bound's centroid partials. The partials of the
+// co.cs their lines or halves (CentsOut) and the larger of the two rows' norms
+// and residuals (f32 bits) in co.part[4 q ..], which the caller appends to the
+// bound's centroid partials. The partials of the
 // blocks the two rows were in stay upper bounds: no other row changed.
 // Workgroup q = pair q. LDS: the two rows' values, then their squares, each
 // row ema_row(d) floats.
@@ -543,16 +548,16 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
                                                      float* __restrict__ usage,
                                                      const uint32_t* __restrict__ pairs, size_t d,
                                                      size_t k, float* __restrict__ norms,
-                                                     char* __restrict__ csplit,
-                                                     uint32_t* __restrict__ cpart, int f16) {
+                                                     const CentsOut co) {
   extern __shared__ __attribute__((aligned(16))) float sl[];
   __shared__ int diff;
-  __shared__ float nv[2];
+  __shared__ float nv[2], rv[2];
   const int tid = threadIdx.x, q = blockIdx.x, len = (int)d, row = ema_row(len);
   float* vs = sl;
   float* sq = sl + 2 * row;
   const uint32_t s = pairs[2 * q], t = pairs[2 * q + 1];
   if (tid == 0) diff = 0;
+  if (tid < 2) rv[tid] = 0.0f;
   __syncthreads();
   float* cs = pos + (size_t)s * d;
   float* ct = pos + (size_t)t * d;
@@ -591,7 +596,7 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
     usage[t] = half;
   }
   __syncthreads();
-  if (csplit) {
+  if (co.cs) {
     // Quads of the two rows (the last slab's dimensions past d are zero),
     // beside the chains of lanes 0 and 1.
     const int nq = ((len + 31) & ~31) >> 2;
@@ -601,12 +606,8 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
       const float4 v4 = make_float4(c4 < len ? vr[c4] : 0.0f, c4 + 1 < len ? vr[c4 + 1] : 0.0f,
                                     c4 + 2 < len ? vr[c4 + 2] : 0.0f,
                                     c4 + 3 < len ? vr[c4 + 3] : 0.0f);
-      uint2 hv, lv;
-      split_quad(v4, hv, lv, f16 != 0);
-      char* o = csplit + ((size_t)(c4 >> 5) * k + (r ? t : s)) * SLAB_BYTES +
-                quad_hi_offset((c4 & 31) >> 2);
-      *reinterpret_cast<uint2*>(o) = hv;
-      *reinterpret_cast<uint2*>(o + 32) = lv;
+      const float res = put_quad(co, k, r ? t : s, (size_t)c4, v4);
+      if (co.scale) atomicAdd(&rv[r], res);
     }
   }
   if (tid < 2) {
@@ -614,12 +615,13 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
     norms[tid ? t : s] = nrm;
     nv[tid] = nrm;
   }
-  if (cpart) {
+  if (co.part) {
     __syncthreads();
+    if (tid < 2 && co.scale) co.norm2[tid ? t : s].y = rv[tid];
     if (tid == 0) {
       const uint32_t m = max(__float_as_uint(nv[0]), __float_as_uint(nv[1]));
-      cpart[2 * q] = m;
-      cpart[2 * q + 1] = m;
+      const uint32_t mr = max(__float_as_uint(rv[0]), __float_as_uint(rv[1]));
+      reinterpret_cast<uint4*>(co.part)[q] = make_uint4(m, m, mr, 0u);
     }
   }
 }
@@ -666,20 +668,19 @@ void launch_normalize_rows(emh_ctx* c, const float* src, size_t rows, size_t d, 
 
 void launch_ema(emh_ctx* c, float* pos, float* usage, const float* sums, const uint32_t* counts,
                 size_t k, size_t d, float alpha, float decay, int replace, float* norms,
-                bool clear_screen_words, uint32_t* tally, bool zero_counts, void* csplit,
-                uint32_t* cpart, uint32_t* zero_words, size_t nzero, float* readout, bool f16) {
+                bool clear_screen_words, uint32_t* tally, bool zero_counts, const CentsOut& co,
+                uint32_t* zero_words, size_t nzero, float* readout) {
   if (k == 0) return;
-  EMH_ENSURE(!csplit || (norms && cpart), "ema: the centroid halves need the norms and maxima");
-  EMH_ENSURE(!readout || (!norms && !csplit && d <= (size_t)ECH),
+  EMH_ENSURE(!co.cs || (norms && co.part), "ema: the split centroids need the norms and maxima");
+  EMH_ENSURE(!readout || (!norms && !co.cs && d <= (size_t)ECH),
              "ema: the fused readout is for spherical runs with d <= %d", ECH);
   const size_t lds = norms || readout ? (size_t)EC * ema_row((int)std::min(d, (size_t)ECH)) *
-                                            sizeof(float) * (csplit || readout ? 2 : 1)
+                                            sizeof(float) * (co.cs || readout ? 2 : 1)
                                       : 0;
   hipLaunchKernelGGL(k_ema, grid1(k, EC), dim3(256), lds, c->stream, pos, usage, sums, counts, k,
                      d, alpha, decay, replace, norms, clear_screen_words ? c->small : nullptr,
                      tally, zero_counts ? const_cast<uint32_t*>(counts) : nullptr,
-                     (char*)csplit, cpart, zero_words, zero_words ? nzero : 0, readout,
-                     f16 ? 1 : 0);
+                     co, zero_words, zero_words ? nzero : 0, readout);
   EMH_HIP(hipGetLastError());
 }
 
@@ -727,13 +728,12 @@ void launch_check_finite(emh_ctx* c, const float* v, size_t n, uint32_t* flag) {
 }
 
 void launch_split_fused(emh_ctx* c, float* pos, float* usage, const uint32_t* pairs_dev,
-                        size_t npairs, size_t d, size_t k, float* norms, void* csplit,
-                        uint32_t* cpart, bool f16) {
+                        size_t npairs, size_t d, size_t k, float* norms, const CentsOut& co) {
   if (npairs == 0) return;
   EMH_ENSURE(d >= 1 && d <= SPLIT_FUSED_MAX_D && norms, "split_fused: shape out of range");
   const size_t lds = 4 * (size_t)ema_row((int)d) * sizeof(float);
   hipLaunchKernelGGL(k_split_fused, dim3((unsigned)npairs), dim3(256), lds, c->stream, pos, usage,
-                     pairs_dev, d, k, norms, (char*)csplit, cpart, f16 ? 1 : 0);
+                     pairs_dev, d, k, norms, co);
   EMH_HIP(hipGetLastError());
 }
 

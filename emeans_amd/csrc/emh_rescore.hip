@@ -764,16 +764,22 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
   static_assert(TALLY_CP % CR == 0, "a check block's rows lie in one tally chunk");
   EMH_ENSURE(!tally || (d % 4 == 0 && lo >= tally->lo && (lo - tally->lo) % TALLY_CP == 0),
              "check: a tally needs d %% 4 == 0 and chunk-aligned positions");
-  EMH_ENSURE(L == L1 || L == L1F || (L == L1S && d % 4 == 0), "check: lists of %d entries", L);
+  EMH_ENSURE(L == L1 || L == L1F || L == L5 || (L == L1S && d % 4 == 0),
+             "check: lists of %d entries", L);
   if (d % 4 == 0)
-    hipLaunchKernelGGL(L == L1S ? k_check1<L1S> : L == L1F ? k_check1<L1F> : k_check1<L1>,
+    hipLaunchKernelGGL(L == L1S   ? k_check1<L1S>
+                       : L == L1F ? k_check1<L1F>
+                       : L == L5  ? k_check1<L5>
+                                  : k_check1<L1>,
                        dim3((unsigned)((n + CR - 1) / CR)), dim3(256), 0, c->stream, x,
                        nx, (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts, xnorm,
                        labels, scores, fb, c->small, bound, tally ? tally->cnt : nullptr,
                        tally ? tally->counts : nullptr, tally ? tally->lo : 0,
                        tally ? tally->stride : 0);
   else
-    hipLaunchKernelGGL((L == L1F ? k_verify<L1F, R1, false, false> : k_verify<L1, R1, false, false>),
+    hipLaunchKernelGGL((L == L1F  ? k_verify<L1F, R1, false, false>
+                        : L == L5 ? k_verify<L5, R1, false, false>
+                                  : k_verify<L1, R1, false, false>),
                        g, dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents, cnorm,
                        (int)k, ip ? 1 : 0, 1, cand, parts, xnorm, labels, scores, fb, c->small,
                        bound);

@@ -34,6 +34,7 @@
 // on both sides (one rounding in the screen's fma, two in the check's). E
 // carries a 12.5% margin for its own rounding.
 
+#include "emh_lines.h"
 #include "emh_screen_kern.h"
 
 namespace emh {
@@ -64,11 +65,13 @@ int choose_parts(int row_tiles, int ntiles, int cus, int per_cu = 2) {
 
 namespace {
 // The screen's launch geometry for n rows against k centroids. split: the
-// call may take the split-operand screen (k_screen4: fp16 or bf16, k >= 64
-// and at most MAX_PARTS tiles of 256 centroids, one tile per part with
-// tagged keys; any d >= 32). Otherwise (and for the no-allocation entry, which
-// has no room to split a selection) the large-tile screen that splits its
-// slabs itself (k_screen3, d % 4 == 0, k >= 64) or the 128 x 128 screens.
+// call may take a split-operand screen (k >= 64, any d >= 32): the one-pass
+// screen over fp16 lines (k_screen5; parts of one tile of 256 centroids while
+// there are at most MAX_PARTS tiles, else of several) or, in SCREEN_F16 with
+// at most MAX_PARTS tiles, the two-pass one (k_screen4). Otherwise (and for
+// the no-allocation entry, which has no room to split a selection) the
+// large-tile screen that splits its slabs itself (k_screen3, d % 4 == 0, k >=
+// 64) or the 128 x 128 screens.
 struct Top1Geom {
   bool screen, big, split;
   int row_tiles, ntiles, parts, tpp;
@@ -87,18 +90,21 @@ Top1Geom top1_geom(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool split
                                queued_direct(c, n, d, k, ip)));
   if (!g.screen) return g;
   const int nt3 = (int)((k + TC3 - 1) / TC3);
-  // (k_screen4 addresses a slab's rows with 32-bit offsets: fewer than 2^25 rows.)
+  // (The split-operand screens address a slab's rows with 32-bit offsets: fewer than 2^25 rows.)
   // A selection that gives the large tiles fewer blocks than half the CUs (an
   // epoch's tail batch: 3,392 rows x 1,024 centroids in 56 blocks took 55 us)
   // takes the 128 x 128 screen, whose 216 blocks there take 45 us.
   const size_t blocks3 = (n + TR3 - 1) / TR3 * (size_t)nt3;
   const bool few = 2 * blocks3 < (size_t)c->cus;
-  if (split && !few && c->screen != SCREEN_F32 && k >= 64 && nt3 <= MAX_PARTS &&
-      n < (1u << 25)) {
+  const bool lines = c->screen != SCREEN_F16;  // the split-operand screen is the one-pass one
+  if (split && !few && c->screen != SCREEN_F32 && k >= 64 && (lines || nt3 <= MAX_PARTS) &&
+      n < (1u << 25) && k < (1u << 25)) {
     g.big = g.split = true;
     g.row_tiles = (int)((n + TR3 - 1) / TR3);
-    g.ntiles = g.parts = nt3;
-    g.tpp = 1;
+    g.ntiles = nt3;
+    g.parts = nt3 <= MAX_PARTS ? nt3 : choose_parts(g.row_tiles, nt3, c->cus, 1);
+    g.tpp = (g.ntiles + g.parts - 1) / g.parts;
+    g.parts = (g.ntiles + g.tpp - 1) / g.tpp;
     return g;
   }
   // The large-tile bf16 screen (one 512-thread block per CU, 256-centroid
@@ -126,6 +132,26 @@ bool top1_tallies(emh_ctx* c, size_t n, size_t d, size_t k, bool ip) {
   return d % 4 == 0 && (top1_screens(c, n, d, k, ip) || queued_direct(c, n, d, k, ip));
 }
 
+SplitCents split_cents(emh_ctx* c, const float* cents, size_t d, size_t k, const float* cnorm,
+                       const float* scale) {
+  void* cw = c->csplit.get(lines_bytes(k, d));
+  const size_t nb = lines_blocks(k);
+  uint32_t* pw = (uint32_t*)c->csplit_part.get((nb + 1) * 16);
+  launch_lines(c, cents, k, d, nullptr, 0, k, scale, cw, (float2*)c->csplit_norm.get(k * 8), cnorm,
+               pw);
+  SplitCents s;
+  s.cs = cw;
+  s.part = pw;
+  s.nparts = (int)nb;
+  s.scale = scale;
+  if (nb > PART_MAX_ONCE) {
+    launch_part_max4(c, pw, nb, pw + 4 * nb);
+    s.part = pw + 4 * nb;
+    s.nparts = 1;
+  }
+  return s;
+}
+
 size_t top1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip) {
   const Top1Geom g = top1_geom(c, n, d, k, ip, false, true);
   if (!g.screen) return exact1_scratch_bytes(c, n, d, k, ip, false);
@@ -135,21 +161,17 @@ size_t top1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip) {
 }
 
 namespace {
-// The screen stage of a top-1 call: its lists, their parts, the rows' |x|^2,
-// the check's queue and the arithmetic the check's bound must follow.
+// The screen stage of a top-1 call: its lists, their parts, the rows' |x|^2
+// (BOUND_LINES: their E), the check's queue and the arithmetic the check's
+// bound must follow.
 struct Top1Screen {
   Top1Geom g;
   Cand* cand = nullptr;
   uint32_t* fb = nullptr;
   float* xnorm = nullptr;
-  bool tagged = false;
-  bool f16 = false;  // the split-operand screen ran in fp16 two-pass arithmetic
-  int L = L1;  // entries per part list: L1S for the sorted insert's, L1F for the fp16 screen's
+  BoundKind bound = BOUND_F32;
+  int L = L1;  // entries per part list
 };
-
-// The split-operand screen's arithmetic: fp16 two-pass in SCREEN_F16, else
-// bf16 three-pass.
-bool split_f16(const emh_ctx* c) { return c->screen == SCREEN_F16; }
 
 Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                        size_t lo, size_t n, const float* cents, const float* cnorm, size_t k,
@@ -159,23 +181,99 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
   s.g = top1_geom(c, n, d, k, ip, !ar, small_exact);
   if (!s.g.screen) return s;
   const Top1Geom& g = s.g;
-  const bool f16 = g.split && split_f16(c);
-  const size_t cbytes = (size_t)g.parts * n * (f16 ? L1F : L1) * sizeof(Cand);
+  const bool f16 = g.split && c->screen == SCREEN_F16;
+  const bool tagged = g.big && g.tpp == 1;
+  s.bound = c->screen == SCREEN_F32 ? BOUND_F32
+            : f16                   ? BOUND_F16_TAGGED
+            : g.split               ? BOUND_LINES
+            : tagged                ? BOUND_BF16_TAGGED
+                                    : BOUND_BF16;
+  s.L = f16 ? L1F : g.split ? L5 : g.big && !tagged ? L1S : L1;
+  const size_t cbytes = (size_t)g.parts * n * s.L * sizeof(Cand);
   s.cand = (Cand*)(ar ? ar->take(cbytes) : c->cand.get(cbytes));
   s.fb = (uint32_t*)(ar ? ar->take(n * 4) : c->fblist.get(n * 4));
-  s.xnorm = (float*)(ar ? ar->take(n * 4) : c->xnorm.get(n * 4));
-  if (!words_clear)  // fallback count, cmax2, cnmax (the screen or the split fills the maxima)
-    launch_fill_u32(c, c->small, 3, 0);
+  const size_t nb = g.split && !f16 ? 2 * n * 4 : n * 4;  // E and its dot term, or |x|^2
+  s.xnorm = (float*)(ar ? ar->take(nb) : c->xnorm.get(nb));
+  // The words a screen starts from: fallback count, cmax2, cnmax (the maxima
+  // filled by the screen or the split).
+  auto clear_words = [&] {
+    if (!words_clear) launch_fill_u32(c, c->small, 3, 0);
+    words_clear = true;
+  };
   const unsigned blocks = (unsigned)(g.row_tiles * g.parts);
-  s.tagged = g.big && g.tpp == 1;
-  s.L = f16 ? L1F : g.big && !s.tagged ? L1S : L1;
   if (g.split) {
-    // The centroids' halves and the bound's centroid maxima (the caller's,
-    // split ahead, or split here), then the rows' halves (the caller's, or
-    // this selection's), all in the call's format.
     EMH_ENSURE(!pre || pre->f16 == f16, "top1: rows split in the other format");
     EMH_ENSURE(!pc || pc->f16 == f16, "top1: centroids split in the other format");
-    s.f16 = f16;
+  }
+  if (g.split && !f16) {
+    // The one-pass screen. Scales and lines that the caller did not bring:
+    // the matrices' scales in one launch (which also clears the words), the
+    // centroids' lines, then the selection's.
+    const float* sx = pre ? pre->scale : nullptr;
+    const float* sc = pc ? pc->scale : nullptr;
+    if (!sx || !sc) {
+      float* wx = c->scales + 2 * SCALE_ROWS;
+      float* wc = c->scales + 2 * SCALE_CENTS;
+      const int nclear = words_clear ? 0 : 3;
+      if (!sx && !sc)
+        launch_scales(c, x, nx * d, wx, cents, k * d, wc, c->small, nclear);
+      else if (!sx)
+        launch_scales(c, x, nx * d, wx, nullptr, 0, nullptr, c->small, nclear);
+      else
+        launch_scales(c, cents, k * d, wc, nullptr, 0, nullptr, c->small, nclear);
+      if (!sx) sx = wx;
+      if (!sc) sc = wc;
+      words_clear = true;
+    }
+    clear_words();
+    Lines5 a{};
+    if (pc && pc->cs) {
+      a.cs = pc->cs;
+      a.part = pc->part;
+      a.nparts = pc->nparts;
+    } else {
+      const SplitCents own = split_cents(c, cents, d, k, ip ? nullptr : cnorm, sc);
+      a.cs = own.cs;
+      a.part = own.part;
+      a.nparts = own.nparts;
+    }
+    if (pre && pre->xs) {
+      a.xs = pre->xs;
+      a.xslab = pre->slab;
+      a.xn = (const float2*)pre->xn;
+      a.nx = pre->nx;
+      a.ids = ids;
+      a.lo = lo;
+    } else {
+      void* xs = c->xsplit.get(lines_bytes(n, d));
+      float2* xn = (float2*)c->xsplit_norm.get(n * 8);
+      launch_lines(c, x, nx, d, ids, lo, n, sx, xs, xn, nullptr, nullptr);
+      a.xs = xs;
+      a.xslab = n * LINE_BYTES;
+      a.xn = xn;
+      a.nx = n;
+    }
+    a.n = n;
+    a.cnorm = cnorm;
+    a.k = k;
+    a.d = d;
+    a.tpp = g.tpp;
+    a.parts = g.parts;
+    a.ntiles = g.ntiles;
+    a.cand = s.cand;
+    a.bound = s.xnorm;
+    a.sx = sx;
+    a.sc = sc;
+    ProfScope prof(c, EMH_PROF_SCREEN, 2.0 * (double)n * (double)k * (double)d,
+                   prof_take(c, EMH_PROF_SCREEN));
+    launch_screen5(c, a, ip);
+    return s;
+  }
+  clear_words();
+  if (g.split) {
+    // The two-pass screen: the centroids' halves and the bound's centroid
+    // maxima (the caller's, split ahead, or split here), then the rows'
+    // halves (the caller's, or this selection's).
     const void* cs;
     const uint32_t* part;
     int nparts;
@@ -185,26 +283,26 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
       nparts = pc->nparts;
     } else {
       void* cw = c->csplit.get(halves_bytes(k, d));
-      uint32_t* pw = (uint32_t*)c->csplit_part.get(halves_blocks(k) * 8);
+      uint32_t* pw = (uint32_t*)c->csplit_part.get(halves_blocks(k) * 16);
       launch_halves(c, cents, k, d, nullptr, 0, k, cw, (float*)c->csplit_norm.get(k * 4),
-                    ip ? nullptr : cnorm, pw, f16);
+                    ip ? nullptr : cnorm, pw);
       cs = cw;
       part = pw;
       nparts = (int)halves_blocks(k);
     }
-    Screen4Args a{blocks,   nullptr,  0,      nullptr, 0,       d,       nullptr,
-                  0,        n,        cs,     k * 128, cnorm,   k,       1,
-                  g.parts,  g.ntiles, s.cand, s.xnorm, part,    nparts,  f16};
+    Screen4Args a{blocks, nullptr, 0,       nullptr, 0,       d,    nullptr, 0,
+                  n,      cs,      k * 128, cnorm,   k,       1,    g.parts, g.ntiles,
+                  s.cand, s.xnorm, part,    nparts};
     if (pre) {
       a.xs = pre->xs;
       a.xslab = pre->slab;
-      a.xn = pre->xn;
+      a.xn = (const float*)pre->xn;
       a.nx = pre->nx;
       a.ids = ids;
       a.lo = lo;
     } else {
       void* xs = c->xsplit.get(halves_bytes(n, d));
-      launch_halves(c, x, nx, d, ids, lo, n, xs, s.xnorm, nullptr, nullptr, f16);
+      launch_halves(c, x, nx, d, ids, lo, n, xs, s.xnorm, nullptr, nullptr);
       a.xs = xs;
       a.xslab = n * 128;
       a.xn = s.xnorm;
@@ -222,18 +320,12 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
   // One tile per part: tagged keys (the cheap fold); more: the sorted
   // insert, which skips most keys once the lists hold good ones.
   if (g.big)
-    launch_screen3(c, a, ip, s.tagged);
+    launch_screen3(c, a, ip, tagged);
   else
     launch_screen_t1(c, a, ip);
   return s;
 }
 
-// The check's bound arithmetic: the screen's (BoundKind).
-int bound_kind(const emh_ctx* c, const Top1Screen& s) {
-  if (c->screen == SCREEN_F32) return BOUND_F32;
-  if (s.f16) return BOUND_F16_TAGGED;
-  return s.tagged ? BOUND_BF16_TAGGED : BOUND_BF16;
-}
 }  // namespace
 
 void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
@@ -257,7 +349,7 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
     return;
   }
   launch_verify1(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, s.cand, s.g.parts, s.xnorm, labels,
-                 scores, s.fb, bound_kind(c, s), tally, s.L);
+                 scores, s.fb, s.bound, tally, s.L);
   launch_exact1(c, x, nx, d, ids, lo, n, s.fb, cents, cnorm, k, ip, labels, scores, ar, tally);
 }
 
@@ -272,13 +364,13 @@ void screen_margin_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const u
       screen_top1(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, false, nullptr, nullptr, nullptr,
                   false);
   if (!s.g.screen) return;  // variant 0: no screen, nothing to measure
-  out->variant = s.f16     ? EMH_SCREEN_BIG_F16
-                 : s.g.big ? (s.tagged ? EMH_SCREEN_BIG_TAGGED : EMH_SCREEN_BIG_SORTED)
+  out->variant = s.bound == BOUND_F16_TAGGED ? EMH_SCREEN_BIG_F16
+                 : s.g.big ? (s.g.tpp == 1 ? EMH_SCREEN_BIG_TAGGED : EMH_SCREEN_BIG_SORTED)
                            : (c->screen == SCREEN_F32 ? EMH_SCREEN_SMALL_F32 : EMH_SCREEN_SMALL_BF16);
   out->parts = s.g.parts;
   out->tiles_per_part = s.g.tpp;
   launch_margin(c, x, nx, d, ids, lo, n, cents, cnorm, ip, s.cand, s.g.parts, s.L, s.xnorm,
-                bound_kind(c, s), out);
+                s.bound, out);
 }
 
 void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,

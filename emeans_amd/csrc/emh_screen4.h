@@ -18,11 +18,9 @@
 //    one line;
 //  - a step's DMAs for the next slab go out between its groups of MFMAs, so
 //    one wave's loads are issued while the other wave on its SIMD runs MFMAs.
-// Two arithmetics, by the halves' format: bf16 three-pass (per 16 dimensions
-// hi.hi, hi.lo, lo.hi: k_screen3's sequence, so the same keys and bound) and
-// fp16 two-pass (centroid hi against row hi, then row lo: a third fewer
-// MFMAs and operand reads, within a bound 2.7 times the bf16 one at d = 768;
-// the centroids' lo halves are not read).
+// fp16 two-pass arithmetic (SCREEN_F16): per 16 dimensions centroid hi against
+// row hi, then row lo (the centroids' lo halves are not read), within a bound
+// that takes the worst case of every element's rounding.
 #pragma once
 
 #include <type_traits>
@@ -50,7 +48,7 @@ constexpr int S4_STAGE = 2 * S4_HALF;      // rows and centroids: 64 KB
 // conflict-free only for the first grouping.)
 __device__ __forceinline__ int swz(int r) { return (((r >> 1) & 3) << 1) | ((r >> 3) & 1); }
 
-// The largest of part[2 i] and of part[2 i + 1] over i < nparts (f32 bits
+// The largest of part[4 i] and of part[4 i + 1] over i < nparts (f32 bits
 // compared as u32: a NaN or negative value wins), in every lane of the wave.
 // Each lane's loads of a batch of PMB partials are issued together: a loop
 // of load-then-max would wait once per 64 partials.
@@ -65,7 +63,7 @@ __device__ __forceinline__ void part_max(const uint32_t* __restrict__ part, int 
 #pragma unroll
     for (int u = 0; u < PMB; u++) {
       const int i = i0 + 64 * u + lane;
-      v[u] = i < nparts ? reinterpret_cast<const uint2*>(part)[i] : make_uint2(0u, 0u);
+      v[u] = i < nparts ? reinterpret_cast<const uint2*>(part)[2 * i] : make_uint2(0u, 0u);
     }
 #pragma unroll
     for (int u = 0; u < PMB; u++) {
@@ -97,12 +95,12 @@ __device__ __forceinline__ void load32(const float* p, int col, int d, float (&v
 }
 
 // Split rows ids[lo + g] (lo + g without ids; an id >= nx reads row 0) for
-// g < n into out (fp16 halves when f16, else bf16), in selection order and
+// g < n into out (fp16 halves), in selection order and
 // slab-major: slab j of row g at
 // out + (j n + g) 128 bytes. norm[g] = the row's |x|^2 (f32, summed in any
 // order: the screen bound's input). With part: block b writes the largest
 // |x|^2 of its rows and, with cnorm, the largest cnorm[g] (f32 bits; a NaN or
-// negative value wins) to part[2 b], part[2 b + 1]: the bound's centroid
+// negative value wins) to part[4 b], part[4 b + 1]: the bound's centroid
 // inputs, which the screen reduces (no atomics on one word).
 // Block b takes rows 8 b .. 8 b + 7, two per wave. A wave reads a row in
 // 256-dimension segments, 16 contiguous bytes per lane (one 1 KB run per
@@ -115,7 +113,7 @@ __global__ __launch_bounds__(256) void k_halves(const float* __restrict__ x, siz
                                                 size_t n, char* __restrict__ out,
                                                 float* __restrict__ norm,
                                                 const float* __restrict__ cnorm,
-                                                uint32_t* __restrict__ part, int f16) {
+                                                uint32_t* __restrict__ part) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int d32 = (d + 31) >> 5, nseg = (d32 + 7) >> 3;
   const int js = lane >> 3, c4 = lane & 7;
@@ -159,7 +157,7 @@ __global__ __launch_bounds__(256) void k_halves(const float* __restrict__ x, siz
       sq[i] = fmaf(v[i].z, v[i].z, sq[i]);
       sq[i] = fmaf(v[i].w, v[i].w, sq[i]);
       uint2 hi, lw;
-      split_quad(v[i], hi, lw, f16 != 0);
+      split_quad(v[i], hi, lw);
       if (valid[i]) {
         char* o = out + ((size_t)j * n + g[i]) * SLAB_BYTES + hoff;
         *reinterpret_cast<uint2*>(o) = hi;
@@ -189,8 +187,8 @@ __global__ __launch_bounds__(256) void k_halves(const float* __restrict__ x, siz
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      part[2 * blockIdx.x] = max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3]));
-      part[2 * blockIdx.x + 1] = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
+      part[4 * blockIdx.x] = max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3]));
+      part[4 * blockIdx.x + 1] = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
     }
   }
 }
@@ -208,7 +206,7 @@ using StageNo = std::integral_constant<int, I>;
 // s % 2. Step s waits for its own DMAs, passes a barrier (every wave's DMAs of
 // step s are in, and every wave is done with stage (s + 1) % 2), then runs
 // its MFMAs while it issues the DMAs of step s + 1 into the other stage.
-template <int L, bool L2, int NW, bool F16>
+template <int L, bool L2, int NW>
 __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
     const char* __restrict__ xs, size_t xslab, const float* __restrict__ xn, size_t nx, int d,
     const uint32_t* __restrict__ ids, size_t lo, int nrows, const char* __restrict__ cs,
@@ -285,8 +283,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
   // half h takes dimensions 16 kk + 8 h .. + 7 (chunk 4 kk + h of the hi
   // half, 4 kk + 2 + h of the lo half).
   const int sw = swz(li);  // rows wr * RW + y * 32 + li: swz(row) = sw
-  // Operand registers: 8 halves of one format (fp16 or bf16).
-  typedef std::conditional_t<F16, v8h, v8bf> Op;
+  typedef v8h Op;  // operand registers: 8 halves
   struct Rows {
     Op bh[WN], bl[WN];
   };
@@ -299,12 +296,11 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
       o.bl[y] = *reinterpret_cast<const Op*>(p + ol);
     }
   };
-  Op ah[WA], al[WA];  // centroid operands: each refreshed right after its MFMAs (al: bf16)
+  Op ah[WA];  // centroid operands (hi halves): each refreshed right after its MFMAs
   auto read_cent = [&](const char* X, int kk, int a) __attribute__((always_inline)) {
-    const int oh = ((4 * kk + h) ^ sw) << 4, ol = ((4 * kk + 2 + h) ^ sw) << 4;
+    const int oh = ((4 * kk + h) ^ sw) << 4;
     const char* p = X + S4_HALF + (wc * 128 + a * 32 + li) * SLAB_BYTES;
     ah[a] = *reinterpret_cast<const Op*>(p + oh);
-    if (!F16) al[a] = *reinterpret_cast<const Op*>(p + ol);
   };
 
   float lkey[WN][L];  // per-row lists, filled by the fold after the loop
@@ -350,7 +346,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
         xv = xn[id < nx ? id : 0];
       }
       thr_e[y] = 2.0f * 1.0078125f *
-                 screen_bound(xv, cm2, cnm, d, L2, F16 ? BOUND_F16_TAGGED : BOUND_BF16_TAGGED);
+                 screen_bound(xv, cm2, cnm, d, L2, BOUND_F16_TAGGED);
     }
   }
   auto threshold = [&](float m, int y) __attribute__((always_inline)) {
@@ -431,22 +427,14 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
 
   constexpr int PER = 2 * ND + (L2 ? 1 : 0);  // DMAs per step per wave
   auto mfma = [](const Op& p, const Op& q, const v16f& c) __attribute__((always_inline)) {
-    if constexpr (F16)
-      return __builtin_amdgcn_mfma_f32_32x32x16_f16(p, q, c, 0, 0, 0);
-    else
-      return __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, q, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(p, q, c, 0, 0, 0);
   };
-  // One centroid block's MFMAs of a 16-dimension step: hi.hi, hi.lo, then
-  // (bf16) lo.hi.
-  auto mfma6 = [&](int a, const Rows& b) __attribute__((always_inline)) {
+  // One centroid block's MFMAs of a 16-dimension step: hi.hi, then hi.lo.
+  auto mfma4 = [&](int a, const Rows& b) __attribute__((always_inline)) {
 #pragma unroll
     for (int y = 0; y < WN; y++) acc[a][y] = mfma(ah[a], b.bh[y], acc[a][y]);
 #pragma unroll
     for (int y = 0; y < WN; y++) acc[a][y] = mfma(ah[a], b.bl[y], acc[a][y]);
-    if constexpr (!F16) {
-#pragma unroll
-      for (int y = 0; y < WN; y++) acc[a][y] = mfma(al[a], b.bh[y], acc[a][y]);
-    }
   };
   // Prologue: steps 0 and 1 into stages 0 and 1; step 0's first operands.
 #pragma unroll
@@ -462,7 +450,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
 #pragma unroll
   for (int a = 0; a < WA; a++) read_cent(s0, 0, a);
   // One step s (a 32-dimension slab in stage s % 2, two MFMA steps), as
-  // groups of 3 WN MFMAs (one centroid block each) with the fences keeping
+  // groups of 2 WN MFMAs (one centroid block each) with the fences keeping
   // each group's other work after it:
   //  - first MFMA step: its groups are followed by the reads of the second
   //    step's operands they no longer need;
@@ -481,7 +469,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
     const char* next = S == 0 ? s1 : s0;
 #pragma unroll
     for (int a = 0; a < WA; a++) {
-      mfma6(a, r0);
+      mfma4(a, r0);
       __builtin_amdgcn_sched_barrier(0);
       if (a == 0) read_rows(cur, 1, r1);
       read_cent(cur, 1, a);
@@ -492,7 +480,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_screen4(
     __builtin_amdgcn_s_barrier();  // ... and every wave's
 #pragma unroll
     for (int a = 0; a < WA; a++) {
-      mfma6(a, r1);
+      mfma4(a, r1);
       __builtin_amdgcn_sched_barrier(0);
       if (a == 0) read_rows(next, 0, r0);
       read_cent(next, 0, a);

@@ -80,7 +80,6 @@ enum Kind5 : int {
   KNN_SELF = 3,  // ... of the rows themselves, each row's own column left out
 };
 constexpr int KTH5 = KMAX;  // kNN: the smallest keys a thread keeps for its row's limit
-constexpr int L5 = 8;       // top-1: entries of a part's list
 constexpr int CAP5 = 12;    // slots of a row's append buffer (each of its two centroid waves)
 constexpr int LOG5_TOP1 = 32, LOG5_KNN = 256;  // entries of a thread's log
 
@@ -569,16 +568,32 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   // within the final limit, into [row][part][L]: a row's best first (top-1),
   // the rest in any order, unused entries {+inf, NONE}. More than L, or a log
   // that did not hold everything: L entries of -inf, which settle no row.
-  constexpr int RS = L | 1;  // a row's entries in LDS: keys, then ids, in the ring
+  constexpr int RS = L | 1, KS = NK | 1;  // LDS strides of a row's entries, and of a thread's keys
   float* OK = reinterpret_cast<float*>(ring);
   uint32_t* OI = reinterpret_cast<uint32_t*>(ring + S5_STAGE);
   uint32_t* on = OI + T5 * RS;
-  static_assert((T5 * RS + T5) * 4 <= S5_STAGE, "output space");
+  float* TK = reinterpret_cast<float*>(ring + 2 * S5_STAGE);
+  static_assert((T5 * RS + T5) * 4 <= S5_STAGE && 512 * KS * 4 <= 2 * S5_STAGE, "output space");
   __syncthreads();  // every wave's DMAs are in and its keys published
   if (tid < T5) on[tid] = 0u;
+  if (TOPK) {
+#pragma unroll
+    for (int e = 0; e < NK; e++) TK[tid * KS + e] = lkey[e];
+  }
   __syncthreads();
   {
-    const float lim = limit_of(published());
+    // The limit from the row's exact kk-th key (the published ones bound it
+    // by a key of rank kk .. 2 kk - 1, whose candidates may not fit the list).
+    float b = TOPK ? INFINITY : published();
+    if (TOPK) {
+      const float *A = TK + prow * KS, *B = TK + (T5 + prow) * KS;
+      for (int e = 0, i = 0; e < kk; e++) {  // i of A's and e - i of B's are the e smallest
+        const float va = A[i], vb = B[e - i];
+        b = fminf(va, vb);
+        i += va <= vb ? 1 : 0;
+      }
+    }
+    const float lim = limit_of(b);
     auto keep = [&](float key, uint32_t id) __attribute__((always_inline)) {
       if (key <= lim) {
         const uint32_t e = atomicAdd(&on[prow], 1u);

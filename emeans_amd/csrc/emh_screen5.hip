@@ -7,32 +7,32 @@
 namespace emh {
 namespace {
 
-// Block b: the power of two that brings the largest of 32,768 elements
-// sampled evenly over a matrix (b = 0: a, 1: b) to 2^7 .. 2^8, and its
-// inverse, into out. A sample: 8 bits of fp16's range are left above it and
-// 21 normal ones below, and a matrix with elements beyond that only costs its
-// rows the exact scan. Also clears `clear` (nclear words). Latency-bound (32
-// loads in flight per thread): ~5 us at any size.
-__global__ __launch_bounds__(1024) void k_scales(const float* __restrict__ a, size_t na,
+// Block b: the power of two that brings the largest of 8,192 elements sampled
+// evenly over a matrix (b = 0: a, 1: b; 128 runs of 64, `step` apart) to 2^7
+// .. 2^8, and its inverse, into out. A sample: 8 bits of fp16's range are left
+// above it and 21 normal ones below, and a matrix with elements beyond that
+// only costs its rows the exact scan. Also clears `clear` (nclear words).
+// Latency-bound: the loads of a thread are all in flight at once.
+constexpr int SRUNS = 8;  // runs per wave of 16
+__global__ __launch_bounds__(1024) void k_scales(const float* __restrict__ a, size_t na, size_t da,
                                                  float* __restrict__ sa,
-                                                 const float* __restrict__ b, size_t nb,
+                                                 const float* __restrict__ b, size_t nb, size_t db,
                                                  float* __restrict__ sb,
                                                  uint32_t* __restrict__ clear, int nclear) {
   const float* p = blockIdx.x ? b : a;
-  const size_t n = blockIdx.x ? nb : na;
+  const size_t n = blockIdx.x ? nb : na, step = blockIdx.x ? db : da;
   float* out = blockIdx.x ? sb : sa;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0 && tid < nclear) clear[tid] = 0u;
-  float v[32];
+  float v[SRUNS];
 #pragma unroll
-  for (int u = 0; u < 32; u++) {
-    const size_t seg = (size_t)(u * 16 + w);
-    const size_t i = (n > 64 ? seg * (n - 64) / 511 : 0) + lane;
+  for (int u = 0; u < SRUNS; u++) {
+    const size_t i = (size_t)(u * 16 + w) * step + lane;
     v[u] = i < n ? p[i] : 0.f;
   }
   float m = 0.f;
 #pragma unroll
-  for (int u = 0; u < 32; u++) {
+  for (int u = 0; u < SRUNS; u++) {
     const float e = fabsf(v[u]);
     m = e < INFINITY ? fmaxf(m, e) : m;  // NaN and infinities say nothing of the scale
   }
@@ -194,8 +194,10 @@ void launch5(emh_ctx* c, unsigned blocks, const Args5& a) {
 
 void launch_scales(emh_ctx* c, const float* a, size_t na, float* sa, const float* b, size_t nb,
                    float* sb, uint32_t* clear, int nclear) {
-  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, na, sa, b, nb, sb,
-                     clear, nclear);
+  // The last run ends within the matrix; matrices below 8,192 elements are read whole.
+  auto step = [](size_t n) { return n > 8192 ? (n - 64) / (16 * SRUNS - 1) : (size_t)64; };
+  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, na, step(na), sa, b,
+                     nb, step(nb), sb, clear, nclear);
   EMH_HIP(hipGetLastError());
 }
 
@@ -213,6 +215,54 @@ void launch_lines(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_
 void launch_part_max4(emh_ctx* c, const uint32_t* part, size_t nparts, uint32_t* out) {
   hipLaunchKernelGGL(k_part_max4, dim3(1), dim3(1024), 0, c->stream, part, nparts, out);
   EMH_HIP(hipGetLastError());
+}
+
+void launch_screen5(emh_ctx* c, const Lines5& l, bool ip) {
+  // The kernel addresses a slab's rows with 32-bit byte offsets (64 per row).
+  EMH_ENSURE(l.nx < (1u << 25) && l.k < (1u << 25), "screen: more than 2^25 rows or centroids");
+  EMH_ENSURE(l.tpp >= 1 && l.parts >= 1 && (l.parts - 1) * l.tpp < l.ntiles &&
+                 l.parts * l.tpp >= l.ntiles,
+             "screen: parts");
+  const bool one = l.tpp == 1;
+  Args5 a{};
+  a.xs = (const char*)l.xs;
+  a.xslab = l.xslab;
+  a.xn = l.xn;
+  a.nx = l.nx;
+  a.ids = l.ids;
+  a.cs = (const char*)l.cs;
+  a.cslab = l.k * (size_t)LINE_BYTES;
+  a.cnorm = l.cnorm;
+  a.k = (int)l.k;
+  a.d = (int)l.d;
+  a.kk = 1;
+  a.tpp = l.tpp;
+  a.parts = l.parts;
+  a.ntiles = l.ntiles;
+  a.bstride = l.n;
+  a.part = l.part;
+  a.nparts = l.nparts;
+  a.sx = l.sx;
+  a.sc = l.sc;
+  // Parts of several tiles keep logs (128 KB a block): launches of at most
+  // four blocks a CU bound them to 128 MB.
+  const int row_tiles = (int)((l.n + T5 - 1) / T5);
+  const int step = one ? row_tiles : std::max(1, 4 * std::max(c->cus, 1) / l.parts);
+  if (!one)
+    a.log = (Cand*)c->log5.get((size_t)std::min(step, row_tiles) * l.parts * 512 * LOG5_TOP1 *
+                               sizeof(Cand));
+  for (int r = 0; r < row_tiles; r += step) {
+    const size_t q0 = (size_t)r * T5, q1 = std::min((size_t)(r + step) * T5, l.n);
+    a.lo = l.lo + q0;
+    a.nrows = (int)(q1 - q0);
+    a.cand = l.cand + q0 * l.parts * L5;
+    a.bound = l.bound + q0;
+    const unsigned blocks = (unsigned)((q1 - q0 + T5 - 1) / T5 * l.parts);
+    if (one)
+      ip ? launch5<TOP1_IP, true>(c, blocks, a) : launch5<TOP1_L2, true>(c, blocks, a);
+    else
+      ip ? launch5<TOP1_IP, false>(c, blocks, a) : launch5<TOP1_L2, false>(c, blocks, a);
+  }
 }
 
 bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d) {
@@ -246,7 +296,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   const float2* qn = xn;
   if (!same) {
     void* qw = c->xsplit.get(lines_bytes(m, d));
-    float2* qnw = (float2*)c->misc.get(m * 8);
+    float2* qnw = (float2*)c->xsplit_norm.get(m * 8);
     launch_lines(c, q, m, d, nullptr, 0, m, sx, qw, qnw, nullptr, nullptr);
     qs = qw;
     qn = qnw;

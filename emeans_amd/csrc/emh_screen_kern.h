@@ -848,9 +848,8 @@ struct Screen4Args {
   int tpp, parts, ntiles;
   Cand* cand;
   float* xnorm;
-  const uint32_t* part;  // the centroid split's per-block maxima (launch_halves' part)
+  const uint32_t* part;  // the centroids' maxima, four words a group (SplitCents)
   int nparts;
-  bool f16;  // both operands in fp16 halves: the two-pass screen (else bf16, three passes)
 };
 void launch_screen4(emh_ctx* c, const Screen4Args& a, bool ip);
 // The 128 x 128 top-1 screen (emh_screen_t1_{bf3,f32}.hip) and the kNN screen

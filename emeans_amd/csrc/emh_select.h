@@ -11,6 +11,7 @@ constexpr uint32_t NONE = 0xffffffffu;
 constexpr int L1 = 6;    // top-1: the smallest screen keys each part keeps
 constexpr int L1S = 5;   // ... with the sorted insert (parts of several 256-centroid tiles)
 constexpr int L1F = 10;  // ... on the fp16 two-pass screen (its bound admits more near-ties)
+constexpr int L5 = 8;    // ... on the one-pass screen
 constexpr int C1 = 16;   // top-1: most candidates a row sends to the exact chains
 constexpr int LK = 24;   // top-k list: kk <= 16 plus 7 spare + the bound
 constexpr int KMAX = 16;  // largest kk of the screened top-k (emeans-core/src/knn.rs:16)
@@ -75,7 +76,7 @@ __device__ __forceinline__ void insert_nb(float (&key)[L], uint32_t (&id)[L], fl
 enum BoundKind : int {
   BOUND_F32 = 0,         // f32 MFMA screen
   BOUND_BF16 = 1,        // bf16 three-pass screen
-  BOUND_BF16_TAGGED = 2, // the same with tagged keys (k_screen4, k_screen3 one tile per part)
+  BOUND_BF16_TAGGED = 2, // the same with tagged keys (k_screen3 one tile per part)
   BOUND_F16_TAGGED = 3,  // fp16 two-pass screen with tagged keys (k_screen4 on fp16 halves)
   BOUND_LINES = 4,       // fp16 one-pass screen (k_screen5): E of row r comes in xnorm[r]
 };
@@ -177,6 +178,30 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
                     const Cand* cand, int parts, const float* xnorm, uint32_t* labels,
                     float* scores, uint32_t* fb, int bound, const LabelTally* tally = nullptr,
                     int L = L1);
+// The one-pass top-1 screen (emh_screen5.hip) over lines: row id r of nx at xs
+// (slab stride xslab) with xn[r] = (|x|^2, residual), positions lo .. lo + n
+// (through ids when given) against k centroids at cs with their maxima in part
+// (SplitCents) and, for L2, cnorm; parts of tpp tiles of 256 centroids. Lists
+// [row][parts][L5] in cand, the rows' E in bound[0 .. n) and its dot term in
+// bound[n ..).
+struct Lines5 {
+  const void* xs;
+  size_t xslab;
+  const float2* xn;
+  size_t nx;
+  const uint32_t* ids;
+  size_t lo, n;
+  const void* cs;
+  const float* cnorm;
+  size_t k, d;
+  int tpp, parts, ntiles;
+  Cand* cand;
+  float* bound;
+  const uint32_t* part;
+  int nparts;
+  const float *sx, *sc;
+};
+void launch_screen5(emh_ctx* c, const Lines5& a, bool ip);
 // The one-pass kNN screen (emh_screen5.hip): whether it takes a call, and the
 // call's screen (candidate lists [m][parts][LK]; the queries' E at bound[r]
 // and its dot term at bound[m + r]; in the context's scratch); returns the parts.

@@ -104,12 +104,19 @@ __device__ __forceinline__ float ordered_sum(const float* v, int len) {
   return s;
 }
 
+// Cluster j's own group of the bound's maxima.
+__device__ __forceinline__ void put_part(const CentsOut& o, size_t j, float norm) {
+  const uint32_t m = __float_as_uint(norm);
+  reinterpret_cast<uint4*>(o.part)[j] =
+      make_uint4(m, m, o.scale ? __float_as_uint(o.norm2[j].y) : 0u, 0u);
+}
+
 struct SmallLds {
   uint32_t lst[USB];                 // the cluster's rows in order
   float sq[UPDATE_SMALL_MAX_D];      // rounded squares of the new row (or of the readout's)
   float wmax[UT / 64];               // readout: each wave's max |v|
   uint32_t cnt;
-  float weight, rnorm;
+  float weight, rnorm, res;
 };
 
 // Cluster j = blockIdx.x, a thread per four columns in whole waves.
@@ -118,9 +125,8 @@ __global__ __launch_bounds__(UT) void k_update_small(
     size_t lo, size_t hi, const uint32_t* __restrict__ labels, size_t k,
     uint32_t* __restrict__ counts, uint32_t* __restrict__ zero_words, size_t nzero,
     float* __restrict__ acc, float* __restrict__ pos, float* __restrict__ usage, float alpha,
-    float decay, int replace, float* __restrict__ norms, char* __restrict__ csplit,
-    uint32_t* __restrict__ cpart, float* __restrict__ readout, uint32_t* __restrict__ tally,
-    uint32_t* __restrict__ small, int f16) {
+    float decay, int replace, float* __restrict__ norms, const CentsOut co,
+    float* __restrict__ readout, uint32_t* __restrict__ tally, uint32_t* __restrict__ small) {
   __shared__ __attribute__((aligned(16))) SmallLds L;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = (int)(blockDim.x >> 6);
   const size_t j = blockIdx.x;
@@ -154,7 +160,7 @@ __global__ __launch_bounds__(UT) void k_update_small(
   __syncthreads();
   const uint32_t cnt = L.cnt;
   if (cnt == 0) {  // the row stays; so do its norm, halves and readout
-    if (tid == 0 && cpart) cpart[2 * j] = cpart[2 * j + 1] = __float_as_uint(norms[j]);
+    if (tid == 0 && co.part) put_part(co, j, norms[j]);
     return;
   }
   float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -218,21 +224,24 @@ __global__ __launch_bounds__(UT) void k_update_small(
       tmx = fmaxf(fmaxf(fmaxf(fmaxf(tmx, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));
     }
   }
-  // The halves, with the zero columns of the last slab.
-  if (csplit && tid < (int)(((d + 31) & ~(size_t)31) / 4)) {
-    uint2 h, l;
-    split_quad(v, h, l, f16 != 0);  // zeros past d
-    const size_t col = 4 * (size_t)tid;
-    char* o = csplit + ((col >> 5) * k + j) * SLAB_BYTES + quad_hi_offset((int)(col & 31) >> 2);
-    *reinterpret_cast<uint2*>(o) = h;
-    *reinterpret_cast<uint2*>(o + 32) = l;
+  // The split row, with the zero columns of the last slab.
+  if (co.cs) {
+    if (tid == 0) L.res = 0.0f;
+    __syncthreads();
+    if (tid < (int)(((d + 31) & ~(size_t)31) / 4)) {
+      const float r = put_quad(co, k, j, 4 * (size_t)tid, v);  // zeros past d
+      if (co.scale) atomicAdd(&L.res, r);  // in any order: the bound allows for it
+    }
   }
   if (norms) {
     __syncthreads();
     if (tid == 0) {
       const float nrm = ordered_sum(L.sq, (int)d);
       norms[j] = nrm;
-      if (cpart) cpart[2 * j] = cpart[2 * j + 1] = __float_as_uint(nrm);
+      if (co.part) {
+        if (co.scale) co.norm2[j].y = L.res;
+        put_part(co, j, nrm);
+      }
     }
     return;
   }
@@ -272,18 +281,17 @@ bool update_small(size_t n, size_t d, bool spherical) {
 void launch_update_small(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                          size_t lo, size_t hi, const uint32_t* labels, size_t k, uint32_t* counts,
                          uint32_t* tcnt, size_t ntcnt, float* acc, float* pos, float* usage,
-                         float alpha, float decay, int replace, float* norms, void* csplit,
-                         uint32_t* cpart, float* readout, uint32_t* tally, bool f16) {
+                         float alpha, float decay, int replace, float* norms, const CentsOut& co,
+                         float* readout, uint32_t* tally) {
   const size_t n = hi > lo ? hi - lo : 0;
   EMH_ENSURE(update_small(n, d, readout != nullptr) && tally && (norms != nullptr) != (readout != nullptr) &&
-                 (!csplit || (norms && cpart)),
+                 (!co.cs || (norms && co.part)),
              "update: shape outside the small-batch path");
   if (k == 0) return;
   const unsigned threads = (unsigned)std::max<size_t>(64, (d / 4 + 63) / 64 * 64);
   hipLaunchKernelGGL(k_update_small, dim3((unsigned)k), dim3(threads), 0, c->stream, x, nx, d, ids,
                      lo, hi, labels, k, counts, tcnt, tcnt ? ntcnt : 0, acc, pos, usage, alpha,
-                     decay, replace, norms, (char*)csplit, cpart, readout, tally, c->small,
-                     f16 ? 1 : 0);
+                     decay, replace, norms, co, readout, tally, c->small);
   EMH_HIP(hipGetLastError());
 }
 

@@ -90,3 +90,74 @@ def test_knn_ranges(dev, case):
         x[100, 3], x[200, 7], x[300] = np.nan, np.inf, 0.0
         q[7, 0], q[8, 1], q[9] = np.nan, -np.inf, 0.0
     _knn(dev, np.ascontiguousarray(q), np.ascontiguousarray(x), 10, False)
+
+
+def _top1(dev, x, c, metric, ids=None):
+    from emeans_amd import Mat, Select
+    n, d = x.shape
+    k = c.shape[0]
+    m = n if ids is None else len(ids)
+    cb, cn = dev.upload_f32(c), None
+    if metric == "l2":
+        cn = dev.zeros_f32(k)
+        dev.row_norms(cb, k, d, cn)
+    lab, sco = dev.zeros_u32(m), dev.zeros_f32(m)
+    idb = None if ids is None else dev.upload_u32(ids)
+    dev.top1(Mat(dev.bind(x), d), Select(idb, (0, m)), cb, cn, k, metric, lab, sco)
+    gl, gs = dev.read_u32(lab), dev.read_f32(sco)
+    ol, os_ = O.top1(x, d, c, metric, ids=ids)
+    assert np.array_equal(gl, ol)
+    assert gs.tobytes() == os_.tobytes()
+
+
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+@pytest.mark.parametrize("n,d,k", [
+    (33000, 32, 64),     # one tile per part, mostly padding; one slab
+    (16384, 33, 512),
+    (8191, 99, 1100),    # five tiles, the last a remainder
+    (4097, 64, 2048),    # eight single-tile parts
+    (4000, 100, 2049),   # nine tiles: parts of several
+    (3000, 384, 5000),
+])
+def test_top1_shapes(dev, metric, n, d, k):
+    ids = ((np.arange(n, dtype=np.uint64) * 7919 + 3) % n).astype(np.uint32)
+    x, c = _rows(n, d, n + k), _rows(k, d, k)
+    x[: n // 2] = c[np.arange(n // 2) % k] + np.float32(0.3) * x[: n // 2]
+    _top1(dev, x, c, metric, ids)
+
+
+@pytest.mark.parametrize("k", [1024, 3000])
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+def test_top1_crowds(dev, metric, k):
+    """Groups of 20 consecutive centroids within 1e-6, some exact duplicates:
+    more near-ties than a part's list keeps, and than its buffers hold."""
+    n, d = 8192, 128
+    c = _rows(k, d, 21)
+    noise = _rows(k, d, 22)
+    for a in range(0, 400, 20):
+        c[a:a + 20] = c[a] + np.float32(1e-6) * noise[a:a + 20]
+        c[a + 7] = c[a + 3]
+    x = c[np.arange(n) % k] + np.float32(0.2) * _rows(n, d, 23)
+    _top1(dev, x, c, metric)
+
+
+@pytest.mark.parametrize("case", ["large", "tiny", "mixed", "beyond", "special"])
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+@pytest.mark.parametrize("k", [600, 2100])
+def test_top1_ranges(dev, metric, case, k):
+    """As test_knn_ranges."""
+    n, d = 16384, 64
+    x, c = _rows(n, d, 31), _rows(k, d, 32)
+    if case == "large":
+        x, c = x * np.float32(1e9), c * np.float32(3e12)
+    elif case == "tiny":
+        x, c = x * np.float32(1e-12), c * np.float32(1e-15)
+    elif case == "mixed":
+        s = np.array([1.0, 1e-3, 1e-6, 1e-9], np.float32)
+        x, c = x * s[np.arange(n) % 4][:, None], c * s[np.arange(k) % 4][:, None]
+    elif case == "beyond":
+        x[5] *= np.float32(1e8)
+        x[6, 9] = np.float32(1e6)
+    else:
+        x[7, 0], x[8, 1], x[9] = np.nan, -np.inf, 0.0
+    _top1(dev, np.ascontiguousarray(x), np.ascontiguousarray(c), metric)
