@@ -108,6 +108,13 @@ __device__ __forceinline__ float seq_sq(const float* __restrict__ xr, int d) {
   return s;
 }
 
+// Entries written of a list whose length came out as n: none of one that
+// overflowed.
+template <int L>
+__device__ __forceinline__ uint32_t list_length(uint32_t n) {
+  return n > (uint32_t)L ? 0u : n;
+}
+
 // Block: 256 threads, R rows (positions lo + r0 ...). KNN: rows are queries,
 // "centroids" the data rows, and the kk best by exact dot are written per
 // query (labels/scores then hold m x kk ids/sims).
@@ -117,8 +124,9 @@ __global__ __launch_bounds__(256) void k_verify(
     int nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
     int kk, const Cand* __restrict__ cand, int parts, const float* __restrict__ xnorm,
     uint32_t* __restrict__ labels, float* __restrict__ scores, uint32_t* __restrict__ fb,
-    uint32_t* __restrict__ small, int bound) {
-  constexpr int PMAX = R * (KNN ? L : C1 + 1);  // pairs (+ the |x|^2 chain per top-1 row)
+    uint32_t* __restrict__ small, int bound, const uint32_t* __restrict__ ncand) {
+  constexpr int CM = L == L5 ? C5 : C1;         // most candidates of a top-1 row
+  constexpr int PMAX = R * (KNN ? L : CM + 1);  // pairs (+ the |x|^2 chain per top-1 row)
   __shared__ Cand cst[R * MAX_PARTS * L];
   __shared__ uint32_t prow[PMAX], pcid[PMAX];
   __shared__ float pres[PMAX];
@@ -147,8 +155,14 @@ __global__ __launch_bounds__(256) void k_verify(
       for (int u = 0; u < 4; u++)
         if (i0 + 256 * u < ne) v[u] = src[i0 + 256 * u];
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (i0 + 256 * u < ne) dst[i0 + 256 * u] = v[u];
+      for (int u = 0; u < 4; u++) {
+        const int i = i0 + 256 * u;
+        if (i >= ne) continue;
+        // (Lists with lengths: what was not written is no entry.)
+        if (ncand && (uint32_t)(i % L) >= list_length<L>(ncand[(size_t)r0 * parts + i / L]))
+          v[u] = make_uint2(__float_as_uint(INFINITY), NONE);
+        dst[i] = v[u];
+      }
     }
   }
   __syncthreads();
@@ -197,13 +211,15 @@ __global__ __launch_bounds__(256) void k_verify(
         int tot = 0;
         for (int q = 0; q < parts; q++) {
           const Cand last = c[q * L + L - 1];
-          if (last.id != NONE && !(last.key > thr)) cert = false;
+          if (ncand ? ncand[(size_t)(r0 + tid) * parts + q] > (uint32_t)L
+                    : last.id != NONE && !(last.key > thr))
+            cert = false;
           for (int e = 0; e < L; e++) {
             const Cand v = c[q * L + e];
             tot += v.id != NONE && (v.key <= thr || thr != thr);
           }
         }
-        complete = anyv && cert && tot <= C1 && !(bound == BOUND_LINES && E != E);
+        complete = anyv && cert && tot <= CM && !(bound == BOUND_LINES && E != E);
         if (complete) nc = tot + (l2 ? 1 : 0);
       }
       if (complete) {
@@ -342,26 +358,45 @@ constexpr int RK = 16;  // rows per block, top-k
 // keeps +inf or NaN), a part's list holds every centroid of the part whose
 // screen key satisfies le when the list is not full or its last key is above
 // thr. The row is settled when some entry is valid, every part is so, and at
-// most C1 entries satisfy le; its candidates are then exactly those entries.
+// most C1 (C5) entries satisfy le; its candidates are then exactly those entries.
 // Eight threads per row scan one part's list each and combine with lane
 // shuffles.
 //
 // Chains. The block's settled rows (x) and their candidates (centroid rows)
-// are staged in CDC-float chunks into a double-buffered LDS tile by waves 2-3,
-// which keep CNR chunks of loads in flight in registers; waves 0-1 run the
-// chains from LDS: wave 0 one lane per (row, candidate) fma chain, wave 1 one
-// lane per row for the |x|^2 chain (L2). Every chunk costs each wave one
-// barrier. Blocks whose rows have more than CCAP candidates in total take
+// are staged in CDC-float chunks into a double-buffered LDS tile by the last
+// waves, which keep CNR chunks of loads in flight in registers; the first run
+// the chains from LDS: one or two waves with a lane per (row, candidate) fma
+// chain, the next with a lane per row for the |x|^2 chain (L2). Every chunk costs each wave one
+// barrier. Blocks whose rows have more candidates than slots in total take
 // further passes over the chunks.
 constexpr int CR = 32;              // rows per block
-constexpr int CCAP = 64;            // candidate slots per pass (one chain lane each)
-constexpr int CSLOT = CR + CCAP;    // staged rows per chunk
 constexpr int CDC = 64;             // floats per chunk
 constexpr int CDC4 = CDC / 4;
 constexpr int CDP4 = CDC4 + 1;      // LDS row stride in float4: conflict-free chain reads
 constexpr int CNR = 2;              // chunks in flight per loading thread
-constexpr int CNQ = CSLOT * CDC4 / 128;  // float4 per loading thread per chunk
-static_assert(CSLOT * CDC4 % 128 == 0, "chunk split");
+// The block's shape by the lists' length. The one-pass screen's bound leaves
+// about 1.8 candidates a row where the others leave 1.1 (200k x 768 L2
+// mixture, k = 1024), 58 a block: 96 slots, with a second dot wave, keep most
+// blocks at one pass over the chunks (64 slots sent a third of them into a
+// second one, and the check from 23 to 31 us a batch), and two blocks still
+// fit a CU's LDS.
+template <int L>
+struct Check1 {
+  static constexpr bool LINES = L == L5;
+  static constexpr int CAP = LINES ? 96 : 64;      // candidate slots per pass (one chain lane each)
+  static constexpr int CM = LINES ? C5 : C1;       // most candidates of a row
+  static constexpr int PAIRS = CR * C1;            // most of a block's settled rows together
+  static constexpr int SLOT = CR + CAP;            // staged rows per chunk
+  static constexpr int DOTW = LINES ? 2 : 1;       // dot waves; then the norm wave
+  static constexpr int LOAD = LINES ? 256 : 128;   // loading threads (the last waves)
+  static constexpr int NT = 64 * (DOTW + 1) + LOAD;
+  static constexpr int NQ = SLOT * CDC4 / LOAD;    // float4 per loading thread per chunk
+  // Operands a chain lane reads ahead of its fmas (half a chunk's with seven
+  // waves a block: two blocks a CU leave a wave 128 registers).
+  static constexpr int HALF = LINES ? CDC4 / 2 : CDC4;
+  static constexpr int WAVES = LINES ? 4 : 2;      // per SIMD, at least
+  static_assert(SLOT * CDC4 % LOAD == 0 && NT >= 256, "chunk split");
+};
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -375,25 +410,30 @@ __device__ __forceinline__ void unroll_steps(F&& f) {
 }
 
 template <int L>
-__global__ __launch_bounds__(256) void k_check1(
+__global__ __launch_bounds__(Check1<L>::NT, Check1<L>::WAVES) void k_check1(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     int nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int ip,
     const Cand* __restrict__ cand, int parts, const float* __restrict__ xnorm,
     uint32_t* __restrict__ labels, float* __restrict__ scores, uint32_t* __restrict__ fb,
     uint32_t* __restrict__ small, int bound, uint32_t* __restrict__ tcnt,
-    uint32_t* __restrict__ tcounts, size_t tlo, size_t tstride) {
-  __shared__ v4f stage[2][CSLOT * CDP4];
+    uint32_t* __restrict__ tcounts, size_t tlo, size_t tstride,
+    const uint32_t* __restrict__ ncand) {
+  using G = Check1<L>;
+  constexpr int CCAP = G::CAP, CNQ = G::NQ, WN = G::DOTW, WL = G::DOTW + 1;
+  __shared__ v4f stage[2][G::SLOT * CDP4];
   __shared__ uint32_t xrow[CR];  // x row of each settled row, NONE otherwise
   __shared__ int rcnt[CR], roff[CR + 1], rset[CR];
-  __shared__ uint32_t prow[CR * C1], pcid[CR * C1];
-  __shared__ float pdot[CR * C1], pcn[CR * C1], rnorm[CR];
+  __shared__ uint32_t prow[G::PAIRS], pcid[G::PAIRS];
+  __shared__ float pdot[G::PAIRS], pcn[G::PAIRS], rnorm[CR];
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * CR;
   const int rows = min(CR, nrows - r0);
   const bool l2 = !ip;
   {
+    // Threads past the first 256 (r >= CR) only pass the barriers.
     const int r = tid >> 3, j = tid & 7;
     const bool live = r < rows;
+    uint32_t nl = (uint32_t)L;  // the list's length, when it comes with one
     float key[L];
     uint32_t idv[L];
 #pragma unroll
@@ -411,9 +451,12 @@ __global__ __launch_bounds__(256) void k_check1(
       xid = badid ? NONE : (uint32_t)xi;
       xn = xnorm[r0 + r];
       if (j < parts) {
-        const Cand* c = cand + ((size_t)(r0 + r) * parts + j) * L;
+        const size_t li = (size_t)(r0 + r) * parts + j;
+        const Cand* c = cand + li * L;
+        if (G::LINES) nl = ncand[li];
 #pragma unroll
         for (int e = 0; e < L; e++) {
+          if (G::LINES && (uint32_t)e >= list_length<L>(nl)) continue;
           const Cand v = c[e];
           key[e] = v.key;
           idv[e] = v.id;
@@ -443,7 +486,8 @@ __global__ __launch_bounds__(256) void k_check1(
         }
       // This part's list holds all of its centroids within thr: not full, or
       // its last key above thr (never with a NaN thr).
-      cert = idv[L - 1] == NONE || key[L - 1] > thr;
+      // Lists with lengths hold them unless they overflowed.
+      cert = G::LINES ? nl <= (uint32_t)L || j >= parts : idv[L - 1] == NONE || key[L - 1] > thr;
     }
     int tot = cj, incl = cj;
 #pragma unroll
@@ -453,8 +497,18 @@ __global__ __launch_bounds__(256) void k_check1(
       const int v = __shfl_up(incl, m, 8);
       if (j >= m) incl += v;
     }
-    const bool settled = vrow && anyv && cert && tot <= C1;
-    if (j == 0) {
+    bool settled = vrow && anyv && cert && tot <= G::CM;
+    if (G::LINES) {
+      // All rows' candidates together fit the block's pairs, or the rows
+      // whose do not go to the exact scan.
+      if (j == 0 && r < CR) rcnt[r] = settled ? tot : 0;
+      __syncthreads();
+      int before = 0;
+      for (int i = 0; i < min(r, CR); i++) before += rcnt[i];
+      settled = settled && before + tot <= G::PAIRS;
+      __syncthreads();
+    }
+    if (j == 0 && r < CR) {
       xrow[r] = settled ? xid : NONE;
       rcnt[r] = settled ? tot : 0;
       rset[r] = settled;
@@ -494,20 +548,21 @@ __global__ __launch_bounds__(256) void k_check1(
   const int wave = tid >> 6, lane = tid & 63;
   for (int pb = 0; pb < npairs; pb += CCAP) {
     const int np = min(CCAP, npairs - pb);
-    const bool dl = wave == 0 && lane < np;
-    const bool nl = l2 && pb == 0 && wave == 1 && lane < CR && rset[lane];
+    const int dlane = wave * 64 + lane;  // dot lanes: the first CCAP of waves 0 .. WN - 1
+    const bool dl = wave < WN && dlane < np;
+    const bool nl = l2 && pb == 0 && wave == WN && lane < CR && rset[lane];
     float acc = 0.f, nrm = 0.f, cn = 0.f;
-    if (wave >= 2) {
+    if (wave >= WL) {
       // Loaders. Float4 i of a chunk is slot i / CDC4, column i % CDC4; past
       // the used slots (and past d in the last chunk) the index is clamped, so
       // every thread issues the same loads each step and the waits stay exact.
       const int nlast = (CR + np) * CDC4 - 1;
-      const int lt = tid - 128;
+      const int lt = tid - 64 * WL;
       const v4f* src[CNQ];
       int col[CNQ], dst[CNQ];
 #pragma unroll
       for (int q = 0; q < CNQ; q++) {
-        const int i = min(lt + 128 * q, nlast);
+        const int i = min(lt + G::LOAD * q, nlast);
         const int slot = i / CDC4;
         const float* base;
         if (slot < CR) {
@@ -546,9 +601,9 @@ __global__ __launch_bounds__(256) void k_check1(
       for (int c0 = 0; c0 < nch; c0 += CNR)
         unroll_steps<CNR>([&](auto U) __attribute__((always_inline)) { step(U, c0); });
     } else {
-      const int xs = dl ? (int)prow[pb + lane] : (nl ? lane : 0);
-      const int cs = CR + (dl ? lane : 0);
-      if (dl && l2) cn = cnorm[pcid[pb + lane]];
+      const int xs = dl ? (int)prow[pb + dlane] : (nl ? lane : 0);
+      const int cs = CR + (dl ? dlane : 0);
+      if (dl && l2) cn = cnorm[pcid[pb + dlane]];
       __syncthreads();
       // As many barriers as the loaders: nch rounded up to a multiple of CNR.
       const int nsteps = (nch + CNR - 1) / CNR * CNR;
@@ -562,19 +617,24 @@ __global__ __launch_bounds__(256) void k_check1(
               // The chunk's operands are read into registers before the
               // chain starts, so the chain waits for LDS once per chunk
               // rather than once per four fmas.
-              v4f xa[CDC4], wa[CDC4];
+              constexpr int HF = G::HALF;
 #pragma unroll
-              for (int f = 0; f < CDC4; f++) {
-                xa[f] = xp[f];
-                wa[f] = cp[f];
-              }
-              __builtin_amdgcn_sched_barrier(0);
+              for (int f0 = 0; f0 < CDC4; f0 += HF) {
+                v4f xa[HF], wa[HF];
 #pragma unroll
-              for (int f = 0; f < CDC4; f++) {
-                acc = fmaf(xa[f].x, wa[f].x, acc);
-                acc = fmaf(xa[f].y, wa[f].y, acc);
-                acc = fmaf(xa[f].z, wa[f].z, acc);
-                acc = fmaf(xa[f].w, wa[f].w, acc);
+                for (int f = 0; f < HF; f++) {
+                  xa[f] = xp[f0 + f];
+                  wa[f] = cp[f0 + f];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int f = 0; f < HF; f++) {
+                  acc = fmaf(xa[f].x, wa[f].x, acc);
+                  acc = fmaf(xa[f].y, wa[f].y, acc);
+                  acc = fmaf(xa[f].z, wa[f].z, acc);
+                  acc = fmaf(xa[f].w, wa[f].w, acc);
+                }
+                __builtin_amdgcn_sched_barrier(0);
               }
             } else {
               for (int f = 0; f < n4; f++) {
@@ -616,8 +676,8 @@ __global__ __launch_bounds__(256) void k_check1(
       }
     }
     if (dl) {
-      pdot[pb + lane] = acc;
-      pcn[pb + lane] = cn;
+      pdot[pb + dlane] = acc;
+      pcn[pb + dlane] = cn;
     }
     if (nl) rnorm[lane] = nrm;
     __syncthreads();
@@ -688,10 +748,12 @@ __global__ __launch_bounds__(256) void k_margin(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     size_t nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int ip,
     const Cand* __restrict__ cand, int per_row, const float* __restrict__ xnorm,
-    const uint32_t* __restrict__ small, int bound, unsigned long long* __restrict__ out) {
+    const uint32_t* __restrict__ small, int bound, unsigned long long* __restrict__ out,
+    const uint32_t* __restrict__ ncand, int L) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nrows * (size_t)per_row) return;
   const size_t r = e / (size_t)per_row;
+  if (ncand && (e % L >= ncand[e / L] || ncand[e / L] > (uint32_t)L)) return;  // not written
   const Cand cd = cand[e];
   if (cd.id == NONE || !isfinite(cd.key)) return;
   const size_t p = lo + r;
@@ -729,7 +791,7 @@ __global__ __launch_bounds__(256) void k_margin(
 void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                    size_t lo, size_t n, const float* cents, const float* cnorm, bool ip,
                    const Cand* cand, int parts, int L, const float* xnorm, int bound,
-                   emh_screen_report* rep) {
+                   emh_screen_report* rep, const uint32_t* ncand) {
   unsigned long long* w = nullptr;
   EMH_HIP(hipMalloc(&w, 4 * sizeof(unsigned long long)));
   unsigned long long h[4] = {0, 0, 0, 0};
@@ -738,7 +800,7 @@ void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
     const size_t total = n * (size_t)parts * L;
     hipLaunchKernelGGL(k_margin, grid1(total, 256), dim3(256), 0, c->stream, x, nx, (int)d, ids,
                        lo, n, cents, cnorm, ip ? 1 : 0, cand, parts * L, xnorm, c->small, bound,
-                       w);
+                       w, ncand, L);
     EMH_HIP(hipGetLastError());
     EMH_HIP(hipMemcpyAsync(h, w, sizeof h, hipMemcpyDeviceToHost, c->stream));
     EMH_HIP(hipStreamSynchronize(c->stream));
@@ -759,30 +821,30 @@ void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
 void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                     size_t lo, size_t n, const float* cents, const float* cnorm, size_t k, bool ip,
                     const Cand* cand, int parts, const float* xnorm, uint32_t* labels,
-                    float* scores, uint32_t* fb, int bound, const LabelTally* tally, int L) {
+                    float* scores, uint32_t* fb, int bound, const LabelTally* tally, int L,
+                    const uint32_t* ncand) {
   const dim3 g((unsigned)((n + R1 - 1) / R1));
   static_assert(TALLY_CP % CR == 0, "a check block's rows lie in one tally chunk");
   EMH_ENSURE(!tally || (d % 4 == 0 && lo >= tally->lo && (lo - tally->lo) % TALLY_CP == 0),
              "check: a tally needs d %% 4 == 0 and chunk-aligned positions");
-  EMH_ENSURE(L == L1 || L == L1F || L == L5 || (L == L1S && d % 4 == 0),
+  EMH_ENSURE(L == L1 || L == L1F || (L == L5 && ncand) || (L == L1S && d % 4 == 0),
              "check: lists of %d entries", L);
-  if (d % 4 == 0)
-    hipLaunchKernelGGL(L == L1S   ? k_check1<L1S>
-                       : L == L1F ? k_check1<L1F>
-                       : L == L5  ? k_check1<L5>
-                                  : k_check1<L1>,
-                       dim3((unsigned)((n + CR - 1) / CR)), dim3(256), 0, c->stream, x,
-                       nx, (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts, xnorm,
+  if (d % 4 == 0) {
+    auto kern = L == L1S ? k_check1<L1S> : L == L1F ? k_check1<L1F> : L == L5 ? k_check1<L5> : k_check1<L1>;
+    const unsigned nt = L == L5 ? Check1<L5>::NT : Check1<L1>::NT;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + CR - 1) / CR)), dim3(nt), 0, c->stream, x, nx,
+                       (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts, xnorm,
                        labels, scores, fb, c->small, bound, tally ? tally->cnt : nullptr,
                        tally ? tally->counts : nullptr, tally ? tally->lo : 0,
-                       tally ? tally->stride : 0);
-  else
-    hipLaunchKernelGGL((L == L1F  ? k_verify<L1F, R1, false, false>
-                        : L == L5 ? k_verify<L5, R1, false, false>
-                                  : k_verify<L1, R1, false, false>),
-                       g, dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents, cnorm,
-                       (int)k, ip ? 1 : 0, 1, cand, parts, xnorm, labels, scores, fb, c->small,
-                       bound);
+                       tally ? tally->stride : 0, ncand);
+  } else {
+    auto kern = L == L1F  ? k_verify<L1F, R1, false, false>
+                : L == L5 ? k_verify<L5, R1, false, false>
+                          : k_verify<L1, R1, false, false>;
+    hipLaunchKernelGGL(kern, g, dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents,
+                       cnorm, (int)k, ip ? 1 : 0, 1, cand, parts, xnorm, labels, scores, fb,
+                       c->small, bound, ncand);
+  }
   EMH_HIP(hipGetLastError());
 }
 
@@ -793,11 +855,11 @@ void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, siz
   if (d % 4 == 0)
     hipLaunchKernelGGL((k_verify<LK, RK, true, true>), g, dim3(256), 0, c->stream, q, m, (int)d,
                        nullptr, (size_t)0, (int)m, data, nullptr, (int)n, 1, (int)kk, cand, parts,
-                       xnorm, ids, sims, fb, c->small, bound);
+                       xnorm, ids, sims, fb, c->small, bound, nullptr);
   else
     hipLaunchKernelGGL((k_verify<LK, RK, true, false>), g, dim3(256), 0, c->stream, q, m,
                        (int)d, nullptr, (size_t)0, (int)m, data, nullptr, (int)n, 1, (int)kk,
-                       cand, parts, xnorm, ids, sims, fb, c->small, bound);
+                       cand, parts, xnorm, ids, sims, fb, c->small, bound, nullptr);
   EMH_HIP(hipGetLastError());
 }
 

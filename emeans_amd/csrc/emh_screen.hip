@@ -167,6 +167,7 @@ namespace {
 struct Top1Screen {
   Top1Geom g;
   Cand* cand = nullptr;
+  uint32_t* ncand = nullptr;  // the lists' lengths (BOUND_LINES)
   uint32_t* fb = nullptr;
   float* xnorm = nullptr;
   BoundKind bound = BOUND_F32;
@@ -190,7 +191,10 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
                                     : BOUND_BF16;
   s.L = f16 ? L1F : g.split ? L5 : g.big && !tagged ? L1S : L1;
   const size_t cbytes = (size_t)g.parts * n * s.L * sizeof(Cand);
-  s.cand = (Cand*)(ar ? ar->take(cbytes) : c->cand.get(cbytes));
+  // (The one-pass screen's lists are followed by their lengths.)
+  const size_t lbytes = g.split && !f16 ? (size_t)g.parts * n * 4 : 0;
+  s.cand = (Cand*)(ar ? ar->take(cbytes) : c->cand.get(cbytes + lbytes));
+  if (lbytes) s.ncand = (uint32_t*)((char*)s.cand + cbytes);
   s.fb = (uint32_t*)(ar ? ar->take(n * 4) : c->fblist.get(n * 4));
   const size_t nb = g.split && !f16 ? 2 * n * 4 : n * 4;  // E and its dot term, or |x|^2
   s.xnorm = (float*)(ar ? ar->take(nb) : c->xnorm.get(nb));
@@ -261,6 +265,7 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
     a.parts = g.parts;
     a.ntiles = g.ntiles;
     a.cand = s.cand;
+    a.ncand = s.ncand;
     a.bound = s.xnorm;
     a.sx = sx;
     a.sc = sc;
@@ -349,7 +354,7 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
     return;
   }
   launch_verify1(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, s.cand, s.g.parts, s.xnorm, labels,
-                 scores, s.fb, s.bound, tally, s.L);
+                 scores, s.fb, s.bound, tally, s.L, s.ncand);
   launch_exact1(c, x, nx, d, ids, lo, n, s.fb, cents, cnorm, k, ip, labels, scores, ar, tally);
 }
 
@@ -370,7 +375,7 @@ void screen_margin_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const u
   out->parts = s.g.parts;
   out->tiles_per_part = s.g.tpp;
   launch_margin(c, x, nx, d, ids, lo, n, cents, cnorm, ip, s.cand, s.g.parts, s.L, s.xnorm,
-                s.bound, out);
+                s.bound, out, s.ncand);
 }
 
 void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,

@@ -97,6 +97,7 @@ struct Args5 {
   int k, d, kk;
   int tpp, parts, ntiles;
   Cand* cand;             // out: [row][part][L], see the end of k_screen5
+  uint32_t* ncand;        // top-1: their lengths
   Cand* log;              // blocks x 512 x LOG5_* entries of scratch (parts of several tiles)
   float* bound;           // out: E of row r at r, its dot term at bstride + r
   size_t bstride;
@@ -565,9 +566,10 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   wait_vm<0>();  // the DMAs past the last step have landed (the output reuses the stages)
 
   // The rows' candidates: of the two threads' logs (ONE: buffers), what lies
-  // within the final limit, into [row][part][L]: a row's best first (top-1),
-  // the rest in any order, unused entries {+inf, NONE}. More than L, or a log
-  // that did not hold everything: L entries of -inf, which settle no row.
+  // within the final limit, into [row][part][L]. Top-1: the length and that
+  // many entries, the best first; more than L, or a log that did not hold
+  // everything: a length beyond L. kNN: in any order, the unused entries
+  // {+inf, NONE}; more than L: L entries of -inf, which settle no row.
   constexpr int RS = L | 1, KS = NK | 1;  // LDS strides of a row's entries, and of a thread's keys
   float* OK = reinterpret_cast<float*>(ring);
   uint32_t* OI = reinterpret_cast<uint32_t*>(ring + S5_STAGE);
@@ -624,15 +626,24 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   }
   __syncthreads();
   if (tid < T5 && row0 + tid < nrows) {
-    Cand* out = a_.cand + ((size_t)(row0 + tid) * parts + part) * L;
+    const size_t at0 = (size_t)(row0 + tid) * parts + part;
+    Cand* out = a_.cand + at0 * L;
     const uint32_t n = on[tid];
     const bool full = n > (uint32_t)L;
-    uint32_t best = 0;
-    if (!TOPK && !full)
-      for (uint32_t e = 1; e < n; e++) best = OK[tid * RS + e] < OK[tid * RS + best] ? e : best;
-    for (uint32_t e = 0; e < (uint32_t)L; e++) {
-      const uint32_t at = tid * RS + (e == 0 ? best : e == best ? 0u : e);
-      out[e] = full ? Cand{-INFINITY, 0u} : e < n ? Cand{OK[at], OI[at]} : Cand{INFINITY, NONE};
+    if (TOPK) {
+      for (uint32_t e = 0; e < (uint32_t)L; e++)
+        out[e] = full ? Cand{-INFINITY, 0u}
+                 : e < n ? Cand{OK[tid * RS + e], OI[tid * RS + e]}
+                         : Cand{INFINITY, NONE};
+    } else {
+      a_.ncand[at0] = n;
+      uint32_t best = 0;
+      for (uint32_t e = 1; e < (full ? 0u : n); e++)
+        best = OK[tid * RS + e] < OK[tid * RS + best] ? e : best;
+      for (uint32_t e = 0; e < (full ? 0u : n); e++) {
+        const uint32_t at = tid * RS + (e == 0 ? best : e == best ? 0u : e);
+        out[e] = Cand{OK[at], OI[at]};
+      }
     }
   }
 }

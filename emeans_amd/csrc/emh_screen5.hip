@@ -256,6 +256,7 @@ void launch_screen5(emh_ctx* c, const Lines5& l, bool ip) {
     a.lo = l.lo + q0;
     a.nrows = (int)(q1 - q0);
     a.cand = l.cand + q0 * l.parts * L5;
+    a.ncand = l.ncand + q0 * l.parts;
     a.bound = l.bound + q0;
     const unsigned blocks = (unsigned)((q1 - q0 + T5 - 1) / T5 * l.parts);
     if (one)

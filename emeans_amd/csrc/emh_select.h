@@ -11,7 +11,8 @@ constexpr uint32_t NONE = 0xffffffffu;
 constexpr int L1 = 6;    // top-1: the smallest screen keys each part keeps
 constexpr int L1S = 5;   // ... with the sorted insert (parts of several 256-centroid tiles)
 constexpr int L1F = 10;  // ... on the fp16 two-pass screen (its bound admits more near-ties)
-constexpr int L5 = 8;    // ... on the one-pass screen
+constexpr int L5 = 16;   // ... on the one-pass screen, whose lists come with their lengths
+constexpr int C5 = 32;   // ... and most candidates of a row there
 constexpr int C1 = 16;   // top-1: most candidates a row sends to the exact chains
 constexpr int LK = 24;   // top-k list: kk <= 16 plus 7 spare + the bound
 constexpr int KMAX = 16;  // largest kk of the screened top-k (emeans-core/src/knn.rs:16)
@@ -177,12 +178,14 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
                     size_t lo, size_t n, const float* cents, const float* cnorm, size_t k, bool ip,
                     const Cand* cand, int parts, const float* xnorm, uint32_t* labels,
                     float* scores, uint32_t* fb, int bound, const LabelTally* tally = nullptr,
-                    int L = L1);
+                    int L = L1, const uint32_t* ncand = nullptr);
 // The one-pass top-1 screen (emh_screen5.hip) over lines: row id r of nx at xs
 // (slab stride xslab) with xn[r] = (|x|^2, residual), positions lo .. lo + n
 // (through ids when given) against k centroids at cs with their maxima in part
 // (SplitCents) and, for L2, cnorm; parts of tpp tiles of 256 centroids. Lists
-// [row][parts][L5] in cand, the rows' E in bound[0 .. n) and its dot term in
+// [row][parts][L5] in cand, of which the first ncand[row][parts] entries are
+// written, the best first (more than L5: none, the part is not complete); the
+// rows' E in bound[0 .. n) and its dot term in
 // bound[n ..).
 struct Lines5 {
   const void* xs;
@@ -196,6 +199,7 @@ struct Lines5 {
   size_t k, d;
   int tpp, parts, ntiles;
   Cand* cand;
+  uint32_t* ncand;
   float* bound;
   const uint32_t* part;
   int nparts;
@@ -219,7 +223,7 @@ void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, siz
 void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                    size_t lo, size_t n, const float* cents, const float* cnorm, bool ip,
                    const Cand* cand, int parts, int L, const float* xnorm, int bound,
-                   emh_screen_report* rep);
+                   emh_screen_report* rep, const uint32_t* ncand = nullptr);
 // ---- emh_verify.hip: the exact scans
 // Exact scan of rows `list[0..*count)` (list != nullptr) or positions lo..lo+n.
 // ar: take the scratch from this fixed block (see Arena) instead of the context's buffers.
