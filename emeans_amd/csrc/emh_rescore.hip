@@ -166,7 +166,8 @@ __global__ __launch_bounds__(256) void k_verify(
     }
   }
   __syncthreads();
-  // One thread per row. kNN: merge (a part's valid entries come first), bound, decide.
+  // One thread per row. kNN: merge (each part's list is ascending, so a part
+  // is done at its first entry not below the current L-th key), bound, decide.
   // Top-1: per part, as k_check1 decides (a part's list holds all of its
   // centroids within thr when not full or when its last key is above thr).
   float key[L];
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(256) void k_verify(
       for (int q = 0; q < parts; q++)
         for (int e = 0; e < L; e++) {
           const Cand v = c[q * L + e];
-          if (v.id == NONE) break;
+          if (v.id == NONE || !(v.key < key[L - 1])) break;
           insert<L>(key, id, v.key, v.id);
         }
     }
@@ -193,8 +194,7 @@ __global__ __launch_bounds__(256) void k_verify(
       bool complete;
       if (KNN) {
         thr = key[kk - 1] + 2.0f * E;
-        // (A NaN bound of the one-pass screen listed nothing.)
-        complete = (id[L - 1] == NONE || key[L - 1] > thr) && !(bound == BOUND_LINES && E != E);
+        complete = id[L - 1] == NONE || key[L - 1] > thr;
         if (complete)
 #pragma unroll
           for (int e = 0; e < L - 1; e++) nc += id[e] != NONE && (key[e] <= thr || thr != thr);
@@ -735,6 +735,162 @@ __global__ __launch_bounds__(Check1<L>::NT, Check1<L>::WAVES) void k_check1(
   }
 }
 
+// ---- Top-k check behind the one-pass screen (lists of up to LK entries a
+// part, any order, {+inf, NONE} after the valid ones; L entries of -inf where
+// a part could not hold its candidates).
+//
+// A part's list holds every data row of the part whose key is within the
+// part's own limit, which is at least the query's kk-th key plus 2E: the
+// query's candidates are the entries of all parts within its kk-th key plus
+// 2E. A wave takes a query's lists in registers (parts x LK entries over its
+// lanes), finds the kk-th key by bisection over the keys' ordered bits (one
+// compare and popcount a register and bit: no list to merge), and compacts the
+// candidates; then one thread per (query, candidate) runs the exact chain, and
+// each pair's place in the output is its rank among the query's pairs.
+// Latency-bound at small calls; it merged lists in one thread a query before
+// (2,000 queries, 8 parts: 104 us).
+// KQ queries per block: few, for calls of few queries (2,000 in blocks of 16 left
+// half the CUs without one).
+constexpr int KC = 64;                         // most candidates of a query
+constexpr int KR = (MAX_PARTS5 * LK + 63) / 64;  // list entries per lane
+
+// Ascending unsigned image of a float's order (not NaN).
+__device__ __forceinline__ uint32_t ord32(float v) {
+  const uint32_t u = __float_as_uint(v);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+template <int KQ, bool VEC4>
+__global__ __launch_bounds__(256) void k_verify_lines(
+    const float* __restrict__ q, int d, int m, const float* __restrict__ data, int kk,
+    const Cand* __restrict__ cand, int parts, const float* __restrict__ bound,
+    uint32_t* __restrict__ ids, float* __restrict__ sims, uint32_t* __restrict__ fb,
+    uint32_t* __restrict__ small) {
+  __shared__ uint32_t pid[KQ * KC];
+  __shared__ float pdot[KQ * KC];
+  __shared__ int cnt[KQ], off[KQ + 1];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int r0 = blockIdx.x * KQ, rows = min(KQ, m - r0);
+  for (int i = w; i < KQ; i += 4) {
+    int c = 0;
+    if (i < rows) {
+      const int n = parts * LK, nr = (n + 63) >> 6;
+      const Cand* src = cand + (size_t)(r0 + i) * n;
+      uint32_t key[KR], id[KR];
+      bool lost = false;
+#pragma unroll
+      for (int u = 0; u < KR; u++) {
+        key[u] = 0xffffffffu;  // no entry
+        id[u] = NONE;
+        if (u < nr && u * 64 + lane < n) {
+          const Cand v = src[u * 64 + lane];
+          if (v.id != NONE) {
+            key[u] = ord32(v.key);
+            id[u] = v.id;
+            lost |= v.key == -INFINITY;
+          }
+        }
+      }
+      const float E = bound[r0 + i];
+      const bool ok = E == E && __ballot(lost) == 0ull;
+      // The kk-th smallest key (the largest valid one when there are fewer):
+      // the least x with kk keys at most x, bit by bit from the top.
+      uint32_t x = 0u;
+      for (int b = 31; b >= 0; b--) {
+        const uint32_t t = x | ((1u << b) - 1u);  // this bit 0, the rest 1
+        int below = 0;
+#pragma unroll
+        for (int u = 0; u < KR; u++)
+          if (u < nr) below += __popcll(__ballot(key[u] <= t));
+        if (below < kk) x |= 1u << b;
+      }
+      // x = 0xffffffff: fewer than kk entries; all of them are candidates.
+      const float kth = __uint_as_float((x & 0x80000000u) ? (x & 0x7fffffffu) : ~x);
+      const float thr = x == 0xffffffffu ? INFINITY : kth + 2.0f * E;
+      const uint32_t xt = ord32(thr);
+#pragma unroll
+      for (int u = 0; u < KR; u++) {
+        if (u >= nr) continue;
+        const bool in = ok && id[u] != NONE && key[u] <= xt;
+        const unsigned long long mk = __ballot(in);
+        const int at = c + (int)__builtin_amdgcn_mbcnt_hi(
+                               (uint32_t)(mk >> 32),
+                               __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
+        if (in && at < KC) pid[i * KC + at] = id[u];
+        c += __popcll(mk);
+      }
+      if (!ok || c > KC) {
+        c = -1;
+        if (lane == 0) fb[atomicAdd(&small[SW_FALLBACK_COUNT], 1u)] = (uint32_t)(r0 + i);
+      }
+    }
+    if (lane == 0) cnt[i] = i < rows ? c : 0;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int s = 0;
+    for (int i = 0; i < KQ; i++) {
+      off[i] = s;
+      s += max(cnt[i], 0);
+    }
+    off[KQ] = s;
+  }
+  __syncthreads();
+  // One thread per pair runs its chain: pair p is candidate p - off[i] of query i.
+  const int np = off[KQ];
+  auto query_of = [&](int p) {
+    int i = 0;
+#pragma unroll
+    for (int b = KQ / 2; b > 0; b >>= 1) i += off[i + b] <= p ? b : 0;
+    return i;
+  };
+  for (int p = tid; p < np; p += 256) {
+    const int i = query_of(p), at = i * KC + p - off[i];
+    pdot[at] = chain<VEC4>(q + (size_t)(r0 + i) * d, data + (size_t)pid[at] * d, d);
+  }
+  __syncthreads();
+  // The kk best by (dot desc, id asc), IEEE; output order: IEEE total order
+  // descending, then id (knn.rs:82-103).
+  for (int p = tid; p < np; p += 256) {
+    const int i = query_of(p), n = off[i + 1] - off[i], at = i * KC + p - off[i];
+    const float v = pdot[at];
+    const uint32_t id = pid[at];
+    auto rank = [&](float a, uint32_t ia) {
+      int r = 0;
+      for (int j = 0; j < n; j++) {
+        const float o = pdot[i * KC + j];
+        r += o > a || (o == a && pid[i * KC + j] < ia) ? 1 : 0;
+      }
+      return r;
+    };
+    const int r = rank(v, id);
+    if (r >= kk) continue;
+    // Among the kept, total order differs from IEEE order only between zeros
+    // of different sign: +0 comes before -0.
+    int place = r;
+    if (v == 0.0f) {
+      const bool neg = __float_as_uint(v) != 0u;
+      for (int j = 0; j < n; j++) {
+        const float o = pdot[i * KC + j];
+        const uint32_t io = pid[i * KC + j];
+        if (!(o == 0.0f) || io == id || rank(o, io) >= kk) continue;
+        const bool oneg = __float_as_uint(o) != 0u;
+        if (neg && !oneg && io > id) place++;
+        if (!neg && oneg && io < id) place--;
+      }
+    }
+    ids[(size_t)(r0 + i) * kk + place] = id;
+    sims[(size_t)(r0 + i) * kk + place] = v;
+  }
+  for (int e = tid; e < rows * kk; e += 256) {  // fewer candidates than kk
+    const int i = e / kk;
+    if (cnt[i] >= 0 && e - i * kk >= cnt[i]) {
+      ids[(size_t)r0 * kk + e] = NONE;
+      sims[(size_t)r0 * kk + e] = -INFINITY;
+    }
+  }
+}
+
 // One thread per list entry: the entry's exact key (the check's fma chain
 // over t = 0..d-1 from +0; IP -dot, L2 cnorm - 2 dot) against its screen key.
 // out[0]: entries measured; out[1]: entries beyond E; out[2]: the largest
@@ -851,6 +1007,16 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                     size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
                     float* sims, uint32_t* fb, int bound) {
+  if (bound == BOUND_LINES) {
+    EMH_ENSURE(parts >= 1 && parts <= MAX_PARTS5 && kk <= KC, "check: %d parts", parts);
+    const int kq = m >= 64 * (size_t)c->cus ? 16 : 4;
+    auto kern = kq == 16 ? (d % 4 == 0 ? k_verify_lines<16, true> : k_verify_lines<16, false>)
+                         : (d % 4 == 0 ? k_verify_lines<4, true> : k_verify_lines<4, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((m + kq - 1) / kq)), dim3(256), 0, c->stream, q,
+                       (int)d, (int)m, data, (int)kk, cand, parts, xnorm, ids, sims, fb, c->small);
+    EMH_HIP(hipGetLastError());
+    return;
+  }
   const dim3 g((unsigned)((m + RK - 1) / RK));
   if (d % 4 == 0)
     hipLaunchKernelGGL((k_verify<LK, RK, true, true>), g, dim3(256), 0, c->stream, q, m, (int)d,

@@ -102,7 +102,7 @@ Top1Geom top1_geom(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool split
     g.big = g.split = true;
     g.row_tiles = (int)((n + TR3 - 1) / TR3);
     g.ntiles = nt3;
-    g.parts = nt3 <= MAX_PARTS ? nt3 : choose_parts(g.row_tiles, nt3, c->cus, 1);
+    g.parts = nt3 <= MAX_PARTS ? nt3 : parts5(g.row_tiles, nt3, c->cus, MAX_PARTS, 0.5);
     g.tpp = (g.ntiles + g.parts - 1) / g.parts;
     g.parts = (g.ntiles + g.tpp - 1) / g.tpp;
     return g;

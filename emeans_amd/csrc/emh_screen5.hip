@@ -304,20 +304,19 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   }
   const int row_tiles = (int)((m + T5 - 1) / T5);
   const int ntiles = (int)((n + T5 - 1) / T5);
-  // Parts (data-tile ranges) per query tile only while there are fewer query
-  // tiles than CUs: the blocks running at once on an XCD then stream the same
-  // data tiles, which its L2 serves.
-  int parts = std::max(1, std::min(std::min((c->cus + row_tiles - 1) / row_tiles, ntiles),
-                                   MAX_PARTS));
+  // Parts (data-tile ranges) where they fill waves of blocks better: up to
+  // MAX_PARTS5, so that a few query tiles still fill the chip (2,000 queries
+  // against 100,000 x 512: 8 parts gave 64 blocks, 0.94 ms; 31 take 0.45).
+  int parts = parts5(row_tiles, ntiles, std::max(c->cus, 1), MAX_PARTS5, 2.0);
   const int tpp = (ntiles + parts - 1) / parts;
-  parts = (ntiles + tpp - 1) / tpp;
   Cand* cand = (Cand*)c->cand.get((size_t)parts * m * LK * sizeof(Cand));
   float* bound = (float*)c->xnorm.get(2 * m * 4);
-  // One launch per block of queries that fills the CUs once: a launch's
-  // threads each keep a log (1 MB a block, 256 MB a launch).
-  const int rt_step = std::max(1, std::max(c->cus, 1) / parts);
+  // A launch's threads each keep a log (1 MB a block): launches of whole waves
+  // of blocks, at most four.
+  const int wave = std::max(1, std::max(c->cus, 1) / parts);
+  const int rt_step = 4 * wave;
   Cand* log = (Cand*)c->log5.get((size_t)std::min(rt_step, row_tiles) * parts * 512 * LOG5_KNN *
-                                    sizeof(Cand));
+                                 sizeof(Cand));
   Args5 a{};
   a.xslab = m * (size_t)LINE_BYTES;
   a.cs = (const char*)xs;

@@ -17,6 +17,7 @@ constexpr int C1 = 16;   // top-1: most candidates a row sends to the exact chai
 constexpr int LK = 24;   // top-k list: kk <= 16 plus 7 spare + the bound
 constexpr int KMAX = 16;  // largest kk of the screened top-k (emeans-core/src/knn.rs:16)
 constexpr int MAX_PARTS = 8;  // centroid parts per row tile: lists per row the verify merges
+constexpr int MAX_PARTS5 = 32;  // ... data parts per query tile of the one-pass kNN screen
 
 // A screen candidate: key (smaller is better: -dot for IP, |c|^2 - 2 dot for L2) and id.
 struct Cand {
@@ -206,6 +207,25 @@ struct Lines5 {
   const float *sx, *sc;
 };
 void launch_screen5(emh_ctx* c, const Lines5& a, bool ip);
+// Parts (of tpp tiles each) for row_tiles x ntiles tiles on `cus` CUs, one block
+// a CU at a time: the fewest tile times of the waves of blocks, where a block
+// costs `fixed` tiles besides its own (its first loads, its lists' start and
+// end). 133 row tiles of 64: 3 parts (two waves of 22) instead of 2 (two of 32).
+inline int parts5(int row_tiles, int ntiles, int cus, int maxp, double fixed) {
+  int best = 1;
+  double cost = 1e300;
+  for (int p = 1; p <= maxp && p <= ntiles; p++) {
+    const int tpp = (ntiles + p - 1) / p, pp = (ntiles + tpp - 1) / tpp;
+    if (pp != p) continue;
+    const double waves = (double)(((long long)row_tiles * p + cus - 1) / cus);
+    const double t = waves * (tpp + fixed);
+    if (t < 0.95 * cost) {  // (more parts are more lists to check)
+      cost = t;
+      best = p;
+    }
+  }
+  return best;
+}
 // The one-pass kNN screen (emh_screen5.hip): whether it takes a call, and the
 // call's screen (candidate lists [m][parts][LK]; the queries' E at bound[r]
 // and its dot term at bound[m + r]; in the context's scratch); returns the parts.
