@@ -23,62 +23,121 @@
 namespace emh {
 namespace {
 
-constexpr int DT = 64;  // queries and data rows per dots tile
-constexpr int DK = 16;  // dimensions per LDS slab
-constexpr int DP = DT + 4;  // padded slab row: the transposed stores hit 64 banks
-
 // S[i ldS + j] = chain over t < d of q[q0 + i][t] * x[j][t], i < qb, j < n.
-// Thread (ty, tx) of 16 x 16 computes queries 4 ty .. + 3 against data rows
-// 4 tx .. + 3: sixteen independent chains, two b128 LDS reads per 16 fmas.
+// A block computes BM queries against BN data rows, a thread TM x TN chains
+// (TM, TN / 4 groups of four consecutive columns, so that LDS reads are 16
+// bytes and a row's stores are contiguous): with 8 x 8 the fmas of a
+// dimension (64 a thread) take twice the time of its four LDS reads, where
+// 4 x 4 was bound by the reads (1,000 x 50,000 x 384: 1.26 ms). Slabs of DK
+// dimensions are double-buffered: the next one's loads are in flight while the
+// present one's fmas run. Few queries take narrow tiles (bound by the reads of
+// the data, and by what is padded).
+constexpr int DK = 16;
+
+template <int BM, int BN, int TM, int TN>
 __global__ __launch_bounds__(256) void k_dots(const float* __restrict__ q, size_t q0, int qb,
                                               const float* __restrict__ x, int n, int d,
                                               float* __restrict__ S, size_t ldS) {
-  __shared__ __attribute__((aligned(16))) float Qs[DK][DP];
-  __shared__ __attribute__((aligned(16))) float Xs[DK][DP];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int j0 = blockIdx.x * DT, i0 = blockIdx.y * DT;
-  // Loader: thread tid stages row tid / 4, dimensions 4 (tid % 4) .. + 3 of a slab.
-  const int lr = tid >> 2, lc = 4 * (tid & 3);
-  const int qi = min(i0 + lr, qb - 1), xj = min(j0 + lr, n - 1);  // clamped: valid rows only
-  const float* qrow = q + (q0 + (size_t)qi) * (size_t)d;
-  const float* xrow = x + (size_t)xj * (size_t)d;
-  float acc[4][4];
+  static_assert((BM / TM) * (BN / TN) == 256, "threads");
+  constexpr int QP = BM + 4, XP = BN + 4;  // padded: the transposed stores spread over the banks
+  constexpr int NTX = BN / TN;             // threads along the data rows
+  constexpr int VT = TN < 4 ? TN : 4;      // columns per group
+  constexpr int GN = TN / VT;              // groups, BN / GN columns apart
+  constexpr int LQ = (BM * DK / 4 + 255) / 256, LX = (BN * DK / 4 + 255) / 256;  // float4 loads
+  __shared__ __attribute__((aligned(16))) float Qs[2][DK][QP];
+  __shared__ __attribute__((aligned(16))) float Xs[2][DK][XP];
+  const int tid = threadIdx.x, tx = tid % NTX, ty = tid / NTX;
+  const int j0 = blockIdx.x * BN, i0 = blockIdx.y * BM;
+  // Loader: float4 e of an operand's slab is row e / 4, dimensions 4 (e % 4) .. + 3.
+  float qr[LQ][4], xr[LX][4];
+  auto load = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+    for (int u = 0; u < LQ; u++) {
+      const int e = u * 256 + tid, r = e >> 2, t = t0 + 4 * (e & 3);
+      const float* p = q + (q0 + (size_t)min(i0 + min(r, BM - 1), qb - 1)) * (size_t)d;
 #pragma unroll
-    for (int b = 0; b < 4; b++) acc[a][b] = 0.f;
-  for (int t0 = 0; t0 < d; t0 += DK) {
-    const int tn = min(DK, d - t0);
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int t = t0 + lc + e;
-      Qs[lc + e][lr] = t < d ? qrow[t] : 0.f;
-      Xs[lc + e][lr] = t < d ? xrow[t] : 0.f;
+      for (int c = 0; c < 4; c++) qr[u][c] = t + c < d ? p[t + c] : 0.f;
     }
-    __syncthreads();
-    for (int t = 0; t < tn; t++) {  // dimensions past d never enter a chain
-      const float4 qa = *reinterpret_cast<const float4*>(&Qs[t][4 * ty]);
-      const float4 xb = *reinterpret_cast<const float4*>(&Xs[t][4 * tx]);
-      const float qv[4] = {qa.x, qa.y, qa.z, qa.w};
-      const float xv[4] = {xb.x, xb.y, xb.z, xb.w};
 #pragma unroll
-      for (int a = 0; a < 4; a++)
+    for (int u = 0; u < LX; u++) {
+      const int e = u * 256 + tid, r = e >> 2, t = t0 + 4 * (e & 3);
+      const float* p = x + (size_t)min(j0 + min(r, BN - 1), n - 1) * (size_t)d;
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = fmaf(qv[a], xv[b], acc[a][b]);
+      for (int c = 0; c < 4; c++) xr[u][c] = t + c < d ? p[t + c] : 0.f;
     }
+  };
+  auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < LQ; u++) {
+      const int e = u * 256 + tid, r = e >> 2, t = 4 * (e & 3);
+      if (r < BM)
+#pragma unroll
+        for (int c = 0; c < 4; c++) Qs[b][t + c][r] = qr[u][c];
+    }
+#pragma unroll
+    for (int u = 0; u < LX; u++) {
+      const int e = u * 256 + tid, r = e >> 2, t = 4 * (e & 3);
+      if (r < BN)
+#pragma unroll
+        for (int c = 0; c < 4; c++) Xs[b][t + c][r] = xr[u][c];
+    }
+  };
+  float acc[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; a++)
+#pragma unroll
+    for (int b = 0; b < TN; b++) acc[a][b] = 0.f;
+  auto dim = [&](int b, int t) __attribute__((always_inline)) {
+    float qv[TM], xv[TN];
+#pragma unroll
+    for (int a = 0; a < TM; a++) qv[a] = Qs[b][t][ty * TM + a];
+#pragma unroll
+    for (int g = 0; g < GN; g++)
+#pragma unroll
+      for (int c = 0; c < VT; c++) xv[g * VT + c] = Xs[b][t][g * (BN / GN) + tx * VT + c];
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int c = 0; c < TN; c++) acc[a][c] = fmaf(qv[a], xv[c], acc[a][c]);
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int t0 = 0, b = 0; t0 < d; t0 += DK, b ^= 1) {
+    const bool more = t0 + DK < d;
+    if (more) load(t0 + DK);
+    const int tn = min(DK, d - t0);  // dimensions past d never enter a chain
+    if (tn == DK) {
+#pragma unroll
+      for (int t = 0; t < DK; t++) dim(b, t);
+    } else {
+      for (int t = 0; t < tn; t++) dim(b, t);
+    }
+    if (more) store(b ^ 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int i = i0 + 4 * ty + a;
+  for (int a = 0; a < TM; a++) {
+    const int i = i0 + ty * TM + a;
     if (i >= qb) break;
     float* o = S + (size_t)i * ldS;
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      const int j = j0 + 4 * tx + b;
-      if (j < n) o[j] = acc[a][b];
-    }
+    for (int g = 0; g < GN; g++)
+#pragma unroll
+      for (int c = 0; c < VT; c++) {
+        const int j = j0 + g * (BN / GN) + tx * VT + c;
+        if (j < n) o[j] = acc[a][g * VT + c];
+      }
   }
+}
+
+template <int BM, int BN, int TM, int TN>
+void dots(emh_ctx* c, const float* q, size_t q0, size_t nb, const float* data, size_t n, size_t d,
+          float* S, size_t ldS) {
+  const dim3 g((unsigned)((n + BN - 1) / BN), (unsigned)((nb + BM - 1) / BM));
+  hipLaunchKernelGGL((k_dots<BM, BN, TM, TN>), g, dim3(256), 0, c->stream, q, q0, (int)nb, data,
+                     (int)n, (int)d, S, ldS);
+  EMH_HIP(hipGetLastError());
 }
 
 // Ascending unsigned image of a float's IEEE total order.
@@ -119,6 +178,33 @@ __device__ __forceinline__ int block_rank(bool f, int* wsum, int& total) {
   return before + below;
 }
 
+// Bitonic sort of sk[0 .. cnt) (P slots, the rest filled), ascending.
+template <int P>
+__device__ __forceinline__ void sort_keys(unsigned long long* sk, uint32_t cnt) {
+  const int tid = threadIdx.x;
+  // (A power of two that holds them: short lists skip the wide stages.)
+  int m = 2;
+  while (m < (int)cnt) m <<= 1;
+  for (int s = tid; s < m; s += NT)
+    if ((uint32_t)s >= cnt) sk[s] = ~0ull;
+  __syncthreads();
+  for (int size = 2; size <= m; size <<= 1) {
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int t = tid; t < m / 2; t += NT) {
+        const int lo = 2 * t - (t & (stride - 1));
+        const int hi = lo + stride;
+        const bool up = (lo & size) == 0;
+        const unsigned long long a = sk[lo], b = sk[hi];
+        if ((a > b) == up) {
+          sk[lo] = b;
+          sk[hi] = a;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // Workgroup i: the kk best data rows of query q0 + i from its scores
 // S[i ldS ..], written to ids / sims row q0 + i. P (a power of two >= kk)
 // slots of sort keys in LDS.
@@ -136,6 +222,58 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
   const float* row = S + (size_t)blockIdx.x * ldS;
   auto key_at = [&](int j) { return sel_key(row[j], exclude_self && (size_t)j == qi); };
 
+  uint32_t cnt = 0;
+  bool listed = false;
+  if (kk <= NT / 2) {
+    // The kk-th largest of the threads' own maxima is at most the kk-th
+    // largest key: the keys not below it are few (about -NT ln(1 - kk / NT) of
+    // them in no particular order), so one more pass lists them all. Two reads
+    // of the row and no histogram, whose atomics meet in a few bins (1,000
+    // rows of 50,000: 593 us with the three radix passes).
+    uint32_t mine = 0u;
+    for (int j0 = tid; j0 < n; j0 += 8 * NT) {
+      uint32_t k8[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) k8[u] = j0 + u * NT < n ? key_at(j0 + u * NT) : 0u;
+#pragma unroll
+      for (int u = 0; u < 8; u++) mine = max(mine, k8[u]);
+    }
+    uint32_t x = 0u;  // the largest x with kk maxima not below it
+    for (int b = 31; b >= 0; b--)
+      if (__syncthreads_count(mine >= (x | (1u << b))) >= kk) x |= 1u << b;
+    if (tid == 0) sh_all = 0u;
+    __syncthreads();
+    for (int j0 = tid; j0 < n; j0 += 8 * NT) {
+      uint32_t k8[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) k8[u] = j0 + u * NT < n ? key_at(j0 + u * NT) : 0u;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        if (k8[u] == 0u || k8[u] < x) continue;
+        const int j = j0 + u * NT;
+        const uint32_t at = atomicAdd(&sh_all, 1u);
+        // Key first (-0 and +0 alike, as the selection compares them), then id.
+        if (at < (uint32_t)P) sk[at] = ((unsigned long long)(~k8[u]) << 32) | (uint32_t)j;
+      }
+    }
+    __syncthreads();
+    const uint32_t got = sh_all;
+    __syncthreads();
+    listed = got <= (uint32_t)P;
+    if (listed) {
+      sort_keys<P>(sk, got);
+      // The kk best; then their own order: IEEE total order, then id.
+      cnt = min(got, (uint32_t)kk);
+      for (uint32_t s = tid; s < (uint32_t)P; s += NT) {
+        if (s < cnt) {
+          const uint32_t j = (uint32_t)sk[s];
+          sk[s] = ((unsigned long long)(~ord_total(row[j])) << 32) | (unsigned long long)j;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if (!listed) {
   // Radix select of the kk-th largest key: digits of 11, 11 and 10 bits.
   uint32_t prefix = 0, pmask = 0;
   uint32_t rem = (uint32_t)kk;
@@ -212,26 +350,9 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
     got_gt += tot_gt;
     got_eq += tot_eq;
   }
-  const uint32_t cnt = all ? got_gt : (uint32_t)kk;
-  for (int s = tid; s < P; s += NT)
-    if ((uint32_t)s >= cnt) sk[s] = ~0ull;
-  __syncthreads();
-  // Bitonic sort of the P keys, ascending: score descending, then id ascending.
-  for (int size = 2; size <= P; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = tid; t < P / 2; t += NT) {
-        const int lo = 2 * t - (t & (stride - 1));
-        const int hi = lo + stride;
-        const bool up = (lo & size) == 0;
-        const unsigned long long a = sk[lo], b = sk[hi];
-        if ((a > b) == up) {
-          sk[lo] = b;
-          sk[hi] = a;
-        }
-      }
-      __syncthreads();
-    }
+  cnt = all ? got_gt : (uint32_t)kk;
   }
+  sort_keys<P>(sk, cnt);
   for (int t = tid; t < kk; t += NT) {
     const size_t o = qi * (size_t)kk + t;
     if ((uint32_t)t < cnt) {
@@ -257,12 +378,12 @@ void select_long(emh_ctx* c, unsigned blocks, const float* S, size_t ldS, size_t
 
 void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, size_t n,
                       size_t d, size_t kk, bool exclude_self, uint32_t* ids, float* sims) {
-  EMH_ENSURE(kk > (size_t)KMAX && kk <= (size_t)KLONG, "topk: kk = %zu outside %d..%d", kk,
-             KMAX + 1, KLONG);
+  EMH_ENSURE(kk >= 1 && kk <= KLONG, "topk: kk = %zu outside 1..%d", kk, KLONG);
   EMH_ENSURE(m < (1u << 31) && n < (1u << 31) && d < (1u << 31), "topk: shape too large");
   if (m == 0) return;
   // Scores of a block of queries against all data rows: about 1 GiB of
-  // scratch, at least one 64-query tile.
+  // scratch, at least one 128-query tile.
+  constexpr size_t DT = 128;
   const size_t ldS = std::max<size_t>((n + 3) & ~size_t(3), 4);
   const size_t budget = size_t(1) << 30;
   size_t qb = std::max<size_t>(budget / (ldS * 4) / DT * DT, DT);
@@ -271,16 +392,19 @@ void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, s
   for (size_t q0 = 0; q0 < m; q0 += qb) {
     const size_t nb = std::min(qb, m - q0);
     if (n > 0) {
-      const dim3 g((unsigned)((n + DT - 1) / DT), (unsigned)((nb + DT - 1) / DT));
-      hipLaunchKernelGGL(k_dots, g, dim3(256), 0, c->stream, q, q0, (int)nb, data, (int)n,
-                         (int)d, S, ldS);
-      EMH_HIP(hipGetLastError());
+      // Tiles by the queries there are; the wide one also needs data rows for
+      // two blocks a CU.
+      const size_t wide = (nb + 127) / 128 * ((n + 127) / 128);
+      if (nb <= 8)
+        dots<8, 256, 4, 2>(c, q, q0, nb, data, n, d, S, ldS);
+      else if (nb <= 64 || wide < 2 * (size_t)c->cus)
+        dots<32, 128, 4, 4>(c, q, q0, nb, data, n, d, S, ldS);
+      else
+        dots<128, 128, 8, 8>(c, q, q0, nb, data, n, d, S, ldS);
     }
     const unsigned blocks = (unsigned)nb;
-    if (kk <= 32)
-      select_long<32>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
-    else if (kk <= 256)
-      select_long<256>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
+    if (kk <= 128)
+      select_long<1024>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
     else
       select_long<KLONG>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
   }
