@@ -1223,7 +1223,7 @@ size_t dedup_groups(const float* x, size_t n, size_t d, const uint32_t* nb_ids,
 // ------------------------------------------------------------- auto-k pieces
 // kmeans_pp (emeans-cluster/src/auto.rs:401-455) on rows resident on the
 // device: each pick's row dots raise every row's best cosine on the device
-// (k_pp_best); the D^2 weights, their f64 sum and the draw run here in row
+// (k_row_chain); the D^2 weights, their f64 sum and the draw run here in row
 // order, as the reference's.
 std::vector<uint32_t> kmeans_pp_dev(emh_ctx* c, const float* x, size_t n, size_t d, size_t kmax,
                                     uint32_t seed) {

@@ -527,6 +527,9 @@ void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t
 constexpr int KLONG = 4096;
 void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                       size_t kk, bool exclude_self, uint32_t* ids, float* sims);
+// out[i nb + j] = the sequential f32 fma chain a[i] . b[j] over d (i < m, j < nb).
+void launch_dots(emh_ctx* c, const float* a, size_t m, size_t d, const float* b, size_t nb,
+                 float* out);
 // The screen stage of a top-1 call, its lists measured instead of checked.
 void screen_margin_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                         size_t lo, size_t hi, const float* cents, const float* cnorm, size_t k,

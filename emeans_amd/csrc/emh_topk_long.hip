@@ -376,6 +376,32 @@ void select_long(emh_ctx* c, unsigned blocks, const float* S, size_t ldS, size_t
 
 }  // namespace
 
+// Tiles by the columns there are: 16 for a handful (four chains a thread, more
+// blocks), 64, or 128 x 128 when such tiles make two blocks a CU (20,000 x 768
+// by 100: 32 x 128 tiles 175 us, 128 x 128 194; a thread a row 4,260). The clusters of the automatic-k sweeps
+// are 2 to 40: 12,000 x 768 rows against 20 took 1,374 us with a thread a row and
+// 64 chains each, 63 us here.
+void launch_dots(emh_ctx* c, const float* a, size_t m, size_t d, const float* b, size_t nb,
+                 float* out) {
+  EMH_ENSURE(d > 0 && d < (1u << 31), "dots: shape too large");
+  // (grid.y, and the int arithmetic on columns, stay in range.)
+  const size_t rows = size_t(1) << 21, cols = size_t(1) << 24;
+  for (size_t i0 = 0; i0 < m; i0 += rows)
+    for (size_t j0 = 0; j0 < nb; j0 += cols) {
+      const size_t mi = std::min(rows, m - i0), nj = std::min(cols, nb - j0);
+      const float* bj = b + j0 * d;
+      float* o = out + i0 * nb + j0;
+      if (nj <= 16)
+        dots<64, 16, 4, 1>(c, a, i0, mi, bj, nj, d, o, nb);
+      else if (nj <= 64)
+        dots<64, 64, 4, 4>(c, a, i0, mi, bj, nj, d, o, nb);
+      else if ((mi + 127) / 128 * ((nj + 127) / 128) < 2 * (size_t)c->cus)
+        dots<32, 128, 4, 4>(c, a, i0, mi, bj, nj, d, o, nb);
+      else
+        dots<128, 128, 8, 8>(c, a, i0, mi, bj, nj, d, o, nb);
+    }
+}
+
 void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, size_t n,
                       size_t d, size_t kk, bool exclude_self, uint32_t* ids, float* sims) {
   EMH_ENSURE(kk >= 1 && kk <= KLONG, "topk: kk = %zu outside 1..%d", kk, KLONG);
