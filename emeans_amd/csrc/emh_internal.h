@@ -132,6 +132,12 @@ constexpr size_t EXACT_BELOW = 4096;
 // (k_queued1: 4 rows x 16 centroids each, plus one per 4 rows for L2) take
 // that scan instead of k_exact1 (~13 us against ~32 us at 64 items).
 constexpr size_t QUEUED_DIRECT = 1024;
+// Direct selections against at most SMALL_DIRECT_K centroids take k_small1 (a
+// block holds all of them) up to SMALL_DIRECT rows times the centroids padded
+// to 16, 32 or 64. Training batches x 128 against 20 centroids: 2,544 rows 20
+// us, 8,192 rows 52 (its label counts are an atomic a row); the screen, its
+// check and its queue 28 and 31.
+constexpr size_t SMALL_DIRECT_K = 64, SMALL_DIRECT = 131072;
 // A top-1 call's exact items.
 inline size_t exact_items(size_t n, size_t k) {
   const size_t g = (k + 63) / 64;
@@ -386,7 +392,7 @@ constexpr size_t ONE_STREAM_ROWS = 65536;
 
 // ---- emh_update.hip: a small training batch's scatter_add and EMA step in one
 // launch (the same bits as launch_scatter_sums then launch_ema).
-constexpr size_t UPDATE_SMALL_BATCH = 256;  // most positions per batch
+constexpr size_t UPDATE_SMALL_BATCH = 1024;  // most positions per batch
 constexpr size_t UPDATE_SMALL_MAX_D = 1024;
 // Whether a batch of n positions with d dimensions takes it.
 bool update_small(size_t n, size_t d, bool spherical);

@@ -255,11 +255,19 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
 size_t exact1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool list);
 // The latency-bound scan's (k_queued1's) items for n rows against k centroids.
 size_t queued_items(size_t n, size_t k, bool ip);
-// Whether a direct selection of n rows takes the latency-bound scan instead
-// of k_exact1: d % 4 == 0 and at most QUEUED_DIRECT of its items (and the
-// context's exact_below not 0, which keeps k_exact1 for every selection).
+// Whether a direct selection of n rows takes the scan whose blocks hold every
+// centroid (k_small1).
+inline bool small_direct(emh_ctx* c, size_t n, size_t d, size_t k) {
+  const size_t kp = k <= 16 ? 16 : k <= 32 ? 32 : 64;
+  return d % 4 == 0 && c->exact_below > 0 && k <= SMALL_DIRECT_K && n <= SMALL_DIRECT / kp;
+}
+// Whether a direct selection of n rows takes a latency-bound scan instead of
+// k_exact1 or the screen: k_small1, or d % 4 == 0 and at most QUEUED_DIRECT of
+// k_queued1's items (and the context's exact_below not 0, which keeps k_exact1
+// for every selection).
 inline bool queued_direct(emh_ctx* c, size_t n, size_t d, size_t k, bool ip) {
-  return d % 4 == 0 && c->exact_below > 0 && queued_items(n, k, ip) <= QUEUED_DIRECT;
+  return small_direct(c, n, d, k) ||
+         (d % 4 == 0 && c->exact_below > 0 && queued_items(n, k, ip) <= QUEUED_DIRECT);
 }
 void launch_exactk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                    size_t kk, bool exclude_self, const uint32_t* fb, uint32_t* ids, float* sims);

@@ -3,13 +3,13 @@
 // (cpu.rs:389-432), for labels the batch's top-1 call tallied. The separate
 // path places every position in a cluster-sorted order (k_place_scan), adds
 // the sums (k_sums) and moves the centroids (k_ema): three launches whose
-// few, small workgroups spend their time waiting on memory, which on the
-// small fits of the automatic-k sweeps (64- to 256-row batches, a hundred
+// few, small workgroups spend their time waiting on memory, which on small
+// fits and those of the automatic-k sweeps (64- to 1,024-row batches, a hundred
 // steps per fit) is most of a step. Here the workgroup of cluster j
 //   - reads the batch's labels and row ids (every position at once: a batch
 //     is at most USB) and keeps the positions with label j, in order, by
 //     ballots: the cluster's rows in selection order;
-//   - adds them in that order from +0 (a thread per four columns), as k_sums;
+//   - adds them in that order from +0 (a thread a column), as k_sums;
 //   - moves the centroid from the sums in registers, as k_ema: the position,
 //     then either the squared norm (one lane adds the rounded squares in
 //     order) with the bf16 halves and the bound's maximum, or the spherical
@@ -25,11 +25,10 @@
 namespace emh {
 namespace {
 
-constexpr int UT = 256;                // most threads per workgroup (d <= 4 UT)
+constexpr int UT = 1024;               // most threads per workgroup (d <= UT)
 constexpr int USB = UPDATE_SMALL_BATCH;  // most positions per batch
-constexpr int USU = 16;                // row loads in flight per thread
 constexpr uint32_t NOROW = 0xffffffffu;
-static_assert(USB % 64 == 0 && UPDATE_SMALL_MAX_D <= 4 * UT, "shape");
+static_assert(USB % 64 == 0 && UPDATE_SMALL_MAX_D <= UT, "shape");
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -111,15 +110,26 @@ __device__ __forceinline__ void put_part(const CentsOut& o, size_t j, float norm
       make_uint4(m, m, o.scale ? __float_as_uint(o.norm2[j].y) : 0u, 0u);
 }
 
+template <int NB>
 struct SmallLds {
-  uint32_t lst[USB];                 // the cluster's rows in order
+  uint32_t lst[64 * NB];             // the cluster's rows in order
   float sq[UPDATE_SMALL_MAX_D];      // rounded squares of the new row (or of the readout's)
+  float nv[UPDATE_SMALL_MAX_D];      // the new row, for its split
   float wmax[UT / 64];               // readout: each wave's max |v|
   uint32_t cnt;
   float weight, rnorm, res;
 };
 
-// Cluster j = blockIdx.x, a thread per four columns in whole waves.
+// Cluster j = blockIdx.x, a thread per column in whole waves; a batch of at
+// most 64 NB positions. Bound by the memory's latency and, where a cluster has
+// hundreds of long rows, by what one CU can fetch: the rows are added in order,
+// so two groups of USU of them are in flight in turn (a thread per four columns
+// had the registers for one group: 15.2 us for 1,052 x 64 with 32 clusters,
+// 11.8 now; 512 x 768 with 5 clusters 27 either way). The separate launches
+// take 7.5 + 11 + 4.8 us and 7.3 + 13.7 + 10.0 there, and two more gaps between
+// launches.
+constexpr int USU = 32;
+template <int NB>
 __global__ __launch_bounds__(UT) void k_update_small(
     const float* __restrict__ x, size_t nx, size_t d, const uint32_t* __restrict__ ids,
     size_t lo, size_t hi, const uint32_t* __restrict__ labels, size_t k,
@@ -127,10 +137,11 @@ __global__ __launch_bounds__(UT) void k_update_small(
     float* __restrict__ acc, float* __restrict__ pos, float* __restrict__ usage, float alpha,
     float decay, int replace, float* __restrict__ norms, const CentsOut co,
     float* __restrict__ readout, uint32_t* __restrict__ tally, uint32_t* __restrict__ small) {
-  __shared__ __attribute__((aligned(16))) SmallLds L;
+  __shared__ __attribute__((aligned(16))) SmallLds<NB> L;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = (int)(blockDim.x >> 6);
   const size_t j = blockIdx.x;
-  const int d4 = (int)(d / 4);
+  const bool own = tid < (int)d;  // this thread has a column
+  const size_t at = j * d + tid;
   const int n = (int)(hi - lo);
   // The next batch's tally starts from zero; the screen's words too.
   for (size_t i = (size_t)blockIdx.x * blockDim.x + tid; i < nzero;
@@ -147,10 +158,10 @@ __global__ __launch_bounds__(UT) void k_update_small(
     L.weight = wgt;
   }
   // The batch's labels and row ids, every position at once (wave 0).
-  uint32_t lab[USB / 64], rw[USB / 64];
+  uint32_t lab[NB], rw[NB];
   if (w == 0) {
 #pragma unroll
-    for (int u = 0; u < USB / 64; u++) {
+    for (int u = 0; u < NB; u++) {
       const int i = 64 * u + lane;
       const size_t p = lo + (size_t)i;
       lab[u] = i < n ? labels[p] : NOROW;
@@ -163,73 +174,72 @@ __global__ __launch_bounds__(UT) void k_update_small(
     if (tid == 0 && co.part) put_part(co, j, norms[j]);
     return;
   }
-  float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (tid < d4) p = reinterpret_cast<const float4*>(pos + j * d)[tid];
+  const float p = own ? pos[at] : 0.0f;
   if (w == 0) {
     uint32_t r = 0;
     bool bad = false;  // a row id past the data adds nothing; reported at the next read
 #pragma unroll
-    for (int u = 0; u < USB / 64; u++) {
+    for (int u = 0; u < NB; u++) {
       const bool m = lab[u] == (uint32_t)j;
       const uint64_t b = __ballot(m);
       if (m) {
         const uint32_t i = r + lanes_below(b);
         const bool ok = (size_t)rw[u] < nx;
         bad |= !ok;
-        if (i < (uint32_t)USB) L.lst[i] = ok ? rw[u] : NOROW;
+        if (i < 64u * NB) L.lst[i] = ok ? rw[u] : NOROW;
       }
       r += (uint32_t)__popcll(b);
     }
     if (bad) small[SW_BAD_ID] = 1;
   }
   __syncthreads();
-  // The rows in order from +0 (as k_sums), USU row loads in flight.
-  const uint32_t nr = min(cnt, (uint32_t)USB);
-  float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  // The rows in order from +0 (as k_sums).
+  const uint32_t nr = min(cnt, 64u * NB);
+  float s = 0.0f, v = 0.0f;
   float tmx = 0.0f;  // readout: max |v| of this thread's values (fold from 0, fmaxf)
-  if (tid < d4) {
-    for (uint32_t q = 0; q < nr; q += USU) {
-      float4 rv[USU];
+  if (own) {
+    const float* const col = x + tid;
+    // Past the list its last row again, never added; a bad row reads row 0 and
+    // adds +0 (s is never -0, so this adds nothing).
+    auto load = [&](float (&g)[USU], uint32_t q) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < USU; u++) {
-        const uint32_t r = q + u < nr ? L.lst[q + u] : NOROW;
-        rv[u] = r != NOROW ? reinterpret_cast<const float4*>(x + (size_t)r * d)[tid]
-                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const uint32_t r = __builtin_amdgcn_readfirstlane(L.lst[min(q + u, nr - 1)]);
+        g[u] = col[(size_t)(r != NOROW ? r : 0u) * d];
+        g[u] = r != NOROW ? g[u] : 0.0f;
       }
+    };
+    auto add = [&](const float (&g)[USU], uint32_t q) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < USU; u++)
-        if (q + u < nr) {  // +0 for a bad row: s is never -0, so this adds nothing
-          s.x = s.x + rv[u].x;
-          s.y = s.y + rv[u].y;
-          s.z = s.z + rv[u].z;
-          s.w = s.w + rv[u].w;
-        }
+        if (q + u < nr) s = s + g[u];
+    };
+    float a[USU], b[USU];
+    load(a, 0);
+    for (uint32_t q = 0; q < nr; q += 2 * USU) {
+      if (q + USU < nr) load(b, q + USU);
+      add(a, q);
+      if (q + 2 * USU < nr) load(a, q + 2 * USU);
+      if (q + USU < nr) add(b, q + USU);
     }
-    if (acc) {
-      float4* ao = reinterpret_cast<float4*>(acc + j * d) + tid;
-      const float4 a0 = *ao;
-      *ao = make_float4(a0.x + s.x, a0.y + s.y, a0.z + s.z, a0.w + s.w);
-    }
-    const float count = (float)cnt, wgt = L.weight;
-    v.x = ema_value(s.x, p.x, count, wgt);
-    v.y = ema_value(s.y, p.y, count, wgt);
-    v.z = ema_value(s.z, p.z, count, wgt);
-    v.w = ema_value(s.w, p.w, count, wgt);
-    reinterpret_cast<float4*>(pos + j * d)[tid] = v;
-    if (norms) {
-      *reinterpret_cast<float4*>(L.sq + 4 * tid) =
-          make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
-    } else if (readout) {
-      tmx = fmaxf(fmaxf(fmaxf(fmaxf(tmx, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));
-    }
+    if (acc) acc[at] = acc[at] + s;
+    v = ema_value(s, p, (float)cnt, L.weight);
+    pos[at] = v;
+    if (norms)
+      L.sq[tid] = v * v;
+    else if (readout)
+      tmx = fmaxf(tmx, fabsf(v));
   }
   // The split row, with the zero columns of the last slab.
   if (co.cs) {
     if (tid == 0) L.res = 0.0f;
+    L.nv[tid] = v;
     __syncthreads();
     if (tid < (int)(((d + 31) & ~(size_t)31) / 4)) {
-      const float r = put_quad(co, k, j, 4 * (size_t)tid, v);  // zeros past d
+      const int t = 4 * tid;
+      const float4 q = t < (int)d ? *reinterpret_cast<const float4*>(L.nv + t)
+                                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      const float r = put_quad(co, k, j, (size_t)t, q);  // zeros past d
       if (co.scale) atomicAdd(&L.res, r);  // in any order: the bound allows for it
     }
   }
@@ -255,20 +265,14 @@ __global__ __launch_bounds__(UT) void k_update_small(
   float mx = L.wmax[0];
   for (int i = 1; i < nw; i++) mx = fmaxf(mx, L.wmax[i]);
   const float s1 = mx > 0.0f ? mx : 1.0f;
-  float4 qv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (tid < d4) {
-    qv = make_float4(v.x / s1, v.y / s1, v.z / s1, v.w / s1);
-    *reinterpret_cast<float4*>(L.sq + 4 * tid) =
-        make_float4(qv.x * qv.x, qv.y * qv.y, qv.z * qv.z, qv.w * qv.w);
-  }
+  const float qv = v / s1;
+  if (own) L.sq[tid] = qv * qv;
   __syncthreads();
   if (tid == 0) L.rnorm = sqrtf(ordered_sum(L.sq, (int)d));
   __syncthreads();
   const float nv = L.rnorm;
   const float s2 = nv > 0.0f ? nv : 1.0f;
-  if (tid < d4)
-    reinterpret_cast<float4*>(readout + j * d)[tid] =
-        make_float4(qv.x / s2, qv.y / s2, qv.z / s2, qv.w / s2);
+  if (own) readout[at] = qv / s2;
 }
 
 }  // namespace
@@ -288,8 +292,9 @@ void launch_update_small(emh_ctx* c, const float* x, size_t nx, size_t d, const 
                  (!co.cs || (norms && co.part)),
              "update: shape outside the small-batch path");
   if (k == 0) return;
-  const unsigned threads = (unsigned)std::max<size_t>(64, (d / 4 + 63) / 64 * 64);
-  hipLaunchKernelGGL(k_update_small, dim3((unsigned)k), dim3(threads), 0, c->stream, x, nx, d, ids,
+  const unsigned threads = (unsigned)std::max<size_t>(64, (d + 63) / 64 * 64);
+  auto kern = n <= 256 ? k_update_small<4> : k_update_small<USB / 64>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)k), dim3(threads), 0, c->stream, x, nx, d, ids,
                      lo, hi, labels, k, counts, tcnt, tcnt ? ntcnt : 0, acc, pos, usage, alpha,
                      decay, replace, norms, co, readout, tally, c->small);
   EMH_HIP(hipGetLastError());

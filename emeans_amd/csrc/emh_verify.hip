@@ -8,6 +8,9 @@
 //  k_queued1   top-1 for the rows the check queues (d % 4 == 0): short
 //              (4 rows x 16 centroids) items, one burst of DMA copies and one
 //              chain per lane each, the winners folded by 64-bit atomics;
+//  k_small1    top-1 for a small direct selection against at most 64
+//              centroids (d % 4 == 0): a block holds all of them and its rows,
+//              so a row's winner is found inside a wave;
 //  k_exactk    top-k: one block per queued query over all data rows.
 //
 // Float order (the reference CPU backend, assign/fused.rs + assign.rs):
@@ -15,6 +18,8 @@
 // roundings); |x|^2 = sequential sum of rounded squares; score = dot (IP) or
 // max(|x|^2 + key, 0) (L2); ties to the lower id; a key that is NaN or +inf
 // never wins, and a row where nothing wins gets label 0 and the initial score.
+
+#include <algorithm>
 
 #include "emh_select.h"
 
@@ -460,6 +465,130 @@ __global__ __launch_bounds__(64) void k_queued1(
   }
 }
 
+// ---------------------------------------- exact top-1, at most 64 centroids
+// A block takes R = 256 / KP rows against all k <= KP centroids: four waves
+// run one chain a lane (row idx / KP, centroid idx % KP), a fifth the rows'
+// |x|^2 for L2. Bound by latency (an id, one burst of DMA copies, one chain of
+// d fmas and the LDS reads of four such waves), so whole rows come at once
+// where 128 KB of LDS hold them, in phases otherwise; LDS slots as in
+// k_queued1. A row's candidates meet inside its wave: no atomics on words in
+// memory, no tickets, no fences. k_queued1 took 17 us for 1,052 rows x 64
+// against 32 centroids (526 items of a wave, their LDS sized for any d: two
+// rounds); this takes 8.4. (One chain wave a block instead of four: 8.3 there,
+// but 30 us instead of 19 for 1,024 x 768 against 20, where every block takes
+// most of a CU's LDS.)
+constexpr int S1_W = 4, S1_T = 64 * S1_W + 64, S1_LDS = 128 * 1024;
+
+template <int KP>
+__global__ __launch_bounds__(S1_T) void k_small1(
+    const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
+    int nrows, uint32_t* __restrict__ small, const float* __restrict__ cents,
+    const float* __restrict__ cnorm, int k, int ip, int pu, uint32_t* __restrict__ labels,
+    float* __restrict__ scores, uint32_t* __restrict__ tcnt, uint32_t* __restrict__ tcounts,
+    size_t tlo, size_t tstride) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  constexpr int R = 64 * S1_W / KP;
+  extern __shared__ __attribute__((aligned(16))) v4f lds[];
+  __shared__ float xn_s[R];
+  v4f* const cs = lds;                          // pu x KP slots (pu: a multiple of 4)
+  v4f* const xs = lds + (size_t)pu * KP;        // pu x R slots, up to whole 64s
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int f0 = blockIdx.x * R;
+  // This lane's copies: row l % R, centroid l % KP.
+  const int fc = f0 + lane % R;
+  size_t xc = 0;
+  bool okc = false;
+  if (fc < nrows) {
+    const size_t p = lo + (size_t)fc;
+    const size_t id = ids ? (size_t)ids[p] : p;
+    okc = id < nx;
+    if (okc)
+      xc = id;
+    else
+      small[SW_BAD_ID] = 1;
+  }
+  const float* const crow = cents + (size_t)min(lane % KP, k - 1) * d;
+  const float* const xrow = x + xc * (size_t)d;  // row 0 where there is none
+  // This lane's chain: row r, centroid j (the last wave: row r's |x|^2).
+  const bool norm = w == S1_W;
+  const int idx = w * 64 + lane;
+  const int r = norm ? lane % R : idx / KP, j = idx % KP;
+  float acc = 0.0f;
+  for (int t0 = 0; t0 < d; t0 += 4 * pu) {
+    const int nu = min(pu, (d - t0) / 4);  // d % 4 == 0
+    for (int i = w; i < (nu * KP + 63) / 64; i += S1_W + 1)
+      __builtin_amdgcn_global_load_lds(crow + min(t0 + 4 * (i * (64 / KP) + lane / KP), d - 4),
+                                       &cs[i * 64], 16, 0, 0);
+    for (int i = w; i < (nu * R + 63) / 64; i += S1_W + 1)
+      __builtin_amdgcn_global_load_lds(xrow + min(t0 + 4 * (i * (64 / R) + lane / R), d - 4),
+                                       &xs[i * 64], 16, 0, 0);
+    __syncthreads();  // waits for the copies
+    if (!norm) {
+#pragma unroll 8
+      for (int u = 0; u < nu; u++) {
+        const v4f cv = cs[u * KP + j], v = xs[u * R + r];
+        acc = fmaf(v.x, cv.x, acc);
+        acc = fmaf(v.y, cv.y, acc);
+        acc = fmaf(v.z, cv.z, acc);
+        acc = fmaf(v.w, cv.w, acc);
+      }
+    } else if (!ip) {
+#pragma unroll 8
+      for (int u = 0; u < nu; u++) {
+        const v4f v = xs[u * R + r];
+        acc = acc + v.x * v.x;
+        acc = acc + v.y * v.y;
+        acc = acc + v.z * v.z;
+        acc = acc + v.w * v.w;
+      }
+    }
+    __syncthreads();  // the next phase's copies overwrite these slots
+  }
+  if (norm && lane < R) xn_s[lane] = acc;
+  __syncthreads();
+  const uint64_t okm = __ballot(okc);  // bit r: the block's row r is there
+  if (norm) return;
+  uint64_t best = 0;
+  if (j < k) {
+    const float key = ip ? -acc : cnorm[j] - 2.0f * acc;
+    if (key < INFINITY) best = pack_best(key, (uint32_t)j);  // NaN or +inf never wins
+  }
+#pragma unroll
+  for (int o = 1; o < KP; o <<= 1) {
+    const uint64_t b2 = __shfl_xor(best, o, WAVE);
+    best = b2 > best ? b2 : best;
+  }
+  if (j == 0 && (okm >> r & 1)) {
+    float bk = INFINITY;
+    uint32_t bid = 0;  // nothing wins: label 0 and the initial score
+    unpack_best(best, bk, bid);
+    const size_t p = lo + (size_t)(f0 + r);
+    labels[p] = bid;
+    scores[p] = ip ? -bk : fmaxf(xn_s[r] + bk, 0.0f);
+    if (tcnt) {
+      atomicAdd(&tcnt[(size_t)bid * tstride + (p - tlo) / TALLY_CP], 1u);
+      atomicAdd(&tcounts[bid], 1u);
+    }
+  }
+}
+
+template <int KP>
+void small1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
+            size_t n, const float* cents, const float* cnorm, size_t k, bool ip, uint32_t* labels,
+            float* scores, const LabelTally* tally) {
+  constexpr int R = 64 * S1_W / KP;
+  // 4-dim slots a phase: all of them where they fit.
+  const size_t most = (S1_LDS - 1024) / ((KP + R) * 16) / 4 * 4;
+  const size_t pu = std::min<size_t>((d / 4 + 3) / 4 * 4, most);
+  const size_t slots = pu * KP + (pu * R + 63) / 64 * 64;
+  hipLaunchKernelGGL(k_small1<KP>, dim3((unsigned)((n + R - 1) / R)), dim3(S1_T), slots * 16,
+                     c->stream, x, nx, (int)d, ids, lo, (int)n, c->small, cents, cnorm, (int)k,
+                     ip ? 1 : 0, (int)pu, labels, scores, tally ? tally->cnt : nullptr,
+                     tally ? tally->counts : nullptr, tally ? tally->lo : 0,
+                     tally ? tally->stride : 0);
+  EMH_HIP(hipGetLastError());
+}
+
 // ------------------------------------------------------------- exact top-k
 // One workgroup per queued query: each thread keeps the kk best of its strided
 // share (j increasing, replace the worst only when strictly better, as
@@ -591,12 +720,12 @@ size_t queued_items(size_t n, size_t k, bool ip) {
 
 size_t exact1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool list) {
   auto r = [](size_t b) { return (b + 255) & ~size_t(255); };
-  if ((list && d % 4 == 0) || (!list && queued_direct(c, n, d, k, ip))) {
-    const size_t ngr = (n + QR - 1) / QR;
-    return r(n * 8 + ngr * 4) + r(n * 4);
-  }
+  const size_t ngq = (n + QR - 1) / QR, queued = r(n * 8 + ngq * 4) + r(n * 4);
+  if (list && d % 4 == 0) return queued;
   const size_t nch = (k + CJ - 1) / CJ, ngr = (n + RG - 1) / RG;
-  return r(n * nch * sizeof(Cand)) + r(ngr * 4);
+  const size_t exact = r(n * nch * sizeof(Cand)) + r(ngr * 4);
+  if (list || !queued_direct(c, n, d, k, ip)) return exact;
+  return std::max(queued, exact);  // (by the buffers' alignment)
 }
 
 void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
@@ -608,10 +737,19 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
              "exact: a tally needs the queued-row scan");
   // Both kernels read row 0 in place of a row whose id is out of range.
   EMH_ENSURE(nx > 0, "top1: a selection of %zu rows over no data rows", n);
+  // (Its copies take 16 bytes: a wrapped buffer may start anywhere.)
+  const bool aligned = (((uintptr_t)x | (uintptr_t)cents) & 15) == 0;
+  if (!list && aligned && small_direct(c, n, d, k)) {
+    auto f = k <= 16 ? small1<16> : k <= 32 ? small1<32> : small1<64>;
+    f(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, labels, scores, tally);
+    return;
+  }
   // Queued rows (few), or a small direct selection: the latency-bound scan.
   // (k_exact1's tiles each wait a memory round trip: ~30 us at any size up
   // to a few thousand rows.)
-  if ((list && d % 4 == 0) || (!list && queued_direct(c, n, d, k, ip))) {
+  if ((list && d % 4 == 0) ||
+      (!list && queued_direct(c, n, d, k, ip) &&
+       (tally || queued_items(n, k, ip) <= QUEUED_DIRECT))) {
     const size_t ngr = (n + QR - 1) / QR;
     const size_t per = (k + QJ - 1) / QJ + (ip ? 0 : 1);
     // Self-cleaning: the best words, then the tickets, all left at zero (a
