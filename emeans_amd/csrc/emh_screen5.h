@@ -78,6 +78,7 @@ enum Kind5 : int {
   TOP1_L2 = 1,   // top-1: key |c|^2 - 2 dot
   KNN = 2,       // top-k, key -dot
   KNN_SELF = 3,  // ... of the rows themselves, each row's own column left out
+  SCORES = 4,    // no lists: every dot to memory (emh_topk_long.hip)
 };
 constexpr int KTH5 = KMAX;  // kNN: the smallest keys a thread keeps for its row's limit
 constexpr int CAP5 = 12;    // slots of a row's append buffer (each of its two centroid waves)
@@ -105,6 +106,8 @@ struct Args5 {
   int nparts;
   const float* sx;        // scales: s, 1 / s
   const float* sc;
+  float* scores;          // SCORES: out, row r's dots at r ldS (a multiple of 4, >= k)
+  size_t ldS;
 };
 
 // ONE: parts of one tile (its lists never leave LDS).
@@ -112,6 +115,7 @@ template <int KIND, bool ONE>
 __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   constexpr bool L2 = KIND == TOP1_L2, SELF = KIND == KNN_SELF;
   constexpr bool TOPK = KIND == KNN || KIND == KNN_SELF;
+  constexpr bool LISTS = KIND != SCORES;
   constexpr int L = TOPK ? LK : L5, NK = TOPK ? KTH5 : 1, CAP = CAP5;
   constexpr int LOG = TOPK ? LOG5_KNN : LOG5_TOP1;
   constexpr int WA = 4, WN = 2;  // centroid (A) and row (B) 32-blocks per wave
@@ -120,7 +124,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   __shared__ __attribute__((aligned(1024))) char ring[NS5 * S5_STAGE];
   __shared__ __attribute__((aligned(16))) float Ns[L2 ? NN5 : 1][L2 ? T5 : 4];  // tile norms, by tile % NN5
   // Append buffers: slot e of wave w's row r (0 .. 63) at (w CAP + e) 64 + r.
-  __shared__ uint32_t buf[8 * CAP * 64];
+  __shared__ uint32_t buf[LISTS ? 8 * CAP * 64 : 1];
   // What the two centroid waves of a row publish for each other's limits
   // (see set_limit): a read that races a write takes either value, both valid.
   __shared__ float pub[2][TOPK ? 2 : 1][T5];
@@ -481,6 +485,27 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     publish();
   };
 
+  // SCORES: a lane's four consecutive columns of its row are 16 bytes, and the
+  // block's four such stores a row fill a 128-byte line in L2.
+  auto store = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < WN; y++) {
+      const int r = row0 + wr * 64 + y * 32 + li;
+      if (r >= nrows) continue;
+      float* o = a_.scores + (size_t)r * a_.ldS;
+#pragma unroll
+      for (int a = 0; a < WA; a++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const size_t col = (size_t)tile * T5 + wc * 128 + a * 32 + 8 * q + 4 * h;
+          if (col < a_.ldS)
+            *reinterpret_cast<float4*>(o + col) =
+                make_float4(f1 * acc[a][y][4 * q], f1 * acc[a][y][4 * q + 1],
+                            f1 * acc[a][y][4 * q + 2], f1 * acc[a][y][4 * q + 3]);
+        }
+    }
+  };
+
   // Prologue: steps 0 .. NS5 - 1 into their stages; step 0's first operands.
   for (int i = tid; i < 2 * (TOPK ? 2 : 1) * T5; i += 512) (&pub[0][0][0])[i] = INFINITY;
 #pragma unroll
@@ -555,7 +580,10 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     st = nx;
     cj++;
     if (last) {
-      fold(ct);
+      if constexpr (LISTS)
+        fold(ct);
+      else
+        store(ct);
       cj = 0;
       ++ct;
       read_rows(st, 0, r0);
@@ -564,6 +592,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     }
   }
   wait_vm<0>();  // the DMAs past the last step have landed (the output reuses the stages)
+  if constexpr (!LISTS) return;
 
   // The rows' candidates: of the two threads' logs (ONE: buffers), what lies
   // within the final limit, into [row][part][L]. Top-1: the length and that

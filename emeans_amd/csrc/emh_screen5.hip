@@ -272,14 +272,14 @@ bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d) {
          m < (1u << 25) && n < (1u << 25);
 }
 
-int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                size_t kk, bool exclude_self, Cand** cand_out, float** bound_out) {
+void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
+            uint32_t* clear, int nclear, Split5* s) {
   // The data's lines once (with their norms, residuals and the maxima of
   // both); the queries' too, unless they are the data.
   const bool same = q == data && m == n;
   float* sc = c->scales + 2 * SCALE_CENTS;
   float* sx = same ? sc : c->scales + 2 * SCALE_ROWS;
-  launch_scales(c, data, n * d, sc, same ? nullptr : q, m * d, sx, c->small, 3);
+  launch_scales(c, data, n * d, sc, same ? nullptr : q, m * d, sx, clear, nclear);
   void* xs = c->csplit.get(lines_bytes(n, d));
   float2* xn = (float2*)c->csplit_norm.get(n * 8);
   // Past PART_MAX_ONCE partials, one workgroup reduces them ahead of the
@@ -287,21 +287,33 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   const size_t hb = lines_blocks(n);
   uint32_t* part = (uint32_t*)c->csplit_part.get((hb + 1) * 16);
   launch_lines(c, data, n, d, nullptr, 0, n, sc, xs, xn, nullptr, part);
-  int nparts = (int)hb;
+  s->part = part;
+  s->nparts = (int)hb;
   if (hb > PART_MAX_ONCE) {
     launch_part_max4(c, part, hb, part + 4 * hb);
-    part += 4 * hb;
-    nparts = 1;
+    s->part = part + 4 * hb;
+    s->nparts = 1;
   }
-  const void* qs = xs;
-  const float2* qn = xn;
+  s->cs = s->xs = xs;
+  s->xn = xn;
   if (!same) {
     void* qw = c->xsplit.get(lines_bytes(m, d));
     float2* qnw = (float2*)c->xsplit_norm.get(m * 8);
     launch_lines(c, q, m, d, nullptr, 0, m, sx, qw, qnw, nullptr, nullptr);
-    qs = qw;
-    qn = qnw;
+    s->xs = qw;
+    s->xn = qnw;
   }
+  s->sx = sx;
+  s->sc = sc;
+  s->m = m;
+  s->n = n;
+  s->d = d;
+}
+
+int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
+                size_t kk, bool exclude_self, Cand** cand_out, float** bound_out) {
+  Split5 s;
+  split5(c, q, m, data, n, d, c->small, 3, &s);
   const int row_tiles = (int)((m + T5 - 1) / T5);
   const int ntiles = (int)((n + T5 - 1) / T5);
   // Parts (data-tile ranges) where they fill waves of blocks better: up to
@@ -319,7 +331,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
                                  sizeof(Cand));
   Args5 a{};
   a.xslab = m * (size_t)LINE_BYTES;
-  a.cs = (const char*)xs;
+  a.cs = (const char*)s.cs;
   a.cslab = n * (size_t)LINE_BYTES;
   a.k = (int)n;
   a.d = (int)d;
@@ -329,14 +341,14 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   a.ntiles = ntiles;
   a.log = log;
   a.bstride = m;
-  a.part = part;
-  a.nparts = nparts;
-  a.sx = sx;
-  a.sc = sc;
+  a.part = s.part;
+  a.nparts = s.nparts;
+  a.sx = s.sx;
+  a.sc = s.sc;
   ProfScope prof(c, EMH_PROF_SCREEN, 2.0 * (double)m * (double)n * (double)d,
                  prof_take(c, EMH_PROF_SCREEN));
-  a.xs = (const char*)qs;
-  a.xn = qn;
+  a.xs = (const char*)s.xs;
+  a.xn = s.xn;
   a.nx = m;
   for (int r = 0; r < row_tiles; r += rt_step) {
     const size_t q0 = (size_t)r * T5, q1 = std::min((size_t)(r + rt_step) * T5, m);
@@ -353,6 +365,38 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   *cand_out = cand;
   *bound_out = bound;
   return parts;
+}
+
+void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* scores, size_t ldS,
+                    float* bound) {
+  EMH_ENSURE(s.m < (1u << 25) && s.n < (1u << 25) && ldS % 4 == 0 && ldS >= s.n && q0 + nb <= s.m,
+             "scores: shape out of range");
+  const int row_tiles = (int)((nb + T5 - 1) / T5), ntiles = (int)((s.n + T5 - 1) / T5);
+  const int parts0 = parts5(row_tiles, ntiles, std::max(c->cus, 1), 1024, 0.5);
+  Args5 a{};
+  a.xs = (const char*)s.xs;
+  a.xslab = s.m * (size_t)LINE_BYTES;
+  a.xn = s.xn;
+  a.nx = s.m;
+  a.lo = q0;
+  a.nrows = (int)nb;
+  a.cs = (const char*)s.cs;
+  a.cslab = s.n * (size_t)LINE_BYTES;
+  a.k = (int)s.n;
+  a.d = (int)s.d;
+  a.kk = 1;
+  a.tpp = (ntiles + parts0 - 1) / parts0;
+  a.parts = (ntiles + a.tpp - 1) / a.tpp;
+  a.ntiles = ntiles;
+  a.bound = bound;
+  a.bstride = nb;
+  a.part = s.part;
+  a.nparts = s.nparts;
+  a.sx = s.sx;
+  a.sc = s.sc;
+  a.scores = scores;
+  a.ldS = ldS;
+  launch5<SCORES, false>(c, (unsigned)(row_tiles * a.parts), a);
 }
 
 }  // namespace emh

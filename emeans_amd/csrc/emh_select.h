@@ -226,6 +226,25 @@ inline int parts5(int row_tiles, int ntiles, int cus, int maxp, double fixed) {
   }
   return best;
 }
+// The lines of m queries and n data rows in the context's scratch (the queries'
+// are the data's when they are the same rows), with the data's maxima in part;
+// clears nclear words of clear on the way.
+struct Split5 {
+  const void *xs, *cs;
+  const float2* xn;
+  const uint32_t* part;
+  int nparts;
+  const float *sx, *sc;
+  size_t m, n, d;
+};
+void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
+            uint32_t* clear, int nclear, Split5* s);
+// Every dot of queries q0 .. q0 + nb with the data, as the one-pass screen sees
+// them, into scores (row r at r ldS; the ldS - n columns past the data hold
+// anything), and the bound E on their distance from the exact chains into
+// bound[0 .. nb) (its dot term in bound[nb ..)).
+void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* scores, size_t ldS,
+                    float* bound);
 // The one-pass kNN screen (emh_screen5.hip): whether it takes a call, and the
 // call's screen (candidate lists [m][parts][LK]; the queries' E at bound[r]
 // and its dot term at bound[m + r]; in the context's scratch); returns the parts.

@@ -7,6 +7,10 @@
 //  - k_dots: the exact dots of a block of queries against every data row,
 //    each the sequential f32 fma chain over the d dimensions (the float order
 //    of every other score in this library), into scratch;
+//  - or, where queries and data rows make it pay, the same dots on the MFMA
+//    within a bound (k_screen5's SCORES), from which k_select_screened lists
+//    every row that can be among the kk best and computes those rows' chains
+//    alone; queries that it cannot settle go through the next two;
 //  - k_select_long: one workgroup per query keeps the kk best data rows by a
 //    radix select over the scores (larger score first, the lower id among
 //    equal scores: the rows the reference keeps by replacing its worst entry
@@ -34,10 +38,12 @@ namespace {
 // the data, and by what is padded).
 constexpr int DK = 16;
 
-template <int BM, int BN, int TM, int TN>
+// LIST: of queries list[1 .. list[0]] (rows of S too) instead, at most qb.
+template <int BM, int BN, int TM, int TN, bool LIST>
 __global__ __launch_bounds__(256) void k_dots(const float* __restrict__ q, size_t q0, int qb,
                                               const float* __restrict__ x, int n, int d,
-                                              float* __restrict__ S, size_t ldS) {
+                                              float* __restrict__ S, size_t ldS,
+                                              const uint32_t* __restrict__ list) {
   static_assert((BM / TM) * (BN / TN) == 256, "threads");
   constexpr int QP = BM + 4, XP = BN + 4;  // padded: the transposed stores spread over the banks
   constexpr int NTX = BN / TN;             // threads along the data rows
@@ -48,13 +54,18 @@ __global__ __launch_bounds__(256) void k_dots(const float* __restrict__ q, size_
   __shared__ __attribute__((aligned(16))) float Xs[2][DK][XP];
   const int tid = threadIdx.x, tx = tid % NTX, ty = tid / NTX;
   const int j0 = blockIdx.x * BN, i0 = blockIdx.y * BM;
+  if (LIST) {
+    qb = min(qb, (int)list[0]);
+    if (i0 >= qb) return;
+  }
+  auto qrow = [&](int i) { return LIST ? (int)list[1 + i] : i; };
   // Loader: float4 e of an operand's slab is row e / 4, dimensions 4 (e % 4) .. + 3.
   float qr[LQ][4], xr[LX][4];
   auto load = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < LQ; u++) {
       const int e = u * 256 + tid, r = e >> 2, t = t0 + 4 * (e & 3);
-      const float* p = q + (q0 + (size_t)min(i0 + min(r, BM - 1), qb - 1)) * (size_t)d;
+      const float* p = q + (q0 + (size_t)qrow(min(i0 + min(r, BM - 1), qb - 1))) * (size_t)d;
 #pragma unroll
       for (int c = 0; c < 4; c++) qr[u][c] = t + c < d ? p[t + c] : 0.f;
     }
@@ -120,7 +131,7 @@ __global__ __launch_bounds__(256) void k_dots(const float* __restrict__ q, size_
   for (int a = 0; a < TM; a++) {
     const int i = i0 + ty * TM + a;
     if (i >= qb) break;
-    float* o = S + (size_t)i * ldS;
+    float* o = S + (size_t)qrow(i) * ldS;
 #pragma unroll
     for (int g = 0; g < GN; g++)
 #pragma unroll
@@ -133,10 +144,14 @@ __global__ __launch_bounds__(256) void k_dots(const float* __restrict__ q, size_
 
 template <int BM, int BN, int TM, int TN>
 void dots(emh_ctx* c, const float* q, size_t q0, size_t nb, const float* data, size_t n, size_t d,
-          float* S, size_t ldS) {
+          float* S, size_t ldS, const uint32_t* list = nullptr) {
   const dim3 g((unsigned)((n + BN - 1) / BN), (unsigned)((nb + BM - 1) / BM));
-  hipLaunchKernelGGL((k_dots<BM, BN, TM, TN>), g, dim3(256), 0, c->stream, q, q0, (int)nb, data,
-                     (int)n, (int)d, S, ldS);
+  if (list)
+    hipLaunchKernelGGL((k_dots<BM, BN, TM, TN, true>), g, dim3(256), 0, c->stream, q, q0, (int)nb,
+                       data, (int)n, (int)d, S, ldS, list);
+  else
+    hipLaunchKernelGGL((k_dots<BM, BN, TM, TN, false>), g, dim3(256), 0, c->stream, q, q0, (int)nb,
+                       data, (int)n, (int)d, S, ldS, list);
   EMH_HIP(hipGetLastError());
 }
 
@@ -205,21 +220,186 @@ __device__ __forceinline__ void sort_keys(unsigned long long* sk, uint32_t cnt) 
   }
 }
 
+// The largest x that kk of the threads' values `mine` are not below (0: fewer
+// than kk are above 0).
+__device__ __forceinline__ uint32_t kth_of_threads(uint32_t mine, int kk) {
+  uint32_t x = 0u;
+  for (int b = 31; b >= 0; b--)
+    if (__syncthreads_count(mine >= (x | (1u << b))) >= kk) x |= 1u << b;
+  return x;
+}
+
+// sk[0 .. got) = (~key, id) of listed scores, any order: sorted, cut to the kk
+// best, and those given their own order (IEEE total order, then id) as keys.
+// Returns how many.
+template <int P>
+__device__ __forceinline__ uint32_t best_of_listed(unsigned long long* sk, uint32_t got, int kk,
+                                                   const float* row) {
+  sort_keys<P>(sk, got);
+  const uint32_t cnt = min(got, (uint32_t)kk);
+  for (uint32_t s = threadIdx.x; s < cnt; s += NT) {
+    const uint32_t j = (uint32_t)sk[s];
+    sk[s] = ((unsigned long long)(~ord_total(row[j])) << 32) | (unsigned long long)j;
+  }
+  __syncthreads();
+  return cnt;
+}
+
+// The sorted result of a query.
+__device__ __forceinline__ void put_result(const unsigned long long* sk, uint32_t cnt, size_t qi,
+                                           int kk, uint32_t* __restrict__ ids,
+                                           float* __restrict__ sims) {
+  for (int t = threadIdx.x; t < kk; t += NT) {
+    const size_t o = qi * (size_t)kk + t;
+    if ((uint32_t)t < cnt) {
+      const unsigned long long e = sk[t];
+      ids[o] = (uint32_t)e;
+      sims[o] = from_ord(~(uint32_t)(e >> 32));
+    } else {
+      ids[o] = NONE;
+      sims[o] = -INFINITY;
+    }
+  }
+}
+
+// Workgroup i: the kk best data rows of query q0 + i from its screen scores
+// S[i ldS ..], each within bound[i] = E of its exact chain. kk of the scores
+// are not below the kk-th largest x of the threads' maxima, so kk exact ones
+// are not below x - E, and a row whose score is below x - 2E is not among the
+// kk best: the others, listed in sk, get their exact chains (into S) and the
+// selection takes it from there. A query with a bound that is not a small
+// number (NaN; 1e32 keeps every chain finite), with fewer than kk candidates
+// or more than KLONG goes to list[1 + list[0]++]. kk <= NT / 2.
+//
+// Bound by its two reads of the scores and the latency of the listed rows'
+// loads: a lane runs one candidate's chain, eight loads ahead, the candidates
+// spread over the waves. 1,000 x 50,000 x 384, k = 100, whole calls: 929 us
+// with every chain computed (k_dots' share is bound by the VALU at 48
+// TFLOP/s), 362 us with the screen's scores.
+template <bool VEC4>
+__global__ __launch_bounds__(NT) void k_select_screened(
+    float* __restrict__ S, size_t ldS, int n, int d, const float* __restrict__ q, size_t q0,
+    const float* __restrict__ x, const float* __restrict__ bound, int kk, int exclude_self,
+    uint32_t* __restrict__ ids, float* __restrict__ sims, uint32_t* __restrict__ list) {
+  constexpr int P = KLONG;  // (32 KB: two workgroups a CU all the same)
+  __shared__ unsigned long long sk[P];
+  __shared__ uint32_t sh_n;
+  const int tid = threadIdx.x;
+  const size_t qi = q0 + blockIdx.x;
+  float* row = S + (size_t)blockIdx.x * ldS;
+  const float E = bound[blockIdx.x];
+  auto give_up = [&]() {
+    if (tid == 0) list[1 + atomicAdd(&list[0], 1u)] = blockIdx.x;
+  };
+  if (!(E < 1e32f)) {  // (uniform)
+    give_up();
+    return;
+  }
+  // Scores four at a time (a row starts at a multiple of 16 bytes and its
+  // padding up to ldS is readable).
+  auto load4 = [&](int j, uint32_t (&k4)[4]) __attribute__((always_inline)) {
+    const float4 v = *reinterpret_cast<const float4*>(row + j);
+    const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      k4[t] = j + t < n ? sel_key(e[t], exclude_self && (size_t)(j + t) == qi) : 0u;
+  };
+  uint32_t mine = 0u;
+  for (int j0 = 4 * tid; j0 < n; j0 += 16 * NT) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      uint32_t k4[4];
+      if (j0 + 4 * u * NT < n) {
+        load4(j0 + 4 * u * NT, k4);
+        mine = max(max(mine, max(k4[0], k4[1])), max(k4[2], k4[3]));
+      }
+    }
+  }
+  if (tid == 0) sh_n = 0u;
+  const uint32_t xk = kth_of_threads(mine, kk);
+  if (xk == 0u) {
+    give_up();
+    return;
+  }
+  const float xv = from_ord(xk);
+  const float lim = xv - 2.0157f * E - fabsf(xv) * 4.7683716e-07f - 1e-42f;
+  const uint32_t lk = sel_key(lim, false);  // (lim is finite)
+  for (int j0 = 4 * tid; j0 < n; j0 += 16 * NT) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      uint32_t k4[4];
+      const int j = j0 + 4 * u * NT;
+      if (j < n) {
+        load4(j, k4);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+          if (k4[t] >= lk) {
+            const uint32_t at = atomicAdd(&sh_n, 1u);
+            if (at < (uint32_t)P) sk[at] = (unsigned long long)(uint32_t)(j + t);
+          }
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t got = sh_n;
+  if (got > (uint32_t)P || got < (uint32_t)kk) {
+    give_up();
+    return;
+  }
+  const float* qr = q + qi * (size_t)d;
+  for (uint32_t s = (uint32_t)((tid & 63) * NW + (tid >> 6)); s < got; s += NT) {
+    const uint32_t j = (uint32_t)sk[s];
+    const float* p = x + (size_t)j * (size_t)d;
+    float acc = 0.f;
+    int t = 0;
+    for (; t + 32 <= d; t += 32) {
+      float v[32];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        if (VEC4) {
+          const float4 f = *reinterpret_cast<const float4*>(p + t + 4 * e);
+          v[4 * e] = f.x;
+          v[4 * e + 1] = f.y;
+          v[4 * e + 2] = f.z;
+          v[4 * e + 3] = f.w;
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; c++) v[4 * e + c] = p[t + 4 * e + c];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 32; e++) acc = fmaf(qr[t + e], v[e], acc);
+    }
+    for (; t < d; t++) acc = fmaf(qr[t], p[t], acc);
+    row[j] = acc;
+    // Key first (-0 and +0 alike, as the selection compares them), then id.
+    sk[s] = ((unsigned long long)(~sel_key(acc, false)) << 32) | (unsigned long long)j;
+  }
+  __syncthreads();
+  const uint32_t cnt = best_of_listed<P>(sk, got, kk, row);
+  sort_keys<P>(sk, cnt);
+  put_result(sk, cnt, qi, kk, ids, sims);
+}
+
 // Workgroup i: the kk best data rows of query q0 + i from its scores
 // S[i ldS ..], written to ids / sims row q0 + i. P (a power of two >= kk)
-// slots of sort keys in LDS.
+// slots of sort keys in LDS. With list, i = list[1 + workgroup] for the first
+// list[0] of them.
 template <int P>
 __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S, size_t ldS,
                                                     int n, size_t q0, int kk, int exclude_self,
                                                     uint32_t* __restrict__ ids,
-                                                    float* __restrict__ sims) {
+                                                    float* __restrict__ sims,
+                                                    const uint32_t* __restrict__ list) {
+  if (list && blockIdx.x >= list[0]) return;
   __shared__ unsigned long long sk[P];
   __shared__ uint32_t hist[2048];
   __shared__ int wsum[NW];
   __shared__ uint32_t sh_prefix, sh_rem, sh_all;
   const int tid = threadIdx.x;
-  const size_t qi = q0 + blockIdx.x;
-  const float* row = S + (size_t)blockIdx.x * ldS;
+  const size_t bi = list ? list[1 + blockIdx.x] : blockIdx.x;
+  const size_t qi = q0 + bi;
+  const float* row = S + bi * ldS;
   auto key_at = [&](int j) { return sel_key(row[j], exclude_self && (size_t)j == qi); };
 
   uint32_t cnt = 0;
@@ -238,9 +418,7 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
 #pragma unroll
       for (int u = 0; u < 8; u++) mine = max(mine, k8[u]);
     }
-    uint32_t x = 0u;  // the largest x with kk maxima not below it
-    for (int b = 31; b >= 0; b--)
-      if (__syncthreads_count(mine >= (x | (1u << b))) >= kk) x |= 1u << b;
+    const uint32_t x = kth_of_threads(mine, kk);
     if (tid == 0) sh_all = 0u;
     __syncthreads();
     for (int j0 = tid; j0 < n; j0 += 8 * NT) {
@@ -260,18 +438,7 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
     const uint32_t got = sh_all;
     __syncthreads();
     listed = got <= (uint32_t)P;
-    if (listed) {
-      sort_keys<P>(sk, got);
-      // The kk best; then their own order: IEEE total order, then id.
-      cnt = min(got, (uint32_t)kk);
-      for (uint32_t s = tid; s < (uint32_t)P; s += NT) {
-        if (s < cnt) {
-          const uint32_t j = (uint32_t)sk[s];
-          sk[s] = ((unsigned long long)(~ord_total(row[j])) << 32) | (unsigned long long)j;
-        }
-      }
-      __syncthreads();
-    }
+    if (listed) cnt = best_of_listed<P>(sk, got, kk, row);
   }
   if (!listed) {
   // Radix select of the kk-th largest key: digits of 11, 11 and 10 bits.
@@ -353,25 +520,39 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
   cnt = all ? got_gt : (uint32_t)kk;
   }
   sort_keys<P>(sk, cnt);
-  for (int t = tid; t < kk; t += NT) {
-    const size_t o = qi * (size_t)kk + t;
-    if ((uint32_t)t < cnt) {
-      const unsigned long long e = sk[t];
-      ids[o] = (uint32_t)e;
-      sims[o] = from_ord(~(uint32_t)(e >> 32));
-    } else {
-      ids[o] = NONE;
-      sims[o] = -INFINITY;
-    }
-  }
+  put_result(sk, cnt, qi, kk, ids, sims);
 }
 
 template <int P>
 void select_long(emh_ctx* c, unsigned blocks, const float* S, size_t ldS, size_t n, size_t q0,
-                 size_t kk, bool exclude_self, uint32_t* ids, float* sims) {
+                 size_t kk, bool exclude_self, uint32_t* ids, float* sims,
+                 const uint32_t* list = nullptr) {
   hipLaunchKernelGGL(k_select_long<P>, dim3(blocks), dim3(NT), 0, c->stream, S, ldS, (int)n, q0,
-                     (int)kk, exclude_self ? 1 : 0, ids, sims);
+                     (int)kk, exclude_self ? 1 : 0, ids, sims, list);
   EMH_HIP(hipGetLastError());
+}
+
+void select_screened(emh_ctx* c, unsigned blocks, float* S, size_t ldS, size_t n, size_t d,
+                     const float* q, size_t q0, const float* data, const float* bound, size_t kk,
+                     bool exclude_self, uint32_t* ids, float* sims, uint32_t* list) {
+  auto kern = d % 4 == 0 ? k_select_screened<true> : k_select_screened<false>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, c->stream, S, ldS, (int)n, (int)d, q, q0,
+                     data, bound, (int)kk, exclude_self ? 1 : 0, ids, sims, list);
+  EMH_HIP(hipGetLastError());
+}
+
+// Whether the screened selection takes a call. Splitting the data into lines,
+// the scores' launch and the (mostly empty) launches over the list cost about
+// 45 us, and the chains of the listed rows grow with kk and not with n: below
+// 10^9 products (us, direct / screened: 20,000 x 64 by 256 queries, k = 100: 70
+// / 75; 8,192 x 768 by 64: 106 / 104; above: 20,000 x 64 by 1,000: 212 / 179),
+// with fewer than 32 rows a neighbour (8,192 x 768 by 1,000, k = 500: 388 /
+// 471; 20,000 x 384, k = 500: 497 / 371) and for fewer than 16 queries (which
+// read the data once, with nothing written) the direct dots stay.
+bool long_screened(emh_ctx* c, size_t m, size_t n, size_t d, size_t kk) {
+  return c->screen != SCREEN_OFF && c->screen != SCREEN_F32 && kk <= NT / 2 && d >= 32 &&
+         d <= 16384 && m >= 16 && m < (1u << 25) && n >= 32 * kk && n < (1u << 25) &&
+         (double)m * (double)n * (double)d >= 1e9;
 }
 
 }  // namespace
@@ -415,24 +596,40 @@ void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, s
   size_t qb = std::max<size_t>(budget / (ldS * 4) / DT * DT, DT);
   qb = std::min(std::min(qb, size_t(65535) * DT), m);  // grid.y of k_dots within 65535
   float* S = (float*)c->klong.get(qb * ldS * 4);
+  const bool screened = long_screened(c, m, n, d, kk);
+  Split5 sp{};
+  uint32_t* list = nullptr;
+  float* bound = nullptr;
+  if (screened) {
+    list = (uint32_t*)c->fblist.get((qb + 1) * 4);
+    bound = (float*)c->xnorm.get(2 * qb * 4);
+    split5(c, q, m, data, n, d, list, 1, &sp);
+  }
   for (size_t q0 = 0; q0 < m; q0 += qb) {
     const size_t nb = std::min(qb, m - q0);
+    if (screened) {
+      if (q0 > 0) launch_fill_u32(c, list, 1, 0);
+      launch_scores5(c, sp, q0, nb, S, ldS, bound);
+      select_screened(c, (unsigned)nb, S, ldS, n, d, q, q0, data, bound, kk, exclude_self, ids,
+                      sims, list);
+    }
+    // (Screened: what is left in the list, by the same kernels.)
     if (n > 0) {
       // Tiles by the queries there are; the wide one also needs data rows for
       // two blocks a CU.
       const size_t wide = (nb + 127) / 128 * ((n + 127) / 128);
       if (nb <= 8)
-        dots<8, 256, 4, 2>(c, q, q0, nb, data, n, d, S, ldS);
+        dots<8, 256, 4, 2>(c, q, q0, nb, data, n, d, S, ldS, list);
       else if (nb <= 64 || wide < 2 * (size_t)c->cus)
-        dots<32, 128, 4, 4>(c, q, q0, nb, data, n, d, S, ldS);
+        dots<32, 128, 4, 4>(c, q, q0, nb, data, n, d, S, ldS, list);
       else
-        dots<128, 128, 8, 8>(c, q, q0, nb, data, n, d, S, ldS);
+        dots<128, 128, 8, 8>(c, q, q0, nb, data, n, d, S, ldS, list);
     }
     const unsigned blocks = (unsigned)nb;
     if (kk <= 128)
-      select_long<1024>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
+      select_long<1024>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims, list);
     else
-      select_long<KLONG>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims);
+      select_long<KLONG>(c, blocks, S, ldS, n, q0, kk, exclude_self, ids, sims, list);
   }
 }
 
