@@ -194,18 +194,18 @@ __device__ __forceinline__ int block_rank(bool f, int* wsum, int& total) {
 }
 
 // Bitonic sort of sk[0 .. cnt) (P slots, the rest filled), ascending.
-template <int P>
+template <int P, int T = NT>
 __device__ __forceinline__ void sort_keys(unsigned long long* sk, uint32_t cnt) {
   const int tid = threadIdx.x;
   // (A power of two that holds them: short lists skip the wide stages.)
   int m = 2;
   while (m < (int)cnt) m <<= 1;
-  for (int s = tid; s < m; s += NT)
+  for (int s = tid; s < m; s += T)
     if ((uint32_t)s >= cnt) sk[s] = ~0ull;
   __syncthreads();
   for (int size = 2; size <= m; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = tid; t < m / 2; t += NT) {
+      for (int t = tid; t < m / 2; t += T) {
         const int lo = 2 * t - (t & (stride - 1));
         const int hi = lo + stride;
         const bool up = (lo & size) == 0;
@@ -232,12 +232,12 @@ __device__ __forceinline__ uint32_t kth_of_threads(uint32_t mine, int kk) {
 // sk[0 .. got) = (~key, id) of listed scores, any order: sorted, cut to the kk
 // best, and those given their own order (IEEE total order, then id) as keys.
 // Returns how many.
-template <int P>
+template <int P, int T = NT>
 __device__ __forceinline__ uint32_t best_of_listed(unsigned long long* sk, uint32_t got, int kk,
                                                    const float* row) {
-  sort_keys<P>(sk, got);
+  sort_keys<P, T>(sk, got);
   const uint32_t cnt = min(got, (uint32_t)kk);
-  for (uint32_t s = threadIdx.x; s < cnt; s += NT) {
+  for (uint32_t s = threadIdx.x; s < cnt; s += T) {
     const uint32_t j = (uint32_t)sk[s];
     sk[s] = ((unsigned long long)(~ord_total(row[j])) << 32) | (unsigned long long)j;
   }
@@ -246,10 +246,11 @@ __device__ __forceinline__ uint32_t best_of_listed(unsigned long long* sk, uint3
 }
 
 // The sorted result of a query.
+template <int T = NT>
 __device__ __forceinline__ void put_result(const unsigned long long* sk, uint32_t cnt, size_t qi,
                                            int kk, uint32_t* __restrict__ ids,
                                            float* __restrict__ sims) {
-  for (int t = threadIdx.x; t < kk; t += NT) {
+  for (int t = threadIdx.x; t < kk; t += T) {
     const size_t o = qi * (size_t)kk + t;
     if ((uint32_t)t < cnt) {
       const unsigned long long e = sk[t];
@@ -264,26 +265,31 @@ __device__ __forceinline__ void put_result(const unsigned long long* sk, uint32_
 
 // Workgroup i: the kk best data rows of query q0 + i from its screen scores
 // S[i ldS ..], each within bound[i] = E of its exact chain. kk of the scores
-// are not below the kk-th largest x of the threads' maxima, so kk exact ones
+// are not below the kk-th largest x of the threads' maxima (two a thread), so kk exact ones
 // are not below x - E, and a row whose score is below x - 2E is not among the
 // kk best: the others, listed in sk, get their exact chains (into S) and the
 // selection takes it from there. A query with a bound that is not a small
 // number (NaN; 1e32 keeps every chain finite), with fewer than kk candidates
-// or more than KLONG goes to list[1 + list[0]++]. kk <= NT / 2.
+// or more than KLONG goes to list[1 + list[0]++]. kk <= ST.
 //
 // Bound by its two reads of the scores and the latency of the listed rows'
 // loads: a lane runs one candidate's chain, eight loads ahead, the candidates
 // spread over the waves. 1,000 x 50,000 x 384, k = 100, whole calls: 929 us
 // with every chain computed (k_dots' share is bound by the VALU at 48
-// TFLOP/s), 362 us with the screen's scores.
+// TFLOP/s), 362 us with the screen's scores, 266 us since the workgroup has 512
+// threads (four a CU, so that one's loads cover another's chains: 1,024 of
+// them made two waves of two a CU), one wave finds x by ballots and short lists
+// are ranked instead of sorted (this kernel: 249 -> 147 us).
+constexpr int ST = 512;  // threads of k_select_screened
 template <bool VEC4>
-__global__ __launch_bounds__(NT) void k_select_screened(
+__global__ __launch_bounds__(ST) void k_select_screened(
     float* __restrict__ S, size_t ldS, int n, int d, const float* __restrict__ q, size_t q0,
     const float* __restrict__ x, const float* __restrict__ bound, int kk, int exclude_self,
     uint32_t* __restrict__ ids, float* __restrict__ sims, uint32_t* __restrict__ list) {
-  constexpr int P = KLONG;  // (32 KB: two workgroups a CU all the same)
+  constexpr int P = KLONG;  // (32 KB: four workgroups a CU all the same)
   __shared__ unsigned long long sk[P];
-  __shared__ uint32_t sh_n;
+  __shared__ uint32_t sh_n, sh_x;
+  uint32_t* mx = (uint32_t*)sk;  // the 2 ST maxima, until the list starts
   const int tid = threadIdx.x;
   const size_t qi = q0 + blockIdx.x;
   float* row = S + (size_t)blockIdx.x * ldS;
@@ -304,19 +310,37 @@ __global__ __launch_bounds__(NT) void k_select_screened(
     for (int t = 0; t < 4; t++)
       k4[t] = j + t < n ? sel_key(e[t], exclude_self && (size_t)(j + t) == qi) : 0u;
   };
-  uint32_t mine = 0u;
-  for (int j0 = 4 * tid; j0 < n; j0 += 16 * NT) {
+  uint32_t mine[2] = {0u, 0u};
+  for (int j0 = 4 * tid; j0 < n; j0 += 32 * ST) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < 8; u++) {
       uint32_t k4[4];
-      if (j0 + 4 * u * NT < n) {
-        load4(j0 + 4 * u * NT, k4);
-        mine = max(max(mine, max(k4[0], k4[1])), max(k4[2], k4[3]));
+      if (j0 + 4 * u * ST < n) {
+        load4(j0 + 4 * u * ST, k4);
+        mine[u & 1] = max(max(mine[u & 1], max(k4[0], k4[1])), max(k4[2], k4[3]));
       }
     }
   }
+  mx[tid] = mine[0];
+  mx[ST + tid] = mine[1];
   if (tid == 0) sh_n = 0u;
-  const uint32_t xk = kth_of_threads(mine, kk);
+  __syncthreads();
+  if (tid < 64) {  // the largest x that kk maxima are not below, by ballots of one wave
+    uint32_t v[2 * ST / 64];
+#pragma unroll
+    for (int i = 0; i < 2 * ST / 64; i++) v[i] = mx[64 * i + tid];
+    uint32_t xk = 0u;
+    for (int b = 31; b >= 0; b--) {
+      const uint32_t t = xk | (1u << b);
+      int c = 0;
+#pragma unroll
+      for (int i = 0; i < 2 * ST / 64; i++) c += __popcll(__ballot(v[i] >= t));
+      if (c >= kk) xk = t;
+    }
+    if (tid == 0) sh_x = xk;
+  }
+  __syncthreads();
+  const uint32_t xk = sh_x;
   if (xk == 0u) {
     give_up();
     return;
@@ -324,11 +348,11 @@ __global__ __launch_bounds__(NT) void k_select_screened(
   const float xv = from_ord(xk);
   const float lim = xv - 2.0157f * E - fabsf(xv) * 4.7683716e-07f - 1e-42f;
   const uint32_t lk = sel_key(lim, false);  // (lim is finite)
-  for (int j0 = 4 * tid; j0 < n; j0 += 16 * NT) {
+  for (int j0 = 4 * tid; j0 < n; j0 += 32 * ST) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < 8; u++) {
       uint32_t k4[4];
-      const int j = j0 + 4 * u * NT;
+      const int j = j0 + 4 * u * ST;
       if (j < n) {
         load4(j, k4);
 #pragma unroll
@@ -347,7 +371,7 @@ __global__ __launch_bounds__(NT) void k_select_screened(
     return;
   }
   const float* qr = q + qi * (size_t)d;
-  for (uint32_t s = (uint32_t)((tid & 63) * NW + (tid >> 6)); s < got; s += NT) {
+  for (uint32_t s = (uint32_t)((tid & 63) * (ST / 64) + (tid >> 6)); s < got; s += ST) {
     const uint32_t j = (uint32_t)sk[s];
     const float* p = x + (size_t)j * (size_t)d;
     float acc = 0.f;
@@ -376,9 +400,32 @@ __global__ __launch_bounds__(NT) void k_select_screened(
     sk[s] = ((unsigned long long)(~sel_key(acc, false)) << 32) | (unsigned long long)j;
   }
   __syncthreads();
-  const uint32_t cnt = best_of_listed<P>(sk, got, kk, row);
-  sort_keys<P>(sk, cnt);
-  put_result(sk, cnt, qi, kk, ids, sims);
+  if (got > (uint32_t)P / 4) {
+    const uint32_t cnt = best_of_listed<P, ST>(sk, got, kk, row);
+    sort_keys<P, ST>(sk, cnt);
+    put_result<ST>(sk, cnt, qi, kk, ids, sims);
+    return;
+  }
+  // Few: each key's rank by comparing it with all (110 of them: 28 stages of
+  // the bitonic sort, with a barrier each, otherwise); then the kk best in
+  // their own order (IEEE total order, then id) the same way.
+  unsigned long long* best = sk + P / 2;
+  for (uint32_t s = tid; s < got; s += ST) {
+    const unsigned long long k = sk[s];
+    uint32_t r = 0;
+    for (uint32_t i = 0; i < got; i++) r += sk[i] < k ? 1u : 0u;
+    if (r < (uint32_t)kk)
+      best[r] = ((unsigned long long)(~ord_total(row[(uint32_t)k])) << 32) | (uint32_t)k;
+  }
+  __syncthreads();
+  for (int s = tid; s < kk; s += ST) {
+    const unsigned long long k = best[s];
+    uint32_t r = 0;
+    for (int i = 0; i < kk; i++) r += best[i] < k ? 1u : 0u;
+    const size_t o = qi * (size_t)kk + r;
+    ids[o] = (uint32_t)k;
+    sims[o] = from_ord(~(uint32_t)(k >> 32));
+  }
 }
 
 // Workgroup i: the kk best data rows of query q0 + i from its scores
@@ -520,7 +567,7 @@ __global__ __launch_bounds__(NT) void k_select_long(const float* __restrict__ S,
   cnt = all ? got_gt : (uint32_t)kk;
   }
   sort_keys<P>(sk, cnt);
-  put_result(sk, cnt, qi, kk, ids, sims);
+  put_result<NT>(sk, cnt, qi, kk, ids, sims);
 }
 
 template <int P>
@@ -536,7 +583,7 @@ void select_screened(emh_ctx* c, unsigned blocks, float* S, size_t ldS, size_t n
                      const float* q, size_t q0, const float* data, const float* bound, size_t kk,
                      bool exclude_self, uint32_t* ids, float* sims, uint32_t* list) {
   auto kern = d % 4 == 0 ? k_select_screened<true> : k_select_screened<false>;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, c->stream, S, ldS, (int)n, (int)d, q, q0,
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(ST), 0, c->stream, S, ldS, (int)n, (int)d, q, q0,
                      data, bound, (int)kk, exclude_self ? 1 : 0, ids, sims, list);
   EMH_HIP(hipGetLastError());
 }
@@ -550,7 +597,7 @@ void select_screened(emh_ctx* c, unsigned blocks, float* S, size_t ldS, size_t n
 // 471; 20,000 x 384, k = 500: 497 / 371) and for fewer than 16 queries (which
 // read the data once, with nothing written) the direct dots stay.
 bool long_screened(emh_ctx* c, size_t m, size_t n, size_t d, size_t kk) {
-  return c->screen != SCREEN_OFF && c->screen != SCREEN_F32 && kk <= NT / 2 && d >= 32 &&
+  return c->screen != SCREEN_OFF && c->screen != SCREEN_F32 && kk <= ST && d >= 32 &&
          d <= 16384 && m >= 16 && m < (1u << 25) && n >= 32 * kk && n < (1u << 25) &&
          (double)m * (double)n * (double)d >= 1e9;
 }
