@@ -16,9 +16,8 @@ reports train seconds, assignment Mrows/s, the rooflines and the CPU baseline:
                    contraction ahead of the exact f32 check): algorithmic
                    2 rows k d FLOP per launch over the HIP-event-timed
                    duration of every 8th launch in the timed steps, against
-                   the 2.5 PFLOP/s dense bf16 peak of the unit it runs on (its
-                   three bf16 passes, x.c ~ xh.ch + xh.cl + xl.ch, are
-                   reported apart as the issued rate);
+                   the 2.5 PFLOP/s dense fp16 peak of the unit it runs on (one
+                   fp16 pass);
   update_rooflines scatter_add and ema_update, algorithmic HBM bytes per
                    call over their HIP-event time in two more steps with every
                    call timed, against 8 TB/s;
@@ -50,21 +49,15 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FP32_MFMA_PEAK = 157.3  # TFLOP/s, MI355X dense
-BF16_MFMA_PEAK = 2500.0  # TFLOP/s, MI355X dense
+F16_MFMA_PEAK = 2500.0   # TFLOP/s, MI355X dense
 HBM_PEAK = 8000.0       # GB/s
 METRIC = "train s & assign Mrows/s at 200k×768 k=1024 FP32; % of FP32 MFMA peak"
-# HBM bytes per screen launch over this workload's launch mix (calibrated
-# FETCH_SIZE + WRITE_SIZE from two rocprofv3 --pmc passes of this script, with
-# a plain copy kernel of known size as the scale;
-# profiles/k_screen_train_assign_200kx768_k1024_hbm_traffic.md): 89.2 MB per
-# 16,384-row batch launch (50.3 MB of split rows, the centroids once per XCD),
-# 335 MB per 65,536-row assignment chunk, 40 MB per epoch-tail batch (the
-# 128 x 128 screen). Measured at commit 2b8405f; the run does not count it
-# again (counters need a profiler pass of their own), so the line names where
-# the figure comes from.
-SCREEN_TRAFFIC_BYTES = 95.6e6
-SCREEN_TRAFFIC_SOURCE = ("profiles/k_screen_train_assign_200kx768_k1024_hbm_traffic.md, "
-                         "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE at commit 2b8405f")
+# HBM bytes of a 16,384-row screen launch of this workload's training (FETCH_SIZE
+# x 2 + WRITE_SIZE of two rocprofv3 --pmc passes; counters need a profiler pass of
+# their own, so the line names where the figure comes from).
+SCREEN_TRAFFIC_BYTES = 78.2e6
+SCREEN_TRAFFIC_SOURCE = ("profiles/k_screen5_train_200kx768_k1024.md, rocprofv3 --pmc "
+                         "FETCH_SIZE / WRITE_SIZE, batch launches")
 # The screen's roofline times every PROFILE_EVERY-th launch of the timed steps
 # with HIP events (an event pair between two kernels costs the stream a few
 # microseconds; on every launch that was ~5 % of the headline step).
@@ -77,17 +70,17 @@ def log(*a):
 
 def screen_roofline(ms, launches, flop, kernel, traffic=None, traffic_source=None):
     """The screen's roofline: algorithmic FLOP (2 rows k d per launch) over its
-    HIP-event time against the dense bf16 MFMA peak of the unit it runs on.
-    Beside it: the bf16 MFMA work it issues (three products per multiply-add)
-    and the ratio of the algorithmic rate to the f32 MFMA peak (above 1 when
-    the exact f32 results come faster than f32 MFMA arithmetic could give)."""
+    HIP-event time against the dense fp16 MFMA peak of the unit it runs on (it
+    issues one product per multiply-add), and the ratio of that rate to the f32
+    MFMA peak (above 1 when the exact f32 results come faster than f32 MFMA
+    arithmetic could give). traffic: HBM bytes per launch where counters of
+    this kernel have been read, else None."""
     alg = flop / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
-    return {"bound": "mfma", "kernel": kernel, "achieved": alg, "peak": BF16_MFMA_PEAK,
-            "unit": "TFLOP/s", "frac": alg / BF16_MFMA_PEAK, "traffic": traffic,
+    return {"bound": "mfma", "kernel": kernel, "achieved": alg, "peak": F16_MFMA_PEAK,
+            "unit": "TFLOP/s", "frac": alg / F16_MFMA_PEAK, "traffic": traffic,
             "traffic_source": traffic_source,
             "launches": launches, "avg_launch_ms": ms / max(launches, 1),
             "flop_per_launch": flop / max(launches, 1),
-            "issued_bf16": {"achieved": 3.0 * alg, "frac": 3.0 * alg / BF16_MFMA_PEAK},
             "vs_fp32_mfma_peak": {"peak": FP32_MFMA_PEAK, "ratio": alg / FP32_MFMA_PEAK}}
 
 
@@ -150,7 +143,7 @@ def headline(args):
 
     def timed(mode, steps, warmup):
         """Warmup, then `steps` timed steps with the screen in `mode`
-        (1: bf16 three-pass, 2: f32), the screen's launches profiled."""
+        (1: the default, 2: f32), the screen's launches profiled."""
         dev.set_screen(mode)
         for i in range(warmup):
             tr, asg, _, info = step()
@@ -214,10 +207,10 @@ def headline(args):
         "fallback_rows_per_run": info["fallback_rows"],
         "roofline": screen_roofline(
             ms, launches, flop,
-            "k_screen4 (bf16 MFMA, three passes xh.ch + xh.cl + xl.ch on operands split "
-            "ahead of time, f32 accumulation, LDS-DMA ring; per-row candidate lists within "
-            "the bound of each lane's best); the epoch tails' 3,392-row batches on the "
-            "128 x 128 k_screen", SCREEN_TRAFFIC_BYTES, SCREEN_TRAFFIC_SOURCE),
+            "k_screen5 (fp16 MFMA, one pass over lines rounded ahead of time, f32 "
+            "accumulation, LDS-DMA ring; per-row candidates within the measured residuals' "
+            "bound); the epoch tails' 3,392-row batches on the 128 x 128 k_screen",
+            SCREEN_TRAFFIC_BYTES, SCREEN_TRAFFIC_SOURCE),
         "update_rooflines": {
             "scatter_add": hbm_roofline(*main["update"]["scatter_add"],
                                         "k_place_scan + k_sums (labels tallied by the "
@@ -236,7 +229,7 @@ def headline(args):
                          "achieved": fa, "peak": FP32_MFMA_PEAK, "unit": "TFLOP/s",
                          "frac": fa / FP32_MFMA_PEAK, "launches": f["launches"],
                          "avg_launch_ms": f["ms"] / max(f["launches"], 1)},
-            "equal_to_bf16_screen": bool(np.array_equal(f["labels"], gpu_labels)
+            "equal_to_default_screen": bool(np.array_equal(f["labels"], gpu_labels)
                                          and f["scores"].tobytes() == gpu_scores.tobytes()
                                          and f["cent"].tobytes() == cent.tobytes()),
         }
@@ -402,7 +395,7 @@ def other_workloads(args):
         "value": 2.0 * n * n * d / step_s / 1e12, "unit": "TFLOP/s", "ms_per_run": step_s * 1e3,
         "steps": args.other_steps,
         "roofline": screen_roofline(ms, launches, flop,
-                                    "k_screen4kn (kNN over rows split once, 24-entry lists)"),
+                                    "k_screen5 (kNN over fp16 lines, one pass)"),
         "cpu_baseline": {"value": 2.0 * len(sample) * n * d / cpu_s / 1e12, "unit": "TFLOP/s",
                          "cores": O.get_threads(), "kind": "port",
                          "sample": f"{len(sample)} queries against all {n} rows"},
@@ -447,8 +440,8 @@ def knn_workload(args):
            "vs_baseline": None, "dtype": "f32", "data": "synthetic",
            "config": {"workload": f"knn_self k=10 {n}x{d} unit rows, 5% near-duplicates, seed 2"},
            "roofline": screen_roofline(ms, launches, flop,
-                                       "k_screen4kn (kNN over rows split once, bf16 three-pass "
-                                       "MFMA, 24-entry lists)")}
+                                       "k_screen5 (kNN over fp16 lines, one pass, 24-entry "
+                                       "lists)")}
     if not args.no_cpu:
         from oracle import oracle as O
         g = np.random.default_rng(0)
@@ -499,7 +492,7 @@ def assign_workload(args):
            "vs_baseline": None, "dtype": "f32", "data": "synthetic",
            "config": {"workload": f"assign {n}x{d} vs {k} centroids, IP, unit rows, seed 1"},
            "tflops": 2.0 * n * k * d / step_s / 1e12,
-           "roofline": screen_roofline(ms, launches, flop, "k_screen (bf16 three-pass MFMA x.C^T + per-row 5-entry candidate lists)")}
+           "roofline": screen_roofline(ms, launches, flop, "k_screen5 (fp16 lines, one pass, x.C^T + per-row candidate lists)")}
     if not args.no_host:
         # The same assignment from host arrays (8.2 GB of queries staged in
         # while earlier chunks run): the PCIe-inclusive rate, not the value.

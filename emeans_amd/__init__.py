@@ -373,9 +373,10 @@ class HipDevice:
         return lib().emh_fallback_rows(self._ctx)
 
     def set_screen(self, mode):
-        """Top-1 / top-k path: 1 or True = bf16 three-pass MFMA screen + exact
-        check (default), 3 = the same with the split-operand top-1 screen in
-        fp16 two-pass arithmetic, 2 = f32 MFMA screen + exact check, 0 or
+        """Top-1 / top-k path: 1 or True = MFMA screen (one fp16 pass over
+        rounded rows; small calls in bf16 three-pass) + exact check (default),
+        3 = the same with the split-operand top-1 screen in fp16 two-pass
+        arithmetic, 2 = f32 MFMA screen + exact check, 0 or
         False = the exact kernels alone. Every mode gives the same bits."""
         check(lib().emh_set_screen(self._ctx, int(mode)))
 

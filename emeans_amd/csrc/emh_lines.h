@@ -2,10 +2,10 @@
 // to fp16, in lines, shared by the kernels that write them (k_lines).
 //
 // A matrix is scaled by one power of two s (scale[0]; scale[1] = 1 / s) that
-// brings its largest sampled element to 2^7 .. 2^8, and cut into slabs of 64
-// dimensions (dimensions past d are zero), each one 128-byte line of fp16
+// brings its largest sampled element to 2^7 .. 2^8, and cut into slabs of 32
+// dimensions (dimensions past d are zero), each a 64-byte line of fp16
 // values h(s x), rounded to nearest even, in order. Lines are stored
-// slab-major: slab j of row g of an n-row matrix at (j n + g) 128 bytes.
+// slab-major: slab j of row g of an n-row matrix at (j n + g) 64 bytes.
 //
 // A row's rounding residual r = |s x - h(s x)| is kept beside |x|^2: the
 // screen's error bound follows from Cauchy-Schwarz on the residuals that the

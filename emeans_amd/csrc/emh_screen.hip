@@ -4,11 +4,13 @@
 //
 // Exactness: the reference CPU backend (cpu-fused, assign/fused.rs) scores
 // every (row, centroid) pair with one sequential f32 fma chain over the d
-// dimensions. The screen computes the same dot products on the bf16 MFMA in
-// three passes (x.c ~ xh.ch + xh.cl + xl.ch, the halves rounded to nearest
-// even, f32 accumulation), so its scores differ from the chain's by about
-// 2^-16 |x| |c| plus the accumulation's rounding. The path therefore has three
-// stages:
+// dimensions. The screen computes the same dot products on the MFMA: in one
+// fp16 pass over rows rounded ahead (k_screen5, whose bound rests on the
+// measured residuals: screen_bound_lines, emh_lines.h), or, for small calls and
+// the no-allocation entry, on the bf16 MFMA in three passes (x.c ~ xh.ch +
+// xh.cl + xl.ch, the halves rounded to nearest even, f32 accumulation), whose
+// scores differ from the chain's by about 2^-16 |x| |c| plus the
+// accumulation's rounding. The path therefore has three stages:
 //
 //  1. screen (MFMA, the dense x . C^T contraction): per part (a range of
 //     centroid tiles) each row keeps the L smallest screen keys (key = -dot
@@ -26,7 +28,7 @@
 // The same stages with a longer list, merged over the parts, give the exact
 // top-k of kNN.
 //
-// Bound (screen_bound, emh_select.h): the chain is within gamma_d sum|x_t c_t|
+// Bound of the bf16 screens (screen_bound, emh_select.h): the chain is within gamma_d sum|x_t c_t|
 // of the exact dot (gamma_d = d u / (1 - d u), u = 2^-24) and sum|x_t c_t| <=
 // |x| |c|; the screen adds the split's dropped and rounded parts
 // (<= 3.05 * 2^-16 |x| |c|) and the MFMA chain's rounding (each MFMA within

@@ -355,11 +355,11 @@ float emh_host_numpy_sum_f32(const float* a, uint64_t n);
 /* ------------------------------------------------------------ diagnostics */
 /* Which screen a top-1 or top-k call ran (emh_screen_report.variant). */
 #define EMH_SCREEN_NONE 0        /* no screen: k < 2, d < 32 or emh_set_screen(ctx, 0) */
-#define EMH_SCREEN_BIG_TAGGED 1  /* large-tile bf16 screen, one tile per part, tagged keys */
-#define EMH_SCREEN_BIG_SORTED 2  /* large-tile bf16 screen, several tiles per part */
+#define EMH_SCREEN_BIG_TAGGED 1  /* large-tile screen, one tile per part, tagged keys */
+#define EMH_SCREEN_BIG_SORTED 2  /* large-tile screen, several tiles per part */
 #define EMH_SCREEN_SMALL_BF16 3  /* 128 x 128 bf16 screen (d % 4 != 0, and small kNN calls) */
 #define EMH_SCREEN_SMALL_F32 4   /* 128 x 128 f32 screen (emh_set_screen(ctx, 2)) */
-#define EMH_SCREEN_BIG_KNN 5     /* kNN: 128 x 256 bf16 screen over operands split once */
+#define EMH_SCREEN_BIG_KNN 5     /* kNN: large-tile screen over operands rounded once */
 #define EMH_SCREEN_BIG_F16 6     /* large-tile fp16 two-pass screen, one tile per part, tagged keys */
 typedef struct emh_screen_report {
   int variant;          /* EMH_SCREEN_* */
@@ -385,8 +385,8 @@ int emh_screen_margin_topk(emh_ctx* ctx, const emh_buf* queries, size_t m, const
 /* Rows the exact top-1 / top-k kernels rescanned since the context was made
  * (the screen's misses; EMEANS_CUDA_SCREEN_STATS analogue, emeans-cuda lib.rs:278-287). */
 uint64_t emh_fallback_rows(emh_ctx* ctx);
-/* Select the top-1 / top-k path: 1 = MFMA screen in bf16 three-pass arithmetic
- * + exact check (default), 3 = the same with the split-operand top-1 screen
+/* Select the top-1 / top-k path: 1 = MFMA screen (one fp16 pass over
+ * rounded rows; small calls in bf16 three-pass arithmetic) + exact check (default), 3 = the same with the split-operand top-1 screen
  * (k_screen4) in fp16 two-pass arithmetic (a third fewer MFMAs, a bound 2.7
  * times looser at d = 768; rows or centroids beyond |x| = 32768 take the exact
  * scan), 2 = MFMA screen in f32 arithmetic + exact check, 0 = exact kernels
