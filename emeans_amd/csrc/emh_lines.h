@@ -64,7 +64,8 @@ __device__ __forceinline__ uint2 line_quad(float4 v, float s, float& res) {
 // roundings apart, plus 127
 // subnormal ulps.
 // A sum of squares that underflows loses at most d 2^-149 (uf). Not finite
-// (an element beyond fp16's range, NaN): NaN, which settles nothing.
+// (an element beyond fp16's range, NaN, a key that may overflow f32): NaN, which
+// settles nothing.
 // edot_out: the dot term alone.
 __device__ __forceinline__ float screen_bound_lines(float xn, float xr, float cmax2, float rmax2,
                                                     float cnmax, float isx, float isc, int d,
@@ -90,7 +91,8 @@ __device__ __forceinline__ float screen_bound_lines(float xn, float xr, float cm
   *edot_out = edot;
   float e = l2 ? 2.0f * edot + 2.0f * u * (cnmax + 2.0f * S) : edot;
   e += 1.5268e-5f * (l2 ? cnmax + 2.0f * H : H) + 1.8e-43f;
-  return e * 1.015625f;  // the rounding of these few operations
+  e *= 1.015625f;  // the rounding of these few operations
+  return e < INFINITY ? e : __builtin_nanf("");
 }
 
 }  // namespace emh

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     const float lim = limit_of(b);
     float g = L2 ? -lim : -lim * rf1;
     if (!L2) g = g - fabsf(g) * 2.384185791015625e-07f - 1e-44f;
-    g = live ? fmaxf(g, -3.0e38f) : __builtin_nanf("");  // (padding's -inf is never within it)
+    g = live ? fmaxf(g, -3.4028235e38f) : __builtin_nanf("");  // (padding's -inf is never within it)
     const float gp = __shfl_xor(g, 32, 64);
     gl[0] = h == 0 ? g : gp;
     gl[1] = h == 1 ? g : gp;
@@ -625,6 +625,9 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
       }
     }
     const float lim = limit_of(b);
+    // A limit past the largest finite key: keys that overflowed may be within
+    // it, and no entry says so.
+    if (L2 && !(lim <= 3.4028235e38f)) spilt = true;
     auto keep = [&](float key, uint32_t id) __attribute__((always_inline)) {
       if (key <= lim) {
         const uint32_t e = atomicAdd(&on[prow], 1u);
@@ -636,7 +639,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     };
     if (ONE) {
       const uint32_t n = h ? cnt[1] : cnt[0];
-      spilt = n > (uint32_t)CAP;
+      spilt = spilt || n > (uint32_t)CAP;
       for (uint32_t i = 0; i < min(n, (uint32_t)CAP); i++) {
         const uint32_t v = mybuf[i * 64 + lane];
         keep(__uint_as_float(v), (uint32_t)(t0 * T5 + wc * 128) + column(v));

@@ -161,3 +161,28 @@ def test_top1_ranges(dev, metric, case, k):
     else:
         x[7, 0], x[8, 1], x[9] = np.nan, -np.inf, 0.0
     _top1(dev, np.ascontiguousarray(x), np.ascontiguousarray(c), metric)
+
+
+@pytest.mark.parametrize("k", [64, 2100])
+@pytest.mark.parametrize("case", ["straddle", "overflow"])
+def test_top1_largest_keys(dev, case, k):
+    """L2 keys at the top of the f32 range. straddle: two centroids whose keys
+    sweep across 3.0e38 from row to row, closer to each other than the screen's
+    error. overflow: |c|^2 + 2 |x| |c| beyond the largest float, so no bound is
+    finite and the exact scan decides."""
+    n, d = 40000, 64
+    g = np.random.default_rng(41)
+    c = _rows(k, d, 42).astype(np.float64) * np.sqrt(3.3e38)
+    if case == "straddle":
+        u = _rows(2, d, 43).astype(np.float64)
+        v = u[0] + 0.01 * (u[1] - (u[1] @ u[0]) * u[0])
+        r = np.sqrt(3.2e38)
+        c[k // 3], c[k // 2] = r * u[0], r * v / np.linalg.norm(v)
+        # |c|^2 - 2 x.c sweeps 5e-6 of 3.0e38 around it
+        t = (r * r - 3.0e38 * (1 + np.linspace(-5e-6, 5e-6, n))) / (2 * r)
+        x = u[0] + 0.02 * _rows(n, d, 44)
+        x *= (t / (x @ u[0]))[:, None]
+    else:
+        c[::k // 8] *= 0.8
+        x = np.sqrt(3.0e38) * _rows(n, d, 45).astype(np.float64) * g.choice([0.3, 1.0], (n, 1))
+    _top1(dev, x.astype(np.float32), c.astype(np.float32), "l2")
