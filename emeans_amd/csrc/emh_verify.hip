@@ -336,6 +336,21 @@ __device__ __forceinline__ bool unpack_best(uint64_t w, float& key, uint32_t& id
   return true;
 }
 
+// Four dimensions (16 bytes) of a lane's row into its slot of LDS (`slots` +
+// the lane): by DMA where rows start at multiples of 16 bytes (AL), else
+// through registers (a wrapped buffer may start at any float).
+typedef float v4f __attribute__((ext_vector_type(4)));
+template <bool AL>
+__device__ __forceinline__ void slot_copy(const float* src, v4f* slots) {
+  if (AL) {
+    __builtin_amdgcn_global_load_lds(src, slots, 16, 0, 0);
+  } else {
+    v4f v = {src[0], src[1], src[2], src[3]};
+    slots[threadIdx.x & 63] = v;
+  }
+}
+
+template <bool AL>
 __global__ __launch_bounds__(64) void k_queued1(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     int n_direct, const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
@@ -343,7 +358,6 @@ __global__ __launch_bounds__(64) void k_queued1(
     unsigned long long* __restrict__ best, uint32_t* __restrict__ tickets,
     float* __restrict__ xnq, uint32_t* __restrict__ labels, float* __restrict__ scores,
     uint32_t* __restrict__ tcnt, uint32_t* __restrict__ tcounts, size_t tlo, size_t tstride) {
-  typedef float v4f __attribute__((ext_vector_type(4)));
   __shared__ v4f cs[QU * QJ];
   __shared__ v4f xs[QU * QR];
   __shared__ uint32_t xid_s[QR];
@@ -384,12 +398,12 @@ __global__ __launch_bounds__(64) void k_queued1(
       const int nu = min(QU, (d - t0) / 4);  // d % 4 == 0
       for (int i = 0; i < (nu + 15) / 16; i++) {
         const int col = min(t0 + 4 * (16 * i + lane / QR), d - 4);
-        __builtin_amdgcn_global_load_lds(xrow + col, &xs[i * 64], 16, 0, 0);
+        slot_copy<AL>(xrow + col, &xs[i * 64]);
       }
       if (!norm)
         for (int i = 0; i < (nu + 3) / 4; i++) {
           const int col = min(t0 + 4 * (4 * i + lane / QJ), d - 4);
-          __builtin_amdgcn_global_load_lds(crow + col, &cs[i * 64], 16, 0, 0);
+          slot_copy<AL>(crow + col, &cs[i * 64]);
         }
       __syncthreads();  // waits for the copies
       if (norm) {  // |x|^2 of row r: sequential sum of rounded squares
@@ -465,6 +479,11 @@ __global__ __launch_bounds__(64) void k_queued1(
   }
 }
 
+// Whether rows of d % 4 == 0 floats at x and c start at multiples of 16 bytes.
+bool aligned16(const float* x, const float* c) {
+  return (((uintptr_t)x | (uintptr_t)c) & 15) == 0;
+}
+
 // ---------------------------------------- exact top-1, at most 64 centroids
 // A block takes R = 256 / KP rows against all k <= KP centroids: four waves
 // run one chain a lane (row idx / KP, centroid idx % KP), a fifth the rows'
@@ -479,14 +498,13 @@ __global__ __launch_bounds__(64) void k_queued1(
 // most of a CU's LDS.)
 constexpr int S1_W = 4, S1_T = 64 * S1_W + 64, S1_LDS = 128 * 1024;
 
-template <int KP>
+template <int KP, bool AL>
 __global__ __launch_bounds__(S1_T) void k_small1(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     int nrows, uint32_t* __restrict__ small, const float* __restrict__ cents,
     const float* __restrict__ cnorm, int k, int ip, int pu, uint32_t* __restrict__ labels,
     float* __restrict__ scores, uint32_t* __restrict__ tcnt, uint32_t* __restrict__ tcounts,
     size_t tlo, size_t tstride) {
-  typedef float v4f __attribute__((ext_vector_type(4)));
   constexpr int R = 64 * S1_W / KP;
   extern __shared__ __attribute__((aligned(16))) v4f lds[];
   __shared__ float xn_s[R];
@@ -517,11 +535,9 @@ __global__ __launch_bounds__(S1_T) void k_small1(
   for (int t0 = 0; t0 < d; t0 += 4 * pu) {
     const int nu = min(pu, (d - t0) / 4);  // d % 4 == 0
     for (int i = w; i < (nu * KP + 63) / 64; i += S1_W + 1)
-      __builtin_amdgcn_global_load_lds(crow + min(t0 + 4 * (i * (64 / KP) + lane / KP), d - 4),
-                                       &cs[i * 64], 16, 0, 0);
+      slot_copy<AL>(crow + min(t0 + 4 * (i * (64 / KP) + lane / KP), d - 4), &cs[i * 64]);
     for (int i = w; i < (nu * R + 63) / 64; i += S1_W + 1)
-      __builtin_amdgcn_global_load_lds(xrow + min(t0 + 4 * (i * (64 / R) + lane / R), d - 4),
-                                       &xs[i * 64], 16, 0, 0);
+      slot_copy<AL>(xrow + min(t0 + 4 * (i * (64 / R) + lane / R), d - 4), &xs[i * 64]);
     __syncthreads();  // waits for the copies
     if (!norm) {
 #pragma unroll 8
@@ -581,8 +597,9 @@ void small1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids
   const size_t most = (S1_LDS - 1024) / ((KP + R) * 16) / 4 * 4;
   const size_t pu = std::min<size_t>((d / 4 + 3) / 4 * 4, most);
   const size_t slots = pu * KP + (pu * R + 63) / 64 * 64;
-  hipLaunchKernelGGL(k_small1<KP>, dim3((unsigned)((n + R - 1) / R)), dim3(S1_T), slots * 16,
-                     c->stream, x, nx, (int)d, ids, lo, (int)n, c->small, cents, cnorm, (int)k,
+  auto kern = aligned16(x, cents) ? k_small1<KP, true> : k_small1<KP, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((n + R - 1) / R)), dim3(S1_T), slots * 16, c->stream,
+                     x, nx, (int)d, ids, lo, (int)n, c->small, cents, cnorm, (int)k,
                      ip ? 1 : 0, (int)pu, labels, scores, tally ? tally->cnt : nullptr,
                      tally ? tally->counts : nullptr, tally ? tally->lo : 0,
                      tally ? tally->stride : 0);
@@ -720,12 +737,13 @@ size_t queued_items(size_t n, size_t k, bool ip) {
 
 size_t exact1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool list) {
   auto r = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t ngq = (n + QR - 1) / QR, queued = r(n * 8 + ngq * 4) + r(n * 4);
-  if (list && d % 4 == 0) return queued;
+  if (!list && small_direct(c, n, d, k)) return 0;
+  if ((list && d % 4 == 0) || (!list && queued_direct(c, n, d, k, ip))) {
+    const size_t ngr = (n + QR - 1) / QR;
+    return r(n * 8 + ngr * 4) + r(n * 4);
+  }
   const size_t nch = (k + CJ - 1) / CJ, ngr = (n + RG - 1) / RG;
-  const size_t exact = r(n * nch * sizeof(Cand)) + r(ngr * 4);
-  if (list || !queued_direct(c, n, d, k, ip)) return exact;
-  return std::max(queued, exact);  // (by the buffers' alignment)
+  return r(n * nch * sizeof(Cand)) + r(ngr * 4);
 }
 
 void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
@@ -737,9 +755,7 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
              "exact: a tally needs the queued-row scan");
   // Both kernels read row 0 in place of a row whose id is out of range.
   EMH_ENSURE(nx > 0, "top1: a selection of %zu rows over no data rows", n);
-  // (Its copies take 16 bytes: a wrapped buffer may start anywhere.)
-  const bool aligned = (((uintptr_t)x | (uintptr_t)cents) & 15) == 0;
-  if (!list && aligned && small_direct(c, n, d, k)) {
+  if (!list && small_direct(c, n, d, k)) {
     auto f = k <= 16 ? small1<16> : k <= 32 ? small1<32> : small1<64>;
     f(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, labels, scores, tally);
     return;
@@ -747,9 +763,7 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
   // Queued rows (few), or a small direct selection: the latency-bound scan.
   // (k_exact1's tiles each wait a memory round trip: ~30 us at any size up
   // to a few thousand rows.)
-  if ((list && d % 4 == 0) ||
-      (!list && queued_direct(c, n, d, k, ip) &&
-       (tally || queued_items(n, k, ip) <= QUEUED_DIRECT))) {
+  if ((list && d % 4 == 0) || (!list && queued_direct(c, n, d, k, ip))) {
     const size_t ngr = (n + QR - 1) / QR;
     const size_t per = (k + QJ - 1) / QJ + (ip ? 0 : 1);
     // Self-cleaning: the best words, then the tickets, all left at zero (a
@@ -765,7 +779,8 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
       xnq = (float*)c->knn_tmp.get(n * 4);
     }
     const unsigned g = (unsigned)std::min<size_t>(ngr * per, (size_t)2 * c->cus);
-    hipLaunchKernelGGL(k_queued1, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo,
+    auto kern = aligned16(x, cents) ? k_queued1<true> : k_queued1<false>;
+    hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo,
                        (int)n, list, c->small, cents, cnorm, (int)k, ip ? 1 : 0,
                        (unsigned long long*)z,
                        (uint32_t*)(z + n * 8), xnq, labels, scores,
