@@ -343,6 +343,8 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
   const size_t n = hi - lo;
   EMH_ENSURE(d <= 16384, "top1: d = %zu above the supported 16384", d);
   EMH_ENSURE(n < (1u << 31) && k < (1u << 31), "top1: shape too large");
+  // (Every kernel reads row 0 in place of a row whose id is out of range.)
+  EMH_ENSURE(nx > 0, "top1: a selection of %zu rows over no data rows", n);
   // A tallying call takes the screen, or the latency-bound exact scan, which
   // tallies too; never k_exact1.
   const bool small_exact = !tally || queued_direct(c, n, d, k, ip);
@@ -367,6 +369,7 @@ void screen_margin_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const u
   if (hi <= lo) return;
   const size_t n = hi - lo;
   EMH_ENSURE(d <= 16384 && n < (1u << 31) && k < (1u << 31), "top1: shape too large");
+  EMH_ENSURE(nx > 0, "top1: a selection of %zu rows over no data rows", n);
   const Top1Screen s =
       screen_top1(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, false, nullptr, nullptr, nullptr,
                   false);

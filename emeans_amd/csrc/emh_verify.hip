@@ -753,8 +753,6 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
   if (n == 0) return;
   EMH_ENSURE(!tally || (d % 4 == 0 && (list || queued_direct(c, n, d, k, ip))),
              "exact: a tally needs the queued-row scan");
-  // Both kernels read row 0 in place of a row whose id is out of range.
-  EMH_ENSURE(nx > 0, "top1: a selection of %zu rows over no data rows", n);
   if (!list && small_direct(c, n, d, k)) {
     auto f = k <= 16 ? small1<16> : k <= 32 ? small1<32> : small1<64>;
     f(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, labels, scores, tally);

@@ -186,3 +186,15 @@ def test_top1_largest_keys(dev, case, k):
         c[::k // 8] *= 0.8
         x = np.sqrt(3.0e38) * _rows(n, d, 45).astype(np.float64) * g.choice([0.3, 1.0], (n, 1))
     _top1(dev, x.astype(np.float32), c.astype(np.float32), "l2")
+
+
+def test_top1_no_data_rows(dev):
+    """Ids over an empty matrix are refused before any kernel reads a row."""
+    from emeans_amd import Mat, Select
+    n, d, k = 40000, 64, 300
+    lab, sco = dev.zeros_u32(n), dev.zeros_f32(n)
+    ids = dev.upload_u32(np.zeros(n, np.uint32))
+    c = dev.upload_f32(_rows(k, d, 1))
+    for m in (3, n):
+        with pytest.raises(Exception, match="no data rows"):
+            dev.top1(Mat(dev.zeros_f32(0), d), Select(ids, (0, m)), c, None, k, "ip", lab, sco)
