@@ -653,7 +653,7 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
       pre_rows.xn = c->xpre_norm.get(n * 8);
       pre_rows.slab = n * LINE_BYTES;
       pre_rows.scale = run_scale;
-      launch_scales(c, x, n * d, run_scale, nullptr, 0, nullptr, nullptr, 0);
+      launch_scales(c, d, ScaleIn{x, n, nullptr, 0, n, run_scale, -50}, nullptr, nullptr, 0);
       launch_lines(c, x, n, d, nullptr, 0, n, run_scale, (void*)pre_rows.xs,
                    (float2*)pre_rows.xn, nullptr, nullptr);
     }
@@ -690,8 +690,9 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
     pcents.scale = tco.scale;
   } else if (pre && !run_f16) {
     // Spherical: the readout is split batch by batch, at one scale (no element
-    // of a unit row is beyond 1, and the largest of d is at least d^-1/2, so
-    // the scale of the first readout keeps every later one in range).
+    // of a unit row is beyond 1, and the largest of each sampled row is at
+    // least d^-1/2 >= 2^-7, so the scale of the first readout is at most 2^14
+    // and keeps every later one in range).
     pcents.scale = c->scales + 2 * SCALE_UNIT;
   }
   const SplitCents* pcp = pre && (keep_csplit || !run_f16) ? &pcents : nullptr;
@@ -782,8 +783,8 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
         if (!ema_readout || readout_stale) launch_normalize_rows(c, pos.f(), k, d, readout.f());
         readout_stale = false;
         if (step == 0 && pcents.scale)
-          launch_scales(c, readout.f(), k * d, c->scales + 2 * SCALE_UNIT, nullptr, 0, nullptr,
-                        nullptr, 0);
+          launch_scales(c, d, ScaleIn{readout.f(), k, nullptr, 0, k, c->scales + 2 * SCALE_UNIT, -6},
+                        nullptr, nullptr, 0);
       } else if (norms_stale) {
         launch_row_norms(c, pos.f(), k, d, readout.f());
         norms_stale = false;
@@ -1575,8 +1576,9 @@ int emh_assign_dev(emh_ctx* c, const emh_buf* x, size_t n, size_t d, const emh_b
     if (!f16 && n > chunk && emh::split_screen(c, chunk, d, k, metric == EMH_IP)) {
       float* sc = c->scales + 2 * emh::SCALE_CENTS;
       float* sx = c->scales + 2 * emh::SCALE_ROWS;
-      emh::launch_scales(c, cp, k * d, sc, reuse ? nullptr : (const float*)x->ptr, n * d, sx,
-                         nullptr, 0);
+      const emh::ScaleIn ic{cp, k, nullptr, 0, k, sc, -50};
+      const emh::ScaleIn ix{(const float*)x->ptr, n, nullptr, 0, n, sx, -50};
+      emh::launch_scales(c, d, ic, reuse ? nullptr : &ix, nullptr, 0);
       if (!reuse) pre.scale = sx;
       pc = emh::split_cents(c, cp, d, k, metric == EMH_L2 ? cn.f() : nullptr, sc);
       once = true;

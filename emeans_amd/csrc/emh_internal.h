@@ -165,6 +165,18 @@ enum ScaleOf : int {
   SCALE_UNIT = 3,   // a spherical run's readout
   SCALE_WORDS = 8,
 };
+// Rows ids[lo + i] (lo + i without ids; an id >= nx reads row 0), i < n, of a
+// matrix of nx rows whose scale goes to out; elements of at most 2^emin are
+// expected whatever the sample shows.
+struct ScaleIn {
+  const float* p;
+  size_t nx;
+  const uint32_t* ids;
+  size_t lo, n;
+  float* out;
+  int emin;
+};
+constexpr int SCALE_ROWS_READ = 64;  // rows that the scale looks at (a quarter beyond 2,048 dimensions)
 
 }  // namespace emh
 
@@ -508,13 +520,13 @@ inline size_t halves_blocks(size_t n) { return (n + 7) / 8; }
 // reduced by one workgroup ahead (launch_part_max4).
 constexpr size_t PART_MAX_ONCE = 1024;
 // Rows as fp16 lines for the one-pass screen (emh_lines.h, emh_screen5.hip):
-// the scales of one or two matrices (nx d elements each; b may be null),
-// clearing nclear words on the way; rows ids[lo .. lo + n) (or lo ..) of x as
+// the scales of one or two selections of rows (b may be null), clearing nclear
+// words on the way; rows ids[lo .. lo + n) (or lo ..) of x as
 // lines in out (lines_bytes(n, d)) with (|x|^2, residual) in norm, and with
 // part each of the lines_blocks(n) blocks' maxima in part[4 b ..]; the maxima
 // over those.
-void launch_scales(emh_ctx* c, const float* a, size_t na, float* sa, const float* b, size_t nb,
-                   float* sb, uint32_t* clear, int nclear);
+void launch_scales(emh_ctx* c, size_t d, const ScaleIn& a, const ScaleIn* b, uint32_t* clear,
+                   int nclear);
 void launch_lines(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
                   size_t n, const float* scale, void* out, float2* norm, const float* cnorm,
                   uint32_t* part);

@@ -221,12 +221,8 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
       float* wx = c->scales + 2 * SCALE_ROWS;
       float* wc = c->scales + 2 * SCALE_CENTS;
       const int nclear = words_clear ? 0 : 3;
-      if (!sx && !sc)
-        launch_scales(c, x, nx * d, wx, cents, k * d, wc, c->small, nclear);
-      else if (!sx)
-        launch_scales(c, x, nx * d, wx, nullptr, 0, nullptr, c->small, nclear);
-      else
-        launch_scales(c, cents, k * d, wc, nullptr, 0, nullptr, c->small, nclear);
+      const ScaleIn ix{x, nx, ids, lo, n, wx, -50}, ic{cents, k, nullptr, 0, k, wc, -50};
+      launch_scales(c, d, sx ? ic : ix, !sx && !sc ? &ic : nullptr, c->small, nclear);
       if (!sx) sx = wx;
       if (!sc) sc = wc;
       words_clear = true;

@@ -7,46 +7,57 @@
 namespace emh {
 namespace {
 
-// Block b: the power of two that brings the largest of 8,192 elements sampled
-// evenly over a matrix (b = 0: a, 1: b; 128 runs of 64, `step` apart) to 2^7
-// .. 2^8, and its inverse, into out. A sample: 8 bits of fp16's range are left
-// above it and 21 normal ones below, and a matrix with elements beyond that
-// only costs its rows the exact scan. Also clears `clear` (nclear words).
-// Latency-bound: the loads of a thread are all in flight at once.
-constexpr int SRUNS = 8;  // runs per wave of 16
-__global__ __launch_bounds__(1024) void k_scales(const float* __restrict__ a, size_t na, size_t da,
-                                                 float* __restrict__ sa,
-                                                 const float* __restrict__ b, size_t nb, size_t db,
-                                                 float* __restrict__ sb,
+// Block b (b = 0: a, 1: b): the power of two that brings the largest element of
+// up to `rows` whole rows, spread over the selection, to 2^7 .. 2^8, and its
+// inverse, into out; no finer than 2^(8 - emin). Whole rows, so that a column
+// in larger units than the others is always seen (runs of 64 elements a fixed
+// step apart could miss the same columns of every row); rows of the selection,
+// because the others may hold anything. 8 bits of fp16's range are left above
+// the sample and 21 normal ones below; elements beyond that cost their row the
+// exact scan (a centroid's or a data row's: every row of the call). Also clears
+// `clear` (nclear words). A thread a column: latency-bound, its loads in flight
+// together.
+constexpr int SCALE_LOADS = 32;
+__global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn b, int d, int rows,
                                                  uint32_t* __restrict__ clear, int nclear) {
-  const float* p = blockIdx.x ? b : a;
-  const size_t n = blockIdx.x ? nb : na, step = blockIdx.x ? db : da;
-  float* out = blockIdx.x ? sb : sa;
+  const ScaleIn in = blockIdx.x ? b : a;
+  __shared__ const float* rp[SCALE_ROWS_READ];
+  __shared__ float wm[16];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0 && tid < nclear) clear[tid] = 0u;
-  float v[SRUNS];
-#pragma unroll
-  for (int u = 0; u < SRUNS; u++) {
-    const size_t i = (size_t)(u * 16 + w) * step + lane;
-    v[u] = i < n ? p[i] : 0.f;
+  const int nr = (int)min((size_t)rows, in.n);
+  if (tid < nr) {
+    // Row i of n: in the i-th of nr equal stretches, at a place in it that
+    // follows no period (multiples of the golden ratio).
+    const uint64_t f = ((uint64_t)tid << 16) + (((uint64_t)tid + 1) * 40503u & 65535u);
+    const size_t at = in.lo + (in.n <= (size_t)rows ? (size_t)tid
+                                                    : (size_t)((f * in.n >> 16) / (uint64_t)nr));
+    const size_t id = in.ids ? (size_t)in.ids[at] : at;
+    rp[tid] = in.p + (id < in.nx ? id : 0) * (size_t)d;
   }
+  __syncthreads();
   float m = 0.f;
+  for (int t = tid; t < d; t += 1024)
+    for (int i0 = 0; i0 < nr; i0 += SCALE_LOADS) {
+      float v[SCALE_LOADS];
 #pragma unroll
-  for (int u = 0; u < SRUNS; u++) {
-    const float e = fabsf(v[u]);
-    m = e < INFINITY ? fmaxf(m, e) : m;  // NaN and infinities say nothing of the scale
-  }
+      for (int u = 0; u < SCALE_LOADS; u++) v[u] = rp[min(i0 + u, nr - 1)][t];
+#pragma unroll
+      for (int u = 0; u < SCALE_LOADS; u++) {
+        const float e = fabsf(v[u]);
+        m = e < INFINITY ? fmaxf(m, e) : m;  // NaN and infinities say nothing of the scale
+      }
+    }
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  __shared__ float wm[16];
   if (lane == 0) wm[w] = m;
   __syncthreads();
   if (tid == 0) {
-    for (int i = 0; i < 16; i++) m = fmaxf(m, wm[i]);
-    int e = 8;  // no sample, or zeros: scale 1
+    for (int i = 1; i < 16; i++) m = fmaxf(m, wm[i]);
+    int e = 8;  // zeros: scale 1
     if (m > 0.f) frexpf(m, &e);  // m in [2^(e - 1), 2^e)
-    e = max(-50, min(e, 60));    // two inverse scales' product stays a normal f32
-    out[0] = ldexpf(1.0f, 8 - e);
-    out[1] = ldexpf(1.0f, e - 8);
+    e = max(max(-50, in.emin), min(e, 60));  // two inverse scales' product stays a normal f32
+    in.out[0] = ldexpf(1.0f, 8 - e);
+    in.out[1] = ldexpf(1.0f, e - 8);
   }
 }
 
@@ -192,12 +203,11 @@ void launch5(emh_ctx* c, unsigned blocks, const Args5& a) {
 
 }  // namespace
 
-void launch_scales(emh_ctx* c, const float* a, size_t na, float* sa, const float* b, size_t nb,
-                   float* sb, uint32_t* clear, int nclear) {
-  // The last run ends within the matrix; matrices below 8,192 elements are read whole.
-  auto step = [](size_t n) { return n > 8192 ? (n - 64) / (16 * SRUNS - 1) : (size_t)64; };
-  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, na, step(na), sa, b,
-                     nb, step(nb), sb, clear, nclear);
+void launch_scales(emh_ctx* c, size_t d, const ScaleIn& a, const ScaleIn* b, uint32_t* clear,
+                   int nclear) {
+  EMH_ENSURE(a.n > 0 && a.nx > 0 && (!b || (b->n > 0 && b->nx > 0)), "scales: no rows");
+  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, b ? *b : a, (int)d,
+                     d <= 2048 ? SCALE_ROWS_READ : SCALE_ROWS_READ / 4, clear, nclear);
   EMH_HIP(hipGetLastError());
 }
 
@@ -279,7 +289,8 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
   const bool same = q == data && m == n;
   float* sc = c->scales + 2 * SCALE_CENTS;
   float* sx = same ? sc : c->scales + 2 * SCALE_ROWS;
-  launch_scales(c, data, n * d, sc, same ? nullptr : q, m * d, sx, clear, nclear);
+  const ScaleIn is{data, n, nullptr, 0, n, sc, -50}, iq{q, m, nullptr, 0, m, sx, -50};
+  launch_scales(c, d, is, same ? nullptr : &iq, clear, nclear);
   void* xs = c->csplit.get(lines_bytes(n, d));
   float2* xn = (float2*)c->csplit_norm.get(n * 8);
   // Past PART_MAX_ONCE partials, one workgroup reduces them ahead of the

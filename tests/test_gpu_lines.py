@@ -198,3 +198,36 @@ def test_top1_no_data_rows(dev):
     for m in (3, n):
         with pytest.raises(Exception, match="no data rows"):
             dev.top1(Mat(dev.zeros_f32(0), d), Select(ids, (0, m)), c, None, k, "ip", lab, sco)
+
+
+@pytest.mark.parametrize("k,d", [(127, 200), (127, 300), (1016, 200), (64, 256), (2159, 320)])
+def test_top1_large_columns(dev, k, d):
+    """One column in units 3,000 times the others', wherever it lies: the
+    screen still settles nearly every row."""
+    n = 40000 if k < 1000 else 20000
+    c, x = _rows(k, d, 51), _rows(n, d, 52)
+    for t in (d // 3, d // 2, d - 40, d - 1):
+        cc, xx = c.copy(), x.copy()
+        cc[:, t] *= np.float32(3000)
+        xx[:, t] *= np.float32(3000)
+        f0 = dev.fallback_rows()
+        _top1(dev, xx, cc, "ip")
+        assert dev.fallback_rows() - f0 < n // 50
+
+
+def test_top1_rows_outside_selection(dev):
+    """Rows that are not selected say nothing of the selected ones' scale."""
+    from emeans_amd import Mat, Select
+    n, d, k = 60000, 64, 300
+    x, c = _rows(n, d, 61), _rows(k, d, 62)
+    x[20000:] *= np.float32(1e12)
+    ids = np.random.default_rng(63).permutation(20000).astype(np.uint32)
+    lab, sco = dev.zeros_u32(n), dev.zeros_f32(n)
+    for i in (None, ids):
+        f0 = dev.fallback_rows()
+        dev.top1(Mat(dev.bind(x), d), Select(None if i is None else dev.upload_u32(i), (0, 20000)),
+                 dev.upload_f32(c), None, k, "ip", lab, sco)
+        ol, os_ = O.top1(x[:20000], d, c, "ip", ids=i)
+        assert np.array_equal(dev.read_u32(lab)[:20000], ol)
+        assert dev.read_f32(sco)[:20000].tobytes() == os_.tobytes()
+        assert dev.fallback_rows() - f0 < 200
