@@ -353,7 +353,7 @@ int emh_destroy(emh_ctx* c) {
     for (emh::Scratch* s : {&c->cand, &c->fblist, &c->order, &c->start, &c->misc, &c->knn_tmp,
                             &c->xnorm, &c->bigj, &c->chunkcnt, &c->tickets,
                             &c->preview_ticket, &c->xsplit, &c->xsplit_norm, &c->csplit, &c->csplit_norm, &c->csplit_part,
-                            &c->xpre, &c->xpre_norm, &c->tsplit, &c->tsplit_norm, &c->tsplit_part, &c->tally_cnt,
+                            &c->cmean, &c->tframe, &c->xpre, &c->xpre_norm, &c->tsplit, &c->tsplit_norm, &c->tsplit_part, &c->tally_cnt,
                             &c->log5, &c->klong, &c->trun, &c->kpp, &c->iscore, &c->cnorm})
       s->release();
     for (emh::Pinned* s : {&c->pin_usage, &c->pin_plan, &c->pin_small, &c->pin_order[0],

@@ -46,23 +46,40 @@ __device__ __forceinline__ void split_quad(float4 v, uint2& hi, uint2& lo) {
   lo = __builtin_bit_cast(uint2, l4);
 }
 
-// Dimensions col .. col + 3 (col % 4 == 0) of row j of k rows; the residual
-// the rounding of the quad left (lines).
-__device__ __forceinline__ float put_quad(const CentsOut& o, size_t k, size_t j, size_t col,
-                                          float4 v) {
+// Dimensions col .. col + 3 (col % 4 == 0, those past d zero) of row j of k
+// rows. Lines: (the squares of the quad's difference from the mean, the
+// residual its rounding left).
+__device__ __forceinline__ float2 put_quad(const CentsOut& o, size_t k, size_t j, size_t col,
+                                           float4 v) {
   if (o.scale) {
+    const float4 m = *reinterpret_cast<const float4*>(o.scale + MEAN_AT + col);  // (zeros past d)
+    v = make_float4(v.x - m.x, v.y - m.y, v.z - m.z, v.w - m.w);
     float res = 0.f;
     const uint2 q = line_quad(v, o.scale[0], res);
     *reinterpret_cast<uint2*>(o.cs + ((col / LINE_DIMS) * k + j) * LINE_BYTES +
                               2 * (col % LINE_DIMS)) = q;
-    return res;
+    return make_float2(fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, v.x * v.x))), res);
   }
   uint2 hi, lo;
   split_quad(v, hi, lo);
   char* p = o.cs + ((col >> 5) * k + j) * SLAB_BYTES + quad_hi_offset((int)(col & 31) >> 2);
   *reinterpret_cast<uint2*>(p) = hi;
   *reinterpret_cast<uint2*>(p + 32) = lo;
-  return 0.f;
+  return make_float2(0.f, 0.f);
+}
+
+// The figures of a row's quads into its two sums in LDS: eight lanes, which
+// hold quads of one row, first add theirs up.
+__device__ __forceinline__ void add_quad(float2 r, float* dif, float* res) {
+#pragma unroll
+  for (int m = 1; m < 8; m <<= 1) {
+    r.x += __shfl_xor(r.x, m, 64);
+    r.y += __shfl_xor(r.y, m, 64);
+  }
+  if ((threadIdx.x & 7) == 0) {
+    atomicAdd(dif, r.x);
+    atomicAdd(res, r.y);
+  }
 }
 
 }  // namespace emh

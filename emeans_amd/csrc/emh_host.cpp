@@ -639,6 +639,7 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
   c->xpre_of = emh_ctx::SplitOf{};  // xpre is rewritten (or left stale) below
   const bool run_f16 = c->screen == SCREEN_F16;
   float* run_scale = c->scales + 2 * SCALE_RUN;
+  float *cent_scale = nullptr, *cent_mean = nullptr;  // the centroids' lines'
   if (split_screen(c, bsz, d, k, sph) && n < (1u << 25)) {
     pre_rows.nx = n;
     pre_rows.f16 = run_f16;
@@ -653,9 +654,13 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
       pre_rows.xn = c->xpre_norm.get(n * 8);
       pre_rows.slab = n * LINE_BYTES;
       pre_rows.scale = run_scale;
-      launch_scales(c, d, ScaleIn{x, n, nullptr, 0, n, run_scale, -50}, nullptr, nullptr, 0);
-      launch_lines(c, x, n, d, nullptr, 0, n, run_scale, (void*)pre_rows.xs,
-                   (float2*)pre_rows.xn, nullptr, nullptr);
+      cent_scale = (float*)c->tframe.get((MEAN_AT + mean_floats(d)) * 4);
+      cent_mean = cent_scale + MEAN_AT;
+      const ScaleIn cents{x, n, nullptr, 0, n, cent_scale, -50, cent_mean};
+      launch_scales(c, d, ScaleIn{x, n, nullptr, 0, n, run_scale, -50}, sph ? nullptr : &cents,
+                    nullptr, 0);
+      launch_lines(c, x, n, d, nullptr, 0, n,
+                   LinesOut{run_scale, (void*)pre_rows.xs, (float2*)pre_rows.xn});
     }
     pre = &pre_rows;
     c->xpre_of.ptr = x;  // which buffer: emh_train_dev names it once the run has ended
@@ -666,8 +671,8 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
   // L2 batches on a split-operand screen keep the centroids split for the
   // run: a full split after each row-norms readout (the first batch, and
   // after a revival moved rows), then the EMA rewrites the rows it moves.
-  // Centroids move within the rows' hull (or, given, towards it), so the rows'
-  // scale serves them.
+  // Centroids move within the rows' hull (or, given, towards it), so the mean
+  // and the scale of the rows' differences from it serve them.
   const bool keep_csplit = pre && !sph;
   CentsOut tco{};
   // The bound's centroid maxima, in groups of four words: halves_blocks(k)
@@ -683,17 +688,18 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
   if (keep_csplit) {
     tco.cs = (char*)c->tsplit.get(run_f16 ? halves_bytes(k, d) : lines_bytes(k, d));
     tco.norm2 = (float2*)c->tsplit_norm.get(k * 8);
-    tco.scale = run_f16 ? nullptr : run_scale;
+    tco.scale = run_f16 ? nullptr : cent_scale;
     tco.part = tpart_h + 4 * full_groups;
     pcents.cs = tco.cs;
     pcents.f16 = run_f16;
     pcents.scale = tco.scale;
   } else if (pre && !run_f16) {
-    // Spherical: the readout is split batch by batch, at one scale (no element
-    // of a unit row is beyond 1, and the largest of each sampled row is at
-    // least d^-1/2 >= 2^-7, so the scale of the first readout is at most 2^14
-    // and keeps every later one in range).
-    pcents.scale = c->scales + 2 * SCALE_UNIT;
+    // Spherical: the readout is split batch by batch, at the first one's scale
+    // and mean. That scale is at most 2^14, and no element of a unit row, nor
+    // its difference from a mean of such rows, is beyond 2: every readout stays
+    // in range.
+    pcents.scale = cent_scale;
+    pcents.mean = cent_mean;
   }
   const SplitCents* pcp = pre && (keep_csplit || !run_f16) ? &pcents : nullptr;
   // When the batches' top-1 runs the screen with d % 4 == 0 (the check and
@@ -783,7 +789,8 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
         if (!ema_readout || readout_stale) launch_normalize_rows(c, pos.f(), k, d, readout.f());
         readout_stale = false;
         if (step == 0 && pcents.scale)
-          launch_scales(c, d, ScaleIn{readout.f(), k, nullptr, 0, k, c->scales + 2 * SCALE_UNIT, -6},
+          launch_scales(c, d,
+                        ScaleIn{readout.f(), k, nullptr, 0, k, cent_scale, -6, cent_mean},
                         nullptr, nullptr, 0);
       } else if (norms_stale) {
         launch_row_norms(c, pos.f(), k, d, readout.f());
@@ -793,8 +800,8 @@ void train_dev(emh_ctx* c, const float* x, size_t n, const emh_config& cfg,
             launch_halves(c, pos.f(), k, d, nullptr, 0, k, tco.cs, (float*)tco.norm2, readout.f(),
                           tpart_h);
           else
-            launch_lines(c, pos.f(), k, d, nullptr, 0, k, run_scale, tco.cs, tco.norm2,
-                         readout.f(), tpart_h);
+            launch_lines(c, pos.f(), k, d, nullptr, 0, k, LinesOut{cent_scale, tco.cs, tco.norm2},
+                         readout.f(), tpart_h, cent_mean);
           pcents.part = tpart_h;
           pcents.nparts = (int)full_groups;
         }
@@ -1576,11 +1583,12 @@ int emh_assign_dev(emh_ctx* c, const emh_buf* x, size_t n, size_t d, const emh_b
     if (!f16 && n > chunk && emh::split_screen(c, chunk, d, k, metric == EMH_IP)) {
       float* sc = c->scales + 2 * emh::SCALE_CENTS;
       float* sx = c->scales + 2 * emh::SCALE_ROWS;
-      const emh::ScaleIn ic{cp, k, nullptr, 0, k, sc, -50};
+      float* mean = (float*)c->cmean.get(emh::mean_floats(d) * 4);
+      const emh::ScaleIn ic{cp, k, nullptr, 0, k, sc, -50, mean};
       const emh::ScaleIn ix{(const float*)x->ptr, n, nullptr, 0, n, sx, -50};
       emh::launch_scales(c, d, ic, reuse ? nullptr : &ix, nullptr, 0);
       if (!reuse) pre.scale = sx;
-      pc = emh::split_cents(c, cp, d, k, metric == EMH_L2 ? cn.f() : nullptr, sc);
+      pc = emh::split_cents(c, cp, d, k, metric == EMH_L2 ? cn.f() : nullptr, sc, mean);
       once = true;
     }
     for (size_t b = 0; b < n; b += chunk) {

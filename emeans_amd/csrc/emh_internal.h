@@ -157,17 +157,19 @@ enum SmallWord : int {
   SW_BAD_INIT = 8,        // set when a training run's initial centroids are not finite
   SW_WORDS = 16,
 };
-// The matrices whose fp16 lines a context may hold at once (emh_lines.h).
+// The rows whose fp16 lines a context may hold at once (emh_lines.h), besides a
+// training run's centroids (tframe).
 enum ScaleOf : int {
   SCALE_ROWS = 0,   // a call's rows
-  SCALE_CENTS = 1,  // a call's centroids (kNN: the data rows)
-  SCALE_RUN = 2,    // a training run's rows (xpre), and its centroids when they lie among them
-  SCALE_UNIT = 3,   // a spherical run's readout
-  SCALE_WORDS = 8,
+  SCALE_CENTS = 1,  // a call's centroids (kNN: the data rows); their mean in cmean
+  SCALE_RUN = 2,    // a training run's rows (xpre)
+  SCALE_WORDS = 6,
 };
 // Rows ids[lo + i] (lo + i without ids; an id >= nx reads row 0), i < n, of a
 // matrix of nx rows whose scale goes to out; elements of at most 2^emin are
-// expected whatever the sample shows.
+// expected whatever the sample shows. With mean (mean_floats(d)), also the
+// sampled rows' mean, zeros where it does not matter; the scale is then that of
+// the differences from it.
 struct ScaleIn {
   const float* p;
   size_t nx;
@@ -175,8 +177,10 @@ struct ScaleIn {
   size_t lo, n;
   float* out;
   int emin;
+  float* mean = nullptr;
 };
-constexpr int SCALE_ROWS_READ = 64;  // rows that the scale looks at (a quarter beyond 2,048 dimensions)
+constexpr int MEAN_AT = 4;  // tframe: (s, 1 / s, -, -), then the mean
+constexpr int SCALE_ROWS_READ = 32;  // rows that the scale looks at (half beyond 2,048 dimensions)
 
 }  // namespace emh
 
@@ -217,6 +221,8 @@ struct emh_ctx {
   uint64_t fallback_total = 0;
   emh::Scratch cand, fblist, order, start, misc, knn_tmp, xnorm, bigj, chunkcnt, tickets;
   emh::Scratch xsplit, xsplit_norm, csplit, csplit_norm, csplit_part;  // split-operand screens: a call's rows, centroids
+  emh::Scratch cmean;  // the mean of a call's centroids
+  emh::Scratch tframe;  // scale and mean (at MEAN_AT) of a training run's centroids
   emh::Scratch xpre, xpre_norm;              // a training run's rows, split once
   // What xpre holds: the rows [0, n) of buffer `serial` at generation `gen`
   // (d dimensions, at address ptr); valid only for a buffer the library owns.
@@ -322,6 +328,17 @@ inline double ema_bytes(size_t k, size_t d) { return 4.0 * (3.0 * (double)k * (d
 void launch_fill_u32(emh_ctx* c, uint32_t* p, size_t n, uint32_t v);
 void launch_row_norms(emh_ctx* c, const float* m, size_t rows, size_t d, float* out);
 void launch_normalize_rows(emh_ctx* c, const float* src, size_t rows, size_t d, float* dst);
+// The split centroids that the kernels which move centroids keep up to date:
+// k rows in lines (scale, with the mean at scale + MEAN_AT: emh_lines.h;
+// norm2[j] is row j's squared distance from the mean and its residual) or,
+// without a scale, in fp16 halves. part: where the kernel leaves the bound's maxima, four words a group
+// of rows: the squared distance (halves: |c|^2), cnorm, the residual, |c|^2.
+struct CentsOut {
+  char* cs = nullptr;
+  const float* scale = nullptr;
+  float2* norm2 = nullptr;
+  uint32_t* part = nullptr;
+};
 // With clear_screen_words, also zeroes the small-block words launch_top1
 // clears before its screen (the fallback count and the bound maxima), so the
 // next top-1 may skip that fill. With tally, also adds counts into it. With
@@ -332,16 +349,6 @@ void launch_normalize_rows(emh_ctx* c, const float* src, size_t rows, size_t d, 
 // zero_words[0..nzero) (a tally's chunk histograms). With readout (spherical
 // runs, no norms, d <= EMA_READOUT_MAX_D), each moved row's normalize_rows
 // readout is written there too (rows that did not move keep theirs).
-// The split centroids that the kernels which move centroids keep up to date:
-// k rows in lines (scale set: emh_lines.h; norm2[j].y is row j's residual) or,
-// without a scale, in fp16 halves. part: where the kernel leaves the bound's
-// maxima, four words a group of rows (|c|^2, cnorm, residual).
-struct CentsOut {
-  char* cs = nullptr;
-  const float* scale = nullptr;
-  float2* norm2 = nullptr;
-  uint32_t* part = nullptr;
-};
 constexpr size_t EMA_READOUT_MAX_D = 1024;
 void launch_ema(emh_ctx* c, float* pos, float* usage, const float* sums, const uint32_t* counts,
                 size_t k, size_t d, float alpha, float decay, int replace, float* norms = nullptr,
@@ -475,14 +482,15 @@ inline size_t scatter_chunks(size_t n) { return (n + TALLY_CP - 1) / TALLY_CP; }
 inline size_t tally_stride(size_t n) { return (scatter_chunks(n) + 3) & ~(size_t)3; }
 // Centroids split ahead of the call (launch_lines or launch_halves over the k
 // centroids, or kept up to date through CentsOut), with the bound's centroid
-// maxima in nparts groups of four words (|c|^2, cnorm, residual; halves: the
-// first two of every four, too).
+// maxima in nparts groups of four words (see CentsOut; halves: the first two).
+// Without cs, the scale and the mean alone, for the call's own split.
 struct SplitCents {
   const void* cs = nullptr;
   const uint32_t* part = nullptr;
   int nparts = 0;
   bool f16 = false;  // fp16 halves (else lines)
   const float* scale = nullptr;
+  const float* mean = nullptr;
 };
 // pre: x's rows already split, pc: the centroids (used when the call takes
 // the split-operand screen; see split_screen).
@@ -497,9 +505,9 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
 // Whether top-1 calls of n rows with d dimensions and k centroids take a
 // split-operand screen, whose rows a caller may split ahead.
 bool split_screen(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);
-// The centroids as lines in the context's scratch (one call's), scale given.
+// The centroids as lines in the context's scratch (one call's), scale and mean given.
 SplitCents split_cents(emh_ctx* c, const float* cents, size_t d, size_t k, const float* cnorm,
-                       const float* scale);
+                       const float* scale, const float* mean);
 // Whether top-1 calls of n rows with d dimensions and k centroids run a
 // screen (and so the check and the queued-row scan). A tallied call always
 // does, whatever its rows.
@@ -521,15 +529,22 @@ inline size_t halves_blocks(size_t n) { return (n + 7) / 8; }
 constexpr size_t PART_MAX_ONCE = 1024;
 // Rows as fp16 lines for the one-pass screen (emh_lines.h, emh_screen5.hip):
 // the scales of one or two selections of rows (b may be null), clearing nclear
-// words on the way; rows ids[lo .. lo + n) (or lo ..) of x as
-// lines in out (lines_bytes(n, d)) with (|x|^2, residual) in norm, and with
-// part each of the lines_blocks(n) blocks' maxima in part[4 b ..]; the maxima
-// over those.
+// words on the way; rows ids[lo .. lo + n) (or lo ..) of x, less mean when
+// given, as lines in out (lines_bytes(n, d)) with their squares and residuals
+// in norm, with part each of the lines_blocks(n) blocks' maxima in part[4 b ..]
+// (see CentsOut), and with `also` the rows themselves as lines there, too; the
+// maxima over those.
+struct LinesOut {
+  const float* scale;
+  void* out;
+  float2* norm;
+};
 void launch_scales(emh_ctx* c, size_t d, const ScaleIn& a, const ScaleIn* b, uint32_t* clear,
                    int nclear);
 void launch_lines(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
-                  size_t n, const float* scale, void* out, float2* norm, const float* cnorm,
-                  uint32_t* part);
+                  size_t n, const LinesOut& o, const float* cnorm = nullptr,
+                  uint32_t* part = nullptr, const float* mean = nullptr,
+                  const LinesOut* also = nullptr);
 inline size_t lines_blocks(size_t n) { return (n + 7) / 8; }
 void launch_part_max4(emh_ctx* c, const uint32_t* part, size_t nparts, uint32_t* out);
 // Bytes of fixed-block scratch launch_top1 takes for a call of n rows (an

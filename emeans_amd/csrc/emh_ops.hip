@@ -245,8 +245,7 @@ __device__ __forceinline__ float ema_mass(float u, uint32_t cnt, float alpha, fl
 // With co.cs (norms too), also the lines or halves of every updated row
 // (CentsOut, emh_halves.h), so the next batch's screen need not split the
 // centroids again (rows without members keep theirs), and the maxima of block
-// b's rows (f32 bits; a NaN wins) in co.part[4 b ..]: norms[] twice, and the
-// residuals.
+// b's rows (f32 bits; a NaN wins) in co.part[4 b ..], as CentsOut says.
 // Workgroup = EC clusters: the 256 threads update the clusters' positions
 // element by element, then lane c of the first wave adds cluster c's rounded
 // squares in order from LDS (rows padded by four floats so the EC lanes read
@@ -274,7 +273,7 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
   // EC rows of min(d, ECH) + 4 floats (norms, or readout): the rounded
   // squares; with co.cs or readout, then as many for the values.
   extern __shared__ __attribute__((aligned(16))) float sq[];
-  __shared__ float wgt[EC], cntf[EC], res[EC];
+  __shared__ float wgt[EC], cntf[EC], res[EC], dif[EC];
   const int tid = threadIdx.x;
   const size_t j0 = (size_t)blockIdx.x * EC;
   const int nc = (int)min((size_t)EC, k - j0);
@@ -289,7 +288,7 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
     usage[j0 + tid] = ema_mass(usage[j0 + tid], cnt, alpha, decay, replace, &weight);
     wgt[tid] = cnt > 0 ? weight : -1.0f;  // -1: no rows, position unchanged
     cntf[tid] = (float)cnt;
-    res[tid] = 0.0f;
+    res[tid] = dif[tid] = 0.0f;
   }
   __syncthreads();
   const int seg = (int)min(d, (size_t)ECH), row = ema_row(seg);
@@ -339,8 +338,8 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
     if (co.cs && tid >= WAVE) {
       // Waves 1-3 write the split rows of the pass's dimensions (c0 is a
       // multiple of 32; the last slab's dimensions past d are zero) while
-      // lanes of wave 0 run the chains. A row's residual is summed in any
-      // order: the bound allows for it.
+      // lanes of wave 0 run the chains. A row's residual and difference are
+      // summed in any order: the bound allows for it.
       const int nq = (((int)len + 31) & ~31) >> 2;  // quads in the pass
       for (int e = tid - WAVE; e < EC * nq; e += 256 - WAVE) {
         const int cc = e / nq, t = 4 * (e % nq);
@@ -349,8 +348,8 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
         const float4 v4 = make_float4(t < len ? vr[t] : 0.0f, t + 1 < len ? vr[t + 1] : 0.0f,
                                       t + 2 < len ? vr[t + 2] : 0.0f,
                                       t + 3 < len ? vr[t + 3] : 0.0f);
-        const float r = put_quad(co, k, j0 + cc, c0 + (size_t)t, v4);
-        if (co.scale) atomicAdd(&res[cc], r);
+        const float2 r = put_quad(co, k, j0 + cc, c0 + (size_t)t, v4);
+        if (co.scale) add_quad(r, &dif[cc], &res[cc]);
       }
     }
     if (tid < nc && wgt[tid] >= 0.0f) nrm = ordered_sum(sq + tid * row, len, nrm);  // in order
@@ -382,22 +381,25 @@ __global__ __launch_bounds__(256) void k_ema(float* __restrict__ pos, float* __r
   }
   if (norms && tid < nc && wgt[tid] >= 0.0f) norms[j0 + tid] = nrm;
   if (co.part && tid < WAVE) {
-    // (The last pass's barrier: every quad's residual is in.)
-    uint32_t m = 0u, mr = 0u;
+    // (The last pass's barrier: every quad's sums are in.)
+    uint32_t m = 0u, md = 0u, mr = 0u;
     if (tid < nc) {
       const bool moved = wgt[tid] >= 0.0f;
-      m = __float_as_uint(moved ? nrm : norms[j0 + tid]);
+      m = md = __float_as_uint(moved ? nrm : norms[j0 + tid]);
       if (co.scale) {
-        if (moved) co.norm2[j0 + tid].y = res[tid];
-        mr = __float_as_uint(moved ? res[tid] : co.norm2[j0 + tid].y);
+        const float2 v = moved ? make_float2(dif[tid], res[tid]) : co.norm2[j0 + tid];
+        if (moved) co.norm2[j0 + tid] = v;
+        md = __float_as_uint(v.x);
+        mr = __float_as_uint(v.y);
       }
     }
 #pragma unroll
     for (int o = 1; o < EC; o <<= 1) {
       m = max(m, (uint32_t)__shfl_xor((int)m, o, WAVE));
+      md = max(md, (uint32_t)__shfl_xor((int)md, o, WAVE));
       mr = max(mr, (uint32_t)__shfl_xor((int)mr, o, WAVE));
     }
-    if (tid == 0) reinterpret_cast<uint4*>(co.part)[blockIdx.x] = make_uint4(m, m, mr, 0u);
+    if (tid == 0) reinterpret_cast<uint4*>(co.part)[blockIdx.x] = make_uint4(md, m, mr, m);
   }
 }
 
@@ -538,10 +540,10 @@ __global__ __launch_bounds__(256) void k_split(float* __restrict__ pos, float* _
 // cluster), d <= SPLIT_FUSED_MAX_D, leaving also what the next batch reads of
 // the two rows it moves, as a full row_norms and halves pass would: norms[s]
 // and norms[t] (k_row_norms' in-order chain of the rounded squares); with
-// co.cs their lines or halves (CentsOut) and the larger of the two rows' norms
-// and residuals (f32 bits) in co.part[4 q ..], which the caller appends to the
-// bound's centroid partials. The partials of the
-// blocks the two rows were in stay upper bounds: no other row changed.
+// co.cs their lines or halves and the larger of the two rows' figures
+// (CentsOut) in co.part[4 q ..], which the caller appends to the bound's
+// centroid partials. The partials of the blocks the two rows were in stay
+// upper bounds: no other row changed.
 // Workgroup q = pair q. LDS: the two rows' values, then their squares, each
 // row ema_row(d) floats.
 __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
@@ -551,13 +553,13 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
                                                      const CentsOut co) {
   extern __shared__ __attribute__((aligned(16))) float sl[];
   __shared__ int diff;
-  __shared__ float nv[2], rv[2];
+  __shared__ float nv[2], rv[2], dv[2];
   const int tid = threadIdx.x, q = blockIdx.x, len = (int)d, row = ema_row(len);
   float* vs = sl;
   float* sq = sl + 2 * row;
   const uint32_t s = pairs[2 * q], t = pairs[2 * q + 1];
   if (tid == 0) diff = 0;
-  if (tid < 2) rv[tid] = 0.0f;
+  if (tid < 2) rv[tid] = dv[tid] = 0.0f;
   __syncthreads();
   float* cs = pos + (size_t)s * d;
   float* ct = pos + (size_t)t * d;
@@ -606,8 +608,8 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
       const float4 v4 = make_float4(c4 < len ? vr[c4] : 0.0f, c4 + 1 < len ? vr[c4 + 1] : 0.0f,
                                     c4 + 2 < len ? vr[c4 + 2] : 0.0f,
                                     c4 + 3 < len ? vr[c4 + 3] : 0.0f);
-      const float res = put_quad(co, k, r ? t : s, (size_t)c4, v4);
-      if (co.scale) atomicAdd(&rv[r], res);
+      const float2 res = put_quad(co, k, r ? t : s, (size_t)c4, v4);
+      if (co.scale) add_quad(res, &dv[r], &rv[r]);
     }
   }
   if (tid < 2) {
@@ -617,11 +619,12 @@ __global__ __launch_bounds__(256) void k_split_fused(float* __restrict__ pos,
   }
   if (co.part) {
     __syncthreads();
-    if (tid < 2 && co.scale) co.norm2[tid ? t : s].y = rv[tid];
+    if (tid < 2 && co.scale) co.norm2[tid ? t : s] = make_float2(dv[tid], rv[tid]);
     if (tid == 0) {
       const uint32_t m = max(__float_as_uint(nv[0]), __float_as_uint(nv[1]));
+      const uint32_t md = max(__float_as_uint(dv[0]), __float_as_uint(dv[1]));
       const uint32_t mr = max(__float_as_uint(rv[0]), __float_as_uint(rv[1]));
-      reinterpret_cast<uint4*>(co.part)[q] = make_uint4(m, m, mr, 0u);
+      reinterpret_cast<uint4*>(co.part)[q] = make_uint4(co.scale ? md : m, m, mr, m);
     }
   }
 }

@@ -905,7 +905,7 @@ __global__ __launch_bounds__(256) void k_margin(
     size_t nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int ip,
     const Cand* __restrict__ cand, int per_row, const float* __restrict__ xnorm,
     const uint32_t* __restrict__ small, int bound, unsigned long long* __restrict__ out,
-    const uint32_t* __restrict__ ncand, int L) {
+    const uint32_t* __restrict__ ncand, int L, const float* __restrict__ mean) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nrows * (size_t)per_row) return;
   const size_t r = e / (size_t)per_row;
@@ -927,7 +927,10 @@ __global__ __launch_bounds__(256) void k_margin(
                                      __uint_as_float(small[SW_CNMAX]), d, !ip, bound, &edot);
   if (bound == BOUND_LINES) edot = xnorm[nrows + r];
   if (!isfinite(kx) || !isfinite(E) || !(E > 0.f) || !(edot > 0.f)) return;
-  const float dk = fabsf(cd.key - kx);
+  double off = 0.0;  // the screen's keys are off by x.mean, whatever the centroid
+  if (mean)
+    for (int t = 0; t < d; t++) off += (double)xr[t] * (double)mean[t];
+  const float dk = (float)fabs((double)cd.key - ((double)kx + (ip ? off : 2.0 * off)));
   const float ratio = dk / E;
   const float u = 5.9604645e-08f;
   const float allow = (ip ? 0.f : 1.0000002f * u * (fabsf(cd.key) + fabsf(kx))) +
@@ -947,7 +950,7 @@ __global__ __launch_bounds__(256) void k_margin(
 void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                    size_t lo, size_t n, const float* cents, const float* cnorm, bool ip,
                    const Cand* cand, int parts, int L, const float* xnorm, int bound,
-                   emh_screen_report* rep, const uint32_t* ncand) {
+                   emh_screen_report* rep, const uint32_t* ncand, const float* mean) {
   unsigned long long* w = nullptr;
   EMH_HIP(hipMalloc(&w, 4 * sizeof(unsigned long long)));
   unsigned long long h[4] = {0, 0, 0, 0};
@@ -956,7 +959,7 @@ void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
     const size_t total = n * (size_t)parts * L;
     hipLaunchKernelGGL(k_margin, grid1(total, 256), dim3(256), 0, c->stream, x, nx, (int)d, ids,
                        lo, n, cents, cnorm, ip ? 1 : 0, cand, parts * L, xnorm, c->small, bound,
-                       w, ncand, L);
+                       w, ncand, L, mean);
     EMH_HIP(hipGetLastError());
     EMH_HIP(hipMemcpyAsync(h, w, sizeof h, hipMemcpyDeviceToHost, c->stream));
     EMH_HIP(hipStreamSynchronize(c->stream));

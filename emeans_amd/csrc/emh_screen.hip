@@ -135,17 +135,17 @@ bool top1_tallies(emh_ctx* c, size_t n, size_t d, size_t k, bool ip) {
 }
 
 SplitCents split_cents(emh_ctx* c, const float* cents, size_t d, size_t k, const float* cnorm,
-                       const float* scale) {
-  void* cw = c->csplit.get(lines_bytes(k, d));
+                       const float* scale, const float* mean) {
+  const LinesOut o{scale, c->csplit.get(lines_bytes(k, d)), (float2*)c->csplit_norm.get(k * 8)};
   const size_t nb = lines_blocks(k);
   uint32_t* pw = (uint32_t*)c->csplit_part.get((nb + 1) * 16);
-  launch_lines(c, cents, k, d, nullptr, 0, k, scale, cw, (float2*)c->csplit_norm.get(k * 8), cnorm,
-               pw);
+  launch_lines(c, cents, k, d, nullptr, 0, k, o, cnorm, pw, mean);
   SplitCents s;
-  s.cs = cw;
+  s.cs = o.out;
   s.part = pw;
   s.nparts = (int)nb;
   s.scale = scale;
+  s.mean = mean;
   if (nb > PART_MAX_ONCE) {
     launch_part_max4(c, pw, nb, pw + 4 * nb);
     s.part = pw + 4 * nb;
@@ -174,6 +174,7 @@ struct Top1Screen {
   float* xnorm = nullptr;
   BoundKind bound = BOUND_F32;
   int L = L1;  // entries per part list
+  const float* mean = nullptr;  // BOUND_LINES: the keys are off by x.mean (L2: 2 x.mean)
 };
 
 Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
@@ -217,11 +218,14 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
     // centroids' lines, then the selection's.
     const float* sx = pre ? pre->scale : nullptr;
     const float* sc = pc ? pc->scale : nullptr;
+    if (sc) s.mean = pc->mean;
     if (!sx || !sc) {
       float* wx = c->scales + 2 * SCALE_ROWS;
       float* wc = c->scales + 2 * SCALE_CENTS;
       const int nclear = words_clear ? 0 : 3;
-      const ScaleIn ix{x, nx, ids, lo, n, wx, -50}, ic{cents, k, nullptr, 0, k, wc, -50};
+      float* mean = sc ? nullptr : (float*)c->cmean.get(mean_floats(d) * 4);
+      if (!sc) s.mean = mean;
+      const ScaleIn ix{x, nx, ids, lo, n, wx, -50}, ic{cents, k, nullptr, 0, k, wc, -50, mean};
       launch_scales(c, d, sx ? ic : ix, !sx && !sc ? &ic : nullptr, c->small, nclear);
       if (!sx) sx = wx;
       if (!sc) sc = wc;
@@ -234,7 +238,7 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
       a.part = pc->part;
       a.nparts = pc->nparts;
     } else {
-      const SplitCents own = split_cents(c, cents, d, k, ip ? nullptr : cnorm, sc);
+      const SplitCents own = split_cents(c, cents, d, k, ip ? nullptr : cnorm, sc, s.mean);
       a.cs = own.cs;
       a.part = own.part;
       a.nparts = own.nparts;
@@ -247,12 +251,11 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
       a.ids = ids;
       a.lo = lo;
     } else {
-      void* xs = c->xsplit.get(lines_bytes(n, d));
-      float2* xn = (float2*)c->xsplit_norm.get(n * 8);
-      launch_lines(c, x, nx, d, ids, lo, n, sx, xs, xn, nullptr, nullptr);
-      a.xs = xs;
+      const LinesOut o{sx, c->xsplit.get(lines_bytes(n, d)), (float2*)c->xsplit_norm.get(n * 8)};
+      launch_lines(c, x, nx, d, ids, lo, n, o);
+      a.xs = o.out;
       a.xslab = n * LINE_BYTES;
-      a.xn = xn;
+      a.xn = o.norm;
       a.nx = n;
     }
     a.n = n;
@@ -376,7 +379,7 @@ void screen_margin_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const u
   out->parts = s.g.parts;
   out->tiles_per_part = s.g.tpp;
   launch_margin(c, x, nx, d, ids, lo, n, cents, cnorm, ip, s.cand, s.g.parts, s.L, s.xnorm,
-                s.bound, out, s.ncand);
+                s.bound, out, s.ncand, s.mean);
 }
 
 void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
@@ -393,14 +396,15 @@ void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t
     // The one-pass large-tile screen, then the same check.
     Cand* cand = nullptr;
     float* xnorm = nullptr;
-    const int parts = screen5_knn(c, q, m, data, n, d, kk, exclude_self, &cand, &xnorm);
+    const float* mean = nullptr;
+    const int parts = screen5_knn(c, q, m, data, n, d, kk, exclude_self, &cand, &xnorm, &mean);
     if (rep) {
       *rep = emh_screen_report{};
       rep->variant = EMH_SCREEN_BIG_KNN;
       rep->parts = parts;
       rep->tiles_per_part = 0;
       launch_margin(c, q, m, d, nullptr, 0, m, data, nullptr, true, cand, parts, LK, xnorm,
-                    BOUND_LINES, rep);
+                    BOUND_LINES, rep, nullptr, mean);
       return;
     }
     uint32_t* fb = (uint32_t*)c->fblist.get(m * 4);

@@ -44,14 +44,14 @@ __device__ __forceinline__ int swz5(int r) { return (((r >> 2) & 1) << 1) | ((r 
 // LDS by address (the ring's stage is a run-time value).
 typedef const v8h __attribute__((address_space(3)))* lds8h;
 
-// Maxima of part[4 i .. 4 i + 2] over i < nparts (f32 bits as u32: a NaN or
+// Maxima of part[4 i .. 4 i + 3] over i < nparts (f32 bits as u32: a NaN or
 // negative value wins), in every lane of the wave; each lane's loads of a
 // batch are issued together.
 __device__ __forceinline__ void part_max4(const uint32_t* __restrict__ part, int nparts,
-                                          uint32_t& ma, uint32_t& mb, uint32_t& mc) {
+                                          uint32_t& ma, uint32_t& mb, uint32_t& mc, uint32_t& md) {
   constexpr int B = 8;
   const int lane = threadIdx.x & 63;
-  ma = mb = mc = 0u;
+  ma = mb = mc = md = 0u;
   for (int i0 = 0; i0 < nparts; i0 += 64 * B) {
     uint4 v[B];
 #pragma unroll
@@ -64,12 +64,14 @@ __device__ __forceinline__ void part_max4(const uint32_t* __restrict__ part, int
       ma = max(ma, v[u].x);
       mb = max(mb, v[u].y);
       mc = max(mc, v[u].z);
+      md = max(md, v[u].w);
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
     ma = max(ma, (uint32_t)__shfl_xor((int)ma, o, 64));
     mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
     mc = max(mc, (uint32_t)__shfl_xor((int)mc, o, 64));
+    md = max(md, (uint32_t)__shfl_xor((int)md, o, 64));
   }
 }
 
@@ -102,7 +104,7 @@ struct Args5 {
   Cand* log;              // blocks x 512 x LOG5_* entries of scratch (parts of several tiles)
   float* bound;           // out: E of row r at r, its dot term at bstride + r
   size_t bstride;
-  const uint32_t* part;   // the centroids' maxima (launch_lines' part)
+  const uint32_t* part;   // the centroids' maxima (CentsOut)
   int nparts;
   const float* sx;        // scales: s, 1 / s
   const float* sc;
@@ -217,8 +219,8 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   const float f1 = a_.sx[1] * a_.sc[1];  // accumulator -> dot, a power of two
   const float rf1 = a_.sx[0] * a_.sc[0];  // its inverse
   {
-    uint32_t ma, mb, mc;
-    part_max4(a_.part, a_.nparts, ma, mb, mc);
+    uint32_t ma, mb, mc, md;
+    part_max4(a_.part, a_.nparts, ma, mb, mc, md);
     const int r = row0 + (tid & (T5 - 1));
     float2 xv = make_float2(0.f, 0.f);
     if (r < nrows) {
@@ -227,9 +229,9 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
       xv = a_.xn[id < a_.nx ? id : 0];
     }
     float edot;
-    const float E = screen_bound_lines(xv.x, xv.y, __uint_as_float(ma), __uint_as_float(mc),
-                                       L2 ? __uint_as_float(mb) : 0.f, a_.sx[1], a_.sc[1], a_.d,
-                                       L2, &edot);
+    const float E = screen_bound_lines(xv.x, xv.y, __uint_as_float(md), __uint_as_float(ma),
+                                       __uint_as_float(mc), L2 ? __uint_as_float(mb) : 0.f,
+                                       a_.sx[1], a_.sc[1], a_.d, L2, &edot);
     thr_q = 2.0f * 1.0078125f * E;
     if (part == 0 && wc == 0 && r < nrows) {
       a_.bound[r] = E;

@@ -14,15 +14,18 @@ namespace {
 // step apart could miss the same columns of every row); rows of the selection,
 // because the others may hold anything. 8 bits of fp16's range are left above
 // the sample and 21 normal ones below; elements beyond that cost their row the
-// exact scan (a centroid's or a data row's: every row of the call). Also clears
-// `clear` (nclear words). A thread a column: latency-bound, its loads in flight
+// exact scan (a centroid's or a data row's: every row of the call). With
+// in.mean: the rows' mean and the scale of the differences, where the mean
+// holds a quarter of the rows' squares or more (the mean of 32 rows without one
+// holds a 32nd, and would only add to them); else zeros. Also clears `clear`
+// (nclear words). A thread a column: latency-bound, its loads in flight
 // together.
-constexpr int SCALE_LOADS = 32;
 __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn b, int d, int rows,
                                                  uint32_t* __restrict__ clear, int nclear) {
+  constexpr int R = SCALE_ROWS_READ, NT = 1024;
   const ScaleIn in = blockIdx.x ? b : a;
-  __shared__ const float* rp[SCALE_ROWS_READ];
-  __shared__ float wm[16];
+  __shared__ const float* rp[R];
+  __shared__ float wr[4][NT / 64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0 && tid < nclear) clear[tid] = 0u;
   const int nr = (int)min((size_t)rows, in.n);
@@ -36,50 +39,89 @@ __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn 
     rp[tid] = in.p + (id < in.nx ? id : 0) * (size_t)d;
   }
   __syncthreads();
-  float m = 0.f;
-  for (int t = tid; t < d; t += 1024)
-    for (int i0 = 0; i0 < nr; i0 += SCALE_LOADS) {
-      float v[SCALE_LOADS];
+  // Largest element and difference; squares of the rows and of the mean.
+  float mv = 0.f, mc = 0.f, sv = 0.f, sm = 0.f;
+  const float inv = 1.0f / (float)nr;
+  for (int t = tid; t < d; t += NT) {
+    float v[R];
 #pragma unroll
-      for (int u = 0; u < SCALE_LOADS; u++) v[u] = rp[min(i0 + u, nr - 1)][t];
+    for (int u = 0; u < R; u++) v[u] = rp[min(u, nr - 1)][t];
+    float m = 0.f;
 #pragma unroll
-      for (int u = 0; u < SCALE_LOADS; u++) {
-        const float e = fabsf(v[u]);
-        m = e < INFINITY ? fmaxf(m, e) : m;  // NaN and infinities say nothing of the scale
-      }
+    for (int u = 0; u < R; u++) {
+      // NaN and infinities say nothing; past the rows read: not counted.
+      v[u] = u < nr && fabsf(v[u]) < INFINITY ? v[u] : 0.f;
+      mv = fmaxf(mv, fabsf(v[u]));
+      sv = fmaf(v[u], v[u], sv);
+      m = fmaf(v[u], inv, m);
     }
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if (lane == 0) wm[w] = m;
+    if (in.mean) {
+#pragma unroll
+      for (int u = 0; u < R; u++) mc = u < nr ? fmaxf(mc, fabsf(v[u] - m)) : mc;
+      sm = fmaf(m, m, sm);
+      in.mean[t] = m;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    mv = fmaxf(mv, __shfl_xor(mv, o, 64));
+    mc = fmaxf(mc, __shfl_xor(mc, o, 64));
+    sv += __shfl_xor(sv, o, 64);
+    sm += __shfl_xor(sm, o, 64);
+  }
+  if (lane == 0) {
+    wr[0][w] = mv;
+    wr[1][w] = mc;
+    wr[2][w] = sv;
+    wr[3][w] = sm;
+  }
   __syncthreads();
+  mv = mc = sv = sm = 0.f;
+  for (int i = 0; i < NT / 64; i++) {
+    mv = fmaxf(mv, wr[0][i]);
+    mc = fmaxf(mc, wr[1][i]);
+    sv += wr[2][i];
+    sm += wr[3][i];
+  }
+  const bool use = in.mean && sv < INFINITY && sm > 0.f && 4.0f * (float)nr * sm >= sv;
+  if (in.mean)
+    for (int t = (use ? d : 0) + tid; t < (d + LINE_DIMS - 1) / LINE_DIMS * LINE_DIMS; t += NT)
+      in.mean[t] = 0.f;
   if (tid == 0) {
-    for (int i = 1; i < 16; i++) m = fmaxf(m, wm[i]);
     int e = 8;  // zeros: scale 1
+    const float m = use ? mc : mv;
     if (m > 0.f) frexpf(m, &e);  // m in [2^(e - 1), 2^e)
+    if (use) {  // (rows that all but agree: any other row as long as they are stays in range)
+      int ev;
+      frexpf(mv, &ev);
+      e = m > 0.f ? max(e, ev - 6) : ev - 6;
+    }
     e = max(max(-50, in.emin), min(e, 60));  // two inverse scales' product stays a normal f32
     in.out[0] = ldexpf(1.0f, 8 - e);
     in.out[1] = ldexpf(1.0f, e - 8);
   }
 }
 
-// Rows ids[lo + g] (lo + g without ids; an id >= nx reads row 0) for g < n as
-// fp16 lines in out (emh_lines.h, scale[0]), in selection order; norm[g] =
-// (|x|^2, the residual), f32 sums in any order. With part: block b writes the
-// largest |x|^2 of its rows, with cnorm the largest cnorm[g], and the largest
-// residual (f32 bits; a NaN wins) to part[4 b .. 4 b + 2].
+// Rows ids[lo + g] (lo + g without ids; an id >= nx reads row 0) for g < n,
+// less `mean` when given, as fp16 lines (emh_lines.h) in o.out, in selection
+// order; o.norm[g] = (their squares, the residual), f32 sums in any order. With
+// BOTH, the rows themselves as lines in p, too. With part: block b writes the
+// largest square of its rows, with cnorm the largest cnorm[g], the largest
+// residual and the largest |x|^2 (f32 bits; a NaN wins) to part[4 b ..].
 // Block b takes rows 8 b .. 8 b + 7, two per wave. HBM-bound: a wave reads a
 // row in 256-dimension segments, 16 contiguous bytes per lane, and eight lanes
 // fill one 64-byte line; the wave's two rows share a cache line in each slab.
-template <bool VEC4>
+template <bool VEC4, bool MEAN, bool BOTH>
 __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size_t nx, int d,
                                                const uint32_t* __restrict__ ids, size_t lo,
-                                               size_t n, const float* __restrict__ scale,
-                                               char* __restrict__ out, float2* __restrict__ norm,
+                                               size_t n, const LinesOut o, const LinesOut p,
+                                               const float* __restrict__ mean,
                                                const float* __restrict__ cnorm,
                                                uint32_t* __restrict__ part) {
+  static_assert(MEAN || !BOTH, "two lines of a row only where they differ");
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int d32 = (d + LINE_DIMS - 1) / LINE_DIMS, nseg = (d32 + 7) >> 3;
   const int js = lane >> 3, q = lane & 7;
-  const float s = scale[0];
+  const float s = o.scale[0], sp = BOTH ? p.scale[0] : 0.f;
   size_t g[2];
   bool valid[2];
   const float* xr[2];
@@ -94,13 +136,18 @@ __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size
     }
     xr[i] = x + id * (size_t)d;
   }
-  float sq[2] = {0.f, 0.f}, rs[2] = {0.f, 0.f};
+  auto square = [](float4 v, float a) __attribute__((always_inline)) {
+    return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, fmaf(v.x, v.x, a))));
+  };
+  // Squares and residuals: the lines' (sv, rv), the rows' (sx, rx with BOTH).
+  float sv[2] = {0.f, 0.f}, rv[2] = {0.f, 0.f}, sx[2] = {0.f, 0.f}, rx[2] = {0.f, 0.f};
 #pragma unroll 3
   for (int sg = 0; sg < nseg; sg++) {
     const int j = 8 * sg + js;
     if (j >= d32) break;
     const int col = LINE_DIMS * j + 4 * q;
-    float4 v[2];
+    float4 v[2], m = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (MEAN) m = *reinterpret_cast<const float4*>(mean + col);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       if (VEC4) {
@@ -114,55 +161,66 @@ __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      sq[i] = fmaf(v[i].x, v[i].x, sq[i]);
-      sq[i] = fmaf(v[i].y, v[i].y, sq[i]);
-      sq[i] = fmaf(v[i].z, v[i].z, sq[i]);
-      sq[i] = fmaf(v[i].w, v[i].w, sq[i]);
-      const uint2 hv = line_quad(v[i], s, rs[i]);
-      if (valid[i])
-        *reinterpret_cast<uint2*>(out + ((size_t)j * n + g[i]) * LINE_BYTES + 8 * q) = hv;
+      const size_t at = ((size_t)j * n + g[i]) * LINE_BYTES + 8 * q;
+      if (MEAN) {
+        sx[i] = square(v[i], sx[i]);
+        if (BOTH) {
+          const uint2 hv = line_quad(v[i], sp, rx[i]);
+          if (valid[i]) *reinterpret_cast<uint2*>((char*)p.out + at) = hv;
+        }
+        v[i] = make_float4(v[i].x - m.x, v[i].y - m.y, v[i].z - m.z, v[i].w - m.w);
+      }
+      sv[i] = square(v[i], sv[i]);
+      const uint2 hv = line_quad(v[i], s, rv[i]);
+      if (valid[i]) *reinterpret_cast<uint2*>((char*)o.out + at) = hv;
     }
   }
 #pragma unroll
   for (int i = 0; i < 2; i++) {
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-      sq[i] += __shfl_xor(sq[i], m, 64);
-      rs[i] += __shfl_xor(rs[i], m, 64);
+    for (int k = 32; k > 0; k >>= 1) {
+      sv[i] += __shfl_xor(sv[i], k, 64);
+      rv[i] += __shfl_xor(rv[i], k, 64);
+      if (MEAN) sx[i] += __shfl_xor(sx[i], k, 64);
+      if (BOTH) rx[i] += __shfl_xor(rx[i], k, 64);
     }
-    if (valid[i] && lane == 0) norm[g[i]] = make_float2(sq[i], rs[i]);
+    if (!MEAN) sx[i] = sv[i];
+    if (valid[i] && lane == 0) {
+      o.norm[g[i]] = make_float2(sv[i], rv[i]);
+      if (BOTH) p.norm[g[i]] = make_float2(sx[i], rx[i]);
+    }
   }
   if (part) {
-    uint32_t ma = 0u, mb = 0u, mc = 0u;
+    uint32_t mx[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       if (valid[i]) {
-        ma = max(ma, __float_as_uint(sq[i]));
-        if (cnorm) mb = max(mb, __float_as_uint(cnorm[g[i]]));
-        mc = max(mc, __float_as_uint(rs[i]));
+        mx[0] = max(mx[0], __float_as_uint(sv[i]));
+        if (cnorm) mx[1] = max(mx[1], __float_as_uint(cnorm[g[i]]));
+        mx[2] = max(mx[2], __float_as_uint(rv[i]));
+        mx[3] = max(mx[3], __float_as_uint(sx[i]));
       }
     }
-    __shared__ uint32_t red[3][4];
+    __shared__ uint32_t red[4][4];
     if (lane == 0) {
-      red[0][w] = ma;
-      red[1][w] = mb;
-      red[2][w] = mc;
+#pragma unroll
+      for (int e = 0; e < 4; e++) red[e][w] = mx[e];
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
+    if (threadIdx.x < 4) {
       const uint32_t* r = red[threadIdx.x];
       part[4 * blockIdx.x + threadIdx.x] = max(max(r[0], r[1]), max(r[2], r[3]));
     }
   }
 }
 
-// out[0 .. 2] = the maxima of part[4 i .. 4 i + 2] over i < nparts.
+// out[0 .. 3] = the maxima of part[4 i .. 4 i + 3] over i < nparts.
 __global__ __launch_bounds__(1024) void k_part_max4(const uint32_t* __restrict__ part,
                                                     size_t nparts, uint32_t* __restrict__ out) {
   constexpr int B = 8;
-  __shared__ uint32_t wm[3][16];
+  __shared__ uint32_t wm[4][16];
   const int tid = threadIdx.x;
-  uint32_t ma = 0u, mb = 0u, mc = 0u;
+  uint32_t m[4] = {0u, 0u, 0u, 0u};
   for (size_t i0 = 0; i0 < nparts; i0 += 1024 * B) {
     uint4 v[B];
 #pragma unroll
@@ -172,26 +230,22 @@ __global__ __launch_bounds__(1024) void k_part_max4(const uint32_t* __restrict__
     }
 #pragma unroll
     for (int u = 0; u < B; u++) {
-      ma = max(ma, v[u].x);
-      mb = max(mb, v[u].y);
-      mc = max(mc, v[u].z);
+      m[0] = max(m[0], v[u].x);
+      m[1] = max(m[1], v[u].y);
+      m[2] = max(m[2], v[u].z);
+      m[3] = max(m[3], v[u].w);
     }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    ma = max(ma, (uint32_t)__shfl_xor((int)ma, o, 64));
-    mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
-    mc = max(mc, (uint32_t)__shfl_xor((int)mc, o, 64));
-  }
-  if ((tid & 63) == 0) {
-    wm[0][tid >> 6] = ma;
-    wm[1][tid >> 6] = mb;
-    wm[2][tid >> 6] = mc;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    for (int o = 32; o > 0; o >>= 1) m[e] = max(m[e], (uint32_t)__shfl_xor((int)m[e], o, 64));
+    if ((tid & 63) == 0) wm[e][tid >> 6] = m[e];
   }
   __syncthreads();
-  if (tid < 3) {
-    uint32_t m = 0u;
-    for (int i = 0; i < 16; i++) m = max(m, wm[tid][i]);
-    out[tid] = m;
+  if (tid < 4) {
+    uint32_t r = 0u;
+    for (int i = 0; i < 16; i++) r = max(r, wm[tid][i]);
+    out[tid] = r;
   }
 }
 
@@ -207,18 +261,23 @@ void launch_scales(emh_ctx* c, size_t d, const ScaleIn& a, const ScaleIn* b, uin
                    int nclear) {
   EMH_ENSURE(a.n > 0 && a.nx > 0 && (!b || (b->n > 0 && b->nx > 0)), "scales: no rows");
   hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, b ? *b : a, (int)d,
-                     d <= 2048 ? SCALE_ROWS_READ : SCALE_ROWS_READ / 4, clear, nclear);
+                     d <= 2048 ? SCALE_ROWS_READ : SCALE_ROWS_READ / 2, clear, nclear);
   EMH_HIP(hipGetLastError());
 }
 
 void launch_lines(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
-                  size_t n, const float* scale, void* out, float2* norm, const float* cnorm,
-                  uint32_t* part) {
+                  size_t n, const LinesOut& o, const float* cnorm, uint32_t* part,
+                  const float* mean, const LinesOut* also) {
   if (n == 0) return;
-  EMH_ENSURE(d >= 1 && n < (1u << 31), "lines: shape out of range");
-  auto kern = d % 4 == 0 ? k_lines<true> : k_lines<false>;
+  EMH_ENSURE(d >= 1 && n < (1u << 31) && (mean || !also), "lines: shape out of range");
+  auto kern = d % 4 == 0 ? (also   ? k_lines<true, true, true>
+                            : mean ? k_lines<true, true, false>
+                                   : k_lines<true, false, false>)
+                         : (also   ? k_lines<false, true, true>
+                            : mean ? k_lines<false, true, false>
+                                   : k_lines<false, false, false>);
   hipLaunchKernelGGL(kern, dim3((unsigned)lines_blocks(n)), dim3(256), 0, c->stream, x, nx, (int)d,
-                     ids, lo, n, scale, (char*)out, norm, cnorm, part);
+                     ids, lo, n, o, also ? *also : o, mean, cnorm, part);
   EMH_HIP(hipGetLastError());
 }
 
@@ -284,20 +343,22 @@ bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d) {
 
 void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
             uint32_t* clear, int nclear, Split5* s) {
-  // The data's lines once (with their norms, residuals and the maxima of
-  // both); the queries' too, unless they are the data.
+  // The data's lines less their mean (with their norms, residuals and the
+  // maxima of both), and the queries' as they are: of the same rows, in one
+  // pass over them.
   const bool same = q == data && m == n;
   float* sc = c->scales + 2 * SCALE_CENTS;
-  float* sx = same ? sc : c->scales + 2 * SCALE_ROWS;
-  const ScaleIn is{data, n, nullptr, 0, n, sc, -50}, iq{q, m, nullptr, 0, m, sx, -50};
-  launch_scales(c, d, is, same ? nullptr : &iq, clear, nclear);
-  void* xs = c->csplit.get(lines_bytes(n, d));
-  float2* xn = (float2*)c->csplit_norm.get(n * 8);
+  float* sx = c->scales + 2 * SCALE_ROWS;
+  float* mean = (float*)c->cmean.get(mean_floats(d) * 4);
+  const ScaleIn is{data, n, nullptr, 0, n, sc, -50, mean}, iq{q, m, nullptr, 0, m, sx, -50};
+  launch_scales(c, d, is, &iq, clear, nclear);
+  const LinesOut xo{sc, c->csplit.get(lines_bytes(n, d)), (float2*)c->csplit_norm.get(n * 8)};
+  const LinesOut qo{sx, c->xsplit.get(lines_bytes(m, d)), (float2*)c->xsplit_norm.get(m * 8)};
   // Past PART_MAX_ONCE partials, one workgroup reduces them ahead of the
   // screen, whose every block would otherwise read them all.
   const size_t hb = lines_blocks(n);
   uint32_t* part = (uint32_t*)c->csplit_part.get((hb + 1) * 16);
-  launch_lines(c, data, n, d, nullptr, 0, n, sc, xs, xn, nullptr, part);
+  launch_lines(c, data, n, d, nullptr, 0, n, xo, nullptr, part, mean, same ? &qo : nullptr);
   s->part = part;
   s->nparts = (int)hb;
   if (hb > PART_MAX_ONCE) {
@@ -305,15 +366,11 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
     s->part = part + 4 * hb;
     s->nparts = 1;
   }
-  s->cs = s->xs = xs;
-  s->xn = xn;
-  if (!same) {
-    void* qw = c->xsplit.get(lines_bytes(m, d));
-    float2* qnw = (float2*)c->xsplit_norm.get(m * 8);
-    launch_lines(c, q, m, d, nullptr, 0, m, sx, qw, qnw, nullptr, nullptr);
-    s->xs = qw;
-    s->xn = qnw;
-  }
+  if (!same) launch_lines(c, q, m, d, nullptr, 0, m, qo);
+  s->cs = xo.out;
+  s->xs = qo.out;
+  s->xn = qo.norm;
+  s->mean = mean;
   s->sx = sx;
   s->sc = sc;
   s->m = m;
@@ -322,7 +379,8 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
 }
 
 int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                size_t kk, bool exclude_self, Cand** cand_out, float** bound_out) {
+                size_t kk, bool exclude_self, Cand** cand_out, float** bound_out,
+                const float** mean_out) {
   Split5 s;
   split5(c, q, m, data, n, d, c->small, 3, &s);
   const int row_tiles = (int)((m + T5 - 1) / T5);
@@ -375,6 +433,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   }
   *cand_out = cand;
   *bound_out = bound;
+  *mean_out = s.mean;
   return parts;
 }
 

@@ -226,21 +226,21 @@ inline int parts5(int row_tiles, int ntiles, int cus, int maxp, double fixed) {
   }
   return best;
 }
-// The lines of m queries and n data rows in the context's scratch (the queries'
-// are the data's when they are the same rows), with the data's maxima in part;
-// clears nclear words of clear on the way.
+// The lines of m queries and of n data rows less their mean in the context's
+// scratch, with the data's maxima in part; clears nclear words of clear on the
+// way.
 struct Split5 {
   const void *xs, *cs;
   const float2* xn;
   const uint32_t* part;
   int nparts;
-  const float *sx, *sc;
+  const float *sx, *sc, *mean;
   size_t m, n, d;
 };
 void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
             uint32_t* clear, int nclear, Split5* s);
-// Every dot of queries q0 .. q0 + nb with the data, as the one-pass screen sees
-// them, into scores (row r at r ldS; the ldS - n columns past the data hold
+// Every dot of queries q0 .. q0 + nb with the data less their mean (a query's
+// all off by the same), as the one-pass screen sees them, into scores (row r at r ldS; the ldS - n columns past the data hold
 // anything), and the bound E on their distance from the exact chains into
 // bound[0 .. nb) (its dot term in bound[nb ..)).
 void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* scores, size_t ldS,
@@ -250,7 +250,7 @@ void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* sc
 // and its dot term at bound[m + r]; in the context's scratch); returns the parts.
 bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d);
 int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                size_t kk, bool exclude_self, Cand** cand, float** bound);
+                size_t kk, bool exclude_self, Cand** cand, float** bound, const float** mean);
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                     size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
                     float* sims, uint32_t* fb, int bound);
@@ -262,7 +262,8 @@ void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, siz
 void launch_margin(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                    size_t lo, size_t n, const float* cents, const float* cnorm, bool ip,
                    const Cand* cand, int parts, int L, const float* xnorm, int bound,
-                   emh_screen_report* rep, const uint32_t* ncand = nullptr);
+                   emh_screen_report* rep, const uint32_t* ncand = nullptr,
+                   const float* mean = nullptr);
 // ---- emh_verify.hip: the exact scans
 // Exact scan of rows `list[0..*count)` (list != nullptr) or positions lo..lo+n.
 // ar: take the scratch from this fixed block (see Arena) instead of the context's buffers.

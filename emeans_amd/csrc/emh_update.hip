@@ -12,7 +12,7 @@
 //   - adds them in that order from +0 (a thread a column), as k_sums;
 //   - moves the centroid from the sums in registers, as k_ema: the position,
 //     then either the squared norm (one lane adds the rounded squares in
-//     order) with the bf16 halves and the bound's maximum, or the spherical
+//     order) with the split row and the bound's maxima, or the spherical
 //     readout (v / max|v| over its sqrt of the in-order sum of squares);
 //   - updates the mass and the epoch's count, and clears its count and the
 //     tally's chunk histograms for the next batch.
@@ -106,8 +106,13 @@ __device__ __forceinline__ float ordered_sum(const float* v, int len) {
 // Cluster j's own group of the bound's maxima.
 __device__ __forceinline__ void put_part(const CentsOut& o, size_t j, float norm) {
   const uint32_t m = __float_as_uint(norm);
-  reinterpret_cast<uint4*>(o.part)[j] =
-      make_uint4(m, m, o.scale ? __float_as_uint(o.norm2[j].y) : 0u, 0u);
+  uint4 g = make_uint4(m, m, 0u, m);
+  if (o.scale) {
+    const float2 v = o.norm2[j];
+    g.x = __float_as_uint(v.x);
+    g.z = __float_as_uint(v.y);
+  }
+  reinterpret_cast<uint4*>(o.part)[j] = g;
 }
 
 template <int NB>
@@ -117,7 +122,7 @@ struct SmallLds {
   float nv[UPDATE_SMALL_MAX_D];      // the new row, for its split
   float wmax[UT / 64];               // readout: each wave's max |v|
   uint32_t cnt;
-  float weight, rnorm, res;
+  float weight, rnorm, dif, res;
 };
 
 // Cluster j = blockIdx.x, a thread per column in whole waves; a batch of at
@@ -232,15 +237,15 @@ __global__ __launch_bounds__(UT) void k_update_small(
   }
   // The split row, with the zero columns of the last slab.
   if (co.cs) {
-    if (tid == 0) L.res = 0.0f;
+    if (tid == 0) L.dif = L.res = 0.0f;
     L.nv[tid] = v;
     __syncthreads();
     if (tid < (int)(((d + 31) & ~(size_t)31) / 4)) {
       const int t = 4 * tid;
       const float4 q = t < (int)d ? *reinterpret_cast<const float4*>(L.nv + t)
                                   : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      const float r = put_quad(co, k, j, (size_t)t, q);  // zeros past d
-      if (co.scale) atomicAdd(&L.res, r);  // in any order: the bound allows for it
+      const float2 r = put_quad(co, k, j, (size_t)t, q);  // zeros past d
+      if (co.scale) add_quad(r, &L.dif, &L.res);  // in any order: the bound allows for it
     }
   }
   if (norms) {
@@ -249,7 +254,7 @@ __global__ __launch_bounds__(UT) void k_update_small(
       const float nrm = ordered_sum(L.sq, (int)d);
       norms[j] = nrm;
       if (co.part) {
-        if (co.scale) co.norm2[j].y = L.res;
+        if (co.scale) co.norm2[j] = make_float2(L.dif, L.res);
         put_part(co, j, nrm);
       }
     }

@@ -231,3 +231,65 @@ def test_top1_rows_outside_selection(dev):
         assert np.array_equal(dev.read_u32(lab)[:20000], ol)
         assert dev.read_f32(sco)[:20000].tobytes() == os_.tobytes()
         assert dev.fallback_rows() - f0 < 200
+
+
+def _common(n, d, s, seed, unit=True):
+    """Rows that share most of their length: a mean and noise s times it."""
+    x = 1.0 + s * np.random.default_rng(seed).standard_normal((n, d))
+    if unit:
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+@pytest.mark.parametrize("n,d,k", [(40000, 33, 256), (16384, 64, 1024), (16384, 128, 2500)])
+def test_top1_common_mean(dev, metric, n, d, k):
+    """The screen's error follows the centroids' distance from their mean, not
+    their length: next to no row goes to the exact scan."""
+    x, c = _common(n, d, 0.1, 71, metric == "ip"), _common(k, d, 0.1, 72, metric == "ip")
+    f0 = dev.fallback_rows()
+    _top1(dev, x, c, metric)
+    assert dev.fallback_rows() - f0 < n // 20
+    from emeans_amd import Mat, Select
+    cb, cn = dev.upload_f32(c), None
+    if metric == "l2":
+        cn = dev.zeros_f32(k)
+        dev.row_norms(cb, k, d, cn)
+    r = dev.screen_margin(Mat(dev.bind(x), d), Select(None, (0, n)), cb, cn, k, metric)
+    assert r["pairs"] > n // 2 and r["over"] == 0 and r["max_dot_ratio"] <= 0.5, r
+
+
+@pytest.mark.parametrize("n,d,s", [(3000, 64, 0.2), (3001, 384, 0.3), (4000, 100, 0.1)])
+def test_knn_common_mean(dev, n, d, s):
+    x = _common(n, d, s, 73)
+    f0 = dev.fallback_rows()
+    _knn(dev, x, x, 10, True)
+    _knn(dev, x[::7].copy(), x, 10, False)
+    assert dev.fallback_rows() - f0 < n // 10
+    _knn(dev, x[:2000].copy(), x, 60, False)
+    r = dev.screen_margin_topk(dev.bind(x), n, dev.bind(x), n, d, True)
+    assert r["pairs"] > n and r["over"] == 0 and r["max_dot_ratio"] <= 0.5, r
+
+
+@pytest.mark.parametrize("spherical", [False, True])
+@pytest.mark.parametrize("n,d,k,batch,s", [
+    (40000, 64, 700, 16384, 0.15),   # the EMA's lines, revivals
+    (30000, 36, 300, 16384, 3.0),
+    (12000, 32, 8200, 1024, 0.2),    # the small batches' lines
+])
+def test_train_common_mean(dev, n, d, k, batch, s, spherical):
+    from emeans_amd import Config
+    x = _common(n, d, s, 74, spherical)
+    x[: n // 2] += (0.3 * x[0]).astype(np.float32)  # two densities, so that some centroids die
+    if spherical:
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+    cfg = Config(d=d, k=k, nepochs=2, batch_size=batch, spherical=spherical, seed=3)
+    f0 = dev.fallback_rows()
+    cent, info = dev.train_dev(dev.bind(x), n, cfg)
+    o = O.train(x, d, k, nepochs=cfg.nepochs, batch_size=cfg.batch_size, alpha0=cfg.alpha0,
+                batch_law=cfg.batch_law, seed=cfg.seed, spherical=cfg.spherical,
+                unused_threshold=cfg.unused_threshold)
+    assert np.array_equal(info["labels"], o["labels"])
+    assert info["positions"].tobytes() == o["positions"].tobytes()
+    assert cent.tobytes() == o["centroids"].tobytes()
+    assert dev.fallback_rows() - f0 < n // 5
