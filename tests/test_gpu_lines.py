@@ -293,3 +293,16 @@ def test_train_common_mean(dev, n, d, k, batch, s, spherical):
     assert info["positions"].tobytes() == o["positions"].tobytes()
     assert cent.tobytes() == o["centroids"].tobytes()
     assert dev.fallback_rows() - f0 < n // 5
+
+
+@pytest.mark.parametrize("d", [32, 36, 61, 64, 65, 96, 127, 128, 129])
+def test_top1_narrow_rows(dev, d):
+    """The lines of rows of up to 128 dimensions: one, two and four slabs a
+    row, their remainders, and the first width past them."""
+    n, k = 16411, 520
+    x, c = _rows(n, d, 81), _rows(k, d, 82)
+    ids = ((np.arange(n, dtype=np.uint64) * 7919 + 3) % n).astype(np.uint32)
+    for i in (None, ids):
+        f0 = dev.fallback_rows()
+        _top1(dev, x, c, "ip", i)
+        assert dev.fallback_rows() - f0 < n // 50
