@@ -22,10 +22,11 @@ namespace {
 // together.
 __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn b, int d, int rows,
                                                  uint32_t* __restrict__ clear, int nclear) {
-  constexpr int R = SCALE_ROWS_READ, NT = 1024;
+  constexpr int R = SCALE_ROWS_READ;
+  const int NT = (int)blockDim.x;
   const ScaleIn in = blockIdx.x ? b : a;
   __shared__ const float* rp[R];
-  __shared__ float wr[4][NT / 64];
+  __shared__ float4 wr[16];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0 && tid < nclear) clear[tid] = 0u;
   const int nr = (int)min((size_t)rows, in.n);
@@ -68,19 +69,15 @@ __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn 
     sv += __shfl_xor(sv, o, 64);
     sm += __shfl_xor(sm, o, 64);
   }
-  if (lane == 0) {
-    wr[0][w] = mv;
-    wr[1][w] = mc;
-    wr[2][w] = sv;
-    wr[3][w] = sm;
-  }
+  if (lane == 0) wr[w] = make_float4(mv, mc, sv, sm);
   __syncthreads();
   mv = mc = sv = sm = 0.f;
   for (int i = 0; i < NT / 64; i++) {
-    mv = fmaxf(mv, wr[0][i]);
-    mc = fmaxf(mc, wr[1][i]);
-    sv += wr[2][i];
-    sm += wr[3][i];
+    const float4 o = wr[i];
+    mv = fmaxf(mv, o.x);
+    mc = fmaxf(mc, o.y);
+    sv += o.z;
+    sm += o.w;
   }
   const bool use = in.mean && sv < INFINITY && sm > 0.f && 4.0f * (float)nr * sm >= sv;
   if (in.mean)
@@ -309,7 +306,8 @@ void launch5(emh_ctx* c, unsigned blocks, const Args5& a) {
 void launch_scales(emh_ctx* c, size_t d, const ScaleIn& a, const ScaleIn* b, uint32_t* clear,
                    int nclear) {
   EMH_ENSURE(a.n > 0 && a.nx > 0 && (!b || (b->n > 0 && b->nx > 0)), "scales: no rows");
-  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(1024), 0, c->stream, a, b ? *b : a, (int)d,
+  const unsigned nt = (unsigned)std::min<size_t>((d + 63) / 64 * 64, 1024);  // a column each
+  hipLaunchKernelGGL(k_scales, dim3(b ? 2 : 1), dim3(nt), 0, c->stream, a, b ? *b : a, (int)d,
                      d <= 2048 ? SCALE_ROWS_READ : SCALE_ROWS_READ / 2, clear, nclear);
   EMH_HIP(hipGetLastError());
 }
