@@ -177,6 +177,31 @@ struct Top1Screen {
   const float* mean = nullptr;  // BOUND_LINES: the keys are off by x.mean (L2: 2 x.mean)
 };
 
+// The one-pass screen's scales and the centroids' mean: the caller's, or this
+// call's, in one launch that also clears the screen's words.
+struct Frames {
+  const float *sx, *sc, *mean;
+};
+Frames top1_frames(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids, size_t lo,
+                   size_t n, const float* cents, size_t k, const SplitRows* pre,
+                   const SplitCents* pc, bool& words_clear) {
+  Frames f{pre ? pre->scale : nullptr, pc ? pc->scale : nullptr, pc ? pc->mean : nullptr};
+  if (f.sx && f.sc) return f;
+  float* wx = c->scales + 2 * SCALE_ROWS;
+  float* wc = c->scales + 2 * SCALE_CENTS;
+  float* mean = f.sc ? nullptr : (float*)c->cmean.get(mean_floats(d) * 4);
+  const ScaleIn ix{x, nx, ids, lo, n, wx, -50}, ic{cents, k, nullptr, 0, k, wc, -50, mean};
+  launch_scales(c, d, f.sx ? ic : ix, !f.sx && !f.sc ? &ic : nullptr, c->small,
+                words_clear ? 0 : 3);
+  words_clear = true;
+  if (!f.sx) f.sx = wx;
+  if (!f.sc) {
+    f.sc = wc;
+    f.mean = mean;
+  }
+  return f;
+}
+
 Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids,
                        size_t lo, size_t n, const float* cents, const float* cnorm, size_t k,
                        bool ip, bool words_clear, Arena* ar, const SplitRows* pre,
@@ -213,24 +238,11 @@ Top1Screen screen_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const ui
     EMH_ENSURE(!pc || pc->f16 == f16, "top1: centroids split in the other format");
   }
   if (g.split && !f16) {
-    // The one-pass screen. Scales and lines that the caller did not bring:
-    // the matrices' scales in one launch (which also clears the words), the
+    // The one-pass screen. What the caller did not bring: the scales, the
     // centroids' lines, then the selection's.
-    const float* sx = pre ? pre->scale : nullptr;
-    const float* sc = pc ? pc->scale : nullptr;
-    if (sc) s.mean = pc->mean;
-    if (!sx || !sc) {
-      float* wx = c->scales + 2 * SCALE_ROWS;
-      float* wc = c->scales + 2 * SCALE_CENTS;
-      const int nclear = words_clear ? 0 : 3;
-      float* mean = sc ? nullptr : (float*)c->cmean.get(mean_floats(d) * 4);
-      if (!sc) s.mean = mean;
-      const ScaleIn ix{x, nx, ids, lo, n, wx, -50}, ic{cents, k, nullptr, 0, k, wc, -50, mean};
-      launch_scales(c, d, sx ? ic : ix, !sx && !sc ? &ic : nullptr, c->small, nclear);
-      if (!sx) sx = wx;
-      if (!sc) sc = wc;
-      words_clear = true;
-    }
+    const Frames f = top1_frames(c, x, nx, d, ids, lo, n, cents, k, pre, pc, words_clear);
+    const float *sx = f.sx, *sc = f.sc;
+    s.mean = f.mean;
     clear_words();
     Lines5 a{};
     if (pc && pc->cs) {
@@ -347,6 +359,26 @@ void launch_top1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t
   // A tallying call takes the screen, or the latency-bound exact scan, which
   // tallies too; never k_exact1.
   const bool small_exact = !tally || queued_direct(c, n, d, k, ip);
+  // Large selections on the one-pass screen go a piece at a time (a multiple of
+  // the tally's chunks), which bounds the copy of the rows as lines and their
+  // lists (1,056 bytes a row at eight parts); scales and centroids once.
+  constexpr size_t PIECE = size_t(1) << 20;
+  static_assert(PIECE % TALLY_CP == 0, "a piece starts a tally chunk");
+  if (n > PIECE && !ar && c->screen != SCREEN_F16 &&
+      top1_geom(c, PIECE, d, k, ip, true, small_exact).split) {
+    const Frames f = top1_frames(c, x, nx, d, ids, lo, n, cents, k, pre, pc, words_clear);
+    SplitRows pr = pre ? *pre : SplitRows{};
+    pr.scale = f.sx;
+    const SplitCents cc = pc && pc->cs ? *pc
+                                       : split_cents(c, cents, d, k, ip ? nullptr : cnorm, f.sc,
+                                                     f.mean);
+    for (size_t b = lo; b < hi; b += PIECE) {
+      launch_top1(c, x, nx, d, ids, b, std::min(b + PIECE, hi), cents, cnorm, k, ip, labels, scores,
+                  words_clear, nullptr, &pr, &cc, tally);
+      words_clear = false;
+    }
+    return;
+  }
   const Top1Screen s = screen_top1(c, x, nx, d, ids, lo, n, cents, cnorm, k, ip, words_clear, ar,
                                    pre, pc, small_exact);
   EMH_ENSURE(!tally || (d % 4 == 0 && (s.g.screen || queued_direct(c, n, d, k, ip))),

@@ -306,3 +306,22 @@ def test_top1_narrow_rows(dev, d):
         f0 = dev.fallback_rows()
         _top1(dev, x, c, "ip", i)
         assert dev.fallback_rows() - f0 < n // 50
+
+
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+def test_top1_pieces(dev, metric):
+    """A selection of more rows than one piece, by ids and from an odd start."""
+    from emeans_amd import Mat, Select
+    n, d, k, lo = (1 << 20) + 70001, 32, 300, 5
+    x, c = _rows(n, d, 91), _rows(k, d, 92)
+    ids = ((np.arange(n, dtype=np.uint64) * 7919 + 3) % n).astype(np.uint32)
+    cb, cn = dev.upload_f32(c), None
+    if metric == "l2":
+        cn = dev.zeros_f32(k)
+        dev.row_norms(cb, k, d, cn)
+    lab, sco = dev.zeros_u32(n), dev.zeros_f32(n)
+    dev.top1(Mat(dev.bind(x), d), Select(dev.upload_u32(ids), (lo, n)), cb, cn, k, metric, lab, sco)
+    ol, os_ = np.zeros(n, np.uint32), np.zeros(n, np.float32)
+    O.top1(x, d, c, metric, ids=ids, rows=(lo, n), labels=ol, scores=os_)
+    assert np.array_equal(dev.read_u32(lab), ol)
+    assert dev.read_f32(sco).tobytes() == os_.tobytes()
