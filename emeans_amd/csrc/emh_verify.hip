@@ -7,7 +7,8 @@
 //              a selection without the screen, and queued rows when d % 4 != 0;
 //  k_queued1   top-1 for the rows the check queues (d % 4 == 0): short
 //              (4 rows x 16 centroids) items, one burst of DMA copies and one
-//              chain per lane each, the winners folded by 64-bit atomics;
+//              chain per lane each, the winners folded by 64-bit atomics; long
+//              queues in tiles of 128 x 128;
 //  k_small1    top-1 for a small direct selection against at most 64
 //              centroids (d % 4 == 0): a block holds all of them and its rows,
 //              so a row's winner is found inside a wave;
@@ -350,21 +351,223 @@ __device__ __forceinline__ void slot_copy(const float* src, v4f* slots) {
   }
 }
 
+// Long queues (more than MANY row-centroid pairs: rows crowded beyond what the
+// screen's bound can tell apart) take tiles instead: 128 rows against 128
+// centroids at a time, a thread 8 x 8 chains, slabs of MD dimensions
+// double-buffered in LDS. Bound by the fmas. Item = (128 rows, a range of
+// centroid tiles), its winners folded by the same words and tickets (one a row
+// tile); the first item of a row tile also runs the rows' |x|^2 for L2.
+// 65,536 rows against 1,024 centroids, d = 768, every row queued: 1.7 ms for the
+// whole call; as short items, 27.8.
+constexpr int MR = 128, MD = 16, MP = MR + 4;
+constexpr uint64_t MANY = 1u << 20;
+
+struct QueuedLds {
+  float xs[2][MD][MP], cs[2][MD][MP];  // a slab of the rows, of the centroids
+  uint32_t rid[MR];
+  int last;
+};
+
 template <bool AL>
-__global__ __launch_bounds__(64) void k_queued1(
+__device__ __forceinline__ void queued_tiles(
+    QueuedLds& L, const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids,
+    int nrows, const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
+    const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
+    unsigned long long* __restrict__ best, uint32_t* __restrict__ tickets,
+    float* __restrict__ xnq, uint32_t* __restrict__ labels, float* __restrict__ scores,
+    uint32_t* __restrict__ tcnt, uint32_t* __restrict__ tcounts, size_t tlo, size_t tstride) {
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int nrt = (nrows + MR - 1) / MR, nct = (k + MR - 1) / MR;
+  const int want = min(nct, max(1, ((int)gridDim.x + nrt - 1) / nrt));
+  const int tpp = (nct + want - 1) / want, parts = (nct + tpp - 1) / tpp;
+  for (int item = blockIdx.x; item < nrt * parts; item += gridDim.x) {
+    const int rt = item / parts, q = item - rt * parts;
+    __syncthreads();  // the previous item is done with L
+    if (tid < MR) {
+      const int f = rt * MR + tid;
+      uint32_t xid = NONE;
+      if (f < nrows) {
+        const size_t p = (size_t)list[f];
+        const size_t id = ids ? (size_t)ids[p] : p;
+        if (id < nx)
+          xid = (uint32_t)id;
+        else
+          small[SW_BAD_ID] = 1;
+      }
+      L.rid[tid] = xid;
+    }
+    __syncthreads();
+    // Loader: 16-byte piece e = 256 u + tid of a slab is row e / 4, dimensions
+    // 4 (e % 4) .. + 3 (d % 4 == 0: all of them in or all past d).
+    const float* xr[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const uint32_t r = L.rid[(256 * u + tid) >> 2];
+      xr[u] = x + (size_t)(r == NONE ? 0u : r) * d + 4 * (tid & 3);
+    }
+    v4f xv[2], cv[2];
+    auto piece = [&](const float* p, int t) __attribute__((always_inline)) {
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      if (t < d) {
+        if (AL) {
+          v = *reinterpret_cast<const v4f*>(p);
+        } else {
+          v4f s = {p[0], p[1], p[2], p[3]};
+          v = s;
+        }
+      }
+      return v;
+    };
+    auto load = [&](int ct, int t0) __attribute__((always_inline)) {
+      const int t = t0 + 4 * (tid & 3);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        xv[u] = piece(xr[u] + t0, t);
+        const int j = min(ct * MR + ((256 * u + tid) >> 2), k - 1);
+        cv[u] = piece(cents + (size_t)j * d + t, t);
+      }
+    };
+    auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int r = (256 * u + tid) >> 2, t = 4 * (tid & 3);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          L.xs[b][t + e][r] = xv[u][e];
+          L.cs[b][t + e][r] = cv[u][e];
+        }
+      }
+    };
+    float bk[8];
+    uint32_t bi[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+      bk[a] = INFINITY;
+      bi[a] = NONE;
+    }
+    float nrm = 0.f;
+    const int c0 = q * tpp, c1 = min(nct, c0 + tpp);
+    for (int ct = c0; ct < c1; ct++) {
+      float acc[8][8];
+#pragma unroll
+      for (int a = 0; a < 8; a++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[a][e] = 0.f;
+      auto dim = [&](int b, int t) __attribute__((always_inline)) {
+        float xa[8], ca[8];
+#pragma unroll
+        for (int a = 0; a < 8; a++) xa[a] = L.xs[b][t][ty * 8 + a];
+#pragma unroll
+        for (int e = 0; e < 8; e++) ca[e] = L.cs[b][t][(e >> 2) * 64 + tx * 4 + (e & 3)];
+#pragma unroll
+        for (int a = 0; a < 8; a++)
+#pragma unroll
+          for (int e = 0; e < 8; e++) acc[a][e] = fmaf(xa[a], ca[e], acc[a][e]);
+      };
+      load(ct, 0);
+      store(0);
+      __syncthreads();
+      for (int t0 = 0, b = 0; t0 < d; t0 += MD, b ^= 1) {
+        const bool more = t0 + MD < d;
+        if (more) load(ct, t0 + MD);
+        const int tn = min(MD, d - t0);  // dimensions past d never enter a chain
+        if (tn == MD) {
+#pragma unroll
+          for (int t = 0; t < MD; t++) dim(b, t);
+        } else {
+          for (int t = 0; t < tn; t++) dim(b, t);
+        }
+        if (!ip && q == 0 && ct == 0 && tid < MR)
+          for (int t = 0; t < tn; t++) {
+            const float v = L.xs[b][t][tid];
+            nrm = nrm + v * v;
+          }
+        if (more) store(b ^ 1);
+        __syncthreads();
+      }
+      // A thread's columns come in rising order: the lower id wins ties.
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int j = ct * MR + (e >> 2) * 64 + tx * 4 + (e & 3);
+        if (j < k) {
+          const float cn = ip ? 0.f : cnorm[j];
+#pragma unroll
+          for (int a = 0; a < 8; a++) {
+            const float key = ip ? -acc[a][e] : cn - 2.0f * acc[a][e];
+            if (key < bk[a]) {  // (NaN or +inf never)
+              bk[a] = key;
+              bi[a] = (uint32_t)j;
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+      uint64_t w = bi[a] == NONE ? 0ull : pack_best(bk[a], bi[a]);
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) {
+        const uint64_t w2 = __shfl_xor(w, o, WAVE);
+        w = w2 > w ? w2 : w;
+      }
+      const int f = rt * MR + ty * 8 + a;
+      if (tx == 0 && w != 0 && f < nrows) atomicMax(&best[f], (unsigned long long)w);
+    }
+    const int f = rt * MR + tid;
+    if (!ip && q == 0 && tid < MR && f < nrows)
+      __hip_atomic_store(&xnq[f], nrm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) L.last = atomicAdd(&tickets[rt], 1u) == (uint32_t)(parts - 1);
+    __syncthreads();
+    if (!L.last) continue;
+    __threadfence();
+    if (tid < MR && f < nrows) {
+      const unsigned long long w = atomicExch(&best[f], 0ull);
+      if (L.rid[tid] != NONE) {
+        float bkey = INFINITY;
+        uint32_t bid = 0;  // nothing wins: label 0 and the initial score
+        unpack_best(w, bkey, bid);
+        const size_t p = (size_t)list[f];
+        labels[p] = bid;
+        scores[p] = ip ? -bkey
+                       : fmaxf(__hip_atomic_load(&xnq[f], __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) + bkey, 0.0f);
+        if (tcnt) {
+          atomicAdd(&tcnt[(size_t)bid * tstride + (p - tlo) / TALLY_CP], 1u);
+          atomicAdd(&tcounts[bid], 1u);
+        }
+      }
+    }
+    if (tid == 0) tickets[rt] = 0;
+  }
+}
+
+// (Four waves; short items take the first alone.)
+template <bool AL>
+__global__ __launch_bounds__(256) void k_queued1(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     int n_direct, const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
     const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
     unsigned long long* __restrict__ best, uint32_t* __restrict__ tickets,
     float* __restrict__ xnq, uint32_t* __restrict__ labels, float* __restrict__ scores,
     uint32_t* __restrict__ tcnt, uint32_t* __restrict__ tcounts, size_t tlo, size_t tstride) {
-  __shared__ v4f cs[QU * QJ];
-  __shared__ v4f xs[QU * QR];
+  __shared__ __attribute__((aligned(16))) char lds[(QU * QJ + QU * QR) * sizeof(v4f)];
+  static_assert(sizeof(QueuedLds) <= sizeof(lds), "tiles");
+  v4f* const cs = reinterpret_cast<v4f*>(lds);
+  v4f* const xs = cs + QU * QJ;
   __shared__ uint32_t xid_s[QR];
   // Queued rows (list: positions, count on the device), or a direct
   // selection of n_direct rows at positions lo, lo + 1, ...
   const int nrows = list ? (int)small[SW_FALLBACK_COUNT] : n_direct;
   if (list && blockIdx.x == 0 && threadIdx.x == 0) small[SW_FALLBACK_TOTAL] += (uint32_t)nrows;
+  if (list && (uint64_t)nrows * (uint64_t)k > MANY) {
+    queued_tiles<AL>(*reinterpret_cast<QueuedLds*>(lds), x, nx, d, ids, nrows, list, small, cents,
+                     cnorm, k, ip, best, tickets, xnq, labels, scores, tcnt, tcounts, tlo,
+                     tstride);
+    return;
+  }
+  if (threadIdx.x >= WAVE) return;
   const int nch = (k + QJ - 1) / QJ;
   const int per = nch + (ip ? 0 : 1);  // items per group (the last one: |x|^2)
   const int ngr = (nrows + QR - 1) / QR;
@@ -778,7 +981,7 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
     }
     const unsigned g = (unsigned)std::min<size_t>(ngr * per, (size_t)2 * c->cus);
     auto kern = aligned16(x, cents) ? k_queued1<true> : k_queued1<false>;
-    hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo,
+    hipLaunchKernelGGL(kern, dim3(g), dim3(256), 0, c->stream, x, nx, (int)d, ids, lo,
                        (int)n, list, c->small, cents, cnorm, (int)k, ip ? 1 : 0,
                        (unsigned long long*)z,
                        (uint32_t*)(z + n * 8), xnq, labels, scores,
