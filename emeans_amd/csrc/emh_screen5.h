@@ -281,7 +281,8 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     const float lim = limit_of(b);
     float g = L2 ? -lim : -lim * rf1;
     if (!L2) g = g - fabsf(g) * 2.384185791015625e-07f - 1e-44f;
-    g = live ? fmaxf(g, -3.4028235e38f) : __builtin_nanf("");  // (padding's -inf is never within it)
+    // (Padding's -inf is never within it; a row that has spilt appends no more.)
+    g = live && !spilt ? fmaxf(g, -3.4028235e38f) : __builtin_nanf("");
     const float gp = __shfl_xor(g, 32, 64);
     gl[0] = h == 0 ? g : gp;
     gl[1] = h == 1 ? g : gp;
