@@ -82,3 +82,44 @@ def test_queued_tiles_train(dev, spherical):
     assert np.array_equal(info["labels"], o["labels"])
     assert info["positions"].tobytes() == o["positions"].tobytes()
     assert cent.tobytes() == o["centroids"].tobytes()
+
+
+@pytest.mark.parametrize("m,n,d,kk,self_", [
+    (700, 3000, 32, 10, False),    # parts of several tiles, the last a remainder
+    (1, 5, 40, 16, False),         # fewer data rows than neighbours
+    (33, 129, 20, 1, False),       # one past a query tile and a data tile; no screen
+    (300, 20000, 33, 16, False),   # 64 parts
+    (2900, 2900, 64, 16, True),
+    (20000, 600, 36, 3, False),    # more query tiles than workgroups: one part
+])
+def test_queued_knn(dev, m, n, d, kk, self_):
+    g = np.random.default_rng(m + n)
+    x = _crowds(n, d, 97, 5)
+    q = x if self_ else g.standard_normal((m, d)).astype(np.float32)
+    if n > 500:
+        x[n // 2, 1], x[n // 3, 2], x[11] = np.nan, np.inf, 0.0
+        q[5 % m] = 0.0                       # every score +0 or -0
+        x[20:60] *= np.where(g.random((40, 1)) < 0.5, -1, 1).astype(np.float32)
+        q[6 % m, 0] = np.nan
+    f0 = dev.fallback_rows()
+    gi, gs = dev.topk(q, x, d, kk, self_)
+    oi, os_ = O.knn(q, x, d, kk, self_)
+    assert np.array_equal(gi, oi)
+    assert gs.tobytes() == os_.tobytes()
+    assert dev.fallback_rows() - f0 >= m // 2
+
+
+def test_queued_knn_few(dev):
+    """A few queued queries among many: the parts' lists and their ranking, call
+    after call (the tickets are left at zero)."""
+    g = np.random.default_rng(8)
+    n, d, m = 9000, 48, 600
+    x = _crowds(n, d, 1, 9)
+    x[4000:4200] = x[4000]
+    q = g.standard_normal((m, d)).astype(np.float32)
+    q[::50] = x[4000] + np.float32(0.01) * q[::50]
+    for kk in (1, 7, 16):
+        gi, gs = dev.topk(q, x, d, kk, False)
+        oi, os_ = O.knn(q, x, d, kk, False)
+        assert np.array_equal(gi, oi)
+        assert gs.tobytes() == os_.tobytes()
