@@ -453,10 +453,10 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   const int tpp = (ntiles + parts - 1) / parts;
   Cand* cand = (Cand*)c->cand.get((size_t)parts * m * LK * sizeof(Cand));
   float* bound = (float*)c->xnorm.get(2 * m * 4);
-  // A launch's threads each keep a log (1 MB a block): a launch is one wave of
-  // blocks, 256 MB on 256 CUs (all pairs of 500,000 x 384: 192.6 ms; four waves
-  // a launch, 1 GB, 195.0).
-  const int rt_step = std::max(1, std::max(c->cus, 1) / parts);
+  // A launch's threads each keep a log (1 MB a block): launches of whole waves
+  // of blocks, at most four.
+  const int wave = std::max(1, std::max(c->cus, 1) / parts);
+  const int rt_step = 4 * wave;
   Cand* log = (Cand*)c->log5.get((size_t)std::min(rt_step, row_tiles) * parts * 512 * LOG5_KNN *
                                  sizeof(Cand));
   Args5 a{};
