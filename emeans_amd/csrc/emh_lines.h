@@ -40,8 +40,12 @@ inline size_t lines_bytes(size_t n, size_t d) {
 
 typedef _Float16 v4h_l __attribute__((ext_vector_type(4)));
 
-// A mean's floats: zeros past d, so that whole lines can read it.
-inline size_t mean_floats(size_t d) { return (d + LINE_DIMS - 1) / LINE_DIMS * LINE_DIMS; }
+// A mean's floats: zeros past d, so that whole lines can read it, then whether
+// it is one (1) or all zeros (0).
+__host__ __device__ inline size_t mean_flag(size_t d) {
+  return (d + LINE_DIMS - 1) / LINE_DIMS * LINE_DIMS;
+}
+inline size_t mean_floats(size_t d) { return mean_flag(d) + 4; }
 
 // Four scaled values rounded to fp16 (8 bytes of a line); res += the squares
 // of what the rounding left (exact differences: v and h are multiples of one

@@ -108,6 +108,8 @@ struct Args5 {
   int nparts;
   const float* sx;        // scales: s, 1 / s
   const float* sc;
+  const float* same;      // kNN: with *same == 0, the rows' lines, norms and scale are
+  const float2* cn;       // the data's (norms cn)
   float* scores;          // SCORES: out, row r's dots at r ldS (a multiple of 4, >= k)
   size_t ldS;
 };
@@ -117,7 +119,7 @@ template <int KIND, bool ONE>
 __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   constexpr bool L2 = KIND == TOP1_L2, SELF = KIND == KNN_SELF;
   constexpr bool TOPK = KIND == KNN || KIND == KNN_SELF;
-  constexpr bool LISTS = KIND != SCORES;
+  constexpr bool LISTS = KIND != SCORES, TOP1 = LISTS && !TOPK;
   constexpr int L = TOPK ? LK : L5, NK = TOPK ? KTH5 : 1, CAP = CAP5;
   constexpr int LOG = TOPK ? LOG5_KNN : LOG5_TOP1;
   constexpr int WA = 4, WN = 2;  // centroid (A) and row (B) 32-blocks per wave
@@ -168,10 +170,14 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   // into a stage nothing reads.
   int lt = t0, lj = 0;
   const int nsteps = (t1 - t0) * d32;
+  const bool own = TOP1 || !a_.same || *a_.same != 0.f;
+  const char* const xs0 = own ? a_.xs : a_.cs;
+  const float2* const xn0 = own ? a_.xn : a_.cn;
+  const float* const sx = own ? a_.sx : a_.sc;
   const uint32_t ring0 = lds_addr(ring);
   const uint32_t ldst = ring0 + (uint32_t)__builtin_amdgcn_readfirstlane(w) * 16 * LINE_BYTES;
   uint32_t ls = 0;                              // the load stage's offset in the ring
-  const char *xp = a_.xs, *cp = a_.cs + (size_t)t0 * T5 * LINE_BYTES;  // slab lj of the rows, the tile
+  const char *xp = xs0, *cp = a_.cs + (size_t)t0 * T5 * LINE_BYTES;  // slab lj of the rows, the tile
   auto dma_part = [&](int q) __attribute__((always_inline)) {
     const int j = q % ND;
     const uint32_t dst = ldst + ls + (q / ND) * S5_HALF + j * 128 * LINE_BYTES;
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     const bool wrap = ++lj == d32;
     lj = wrap ? 0 : lj;
     lt += wrap ? 1 : 0;
-    xp = wrap ? a_.xs : xp + a_.xslab;
+    xp = wrap ? xs0 : xp + a_.xslab;
     cp = wrap ? a_.cs + (size_t)min(lt, t1 - 1) * T5 * LINE_BYTES : cp + a_.cslab;
     ls = (ls + S5_STAGE) % (NS5 * S5_STAGE);
   };
@@ -216,8 +222,8 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   // from bound[], and the fold keeps what lies within 2E' (E' >= E, with a
   // margin for the rounding of the sums that use it).
   float thr_q;  // 2E' of the row this lane keeps (block h's)
-  const float f1 = a_.sx[1] * a_.sc[1];  // accumulator -> dot, a power of two
-  const float rf1 = a_.sx[0] * a_.sc[0];  // its inverse
+  const float f1 = sx[1] * a_.sc[1];  // accumulator -> dot, a power of two
+  const float rf1 = sx[0] * a_.sc[0];  // its inverse
   {
     uint32_t ma, mb, mc, md;
     part_max4(a_.part, a_.nparts, ma, mb, mc, md);
@@ -226,12 +232,12 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     if (r < nrows) {
       const size_t p = a_.lo + (size_t)r;
       const size_t id = a_.ids ? (size_t)a_.ids[p] : p;
-      xv = a_.xn[id < a_.nx ? id : 0];
+      xv = xn0[id < a_.nx ? id : 0];
     }
     float edot;
     const float E = screen_bound_lines(xv.x, xv.y, __uint_as_float(md), __uint_as_float(ma),
                                        __uint_as_float(mc), L2 ? __uint_as_float(mb) : 0.f,
-                                       a_.sx[1], a_.sc[1], a_.d, L2, &edot);
+                                       sx[1], a_.sc[1], a_.d, L2, &edot);
     thr_q = 2.0f * 1.0078125f * E;
     if (part == 0 && wc == 0 && r < nrows) {
       a_.bound[r] = E;

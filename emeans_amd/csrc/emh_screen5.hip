@@ -80,9 +80,10 @@ __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn 
     sm += o.w;
   }
   const bool use = in.mean && sv < INFINITY && sm > 0.f && 4.0f * (float)nr * sm >= sv;
-  if (in.mean)
-    for (int t = (use ? d : 0) + tid; t < (d + LINE_DIMS - 1) / LINE_DIMS * LINE_DIMS; t += NT)
-      in.mean[t] = 0.f;
+  if (in.mean) {
+    for (int t = (use ? d : 0) + tid; t < (int)mean_flag(d); t += NT) in.mean[t] = 0.f;
+    if (tid == 0) in.mean[mean_flag(d)] = use ? 1.f : 0.f;
+  }
   if (tid == 0) {
     int e = 8;  // zeros: scale 1
     const float m = use ? mc : mv;
@@ -101,7 +102,8 @@ __global__ __launch_bounds__(1024) void k_scales(const ScaleIn a, const ScaleIn 
 // Rows ids[lo + g] (lo + g without ids; an id >= nx reads row 0) for g < n,
 // less `mean` when given, as fp16 lines (emh_lines.h) in o.out, in selection
 // order; o.norm[g] = (their squares, the residual), f32 sums in any order. With
-// BOTH, the rows themselves as lines in p, too. With part: block b writes the
+// BOTH, the rows themselves as lines in p, too, unless the mean is all zeros
+// (they would be the same: the screen reads o's instead). With part: block b writes the
 // largest square of its rows, with cnorm the largest cnorm[g], the largest
 // residual and the largest |x|^2 (f32 bits; a NaN wins) to part[4 b ..].
 // Block b takes rows 8 b .. 8 b + 7, two per wave. HBM-bound: a wave reads a
@@ -120,6 +122,7 @@ __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size
   const int d32 = (d + LINE_DIMS - 1) / LINE_DIMS, nseg = (d32 + 7) >> 3;
   const int js = lane >> 3, q = lane & 7;
   const float s = o.scale[0], sp = BOTH ? p.scale[0] : 0.f;
+  const bool both = BOTH && mean[mean_flag(d)] != 0.f;
   size_t g[2];
   bool valid[2];
   const float* xr[2];
@@ -162,7 +165,7 @@ __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size
       const size_t at = ((size_t)j * n + g[i]) * LINE_BYTES + 8 * q;
       if (MEAN) {
         sx[i] = square(v[i], sx[i]);
-        if (BOTH) {
+        if (both) {
           const uint2 hv = line_quad(v[i], sp, rx[i]);
           if (valid[i]) *reinterpret_cast<uint2*>((char*)p.out + at) = hv;
         }
@@ -180,12 +183,12 @@ __global__ __launch_bounds__(256) void k_lines(const float* __restrict__ x, size
       sv[i] += __shfl_xor(sv[i], k, 64);
       rv[i] += __shfl_xor(rv[i], k, 64);
       if (MEAN) sx[i] += __shfl_xor(sx[i], k, 64);
-      if (BOTH) rx[i] += __shfl_xor(rx[i], k, 64);
+      if (both) rx[i] += __shfl_xor(rx[i], k, 64);
     }
     if (!MEAN) sx[i] = sv[i];
     if (valid[i] && lane == 0) {
       o.norm[g[i]] = make_float2(sv[i], rv[i]);
-      if (BOTH) p.norm[g[i]] = make_float2(sx[i], rx[i]);
+      if (both) p.norm[g[i]] = make_float2(sx[i], rx[i]);
     }
   }
   if (part) {
@@ -432,6 +435,11 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
   s->xs = qo.out;
   s->xn = qo.norm;
   s->mean = mean;
+  s->same = nullptr;
+  if (same) {
+    s->same = mean + mean_flag(d);
+    s->cn = xo.norm;
+  }
   s->sx = sx;
   s->sc = sc;
   s->m = m;
@@ -481,6 +489,8 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
                  prof_take(c, EMH_PROF_SCREEN));
   a.xs = (const char*)s.xs;
   a.xn = s.xn;
+  a.same = s.same;
+  a.cn = s.cn;
   a.nx = m;
   for (int r = 0; r < row_tiles; r += rt_step) {
     const size_t q0 = (size_t)r * T5, q1 = std::min((size_t)(r + rt_step) * T5, m);
@@ -510,6 +520,8 @@ void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* sc
   a.xs = (const char*)s.xs;
   a.xslab = s.m * (size_t)LINE_BYTES;
   a.xn = s.xn;
+  a.same = s.same;
+  a.cn = s.cn;
   a.nx = s.m;
   a.lo = q0;
   a.nrows = (int)nb;

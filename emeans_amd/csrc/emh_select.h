@@ -235,6 +235,10 @@ struct Split5 {
   const uint32_t* part;
   int nparts;
   const float *sx, *sc, *mean;
+  // Queries that are the data rows: where the word is 0 (no mean), their lines,
+  // norms and scale are the data's.
+  const float* same;
+  const float2* cn;
   size_t m, n, d;
 };
 void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
