@@ -124,9 +124,8 @@ __global__ __launch_bounds__(256) void k_verify(
     int nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
     int kk, const Cand* __restrict__ cand, int parts, const float* __restrict__ xnorm,
     uint32_t* __restrict__ labels, float* __restrict__ scores, uint32_t* __restrict__ fb,
-    uint32_t* __restrict__ small, int bound, const uint32_t* __restrict__ ncand) {
-  constexpr int CM = L == L5 ? C5 : C1;         // most candidates of a top-1 row
-  constexpr int PMAX = R * (KNN ? L : CM + 1);  // pairs (+ the |x|^2 chain per top-1 row)
+    uint32_t* __restrict__ small, int bound) {
+  constexpr int PMAX = R * (KNN ? L : C1 + 1);  // pairs (+ the |x|^2 chain per top-1 row)
   __shared__ Cand cst[R * MAX_PARTS * L];
   __shared__ uint32_t prow[PMAX], pcid[PMAX];
   __shared__ float pres[PMAX];
@@ -155,14 +154,8 @@ __global__ __launch_bounds__(256) void k_verify(
       for (int u = 0; u < 4; u++)
         if (i0 + 256 * u < ne) v[u] = src[i0 + 256 * u];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int i = i0 + 256 * u;
-        if (i >= ne) continue;
-        // (Lists with lengths: what was not written is no entry.)
-        if (ncand && (uint32_t)(i % L) >= list_length<L>(ncand[(size_t)r0 * parts + i / L]))
-          v[u] = make_uint2(__float_as_uint(INFINITY), NONE);
-        dst[i] = v[u];
-      }
+      for (int u = 0; u < 4; u++)
+        if (i0 + 256 * u < ne) dst[i0 + 256 * u] = v[u];
     }
   }
   __syncthreads();
@@ -190,7 +183,8 @@ __global__ __launch_bounds__(256) void k_verify(
     }
     int state = 0, nc = 0;
     if (rowid[tid] != NONE) {
-      const float E = row_bound(xnorm[r0 + tid], small, d, l2, bound);
+      const float E = screen_bound(xnorm[r0 + tid], __uint_as_float(small[SW_CMAX2]),
+                                   __uint_as_float(small[SW_CNMAX]), d, l2, bound);
       bool complete;
       if (KNN) {
         thr = key[kk - 1] + 2.0f * E;
@@ -211,15 +205,13 @@ __global__ __launch_bounds__(256) void k_verify(
         int tot = 0;
         for (int q = 0; q < parts; q++) {
           const Cand last = c[q * L + L - 1];
-          if (ncand ? ncand[(size_t)(r0 + tid) * parts + q] > (uint32_t)L
-                    : last.id != NONE && !(last.key > thr))
-            cert = false;
+          if (last.id != NONE && !(last.key > thr)) cert = false;
           for (int e = 0; e < L; e++) {
             const Cand v = c[q * L + e];
             tot += v.id != NONE && (v.key <= thr || thr != thr);
           }
         }
-        complete = anyv && cert && tot <= CM && !(bound == BOUND_LINES && E != E);
+        complete = anyv && cert && tot <= C1;
         if (complete) nc = tot + (l2 ? 1 : 0);
       }
       if (complete) {
@@ -345,6 +337,131 @@ __global__ __launch_bounds__(256) void k_verify(
         so[e] = e < kept ? dv[e] : -INFINITY;
       }
     }
+  }
+}
+
+// Top-1 behind the one-pass screen when d % 4 != 0: lists with lengths (their
+// first entry the best), read where they lie. Block: AR rows, a thread each to
+// decide, then a thread per (row, candidate) pair to run its chain. Bound by the
+// chains' latency, so by the pairs a CU holds at once: 64 rows make about two
+// waves of them, where k_verify's 16 rows with every list in LDS made half a one
+// (65,536 x 301 against 300 centroids: 220 us; 157 here).
+constexpr int AR = 64;
+
+__global__ __launch_bounds__(256) void k_check1_any(
+    const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
+    int nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int ip,
+    const Cand* __restrict__ cand, int parts, const float* __restrict__ bound,
+    uint32_t* __restrict__ labels, float* __restrict__ scores, uint32_t* __restrict__ fb,
+    uint32_t* __restrict__ small, const uint32_t* __restrict__ ncand) {
+  constexpr int PMAX = AR * (C5 + 1);
+  __shared__ uint32_t pcid[PMAX];
+  __shared__ float pres[PMAX];
+  __shared__ uint16_t prow[PMAX];
+  __shared__ uint32_t rowid[AR];
+  __shared__ int off[AR + 1];
+  static_assert(AR == 64, "the offsets are one wave's scan");
+  const int tid = threadIdx.x;
+  const int r0 = blockIdx.x * AR;
+  if (tid < AR) {
+    const bool live = r0 + tid < nrows;
+    const size_t at0 = (size_t)(live ? r0 + tid : r0) * parts;
+    const Cand* const c = cand + at0 * L5;
+    uint32_t nl[MAX_PARTS];
+    Cand first[MAX_PARTS];
+#pragma unroll
+    for (int q = 0; q < MAX_PARTS; q++) {
+      nl[q] = q < parts ? ncand[at0 + q] : 0u;
+      first[q] = c[min(q, parts - 1) * L5];
+    }
+    uint32_t xid = NONE;
+    if (live) {
+      const size_t p = lo + (size_t)(r0 + tid);
+      const size_t id = ids ? (size_t)ids[p] : p;
+      if (id < nx)
+        xid = (uint32_t)id;
+      else
+        small[SW_BAD_ID] = 1;
+    }
+    const float E = bound[live ? r0 + tid : r0];
+    float best = INFINITY;
+    bool any = false, whole = E == E;
+#pragma unroll
+    for (int q = 0; q < MAX_PARTS; q++) {
+      whole = whole && nl[q] <= (uint32_t)L5;
+      if (nl[q] > 0u && nl[q] <= (uint32_t)L5) {
+        any = true;
+        best = fminf(best, first[q].key);
+      }
+    }
+    const float thr = best + 2.0f * E;
+    const bool open = xid != NONE && any && whole;
+    // The candidates, counted, then listed.
+    auto each = [&](auto&& f) __attribute__((always_inline)) {
+      for (int q = 0; q < parts; q++)
+        for (uint32_t e = 0; e < nl[q]; e++) {
+          const Cand v = c[q * L5 + e];
+          if (v.key <= thr) f(v.id);
+        }
+    };
+    int n = 0;
+    if (open) each([&](uint32_t) { n++; });
+    const bool settled = open && n <= C5;
+    n = settled ? n + (ip ? 0 : 1) : 0;
+    int inc = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(inc, o, 64);
+      if (tid >= o) inc += t;
+    }
+    int o = inc - n;
+    off[tid] = o;
+    if (tid == AR - 1) off[AR] = inc;
+    rowid[tid] = settled ? xid : NONE;
+    if (settled) {
+      each([&](uint32_t id) {
+        prow[o] = (uint16_t)tid;
+        pcid[o++] = id;
+      });
+      if (!ip) {  // the row's |x|^2
+        prow[o] = (uint16_t)tid;
+        pcid[o] = NONE;
+      }
+    } else if (xid != NONE) {
+      fb[atomicAdd(&small[SW_FALLBACK_COUNT], 1u)] = (uint32_t)(lo + r0 + tid);
+    }
+  }
+  __syncthreads();
+  const int np = off[AR];
+  for (int s = tid; s < np; s += 256) {
+    const float* xr = x + (size_t)rowid[prow[s]] * d;
+    const uint32_t cid = pcid[s];
+    pres[s] = cid == NONE ? seq_sq<false>(xr, d) : chain<false>(xr, cents + (size_t)cid * d, d);
+  }
+  __syncthreads();
+  if (tid < AR && rowid[tid] != NONE) {
+    float best = INFINITY, xn = 0.f;
+    uint32_t bid = NONE;
+    for (int s = off[tid]; s < off[tid + 1]; s++) {
+      const uint32_t cid = pcid[s];
+      if (cid == NONE) {
+        xn = pres[s];
+        continue;
+      }
+      const float two = 2.0f * pres[s];
+      const float kx = ip ? -pres[s] : cnorm[cid] - two;
+      if (kx < best || (kx == best && cid < bid)) {
+        best = kx;
+        bid = cid;
+      }
+    }
+    if (bid == NONE) {
+      bid = 0;
+      best = INFINITY;
+    }
+    const size_t p = lo + (size_t)(r0 + tid);
+    labels[p] = bid;
+    scores[p] = ip ? -best : fmaxf(xn + best, 0.0f);
   }
 }
 
@@ -997,12 +1114,16 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
                        tally ? tally->counts : nullptr, tally ? tally->lo : 0,
                        tally ? tally->stride : 0, ncand);
   } else {
-    auto kern = L == L1F  ? k_verify<L1F, R1, false, false>
-                : L == L5 ? k_verify<L5, R1, false, false>
-                          : k_verify<L1, R1, false, false>;
-    hipLaunchKernelGGL(kern, g, dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents,
-                       cnorm, (int)k, ip ? 1 : 0, 1, cand, parts, xnorm, labels, scores, fb,
-                       c->small, bound, ncand);
+    if (L == L5) {
+      hipLaunchKernelGGL(k_check1_any, dim3((unsigned)((n + AR - 1) / AR)), dim3(256), 0, c->stream,
+                         x, nx, (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts,
+                         xnorm, labels, scores, fb, c->small, ncand);
+    } else {
+      auto kern = L == L1F ? k_verify<L1F, R1, false, false> : k_verify<L1, R1, false, false>;
+      hipLaunchKernelGGL(kern, g, dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents,
+                         cnorm, (int)k, ip ? 1 : 0, 1, cand, parts, xnorm, labels, scores, fb,
+                         c->small, bound);
+    }
   }
   EMH_HIP(hipGetLastError());
 }
@@ -1024,11 +1145,11 @@ void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, siz
   if (d % 4 == 0)
     hipLaunchKernelGGL((k_verify<LK, RK, true, true>), g, dim3(256), 0, c->stream, q, m, (int)d,
                        nullptr, (size_t)0, (int)m, data, nullptr, (int)n, 1, (int)kk, cand, parts,
-                       xnorm, ids, sims, fb, c->small, bound, nullptr);
+                       xnorm, ids, sims, fb, c->small, bound);
   else
     hipLaunchKernelGGL((k_verify<LK, RK, true, false>), g, dim3(256), 0, c->stream, q, m,
                        (int)d, nullptr, (size_t)0, (int)m, data, nullptr, (int)n, 1, (int)kk,
-                       cand, parts, xnorm, ids, sims, fb, c->small, bound, nullptr);
+                       cand, parts, xnorm, ids, sims, fb, c->small, bound);
   EMH_HIP(hipGetLastError());
 }
 
