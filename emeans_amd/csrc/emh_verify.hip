@@ -162,10 +162,11 @@ __device__ __attribute__((noinline)) void finish_group(const float* __restrict__
   }
 }
 
+// One wave.
 template <bool VEC4>
-__global__ __launch_bounds__(64) void k_exact1(
+__device__ __forceinline__ void exact_items(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
-    int n_direct, const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
+    int nrows, const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
     const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
     Cand* __restrict__ partial, uint32_t* __restrict__ tickets, uint32_t* __restrict__ labels,
     float* __restrict__ scores) {
@@ -173,8 +174,6 @@ __global__ __launch_bounds__(64) void k_exact1(
   __shared__ __attribute__((aligned(16))) float xt[RG * TD];
   __shared__ uint32_t xid_s[RG];
   __shared__ int last_s;
-  const int nrows = list ? (int)small[SW_FALLBACK_COUNT] : n_direct;
-  if (list && blockIdx.x == 0 && threadIdx.x == 0) small[SW_FALLBACK_TOTAL] += (uint32_t)nrows;
   const int nch = (k + CJ - 1) / CJ;
   const int ngr = (nrows + RG - 1) / RG;
   const int ntd = (d + TD - 1) / TD;
@@ -292,6 +291,16 @@ __global__ __launch_bounds__(64) void k_exact1(
   }
 }
 
+template <bool VEC4>
+__global__ __launch_bounds__(64) void k_exact1(
+    const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
+    int n, uint32_t* __restrict__ small, const float* __restrict__ cents,
+    const float* __restrict__ cnorm, int k, int ip, Cand* __restrict__ partial,
+    uint32_t* __restrict__ tickets, uint32_t* __restrict__ labels, float* __restrict__ scores) {
+  exact_items<VEC4>(x, nx, d, ids, lo, n, nullptr, small, cents, cnorm, k, ip, partial, tickets,
+                    labels, scores);
+}
+
 // ------------------------------------------------- exact top-1, queued rows
 // The check queues few rows (often one to eight per batch), so this scan is
 // built for latency: many short items, each a single wave that copies its
@@ -399,7 +408,7 @@ __device__ __forceinline__ void queued_tiles(
     }
     __syncthreads();
     // Loader: 16-byte piece e = 256 u + tid of a slab is row e / 4, dimensions
-    // 4 (e % 4) .. + 3 (d % 4 == 0: all of them in or all past d).
+    // 4 (e % 4) .. + 3 (AL: d % 4 == 0, all of them in or all past d).
     const float* xr[2];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
@@ -409,13 +418,12 @@ __device__ __forceinline__ void queued_tiles(
     v4f xv[2], cv[2];
     auto piece = [&](const float* p, int t) __attribute__((always_inline)) {
       v4f v = {0.f, 0.f, 0.f, 0.f};
-      if (t < d) {
-        if (AL) {
-          v = *reinterpret_cast<const v4f*>(p);
-        } else {
-          v4f s = {p[0], p[1], p[2], p[3]};
-          v = s;
-        }
+      if (AL) {
+        if (t < d) v = *reinterpret_cast<const v4f*>(p);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (t + e < d) v[e] = p[e];
       }
       return v;
     };
@@ -542,6 +550,28 @@ __device__ __forceinline__ void queued_tiles(
     }
     if (tid == 0) tickets[rt] = 0;
   }
+}
+
+// Queued rows of any width (d % 4 != 0): short items as k_exact1's by the first
+// wave, or, with `best`, tiles.
+__global__ __launch_bounds__(256) void k_exact1_list(
+    const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
+    const uint32_t* __restrict__ list, uint32_t* __restrict__ small,
+    const float* __restrict__ cents, const float* __restrict__ cnorm, int k, int ip,
+    Cand* __restrict__ partial, uint32_t* __restrict__ tickets,
+    unsigned long long* __restrict__ best, float* __restrict__ xnq, uint32_t* __restrict__ labels,
+    float* __restrict__ scores) {
+  __shared__ __attribute__((aligned(16))) QueuedLds tiles;
+  const int nrows = (int)small[SW_FALLBACK_COUNT];
+  if (blockIdx.x == 0 && threadIdx.x == 0) small[SW_FALLBACK_TOTAL] += (uint32_t)nrows;
+  if (best && (uint64_t)nrows * (uint64_t)k > MANY) {
+    queued_tiles<false>(tiles, x, nx, d, ids, nrows, list, small, cents, cnorm, k, ip, best,
+                        tickets, xnq, labels, scores, nullptr, nullptr, 0, 0);
+    return;
+  }
+  if (threadIdx.x >= WAVE) return;
+  exact_items<false>(x, nx, d, ids, lo, nrows, list, small, cents, cnorm, k, ip, partial, tickets,
+                     labels, scores);
 }
 
 // (Four waves; short items take the first alone.)
@@ -1159,27 +1189,31 @@ void launch_exact1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32
   const size_t ngr = (n + RG - 1) / RG;
   Cand* partial;
   uint32_t* tickets;
+  unsigned long long* best = nullptr;  // tiles: left at zero, as the tickets
   if (ar) {
     partial = (Cand*)ar->take(n * nch * sizeof(Cand));
     tickets = (uint32_t*)ar->take(ngr * 4);
     launch_fill_u32(c, tickets, ngr, 0);
   } else {
     partial = (Cand*)c->knn_tmp.get(n * nch * sizeof(Cand));
-    tickets = (uint32_t*)c->tickets.get_zeroed(ngr * 4, c->stream);
+    best = (unsigned long long*)c->tickets.get_zeroed((list ? n * 8 : 0) + ngr * 4, c->stream);
+    tickets = (uint32_t*)(best + (list ? n : 0));
   }
   // Queued rows: the count lives on the device, so the grid covers the worst
   // case. Queued rows are few: a grid of 2 blocks per CU covers them, and
   // blocks past the device-side count exit at once.
   const size_t items = ngr * nch;
   const unsigned g = (unsigned)std::min<size_t>(items, (size_t)(list ? 2 : 8) * c->cus);
-  if (d % 4 == 0)
-    hipLaunchKernelGGL(k_exact1<true>, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo,
-                       (int)n, list, c->small, cents, cnorm, (int)k, ip ? 1 : 0, partial, tickets,
-                       labels, scores);
-  else
-    hipLaunchKernelGGL(k_exact1<false>, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo,
-                       (int)n, list, c->small, cents, cnorm, (int)k, ip ? 1 : 0, partial, tickets,
-                       labels, scores);
+  if (list) {  // (d % 4 != 0; the tiles' |x|^2 where the items' winners would be)
+    hipLaunchKernelGGL(k_exact1_list, dim3(g), dim3(256), 0, c->stream, x, nx, (int)d, ids, lo,
+                       list, c->small, cents, cnorm, (int)k, ip ? 1 : 0, partial, tickets, best,
+                       (float*)partial, labels, scores);
+  } else {
+    auto kern = d % 4 == 0 ? k_exact1<true> : k_exact1<false>;
+    hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, c->stream, x, nx, (int)d, ids, lo, (int)n,
+                       c->small, cents, cnorm, (int)k, ip ? 1 : 0, partial, tickets, labels,
+                       scores);
+  }
   EMH_HIP(hipGetLastError());
 }
 

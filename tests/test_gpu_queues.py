@@ -36,6 +36,8 @@ def _crowds(n, d, each, seed):
     (2049, 100, 2100, 0),    # ranges of centroid tiles
     (40000, 64, 129, 0),     # more items than workgroups
     (4200, 388, 257, 3),
+    (5000, 33, 1000, 0),     # odd widths
+    (3000, 102, 700, 1),
 ])
 def test_queued_tiles(dev, n, d, k, metric, off):
     from emeans_amd import Mat, Select
