@@ -94,11 +94,16 @@ Top1Geom top1_geom(emh_ctx* c, size_t n, size_t d, size_t k, bool ip, bool split
   const int nt3 = (int)((k + TC3 - 1) / TC3);
   // (The split-operand screens address a slab's rows with 32-bit offsets: fewer than 2^25 rows.)
   // A selection that gives the large tiles fewer blocks than half the CUs (an
-  // epoch's tail batch: 3,392 rows x 1,024 centroids in 56 blocks took 55 us)
-  // takes the 128 x 128 screen, whose 216 blocks there take 45 us.
+  // epoch's tail batch) takes the 128 x 128 screen, which splits its rows
+  // itself: two launches less. Whole IP calls in us, one-pass / 128 x 128, d =
+  // 64, 384, 1,024: 3,392 rows x 1,024 centroids (56 tiles) 38 / 29, 47 / 42, 68 /
+  // 72; 16,384 x 128 (64 tiles) 39 / 29, 52 / 44, 82 / 75; 12,000 x 512 (94 tiles)
+  // 40 / 34, 51 / 50, 78 / 83. Not past MAX_PARTS tiles of centroids, where the
+  // 128 x 128 screen takes several a part: 2,545 x 3,000 (120 tiles) 49 / 47, 66 /
+  // 85, 96 / 159; 600 x 10,000 66 / 106, 103 / 224, 169 / 461.
   const size_t blocks3 = (n + TR3 - 1) / TR3 * (size_t)nt3;
-  const bool few = 2 * blocks3 < (size_t)c->cus;
   const bool lines = c->screen != SCREEN_F16;  // the split-operand screen is the one-pass one
+  const bool few = 2 * blocks3 < (size_t)c->cus && (nt3 <= MAX_PARTS || !lines);
   if (split && !few && c->screen != SCREEN_F32 && k >= 64 && (lines || nt3 <= MAX_PARTS) &&
       n < (1u << 25) && k < (1u << 25)) {
     g.big = g.split = true;

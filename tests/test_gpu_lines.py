@@ -325,3 +325,12 @@ def test_top1_pieces(dev, metric):
     O.top1(x, d, c, metric, ids=ids, rows=(lo, n), labels=ol, scores=os_)
     assert np.array_equal(dev.read_u32(lab), ol)
     assert dev.read_f32(sco).tobytes() == os_.tobytes()
+
+
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+@pytest.mark.parametrize("n,d,k", [(300, 64, 2049), (2545, 100, 3000), (257, 33, 9000)])
+def test_top1_few_rows_many_centroids(dev, metric, n, d, k):
+    """A few row tiles against more than eight tiles of centroids."""
+    x, c = _rows(n, d, n), _rows(k, d, k)
+    x[: n // 2] = c[np.arange(n // 2) % k] + np.float32(0.3) * x[: n // 2]
+    _top1(dev, x, c, metric)
