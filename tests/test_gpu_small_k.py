@@ -56,6 +56,48 @@ def test_small_k(dev, n, d, k, metric):
         assert same.all()
 
 
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("n,d,k", [(8192, 32, 16), (8193, 32, 16), (4096, 36, 32), (4097, 36, 17),
+                                   (2048, 64, 64), (2049, 64, 33)])
+def test_small_k_row_limit(dev, n, d, k, metric):
+    """The most rows of each centroid padding that one block's scan takes, and
+    one more (the screen)."""
+    from emeans_amd import Mat, Select
+    g = np.random.default_rng(n + k)
+    x = g.standard_normal((n, d)).astype(np.float32)
+    c = g.standard_normal((k, d)).astype(np.float32)
+    cb, cn = dev.upload_f32(c), None
+    if metric == "l2":
+        cn = dev.zeros_f32(k)
+        dev.row_norms(cb, k, d, cn)
+    lab, sc = dev.zeros_u32(n), dev.zeros_f32(n)
+    dev.top1(Mat(dev.bind(x), d), Select(None, (0, n)), cb, cn, k, metric, lab, sc)
+    ol, osc = O.top1(x, d, c, metric)
+    assert np.array_equal(dev.read_u32(lab), ol)
+    assert dev.read_f32(sc).tobytes() == osc.tobytes()
+
+
+@pytest.mark.parametrize("spherical", [False, True])
+@pytest.mark.parametrize("batch,k,d", [(8193, 10, 32), (4100, 20, 36), (2049, 50, 64)])
+def test_small_k_train_over_limit(dev, batch, k, d, spherical):
+    """Tallied batches just past the limit, their tails below it."""
+    from emeans_amd import Config, Emeans
+    g = np.random.default_rng(batch)
+    n = 2 * batch + 301
+    x = (g.standard_normal((n, d)) + 3 * g.standard_normal((k, d))[g.integers(0, k, n)])
+    x = x.astype(np.float32)
+    if spherical:
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+    cfg = Config(d=d, k=k, nepochs=2, batch_size=batch, spherical=spherical, seed=6)
+    m = Emeans(cfg, dev)
+    t = m.train_from(x, None)
+    o = O.train(x, d, k, nepochs=cfg.nepochs, batch_size=cfg.batch_size, alpha0=cfg.alpha0,
+                batch_law=cfg.batch_law, seed=cfg.seed, spherical=cfg.spherical,
+                unused_threshold=cfg.unused_threshold)
+    assert np.array_equal(t.labels, o["labels"])
+    assert t.centroids.tobytes() == o["centroids"].tobytes()
+
+
 def test_small_k_bad_id(dev):
     """A row id past the data is still reported."""
     from emeans_amd import Mat, Select
