@@ -354,7 +354,7 @@ def other_workloads(args):
     res["assign_2Mx1024_k16384_ip"] = {
         "value": n / step_s / 1e6, "unit": "Mrows/s", "ms_per_run": step_s * 1e3,
         "steps": args.other_steps,
-        "roofline": screen_roofline(ms, launches, flop, "k_screen3 (sorted-insert lists)"),
+        "roofline": screen_roofline(ms, launches, flop, "k_screen5 (fp16 lines, one pass)"),
         "cpu_baseline": {"value": len(sample) / cpu_s / 1e6, "unit": "Mrows/s",
                          "cores": O.get_threads(), "kind": "port",
                          "sample": f"{len(sample)} of the {n} queries against all {k} centroids"},

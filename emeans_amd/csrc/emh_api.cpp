@@ -317,7 +317,7 @@ int emh_create(int device, emh_ctx** out) {
     c->cus = p.multiProcessorCount;
     if (const char* s = getenv("EMEANS_HIP_SCREEN")) {
       const int m = atoi(s);
-      c->screen = m >= emh::SCREEN_OFF && m <= emh::SCREEN_F16 ? m : emh::SCREEN_BF3;
+      c->screen = m >= emh::SCREEN_OFF && m <= emh::SCREEN_F16 ? m : emh::SCREEN_ON;
     }
     try {
       EMH_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
@@ -810,7 +810,7 @@ uint64_t emh_fallback_rows(emh_ctx* c) {
 int emh_set_screen(emh_ctx* c, int on) {
   return guard([&] {
     EMH_ENSURE(c, "null context");
-    EMH_ENSURE(on >= 0 && on <= 3, "screen mode %d: 0 (off), 1 (bf16), 2 (f32) or 3 (fp16)",
+    EMH_ENSURE(on >= 0 && on <= 3, "screen mode %d: 0 (off), 1 (on), 2 (f32) or 3 (fp16 two-pass)",
                on);
     c->screen = on;
   });

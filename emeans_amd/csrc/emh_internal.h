@@ -118,11 +118,12 @@ struct Pinned {
 };
 
 // Top-1 / top-k path (emh_set_screen): the exact kernels alone, or the MFMA
-// screen ahead of the exact check: bf16 three-pass (SCREEN_BF3), f32, or
-// (SCREEN_F16) fp16 two-pass on the split-operand top-1 screen with every
-// other screen in bf16 three-pass. Rows or centroids beyond |x| = 32768 make
-// the fp16 bound NaN: those rows take the exact scan.
-enum ScreenMode : int { SCREEN_OFF = 0, SCREEN_BF3 = 1, SCREEN_F32 = 2, SCREEN_F16 = 3 };
+// screen ahead of the exact check: the one-pass screen over fp16 lines, with the
+// bf16 three-pass ones for small calls and the no-allocation entry (SCREEN_ON);
+// f32; or (SCREEN_F16) as SCREEN_ON with the fp16 two-pass screen for top-1
+// against up to eight tiles of centroids (rows or centroids beyond |x| = 32768
+// make its bound NaN: those rows take the exact scan).
+enum ScreenMode : int { SCREEN_OFF = 0, SCREEN_ON = 1, SCREEN_F32 = 2, SCREEN_F16 = 3 };
 // Top-1 calls of at most this many exact items (rows x max(ceil(k / 64), 2))
 // run the exact kernels alone by default: there one launch takes less time
 // than the screen's three (d = 768: the screen ~60 us at any size up to 8,192
@@ -213,7 +214,7 @@ struct emh_ctx {
     return copy_stream;
   }
   int cus = 256;
-  int screen = emh::SCREEN_BF3;
+  int screen = emh::SCREEN_ON;
   size_t exact_below = emh::EXACT_BELOW;  // emh_set_exact_below
   uint32_t* small = nullptr;  // SW_WORDS u32 on the device
   float* scales = nullptr;    // (s, 1 / s) of each SCALE_* matrix (emh_lines.h), after small
@@ -556,7 +557,8 @@ size_t top1_scratch_bytes(emh_ctx* c, size_t n, size_t d, size_t k, bool ip);
 void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                  size_t kk, bool exclude_self, uint32_t* ids, float* sims,
                  emh_screen_report* rep = nullptr);
-// Exact top-k for 16 < kk <= KLONG (emh_topk_long.hip): no screen.
+// Exact top-k for 16 < kk <= KLONG (emh_topk_long.hip): from the one-pass
+// screen's scores where that pays, else from exact dots alone.
 constexpr int KLONG = 4096;
 void launch_topk_long(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
                       size_t kk, bool exclude_self, uint32_t* ids, float* sims);

@@ -3,9 +3,12 @@
 //
 // The screen only has to name every row's possible winners; the check's exact
 // chains decide. One fp16 MFMA per 16 dimensions (where the bf16 three-pass
-// screens issue three) leaves an error bound about twice theirs, because it
-// rests on each row's measured rounding residual instead of the worst case,
-// and the operands take half the bytes from HBM to LDS.
+// screens issue three) leaves an error bound, in units of |x||c - m|
+// (emh_lines.h; theirs in |x||c|), of 1.6 times theirs at d = 1,024, 2.9 at 384,
+// 6 at 64 and 10 at 32, because it rests on each row's measured rounding residual
+// instead of the worst case, and the operands take half the bytes from HBM to
+// LDS. Rows that the longer lists cannot settle all the same go to exact scans
+// that take long queues in tiles (emh_verify.hip).
 //
 // Tile: 256 rows x 256 centroids (kNN: queries x data rows), 8 waves; wave w
 // owns rows 64 (w % 4) .. + 64 and centroids 128 (w / 4) .. + 128, as 2 x 4
@@ -436,7 +439,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
           }
         float v = s[0];
 #pragma unroll
-        for (int e = 1; e < 8; e++) v = fmaxf(v, e < kh ? s[e] : -INFINITY);
+        for (int e = 1; e < 8; e++) v = fmaxf(v, e < nh ? s[e] : -INFINITY);
         t[y] = v;  // minus the kh-th largest
       }
       const float own = h ? t[1] : t[0], give = h ? t[0] : t[1];

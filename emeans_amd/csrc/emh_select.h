@@ -43,12 +43,6 @@ __device__ __forceinline__ void insert(float (&key)[L], uint32_t (&id)[L], float
   }
 }
 
-// The same insertion without a branch: every slot takes its new value at once
-// from the comparisons c[e] = v < key[e] of the old list. For a sorted list,
-// slot e becomes key[e - 1] if v < key[e - 1], else min(v, key[e]), which is
-// med3(key[e - 1], v, key[e]). v is first mapped to +inf when it is NaN or
-// +inf, so such a key leaves the list unchanged; equal keys stay after the
-// ones already in the list.
 // Insert v into an ascending list of L keys that keeps the L smallest (no
 // ids; v and the keys are numbers or +inf, never NaN). Branch-free.
 template <int L>
@@ -58,6 +52,12 @@ __device__ __forceinline__ void insert_key(float (&key)[L], float v) {
   key[0] = fminf(v, key[0]);
 }
 
+// insert<L> without a branch: every slot takes its new value at once
+// from the comparisons c[e] = v < key[e] of the old list. For a sorted list,
+// slot e becomes key[e - 1] if v < key[e - 1], else min(v, key[e]), which is
+// med3(key[e - 1], v, key[e]). v is first mapped to +inf when it is NaN or
+// +inf, so such a key leaves the list unchanged; equal keys stay after the
+// ones already in the list.
 template <int L>
 __device__ __forceinline__ void insert_nb(float (&key)[L], uint32_t (&id)[L], float v,
                                           uint32_t j) {

@@ -375,7 +375,8 @@ typedef struct emh_screen_report {
  * reference): run the screen of emh_top1 (or of emh_topk_dev) on the same
  * arguments, then re-score every entry of its candidate lists with the exact
  * fma-chain key the check uses and report how far the screen's key was from
- * it, relative to the per-row bound E the check trusts. Writes no labels,
+ * it (less the constant by which a screen that takes the mean off the centroids
+ * is off for all of a row's), relative to the per-row bound E the check trusts. Writes no labels,
  * scores, ids or sims; waits for the device. */
 int emh_screen_margin(emh_ctx* ctx, const emh_buf* x, size_t d, const emh_buf* ids, size_t lo,
                       size_t hi, const emh_buf* centroids, const emh_buf* cnorm, size_t k,
@@ -385,11 +386,11 @@ int emh_screen_margin_topk(emh_ctx* ctx, const emh_buf* queries, size_t m, const
 /* Rows the exact top-1 / top-k kernels rescanned since the context was made
  * (the screen's misses; EMEANS_CUDA_SCREEN_STATS analogue, emeans-cuda lib.rs:278-287). */
 uint64_t emh_fallback_rows(emh_ctx* ctx);
-/* Select the top-1 / top-k path: 1 = MFMA screen (one fp16 pass over
- * rounded rows; small calls in bf16 three-pass arithmetic) + exact check (default), 3 = the same with the split-operand top-1 screen
- * (k_screen4) in fp16 two-pass arithmetic (a third fewer MFMAs, a bound 2.7
- * times looser at d = 768; rows or centroids beyond |x| = 32768 take the exact
- * scan), 2 = MFMA screen in f32 arithmetic + exact check, 0 = exact kernels
+/* Select the top-1 / top-k path: 1 = MFMA screen (one fp16 pass over rounded
+ * rows; small calls in bf16 three-pass arithmetic) + exact check (default), 3 =
+ * the same with top-1 against 64 to 2,048 centroids in fp16 two-pass arithmetic
+ * (k_screen4: twice the MFMAs; rows or centroids beyond |x| = 32768 take the
+ * exact scan), 2 = MFMA screen in f32 arithmetic + exact check, 0 = exact kernels
  * only (the reference "FP32 kernel alone", emeans-cuda tests/contract.rs:27-37).
  * Results are the same bits in every mode. */
 int emh_set_screen(emh_ctx* ctx, int on);

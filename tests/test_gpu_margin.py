@@ -2,7 +2,8 @@
 
 Every top-1 and top-k result is exact only if the screen's key of each listed
 candidate is within the per-row bound E (screen_bound) of the exact fma-chain
-key the check computes. emh_screen_margin runs the screen on a call's
+key the check computes (the one-pass screen's: less a constant per row).
+emh_screen_margin runs the screen on a call's
 arguments and re-scores every list entry with that chain; these tests assert
 that no entry is beyond E, and that the dot error stays within half of the
 bound's dot term (the split and the MFMA rounding model, the part that rests
@@ -14,9 +15,9 @@ adversarial: crowds of centroids within 1e-6,
 exact duplicates, rows at scales 1e3 .. 1e-15, rows in the bf16 subnormal
 range, centroids up to 5e17 (1e34 overflows the bound's |c|^2 and sends every
 row to the exact scan), d from 36 to 2500 (d < 32 runs no screen), both
-screen arithmetics, the split-operand screen's filtered single-tile lists
-(k <= 2048), the sorted many-tile lists of larger k, the 128 x 128 screen of
-small k, and the kNN screen's 24-entry lists. They
+screen arithmetics, the large-tile screens' single-tile lists (k <= 2048) and
+many-tile ones of larger k, the 128 x 128 screen of small k, and the kNN screen's
+24-entry lists. They
 also pin which screen variant ran, whatever the CU count. With
 EMEANS_MARGIN_OUT set, each case's report is appended to that file (JSON lines).
 """
@@ -106,7 +107,7 @@ def _crowds(k, d, seed):
     return c, groups
 
 
-@pytest.mark.parametrize("mode", [1, 2, 3], ids=["bf16x3", "f32", "f16x2"])
+@pytest.mark.parametrize("mode", [1, 2, 3], ids=["default", "f32", "f16x2"])
 @pytest.mark.parametrize("metric", ["ip", "l2"])
 @pytest.mark.parametrize("d", [36, 99, 768, 2500])
 def test_margin_near_tie_crowds(dev, mode, metric, d):
@@ -220,7 +221,7 @@ def test_margin_tagged_and_sorted_lists(dev, metric):
         assert (r["tiles_per_part"] == 1) == (want == "big_tagged")
 
 
-@pytest.mark.parametrize("mode", [1, 2], ids=["bf16x3", "f32"])
+@pytest.mark.parametrize("mode", [1, 2], ids=["default", "f32"])
 @pytest.mark.parametrize("k", [2, 21, 63])
 def test_margin_small_k(dev, mode, k):
     """Small k on the 128 x 128 screen (one partly filled tile) at d = 768,
@@ -263,7 +264,7 @@ def test_margin_headline_batch(dev):
         dev.set_screen(1)
 
 
-@pytest.mark.parametrize("mode", [1, 2], ids=["bf16x3", "f32"])
+@pytest.mark.parametrize("mode", [1, 2], ids=["default", "f32"])
 def test_margin_knn_lists(dev, mode):
     """The kNN screen's merged lists on unit rows with near-duplicates (d = 384)."""
     from emeans_amd import synth

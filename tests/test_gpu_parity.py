@@ -24,9 +24,9 @@ def dev():
     d.close()
 
 
-@pytest.fixture(params=[1, 2, 3], ids=["bf16x3", "f32", "f16x2"])
+@pytest.fixture(params=[1, 2, 3], ids=["default", "f32", "f16x2"])
 def screen(request, dev):
-    """The MFMA screen's arithmetic: bf16 three-pass (default) or f32."""
+    """The MFMA screen's arithmetic: the default's, f32, or fp16 two-pass."""
     dev.set_screen(request.param)
     yield request.param
     dev.set_screen(1)
@@ -109,7 +109,7 @@ def test_top1_parts_of_several_tiles(dev, screen, n, k, metric):
     (tagged keys); 4,096 centroids (16 tiles, more than eight parts): the
     large-tile screen that splits its own slabs, on 256 CUs eight parts of two
     tiles each, so its lists take the sorted insert across tiles. Bit-equal to
-    the oracle; with the bf16 screen, the variant that ran is the intended one
+    the oracle; with the default screen, the variant that ran is the intended one
     (the parts follow the device's CU count)."""
     from emeans_amd import Mat, Select
     d = 256
@@ -209,7 +209,7 @@ def test_screen_bit_equal_on_near_ties(dev, n, d, k, metric):
     x = (rows * scale[:, None]).astype(np.float32)
     perm = ((np.arange(n, dtype=np.uint64) * 7919 + 5) % n).astype(np.uint32)
     outs = []
-    for mode in (1, 2, 0):  # bf16 screen, f32 screen, exact kernel alone
+    for mode in (1, 2, 0):  # default screen, f32 screen, exact kernel alone
         dev.set_screen(mode)
         outs.append(_gpu_top1(dev, x, c, metric, ids=perm))
     dev.set_screen(1)
@@ -487,7 +487,7 @@ def test_topk_production_duplicates(dev, screen):
 ])
 def test_topk_split_screen(dev, screen, m, n, d, kk, self_):
     """Calls of at least 256 queries against at least 512 rows take the kNN
-    screen over operands split once (k_screen4kn): ids and sims bit-equal to
+    screen over operands rounded once (k_screen5): ids and sims bit-equal to
     the oracle, with exact duplicates among the data rows."""
     data = _mix(n, d, 12, 0.25, True, m + n + d)
     data[n // 2:n // 2 + 64] = data[:64]  # exact duplicates: equal scores, lower id first

@@ -1,6 +1,6 @@
 """A chain per row (k-means++'s dots, internal_scores' f64 squares) and the
 exact dots of rows with cluster sums, at the edges of their 16-row groups,
-768-column passes, 4-column loads and column tiles: bit-equal to the oracle."""
+256-column passes, 4-column loads and column tiles: bit-equal to the oracle."""
 
 import numpy as np
 import pytest

@@ -112,7 +112,7 @@ def test_spherical_blobs_config(dev):
     assert a.mean_objective(True) == O.mean_objective(osc, True)
 
 
-@pytest.mark.parametrize("mode", [1, 3], ids=["bf16x3", "f16x2"])
+@pytest.mark.parametrize("mode", [1, 3], ids=["default", "f16x2"])
 def test_l2_gmm_mid_size(dev, mode):
     """A 40,000 x 256, k = 512 L2 run through the MFMA screen, with revival,
     in either arithmetic of the split-operand screen."""
@@ -128,7 +128,7 @@ def test_l2_gmm_mid_size(dev, mode):
     assert sum(s.nsplit for s in m.iteration_stats()) > 0
 
 
-@pytest.mark.parametrize("mode", [1, 3], ids=["bf16x3", "f16x2"])
+@pytest.mark.parametrize("mode", [1, 3], ids=["default", "f16x2"])
 def test_headline_config_bit_exact(dev, mode):
     """200,000 x 768, k = 1024, exact FP32, L2, seed 0: the whole training run and
     the final assignment equal the oracle's CPU run bit for bit (with either
@@ -150,10 +150,10 @@ def test_headline_config_bit_exact(dev, mode):
 
 
 def test_assign_after_training_reuses_split_rows_only_while_unchanged(dev):
-    """A training run on bound rows leaves them split in bf16 halves, and an
-    assignment of the same buffer takes those halves instead of splitting
+    """A training run on bound rows leaves them split (as lines, or as halves),
+    and an assignment of the same buffer takes those instead of splitting
     again. The results must be those of the rows as they are: right after the
-    run, after a write into the bound rows (the halves are stale then), and
+    run, after a write into the bound rows (they are stale then), and
     after the buffer's address was handed out (writes may come from outside)."""
     from emeans_amd import Config, synth
     n, d, k = 40_000, 256, 512
