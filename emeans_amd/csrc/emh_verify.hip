@@ -843,17 +843,17 @@ void small1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids
 // ------------------------------------------------------------- exact top-k
 // Items of KQ queued queries x a range (part) of the data rows, few enough parts
 // that the items fill the chip. A tile is KQ queries x KT data rows, a thread 4
-// x 4 chains, slabs of KD dimensions double-buffered in LDS (bound by the fmas
-// and the LDS reads that feed them). A query keeps its kk best in LDS, behind
+// x 4 chains, slabs of KD dimensions in LDS with the next one in registers (bound
+// by the fmas, the LDS reads that feed them and the loads' latency). A query keeps its kk best in LDS, behind
 // them the rows of the last tiles that beat the kk-th of those it had (data rows
 // come in rising order, so an equal score never does); when a tile may not fit
 // any more, one wave keeps the kk best of the query's entries. With several
 // parts, each leaves its kk best in memory and the last to finish picks from
 // those of all parts. 20,000 queued
-// queries of 128 dimensions against as many rows: 5.9 ms for the whole call; a
-// workgroup a query, a data row a thread, 170. 95 against 2,000 x 64: 106 us
-// (147).
-constexpr int KQ = 32, KT = 128, KD = 16, KB = 160, KPARTS = 64;
+// queries of 128 dimensions against as many rows: 4.5 ms for the whole call; with
+// slabs of 16 dimensions double-buffered 5.9; a workgroup a query, a data row a
+// thread, 170.
+constexpr int KQ = 32, KT = 128, KD = 32, KB = 160, KPARTS = 64;
 constexpr int KQP = KQ + 4, KTP = KT + 4;
 
 // The kk best (larger score, then lower id; NaN and -inf never came in) of the
@@ -928,8 +928,8 @@ __global__ __launch_bounds__(256) void k_exactk(const float* __restrict__ q, int
                                                 float* __restrict__ sims_out,
                                                 Cand* __restrict__ plist,
                                                 uint32_t* __restrict__ tickets) {
-  __shared__ __attribute__((aligned(16))) float Qs[2][KD][KQP];
-  __shared__ __attribute__((aligned(16))) float Xs[2][KD][KTP];
+  __shared__ __attribute__((aligned(16))) float Qs[KD][KQP];
+  __shared__ __attribute__((aligned(16))) float Xs[KD][KTP];
   __shared__ __attribute__((aligned(16))) float bv[KQ][KB];
   __shared__ __attribute__((aligned(16))) uint32_t bi[KQ][KB];
   __shared__ float thr[KQ];  // the kk-th best, -inf while there are fewer
@@ -954,33 +954,29 @@ __global__ __launch_bounds__(256) void k_exactk(const float* __restrict__ q, int
       cnt[tid] = 0;
     }
     __syncthreads();
-    // Loader: piece e of a slab is row e / 4, dimensions 4 (e % 4) .. + 3; the
-    // first 128 threads take the queries', all of them two of the data's.
-    const int pr = tid >> 2, pt = 4 * (tid & 3);
-    const float* const qrow = q + (size_t)qid[pr & (KQ - 1)] * d;
-    float qv[4], xv[2][4];
+    // Loader: a thread takes dimensions 4 (tid % 8) .. + 3 of query tid / 8 and
+    // of the data rows tid / 8 + 32 u (a slab is a whole line of a row).
+    const int pr = tid >> 3, pt = 4 * (tid & 7);
+    const float* const qrow = q + (size_t)qid[pr] * d;
+    float qv[4], xv[4][4];
     auto load = [&](int j0, int t0) __attribute__((always_inline)) {
       const int t = t0 + pt;
-      if (tid < 4 * KQ) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) qv[c] = t + c < d ? qrow[t + c] : 0.f;
-      }
+      for (int c = 0; c < 4; c++) qv[c] = t + c < d ? qrow[t + c] : 0.f;
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const float* p = data + (size_t)min(j0 + 64 * u + pr, n - 1) * d;
+      for (int u = 0; u < 4; u++) {
+        const float* p = data + (size_t)min(j0 + 32 * u + pr, n - 1) * d;
 #pragma unroll
         for (int c = 0; c < 4; c++) xv[u][c] = t + c < d ? p[t + c] : 0.f;
       }
     };
-    auto store = [&](int b) __attribute__((always_inline)) {
-      if (tid < 4 * KQ) {
+    auto store = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) Qs[b][pt + c][pr] = qv[c];
+      for (int c = 0; c < 4; c++) {
+        Qs[pt + c][pr] = qv[c];
+#pragma unroll
+        for (int u = 0; u < 4; u++) Xs[pt + c][32 * u + pr] = xv[u][c];
       }
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) Xs[b][pt + c][64 * u + pr] = xv[u][c];
     };
     const int c0 = part * tpp, c1 = min(ntile, c0 + tpp);
     for (int ct = c0; ct < c1; ct++) {
@@ -990,31 +986,33 @@ __global__ __launch_bounds__(256) void k_exactk(const float* __restrict__ q, int
       for (int a = 0; a < 4; a++)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[a][e] = 0.f;
-      auto dim = [&](int b, int t) __attribute__((always_inline)) {
+      auto dim = [&](int t) __attribute__((always_inline)) {
         float qa[4], xa[4];
 #pragma unroll
-        for (int a = 0; a < 4; a++) qa[a] = Qs[b][t][ty * 4 + a];
+        for (int a = 0; a < 4; a++) qa[a] = Qs[t][ty * 4 + a];
 #pragma unroll
-        for (int e = 0; e < 4; e++) xa[e] = Xs[b][t][tx * 4 + e];
+        for (int e = 0; e < 4; e++) xa[e] = Xs[t][tx * 4 + e];
 #pragma unroll
         for (int a = 0; a < 4; a++)
 #pragma unroll
           for (int e = 0; e < 4; e++) acc[a][e] = fmaf(qa[a], xa[e], acc[a][e]);
       };
-      load(j0, 0);
-      store(0);
-      __syncthreads();
-      for (int t0 = 0, b = 0; t0 < d; t0 += KD, b ^= 1) {
-        const bool more = t0 + KD < d;
-        if (more) load(j0, t0 + KD);
+      if (ct == c0) load(j0, 0);
+      for (int t0 = 0; t0 < d; t0 += KD) {
+        store();
+        __syncthreads();
+        // The next slab (of the next tile, after the last) is on its way meanwhile.
+        if (t0 + KD < d)
+          load(j0, t0 + KD);
+        else if (ct + 1 < c1)
+          load(j0 + KT, 0);
         const int tn = min(KD, d - t0);  // dimensions past d never enter a chain
         if (tn == KD) {
 #pragma unroll
-          for (int t = 0; t < KD; t++) dim(b, t);
+          for (int t = 0; t < KD; t++) dim(t);
         } else {
-          for (int t = 0; t < tn; t++) dim(b, t);
+          for (int t = 0; t < tn; t++) dim(t);
         }
-        if (more) store(b ^ 1);
         __syncthreads();
       }
 #pragma unroll
