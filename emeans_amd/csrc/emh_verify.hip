@@ -844,15 +844,14 @@ void small1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint32_t* ids
 // Items of KQ queued queries x a range (part) of the data rows, few enough parts
 // that the items fill the chip. A tile is KQ queries x KT data rows, a thread 4
 // x 4 chains, slabs of KD dimensions in LDS with the next one in registers (bound
-// by the fmas, the LDS reads that feed them and the loads' latency). A query keeps its kk best in LDS, behind
-// them the rows of the last tiles that beat the kk-th of those it had (data rows
-// come in rising order, so an equal score never does); when a tile may not fit
-// any more, one wave keeps the kk best of the query's entries. With several
-// parts, each leaves its kk best in memory and the last to finish picks from
-// those of all parts. 20,000 queued
-// queries of 128 dimensions against as many rows: 4.5 ms for the whole call; with
-// slabs of 16 dimensions double-buffered 5.9; a workgroup a query, a data row a
-// thread, 170.
+// by the fmas, the LDS reads that feed them and the loads' latency). A query keeps
+// its kk best in LDS, behind them the rows of the last tiles that beat the kk-th
+// of those it had (data rows come in rising order, so an equal score never does);
+// when a tile may not fit any more, one wave keeps the kk best of the query's
+// entries. With several parts, each leaves its kk best in memory and the last to
+// finish picks from those of all parts. 20,000 queued queries of 128 dimensions
+// against as many rows: 4.5 ms for the whole call; with slabs of 16 dimensions
+// double-buffered 5.9; a workgroup a query, a data row a thread, 170.
 constexpr int KQ = 32, KT = 128, KD = 32, KB = 160, KPARTS = 64;
 constexpr int KQP = KQ + 4, KTP = KT + 4;
 
