@@ -852,14 +852,14 @@ __global__ __launch_bounds__(Check1<L>::NT, Check1<L>::WAVES) void k_check1(
   }
 }
 
-// ---- Top-k check behind the one-pass screen (lists of up to LK entries a
+// ---- Top-k check behind the one-pass screen (lists of L = LK or LK5 entries a
 // part, any order, {+inf, NONE} after the valid ones; L entries of -inf where
 // a part could not hold its candidates).
 //
 // A part's list holds every data row of the part whose key is within the
 // part's own limit, which is at least the query's kk-th key plus 2E: the
 // query's candidates are the entries of all parts within its kk-th key plus
-// 2E. A wave takes a query's lists in registers (parts x LK entries over its
+// 2E. A wave takes a query's lists in registers (parts x L entries over its
 // lanes), finds the kk-th key by bisection over the keys' ordered bits (one
 // compare and popcount a register and bit: no list to merge), and compacts the
 // candidates; then one thread per (query, candidate) runs the exact chain, and
@@ -869,7 +869,6 @@ __global__ __launch_bounds__(Check1<L>::NT, Check1<L>::WAVES) void k_check1(
 // KQ queries per block: few, for calls of few queries (2,000 in blocks of 16 left
 // half the CUs without one).
 constexpr int KC = 64;                         // most candidates of a query
-constexpr int KR = (MAX_PARTS5 * LK + 63) / 64;  // list entries per lane
 
 // Ascending unsigned image of a float's order (not NaN).
 __device__ __forceinline__ uint32_t ord32(float v) {
@@ -877,12 +876,13 @@ __device__ __forceinline__ uint32_t ord32(float v) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-template <int KQ, bool VEC4>
+template <int KQ, bool VEC4, int L>
 __global__ __launch_bounds__(256) void k_verify_lines(
     const float* __restrict__ q, int d, int m, const float* __restrict__ data, int kk,
     const Cand* __restrict__ cand, int parts, const float* __restrict__ bound,
     uint32_t* __restrict__ ids, float* __restrict__ sims, uint32_t* __restrict__ fb,
     uint32_t* __restrict__ small) {
+  constexpr int KR = (MAX_PARTS5 * L + 255) / 256 * 4;  // list entries per lane
   __shared__ uint32_t pid[KQ * KC];
   __shared__ float pdot[KQ * KC];
   __shared__ int cnt[KQ], off[KQ + 1];
@@ -891,7 +891,7 @@ __global__ __launch_bounds__(256) void k_verify_lines(
   for (int i = w; i < KQ; i += 4) {
     int c = 0;
     if (i < rows) {
-      const int n = parts * LK, nr = (n + 63) >> 6;
+      const int n = parts * L, nr = (n + 63) >> 6;
       const Cand* src = cand + (size_t)(r0 + i) * n;
       uint32_t key[KR], id[KR];
       bool lost = false;
@@ -917,8 +917,11 @@ __global__ __launch_bounds__(256) void k_verify_lines(
         const uint32_t t = x | ((1u << b) - 1u);  // this bit 0, the rest 1
         int below = 0;
 #pragma unroll
-        for (int u = 0; u < KR; u++)
-          if (u < nr) below += __popcll(__ballot(key[u] <= t));
+        for (int u = 0; u < KR; u += 4) {  // (a branch for each costs as much as its compare)
+          if (u >= nr) break;
+#pragma unroll
+          for (int e = 0; e < 4; e++) below += __popcll(__ballot(key[u + e] <= t));
+        }
         if (below < kk) x |= 1u << b;
       }
       // x = 0xffffffff: fewer than kk entries; all of them are candidates.
@@ -1129,13 +1132,17 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
 }
 
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                    size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
-                    float* sims, uint32_t* fb, int bound) {
+                    size_t kk, const Cand* cand, int parts, int L, const float* xnorm,
+                    uint32_t* ids, float* sims, uint32_t* fb, int bound) {
+  EMH_ENSURE(L == LK || (L == LK5 && bound == BOUND_LINES), "check: lists of %d entries", L);
   if (bound == BOUND_LINES) {
     EMH_ENSURE(parts >= 1 && parts <= MAX_PARTS5 && kk <= KC, "check: %d parts", parts);
     const int kq = m >= 64 * (size_t)c->cus ? 16 : 4;
-    auto kern = kq == 16 ? (d % 4 == 0 ? k_verify_lines<16, true> : k_verify_lines<16, false>)
-                         : (d % 4 == 0 ? k_verify_lines<4, true> : k_verify_lines<4, false>);
+    const bool v = d % 4 == 0;
+    auto kern = L == LK5 ? (kq == 16 ? (v ? k_verify_lines<16, true, LK5> : k_verify_lines<16, false, LK5>)
+                                     : (v ? k_verify_lines<4, true, LK5> : k_verify_lines<4, false, LK5>))
+                         : (kq == 16 ? (v ? k_verify_lines<16, true, LK> : k_verify_lines<16, false, LK>)
+                                     : (v ? k_verify_lines<4, true, LK> : k_verify_lines<4, false, LK>));
     hipLaunchKernelGGL(kern, dim3((unsigned)((m + kq - 1) / kq)), dim3(256), 0, c->stream, q,
                        (int)d, (int)m, data, (int)kk, cand, parts, xnorm, ids, sims, fb, c->small);
     EMH_HIP(hipGetLastError());

@@ -434,18 +434,19 @@ void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t
     Cand* cand = nullptr;
     float* xnorm = nullptr;
     const float* mean = nullptr;
-    const int parts = screen5_knn(c, q, m, data, n, d, kk, exclude_self, &cand, &xnorm, &mean);
+    int L = 0;
+    const int parts = screen5_knn(c, q, m, data, n, d, kk, exclude_self, &cand, &L, &xnorm, &mean);
     if (rep) {
       *rep = emh_screen_report{};
       rep->variant = EMH_SCREEN_BIG_KNN;
       rep->parts = parts;
       rep->tiles_per_part = 0;
-      launch_margin(c, q, m, d, nullptr, 0, m, data, nullptr, true, cand, parts, LK, xnorm,
+      launch_margin(c, q, m, d, nullptr, 0, m, data, nullptr, true, cand, parts, L, xnorm,
                     BOUND_LINES, rep, nullptr, mean);
       return;
     }
     uint32_t* fb = (uint32_t*)c->fblist.get(m * 4);
-    launch_verifyk(c, q, m, data, n, d, kk, cand, parts, xnorm, ids, sims, fb, BOUND_LINES);
+    launch_verifyk(c, q, m, data, n, d, kk, cand, parts, L, xnorm, ids, sims, fb, BOUND_LINES);
     launch_exactk(c, q, m, data, n, d, kk, exclude_self, fb, ids, sims);
     return;
   }
@@ -481,7 +482,7 @@ void launch_topk(emh_ctx* c, const float* q, size_t m, const float* data, size_t
                   c->screen != SCREEN_F32 ? BOUND_BF16 : BOUND_F32, rep);
     return;
   }
-  launch_verifyk(c, q, m, data, n, d, kk, cand, parts, xnorm, ids, sims, fb,
+  launch_verifyk(c, q, m, data, n, d, kk, cand, parts, LK, xnorm, ids, sims, fb,
                  c->screen == SCREEN_F32 ? BOUND_F32 : BOUND_BF16);
   launch_exactk(c, q, m, data, n, d, kk, exclude_self, fb, ids, sims);
 }

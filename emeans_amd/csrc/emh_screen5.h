@@ -101,6 +101,7 @@ struct Args5 {
   size_t cslab;
   const float* cnorm;     // L2: the centroids' given squared norms
   int k, d, kk;
+  int L;                  // kNN: entries of a list, at most LK5 (top-1: L5)
   int tpp, parts, ntiles;
   Cand* cand;             // out: [row][part][L], see the end of k_screen5
   uint32_t* ncand;        // top-1: their lengths
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   constexpr bool L2 = KIND == TOP1_L2, SELF = KIND == KNN_SELF;
   constexpr bool TOPK = KIND == KNN || KIND == KNN_SELF;
   constexpr bool LISTS = KIND != SCORES, TOP1 = LISTS && !TOPK;
-  constexpr int L = TOPK ? LK : L5, NK = TOPK ? KTH5 : 1, CAP = CAP5;
+  constexpr int NK = TOPK ? KTH5 : 1, CAP = CAP5;
   constexpr int LOG = TOPK ? LOG5_KNN : LOG5_TOP1;
   constexpr int WA = 4, WN = 2;  // centroid (A) and row (B) 32-blocks per wave
   constexpr int ND = 2;          // DMAs per operand per step per wave
@@ -611,12 +612,13 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
   // many entries, the best first; more than L, or a log that did not hold
   // everything: a length beyond L. kNN: in any order, the unused entries
   // {+inf, NONE}; more than L: L entries of -inf, which settle no row.
-  constexpr int RS = L | 1, KS = NK | 1;  // LDS strides of a row's entries, and of a thread's keys
+  const int L = TOPK ? a_.L : L5;
+  constexpr int RS = (TOPK ? LK5 : L5) | 1, KS = NK | 1;  // LDS strides of a row's entries, and of a thread's keys
   float* OK = reinterpret_cast<float*>(ring);
-  uint32_t* OI = reinterpret_cast<uint32_t*>(ring + S5_STAGE);
+  uint32_t* OI = reinterpret_cast<uint32_t*>(OK + T5 * RS);
   uint32_t* on = OI + T5 * RS;
-  float* TK = reinterpret_cast<float*>(ring + 2 * S5_STAGE);
-  static_assert((T5 * RS + T5) * 4 <= S5_STAGE && 512 * KS * 4 <= 2 * S5_STAGE, "output space");
+  float* TK = reinterpret_cast<float*>(on + T5);
+  static_assert((2 * T5 * RS + T5 + 512 * KS) * 4 <= NS5 * S5_STAGE, "output space");
   __syncthreads();  // every wave's DMAs are in and its keys published
   if (tid < T5) on[tid] = 0u;
   if (TOPK) {
@@ -669,25 +671,27 @@ __global__ __launch_bounds__(512, 1) void k_screen5(const Args5 a_) {
     if (spilt) atomicAdd(&on[prow], (uint32_t)(2 * L));
   }
   __syncthreads();
-  if (tid < T5 && row0 + tid < nrows) {
+  if (TOPK) {  // eight lanes a row: 64 bytes of its list at a time
+    for (int r = tid >> 3; r < min(T5, nrows - row0); r += 64) {
+      Cand* out = a_.cand + ((size_t)(row0 + r) * parts + part) * L;
+      const int n = (int)on[r];
+      for (int e = tid & 7; e < L; e += 8)
+        out[e] = n > L ? Cand{-INFINITY, 0u}
+                 : e < n ? Cand{OK[r * RS + e], OI[r * RS + e]}
+                         : Cand{INFINITY, NONE};
+    }
+  } else if (tid < T5 && row0 + tid < nrows) {
     const size_t at0 = (size_t)(row0 + tid) * parts + part;
     Cand* out = a_.cand + at0 * L;
     const uint32_t n = on[tid];
     const bool full = n > (uint32_t)L;
-    if (TOPK) {
-      for (uint32_t e = 0; e < (uint32_t)L; e++)
-        out[e] = full ? Cand{-INFINITY, 0u}
-                 : e < n ? Cand{OK[tid * RS + e], OI[tid * RS + e]}
-                         : Cand{INFINITY, NONE};
-    } else {
-      a_.ncand[at0] = n;
-      uint32_t best = 0;
-      for (uint32_t e = 1; e < (full ? 0u : n); e++)
-        best = OK[tid * RS + e] < OK[tid * RS + best] ? e : best;
-      for (uint32_t e = 0; e < (full ? 0u : n); e++) {
-        const uint32_t at = tid * RS + (e == 0 ? best : e == best ? 0u : e);
-        out[e] = Cand{OK[at], OI[at]};
-      }
+    a_.ncand[at0] = n;
+    uint32_t best = 0;
+    for (uint32_t e = 1; e < (full ? 0u : n); e++)
+      best = OK[tid * RS + e] < OK[tid * RS + best] ? e : best;
+    for (uint32_t e = 0; e < (full ? 0u : n); e++) {
+      const uint32_t at = tid * RS + (e == 0 ? best : e == best ? 0u : e);
+      out[e] = Cand{OK[at], OI[at]};
     }
   }
 }

@@ -448,7 +448,7 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
 }
 
 int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                size_t kk, bool exclude_self, Cand** cand_out, float** bound_out,
+                size_t kk, bool exclude_self, Cand** cand_out, int* L_out, float** bound_out,
                 const float** mean_out) {
   Split5 s;
   split5(c, q, m, data, n, d, c->small, 3, &s);
@@ -459,7 +459,12 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   // against 100,000 x 512: 8 parts gave 64 blocks, 0.94 ms; 31 take 0.45).
   int parts = parts5(row_tiles, ntiles, std::max(c->cus, 1), MAX_PARTS5, 2.0);
   const int tpp = (ntiles + parts - 1) / parts;
-  Cand* cand = (Cand*)c->cand.get((size_t)parts * m * LK * sizeof(Cand));
+  // Lists of 24 leave room for the near-ties of at most 12 neighbours: among
+  // 1,000,000 unit rows with a common mean (d = 32) 10 queue 2,557 rows (160 ms),
+  // 16 queued 311,078 (732 ms; 171 with lists of 40, 99 rows). Where both hold
+  // everything 40 entries cost 1%.
+  const int L = kk > (size_t)LK_KK ? LK5 : LK;
+  Cand* cand = (Cand*)c->cand.get((size_t)parts * m * L * sizeof(Cand));
   float* bound = (float*)c->xnorm.get(2 * m * 4);
   // A launch's threads each keep a log (1 MB a block): launches of whole waves
   // of blocks, at most four: 1 GB on 256 CUs, kept with the context. One wave a
@@ -476,6 +481,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
   a.k = (int)n;
   a.d = (int)d;
   a.kk = (int)kk;
+  a.L = L;
   a.tpp = tpp;
   a.parts = parts;
   a.ntiles = ntiles;
@@ -496,7 +502,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
     const size_t q0 = (size_t)r * T5, q1 = std::min((size_t)(r + rt_step) * T5, m);
     a.lo = q0;
     a.nrows = (int)(q1 - q0);
-    a.cand = cand + q0 * parts * LK;
+    a.cand = cand + q0 * parts * L;
     a.bound = bound + q0;
     const unsigned blocks = (unsigned)((q1 - q0 + T5 - 1) / T5 * parts);
     if (exclude_self)
@@ -505,6 +511,7 @@ int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t 
       launch5<KNN, false>(c, blocks, a);
   }
   *cand_out = cand;
+  *L_out = L;
   *bound_out = bound;
   *mean_out = s.mean;
   return parts;

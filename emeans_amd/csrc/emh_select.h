@@ -15,6 +15,8 @@ constexpr int L5 = 16;   // ... on the one-pass screen, whose lists come with th
 constexpr int C5 = 32;   // ... and most candidates of a row there
 constexpr int C1 = 16;   // top-1: most candidates a row sends to the exact chains
 constexpr int LK = 24;   // top-k list: kk <= 16 plus 7 spare + the bound
+constexpr int LK5 = 40;  // ... on the one-pass screen, past LK_KK neighbours
+constexpr int LK_KK = 12;
 constexpr int KMAX = 16;  // largest kk of the screened top-k (emeans-core/src/knn.rs:16)
 constexpr int MAX_PARTS = 8;  // centroid parts per row tile: lists per row the verify merges
 constexpr int MAX_PARTS5 = 32;  // ... data parts per query tile of the one-pass kNN screen
@@ -250,14 +252,16 @@ void split5(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, s
 void launch_scores5(emh_ctx* c, const Split5& s, size_t q0, size_t nb, float* scores, size_t ldS,
                     float* bound);
 // The one-pass kNN screen (emh_screen5.hip): whether it takes a call, and the
-// call's screen (candidate lists [m][parts][LK]; the queries' E at bound[r]
-// and its dot term at bound[m + r]; in the context's scratch); returns the parts.
+// call's screen (candidate lists [m][parts][L], L = LK or LK5; the queries' E at
+// bound[r] and its dot term at bound[m + r]; in the context's scratch); returns
+// the parts.
 bool screen5_knn_fits(emh_ctx* c, size_t m, size_t n, size_t d);
 int screen5_knn(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                size_t kk, bool exclude_self, Cand** cand, float** bound, const float** mean);
+                size_t kk, bool exclude_self, Cand** cand, int* L, float** bound,
+                const float** mean);
 void launch_verifyk(emh_ctx* c, const float* q, size_t m, const float* data, size_t n, size_t d,
-                    size_t kk, const Cand* cand, int parts, const float* xnorm, uint32_t* ids,
-                    float* sims, uint32_t* fb, int bound);
+                    size_t kk, const Cand* cand, int parts, int L, const float* xnorm,
+                    uint32_t* ids, float* sims, uint32_t* fb, int bound);
 // Re-score every entry of the screen's lists (rows lo..lo+n, parts x L
 // entries each, laid out [row][part][L]) with the check's exact key and fill
 // rep's pair count, pairs beyond the bound and max |screen key - exact key| / E

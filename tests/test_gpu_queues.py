@@ -111,6 +111,27 @@ def test_queued_knn(dev, m, n, d, kk, self_):
     assert dev.fallback_rows() - f0 >= m // 2
 
 
+@pytest.mark.parametrize("each,kk,queued", [
+    (24, 12, False), (25, 12, True),   # lists of 24
+    (33, 13, False), (40, 16, False), (41, 16, True),  # lists of 40
+])
+@pytest.mark.parametrize("n,d", [(600, 64), (9000, 33)])
+def test_near_ties_within_the_lists(dev, n, d, each, kk, queued):
+    """Near-ties that a list has room for beside the neighbours are settled from
+    it; a list of more goes to the exact scan."""
+    g = np.random.default_rng(n + each)
+    x = _crowds(n, d, 1, 9)
+    x[10:10 + each] = _crowds(each, d, each, 3)
+    q = (x[10] + np.float32(0.01) * g.standard_normal((300, d))).astype(np.float32)
+    f0 = dev.fallback_rows()
+    gi, gs = dev.topk(q, x, d, kk, False)
+    f1 = dev.fallback_rows() - f0
+    oi, os_ = O.knn(q, x, d, kk, False)
+    assert np.array_equal(gi, oi)
+    assert gs.tobytes() == os_.tobytes()
+    assert f1 == (len(q) if queued else 0)
+
+
 def test_queued_knn_few(dev):
     """A few queued queries among many: the parts' lists and their ranking, call
     after call (the tickets are left at zero)."""
