@@ -343,11 +343,10 @@ __global__ __launch_bounds__(256) void k_verify(
 // Top-1 behind the one-pass screen when d % 4 != 0: lists with lengths (their
 // first entry the best), read where they lie. Block: AR rows, a thread each to
 // decide, then a thread per (row, candidate) pair to run its chain. Bound by the
-// chains' latency, so by the pairs a CU holds at once: 64 rows make about two
-// waves of them, where k_verify's 16 rows with every list in LDS made half a one
-// (65,536 x 301 against 300 centroids: 220 us; 157 here).
-constexpr int AR = 64;
-
+// chains' latency, so by the pairs a CU holds at once (k_verify's 16 rows with
+// every list in LDS, six blocks a CU: 65,536 x 301 against 300 centroids 220 us;
+// 157 here with 64 rows, 154 with 32).
+template <int AR>
 __global__ __launch_bounds__(256) void k_check1_any(
     const float* __restrict__ x, size_t nx, int d, const uint32_t* __restrict__ ids, size_t lo,
     int nrows, const float* __restrict__ cents, const float* __restrict__ cnorm, int ip,
@@ -360,7 +359,7 @@ __global__ __launch_bounds__(256) void k_check1_any(
   __shared__ uint16_t prow[PMAX];
   __shared__ uint32_t rowid[AR];
   __shared__ int off[AR + 1];
-  static_assert(AR == 64, "the offsets are one wave's scan");
+  static_assert(AR <= 64, "the offsets are one wave's scan");
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * AR;
   if (tid < AR) {
@@ -410,7 +409,7 @@ __global__ __launch_bounds__(256) void k_check1_any(
     n = settled ? n + (ip ? 0 : 1) : 0;
     int inc = n;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+    for (int o = 1; o < AR; o <<= 1) {
       const int t = __shfl_up(inc, o, 64);
       if (tid >= o) inc += t;
     }
@@ -1118,8 +1117,13 @@ void launch_verify1(emh_ctx* c, const float* x, size_t nx, size_t d, const uint3
                        tally ? tally->stride : 0, ncand);
   } else {
     if (L == L5) {
-      hipLaunchKernelGGL(k_check1_any, dim3((unsigned)((n + AR - 1) / AR)), dim3(256), 0, c->stream,
-                         x, nx, (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts,
+      // 16 rows a block while a CU holds all its blocks at once (8 of 4 waves): a
+      // row's few chains wait for loads, and more, shorter waves overlap them. 16,384
+      // x 301 by 300: 67 us against 75; 32,768 x 567 by 1,155: 163 against 170;
+      // 40,000: 267 against 188.
+      const int ar = n <= (size_t)128 * std::max(c->cus, 1) ? 16 : 32;
+      auto kern = ar == 16 ? k_check1_any<16> : k_check1_any<32>;
+      hipLaunchKernelGGL(kern, dim3((unsigned)((n + ar - 1) / ar)), dim3(256), 0, c->stream, x, nx, (int)d, ids, lo, (int)n, cents, cnorm, ip ? 1 : 0, cand, parts,
                          xnorm, labels, scores, fb, c->small, ncand);
     } else {
       auto kern = L == L1F ? k_verify<L1F, R1, false, false> : k_verify<L1, R1, false, false>;

@@ -334,3 +334,15 @@ def test_top1_few_rows_many_centroids(dev, metric, n, d, k):
     x, c = _rows(n, d, n), _rows(k, d, k)
     x[: n // 2] = c[np.arange(n // 2) % k] + np.float32(0.3) * x[: n // 2]
     _top1(dev, x, c, metric)
+
+
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+@pytest.mark.parametrize("n,d,k", [(16401, 35, 600), (32768, 33, 80), (32769, 34, 80)])
+def test_top1_odd_width_check_blocks(dev, metric, n, d, k):
+    """Odd widths: the check's blocks of 16 rows, up to the most that take them,
+    and of 32, each with a remainder; near-ties and rows of NaN and zeros."""
+    x, c = _rows(n, d, n), _rows(k, d, k)
+    c[1:12] = c[0] * (1 + np.float32(1e-6) * np.arange(11, dtype=np.float32)[:, None])
+    x[::3] = c[0] + np.float32(0.05) * x[::3]
+    x[n - 1], x[n - 2, 1] = 0.0, np.nan
+    _top1(dev, x, c, metric)
